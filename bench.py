@@ -405,8 +405,8 @@ def run_conv(name, mode, policy, args, traffic_table):
         "bwd_weights": esize * (x.numel() + gr.numel() + dw.numel()),
     }
     per_pass = dict(zip(PASSES, t.kernel_ms))
-    compute = {p: "f32" if (dt == "f32" or policy == "fp32" or (policy == "backward32" and p != "fwd")) else "f16"
-               for p in PASSES}
+    # (fp32 arithmetic on fp16 tensors runs on the fp16 matrix instructions, whose products of fp16 values are exact)
+    compute = {p: "f32" if "_f32mfma" in names[p] else dt for p in PASSES}
     roofs = {p: roofline_of(p, names[p], flops_pass, bytes_pass[p], per_pass[p], compute[p],
                             traffic_table.get((name, names[p]))) for p in PASSES}
     dominant = max(per_pass, key=per_pass.get)

@@ -74,9 +74,11 @@ enum phx_product_mode { PHX_PRODUCT_16 = 16, PHX_PRODUCT_8 = 8 };
 
 /* UPSTRIDE_CONV_FP16_POLICY (src/backend/backend.cc:35-42, src/backend/backend.hpp:60-66).
  * Applies to PHX_F16 tensors only; accumulation is fp32 under every policy.
- *   FULL32      fp32 MFMA in every pass (operands widened while staged)
- *   BACKWARD32  fp16 MFMA forward, fp32 MFMA backward
- *   FULL16      fp16 MFMA in every pass */
+ *   FULL32      fp32 arithmetic in every pass
+ *   BACKWARD32  fp16 arithmetic forward, fp32 arithmetic backward
+ *   FULL16      fp16 arithmetic in every pass
+ * fp32 arithmetic on fp16 tensors runs on the fp16 matrix instructions too, in 16-product form: products of fp16 values
+ * are exact in fp32 and are summed there.  fp16 arithmetic may also round sums of components to fp16 (the 8-product form). */
 enum phx_fp16_policy { PHX_FP16_FULL32 = 0, PHX_FP16_BACKWARD32 = 1, PHX_FP16_FULL16 = 2 };
 
 enum phx_pass { PHX_PASS_FWD = 0, PHX_PASS_BWD_DATA = 1, PHX_PASS_BWD_WEIGHTS = 2 };

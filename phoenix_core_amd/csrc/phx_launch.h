@@ -27,8 +27,6 @@ bool tuning_thin_notile();  // PHX_TUNE_THIN_NOTILE
 
 // which instantiation of the forward / input-gradient kernel to run
 struct FwdVariant {
-    bool half_storage;  // tensors are fp16 (else fp32)
-    bool f16_mfma;      // fp16 matrix-core arithmetic (else fp32)
     int mode, map;      // 16 / 8, MAP_FWD / MAP_DGRAD
     int WCO, NTW, CK, P2LOG;
     bool lds_filters;   // fp16 MFMA only: filters staged through LDS (qconv_fwd_f16_lds_kernel)
@@ -64,7 +62,6 @@ enum PackKind { PACK_F32 = 0, PACK_F16 = 1, PACK_F16_LDS = 2, PACK_PWX = 3 };
 struct PackJob {
     PackArgs a;
     int kind;                    // PackKind
-    int half_storage;            // PACK_F32: the filter is stored as fp16
     int mode, map;               // 16 / 8, MAP_FWD / MAP_DGRAD
     int WCO, ngroups, pw;        // PACK_F16_LDS (PackLdsArgs), PACK_PWX (WCO)
     int nsteps;                  // PACK_PWX

@@ -3,11 +3,11 @@
 
 namespace phx {
 
-template <typename TS, int MODE>
+template <int MODE>
 static int launch_variant(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
 #define PHX_CASE(WCO_, NTW_, CK_, P2_, VS_)                                                                   \
     if (v.WCO == WCO_ && v.NTW == NTW_ && v.CK == CK_ && v.P2LOG == P2_ && v.vstage == VS_) {                 \
-        hipLaunchKernelGGL((qconv_fwd_f32_kernel<TS, MODE, WCO_, NTW_, CK_, P2_, VS_>), dim3(v.wgs, grid_rows(a.groups)),          \
+        hipLaunchKernelGGL((qconv_fwd_f32_kernel<float, MODE, WCO_, NTW_, CK_, P2_, VS_>), dim3(v.wgs, grid_rows(a.groups)),          \
                            dim3(WG_THREADS), v.lds_bytes, st, a);                                             \
         return 0;                                                                                             \
     }
@@ -24,29 +24,19 @@ static int launch_variant(const FwdVariant& v, const ConvArgs& a, hipStream_t st
     return -1;
 }
 
-template <typename TS>
-static int launch_ts(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
-    // one kernel for both passes: the input gradient differs only in how its filters are packed
-    if (v.mode == 16) return launch_variant<TS, 16>(v, a, st);
-    return launch_variant<TS, 8>(v, a, st);
-}
-
+// (fp32 tensors only: fp16 tensors run on the fp16 matrix instructions under every policy)
 int launch_fwd_f32(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
-    return v.half_storage ? launch_ts<_Float16>(v, a, st) : launch_ts<float>(v, a, st);
-}
-
-template <typename TS>
-static int pack_ts(const FwdVariant& v, const PackArgs& a, int blocks, hipStream_t st) {
-    const dim3 g(blocks, grid_rows(a.groups)), b(WG_THREADS);
-    if (v.mode == 16 && v.map == MAP_FWD) hipLaunchKernelGGL((pack_filters_f32_kernel<TS, 16, MAP_FWD>), g, b, 0, st, a);
-    else if (v.mode == 16) hipLaunchKernelGGL((pack_filters_f32_kernel<TS, 16, MAP_DGRAD>), g, b, 0, st, a);
-    else if (v.map == MAP_FWD) hipLaunchKernelGGL((pack_filters_f32_kernel<TS, 8, MAP_FWD>), g, b, 0, st, a);
-    else hipLaunchKernelGGL((pack_filters_f32_kernel<TS, 8, MAP_DGRAD>), g, b, 0, st, a);
-    return 0;
+    // one kernel for both passes: the input gradient differs only in how its filters are packed
+    return v.mode == 16 ? launch_variant<16>(v, a, st) : launch_variant<8>(v, a, st);
 }
 
 int launch_pack_filters(const FwdVariant& v, const PackArgs& a, int blocks, hipStream_t st) {
-    return v.half_storage ? pack_ts<_Float16>(v, a, blocks, st) : pack_ts<float>(v, a, blocks, st);
+    const dim3 g(blocks, grid_rows(a.groups)), b(WG_THREADS);
+    if (v.mode == 16 && v.map == MAP_FWD) hipLaunchKernelGGL((pack_filters_f32_kernel<float, 16, MAP_FWD>), g, b, 0, st, a);
+    else if (v.mode == 16) hipLaunchKernelGGL((pack_filters_f32_kernel<float, 16, MAP_DGRAD>), g, b, 0, st, a);
+    else if (v.map == MAP_FWD) hipLaunchKernelGGL((pack_filters_f32_kernel<float, 8, MAP_FWD>), g, b, 0, st, a);
+    else hipLaunchKernelGGL((pack_filters_f32_kernel<float, 8, MAP_DGRAD>), g, b, 0, st, a);
+    return 0;
 }
 
 }  // namespace phx

@@ -8,8 +8,7 @@ namespace phx {
 template <int MODE, int MAP>
 static __device__ __forceinline__ void pack_job_as(const PackJob& j, long first, long stride) {
     if (j.kind == PACK_F32) {
-        if (j.half_storage) pack_filters_f32_body<_Float16, MODE, MAP>(j.a, first, stride);
-        else pack_filters_f32_body<float, MODE, MAP>(j.a, first, stride);
+        pack_filters_f32_body<float, MODE, MAP>(j.a, first, stride);
     } else if (j.kind == PACK_F16) {
         pack_filters_f16_body<MODE, MAP>(j.a, first, stride);
     } else if (j.kind == PACK_F16_LDS) {

@@ -679,13 +679,32 @@ static bool plan_forward(const Corr& c, int mode, bool f16mfma, FwdPlan& best, b
     return true;
 }
 
-// fp16 tensors use fp16 matrix-core arithmetic where UPSTRIDE_CONV_FP16_POLICY allows it for the
-// pass (forward: full16 or backward32; backward: full16 only), fp32 arithmetic otherwise
-static bool use_f16_mfma(const Problem& p, int pass) {
+// UPSTRIDE_CONV_FP16_POLICY allows fp16 arithmetic for the pass (forward: full16 or backward32; backward: full16
+// only): operands may be rounded to fp16 on their way into the products, as the factorized form rounds its lanes.
+static bool fp16_arithmetic(const Problem& p, int pass) {
     if (p.dtype != PHX_F16) return false;
     if (pass == PHX_PASS_FWD) return p.policy == PHX_FP16_FULL16 || p.policy == PHX_FP16_BACKWARD32;
     return p.policy == PHX_FP16_FULL16;
 }
+
+// Every pass on fp16 tensors runs on the fp16 matrix instructions, fp32 arithmetic included: the product of two fp16
+// values has 22 significant bits and is exact in fp32, subnormal operands are kept, and the sums are fp32 sums, so the
+// 16-product form, whose operands are the tensors' own values and their negatives, IS fp32 arithmetic.  (It rounds
+// less often than the fp32 matrix instructions on widened operands: a 32x32x16 instruction adds sixteen products
+// between two roundings, a 32x32x2 one two.  Against fp64, N(0,1) operands, 4608 products per sum: 2-norm error 4.3e-7 on
+// fp16 instructions, 1.3e-6 on fp32 ones; operands in the subnormal range 5.9e-7 and 6.5e-7.)  At 16 times the
+// instruction rate: backward32, N=128, 3x3 256 -> 256 at 14x14, input gradient 2.65 -> 0.46 ms, filter gradient 3.22 -> 0.42.
+static bool use_f16_mfma(const Problem& p) { return p.dtype == PHX_F16; }
+
+// The product formulation a pass may run in: the factorized form sums and differences components before it multiplies,
+// which fp16 rounds, so fp32 arithmetic on the fp16 instructions is always the 16-product form.
+static int pass_mode(const Problem& p, int pass) {
+    return use_f16_mfma(p) && !fp16_arithmetic(p, pass) ? PHX_PRODUCT_16 : p.mode;
+}
+
+// Kernel labels tell the two apart: f16mfma = fp16 arithmetic allowed, exact16mfma = fp32 arithmetic on fp16 instructions.
+static const char* f16_tag(const Problem& p, int pass) { return fp16_arithmetic(p, pass) ? "f16" : "exact16"; }
+static int map_pass(int map) { return map == MAP_FWD ? PHX_PASS_FWD : PHX_PASS_BWD_DATA; }
 
 // A pointwise fp16 correlation on one long row per image has a single tap, which would leave the LDS
 // kernels one MFMA block per barrier.  It is run instead as a column of PW_TAPS virtual taps: window
@@ -871,8 +890,8 @@ static int run_pwx(const Problem& p, const Corr& c, const FwdPlan& pl, int map, 
         }
         if (prc != 0) return PHX_ERR_NOT_SUPPORTED;
         PHX_HIP(hipGetLastError());
-        snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_f16mfmapwr_p16_f16_wco%d_k%d_wgs%d_sub%d%s", g_name_prefix,
-                 map == MAP_FWD ? "fwd" : "dgrad", pl.pwx, pl.pwx_steps, wgs, a.items - a.items_whole, a.addend ? "_add" : "");
+        snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_%smfmapwr_p16_f16_wco%d_k%d_wgs%d_sub%d%s", g_name_prefix,
+                 map == MAP_FWD ? "fwd" : "dgrad", f16_tag(p, map_pass(map)), pl.pwx, pl.pwx_steps, wgs, a.items - a.items_whole, a.addend ? "_add" : "");
         label_groups(gb.n);
         g_last_kernel = g_name_buf;
         say(p, map == MAP_FWD ? "forward" : "input gradient");
@@ -897,8 +916,8 @@ static int run_pwx(const Problem& p, const Corr& c, const FwdPlan& pl, int map, 
     }
     if (rc != 0) return PHX_ERR_NOT_SUPPORTED;
     PHX_HIP(hipGetLastError());
-    snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_f16mfmapwx_p16_f16_wco%d_px%d_k%d_wgs%d_half%d%s", g_name_prefix,
-             map == MAP_FWD ? "fwd" : "dgrad", pl.pwx, 64 * (4 / pl.pwx), pl.pwx_steps, blocks, a.items - a.items_whole,
+    snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_%smfmapwx_p16_f16_wco%d_px%d_k%d_wgs%d_half%d%s", g_name_prefix,
+             map == MAP_FWD ? "fwd" : "dgrad", f16_tag(p, map_pass(map)), pl.pwx, 64 * (4 / pl.pwx), pl.pwx_steps, blocks, a.items - a.items_whole,
              a.addend ? "_add" : "");
     label_groups(gb.n);
     g_last_kernel = g_name_buf;
@@ -925,7 +944,7 @@ static int pwx_wco_nhwc(int cin, int cout) {
 
 static bool nhwc_native(const Problem& p, int pass) {
     return p.nhwc && (pass == PHX_PASS_FWD || pass == PHX_PASS_BWD_DATA) && is_pointwise_unit(p) && !is_empty(p) &&
-           use_f16_mfma(p, pass) && !p.real_input && p.groups == 1 && p.ci % 8 == 0 && p.co % 8 == 0 &&
+           use_f16_mfma(p) && !p.real_input && p.groups == 1 && p.ci % 8 == 0 && p.co % 8 == 0 &&
            (long)p.n * p.h * p.w < (1L << 30) && !tune().nopwx;
 }
 
@@ -1017,8 +1036,8 @@ static int run_pwx_nhwc(const Problem& p, int map, hipStream_t st, const void* i
         PHX_HIP(hipGetLastError());
         if (add) g_addend.fused = true;
     }
-    snprintf(g_name_buf, sizeof(g_name_buf), "qconv_%s_f16mfmapwxcl_p16_f16_wco%d_px%d_k%d_wgs%d", map == MAP_FWD ? "fwd" : "dgrad",
-             wco, 64 * (4 / wco), nsteps, blocks);
+    snprintf(g_name_buf, sizeof(g_name_buf), "qconv_%s_%s_p16_f16_wco%d_px%d_k%d_wgs%d", map == MAP_FWD ? "fwd" : "dgrad",
+             fp16_arithmetic(p, map_pass(map)) ? "f16mfmapwxcl" : "exact16mfmapwx_cl", wco, 64 * (4 / wco), nsteps, blocks);
     if (Z) snprintf(g_name_buf + strlen(g_name_buf), sizeof(g_name_buf) - strlen(g_name_buf), "_kslices%d", Z);
     g_last_kernel = g_name_buf;
     say(p, map == MAP_FWD ? "forward (channels-last)" : "input gradient (channels-last)");
@@ -1027,11 +1046,11 @@ static int run_pwx_nhwc(const Problem& p, int map, hipStream_t st, const void* i
 
 static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st, const void* in, const void* w,
                     const void* bias, void* out, void* ws, size_t ws_bytes) {
-    const bool f16 = use_f16_mfma(p, map == MAP_FWD ? PHX_PASS_FWD : PHX_PASS_BWD_DATA);
+    const bool f16 = use_f16_mfma(p);
     int pw = 0;
     Corr c;
     FwdPlan pl;
-    if (!plan_corr(creal, p.mode, f16, c, pl, pw)) return PHX_ERR_NOT_SUPPORTED;
+    if (!plan_corr(creal, pass_mode(p, map_pass(map)), f16, c, pl, pw)) return PHX_ERR_NOT_SUPPORTED;
     if (pl.pwx) return run_pwx(p, creal, pl, map, st, in, w, bias, out, ws, ws_bytes);
     const GroupBatch gb = g_batch;
     const size_t image = align_up(pl.wpk_bytes, 256);  // (group after group where one launch runs them all)
@@ -1040,7 +1059,7 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     ws = slot.dst;
 
     FwdVariant v;
-    v.half_storage = p.dtype == PHX_F16; v.f16_mfma = f16; v.mode = pl.kmode; v.map = map;
+    v.mode = pl.kmode; v.map = map;
     v.WCO = pl.WCO; v.NTW = pl.NTW; v.CK = pl.CK; v.P2LOG = pl.P2LOG; v.wgs = pl.wgs; v.lds_bytes = pl.lds_bytes;
     v.lds_filters = pl.lds_filters; v.ngroups = pl.ngroups; v.pairs = pl.pairs; v.chunks = pl.chunks; v.pw = pw; v.vstage = pl.vstage;
 
@@ -1092,7 +1111,7 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
             j.a.w = at_bytes(pa.w, g * gb.w);
             j.a.out = at_bytes(pa.out, g * image);
             j.kind = !f16 ? PACK_F32 : pl.lds_filters ? PACK_F16_LDS : PACK_F16;
-            j.half_storage = v.half_storage; j.mode = pl.kmode; j.map = map; j.WCO = pl.WCO; j.ngroups = pl.ngroups; j.pw = pw;
+            j.mode = pl.kmode; j.map = map; j.WCO = pl.WCO; j.ngroups = pl.ngroups; j.pw = pw;
             if (const int rrc = record_pack_job(j, pack_items)) return rrc;
         }
     }
@@ -1104,7 +1123,7 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     if (rc != 0) return PHX_ERR_NOT_SUPPORTED;
     PHX_HIP(hipGetLastError());
     snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_%smfma%s%s_p%d_%s_wco%d_ntw%d_ck%d_%s%dx%dx%d", g_name_prefix,
-             map == MAP_FWD ? "fwd" : "dgrad", f16 ? "f16" : "f32", pl.lds_filters ? (pw ? "ldspw" : pl.chunks ? "ldsc" : "lds") : "",
+             map == MAP_FWD ? "fwd" : "dgrad", f16 ? f16_tag(p, map_pass(map)) : "f32", pl.lds_filters ? (pw ? "ldspw" : pl.chunks ? "ldsc" : "lds") : "",
              cl ? "cl" : "", pl.kmode, p.dtype == PHX_F32 ? "f32" : "f16", pl.WCO, pl.NTW, pl.CK, pl.tall ? "flat" : "tile", pl.NB, pl.TH, pl.TW);
     label_groups(gb.n);
     g_last_kernel = g_name_buf;
@@ -1246,7 +1265,8 @@ static bool plan_wgrad_f32(const Problem& p, WgPlan& best) {
 // speed" (src/backend/backend.hpp:36-66), so the 8-product mode runs this pass on the 16-product kernel;
 // PHX_TUNE_WG8 keeps the factorized kernel (tests exercise it).
 static int wgrad_f16_formulation(const Problem& p) {
-    return (p.mode == 8 && !tune().wg8) ? 16 : p.mode;
+    const int mode = pass_mode(p, PHX_PASS_BWD_WEIGHTS);
+    return (mode == 8 && !tune().wg8) ? 16 : mode;
 }
 
 // Real-valued input with few channels (the first layer of a network on images): one matrix product holds the whole
@@ -1330,7 +1350,7 @@ static bool plan_wgrad_f16(const Problem& p, WgPlan& best) {
 static bool wgrad_on_f16_mfma(const Problem& p) {
     // the kernel addresses one component with 32-bit element offsets
     const long lim = (1L << 31) - 64;
-    return use_f16_mfma(p, PHX_PASS_BWD_WEIGHTS) && (p.sw == 1 || p.sw == 2) && (long)p.n * p.ci_mem * p.h * p.w < lim &&
+    return use_f16_mfma(p) && (p.sw == 1 || p.sw == 2) && (long)p.n * p.ci_mem * p.h * p.w < lim &&
            (long)p.n * p.co_mem * p.ho * p.wo < lim;
 }
 
@@ -1338,7 +1358,7 @@ static bool plan_wgrad(const Problem& p, bool f16mfma, WgPlan& best) {
     struct Entry { WgPlan pl; bool ok; };
     static PlanMemo<Entry> memo;
     // everything the two planners read
-    const PlanKey key{{p.mode, p.n, p.ci, p.co, p.h, p.w, p.kh, p.kw, p.sh, p.sw, p.dh, p.dw, p.pt, p.pl, p.pb, p.pr,
+    const PlanKey key{{f16mfma ? pass_mode(p, PHX_PASS_BWD_WEIGHTS) : p.mode, p.n, p.ci, p.co, p.h, p.w, p.kh, p.kw, p.sh, p.sw, p.dh, p.dw, p.pt, p.pl, p.pb, p.pr,
                        p.ho, p.wo, (int)f16mfma, (int)p.real_input, (int)p.dtype, p.groups, (int)p.nhwc}};
     std::lock_guard<std::mutex> lock(g_plan_mutex);
     const Entry& hit = memo.get(key, [&] {
@@ -1380,7 +1400,8 @@ static int run_wgrad(const Problem& p, hipStream_t st, const void* x, const void
         r.Z = pl.Z; r.Co = p.co; r.Ci = p.ci; r.Kh = p.kh; r.Kw = p.kw; r.CoP = pl.CoP; r.CiP = pl.CiP;
         launch_reduce_wgrad(true, r, st);
         PHX_HIP(hipGetLastError());
-        snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_wgrad_f16mfma_realx_f16_cols%d_rows%d_z%d", g_name_prefix, ra.ncol,
+        snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_wgrad_%s_f16_cols%d_rows%d_z%d", g_name_prefix,
+                 fp16_arithmetic(p, PHX_PASS_BWD_WEIGHTS) ? "f16mfma_realx" : "exact16mfma_real_x", ra.ncol,
                  pl.rows_per_wg, pl.Z);
         say(p, "filter gradient (real-valued input)");
         return PHX_OK;
@@ -1424,7 +1445,8 @@ static int run_wgrad(const Problem& p, hipStream_t st, const void* x, const void
     launch_reduce_wgrad(half_storage, r, st);
     PHX_HIP(hipGetLastError());
     if (f16)
-        snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_wgrad_f16mfma%s_p%d_f16_ch%dx%d_taps%d_sw%d%s_z%d", g_name_prefix, cl ? "cl" : "",
+        snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_wgrad_%smfma%s_p%d_f16_ch%dx%d_taps%d_sw%d%s_z%d", g_name_prefix,
+                 f16_tag(p, PHX_PASS_BWD_WEIGHTS), cl ? "cl" : "",
                  pl.kmode, 32 * pl.MT, 32 * pl.NT, pl.TPW, pl.SW, pl.flat ? "_flat" : "", pl.Z);
     else
         snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_wgrad_f32mfma%s_p%d_%s_tile%dx%dx%d_z%d", g_name_prefix, pl.vec ? "v" : "", pl.kmode,
@@ -1485,7 +1507,7 @@ static bool dgrad_by_phases(const Problem& p) {
     // 28x28 2174 / 789; but 64 at 28x28 83 / 103, 128 at 14x14 78 / 153, 512 at 7x7 346 / 463)
     // In fp32 arithmetic the phases win at every size measured (N=64, 3x3: 16 channels at 56x56 359 / 125 us, 128 at
     // 14x14 622 / 353, 512 at 7x7 2967 / 1281, 256 at 28x28 10325 / 1809).
-    if (!use_f16_mfma(p, PHX_PASS_BWD_DATA)) return true;
+    if (!use_f16_mfma(p)) return true;
     const double flops = 32.0 * p.n * p.ci * p.co * p.ho * p.wo * p.kh * p.kw;
     return flops >= 40e9 && (long)p.h * p.w >= 196;
 }
@@ -1519,12 +1541,12 @@ static size_t workspace_plain(const Problem& p, int pass) {
                 const PhaseAxis ah = phase_axis(a, p.h, p.kh, p.dh, p.sh, p.pt), aw = phase_axis(b, p.w, p.kw, p.dw, p.sw, p.pl);
                 if (!ah.taps || !aw.taps || !ah.size || !aw.size) continue;
                 bufs += align_up((size_t)4 * p.n * p.ci * ah.size * aw.size * esize, 256);
-                if (!plan_corr(phase_corr(p, ah, aw), p.mode, use_f16_mfma(p, pass), c, pl, pw)) return 0;
+                if (!plan_corr(phase_corr(p, ah, aw), pass_mode(p, pass), use_f16_mfma(p), c, pl, pw)) return 0;
                 wpk = std::max(wpk, align_up(pl.wpk_bytes, 256));
             }
         return bufs + wpk;
     }
-    return plan_corr((pass == PHX_PASS_FWD) ? corr_forward(p) : corr_dgrad(p), p.mode, use_f16_mfma(p, pass), c, pl, pw)
+    return plan_corr((pass == PHX_PASS_FWD) ? corr_forward(p) : corr_dgrad(p), pass_mode(p, pass), use_f16_mfma(p), c, pl, pw)
                ? align_up(pl.wpk_bytes, 256)
                : 0;
 }
@@ -1620,7 +1642,7 @@ static bool patch_view(const Problem& p, int pass, PatchView& v) {
     // four phases against one pointwise pass and a scatter: 99 / 71, 102 / 53) and the filter gradient in fp32 arithmetic
     // (267 / 148) do not.  From 3x3 on every pass gains (4x4 stride 4, 32 -> 64 at 56x56: 45 / 141 / 258 -> 97 / 57 / 93).
     if (p.kh * p.kw < 9 && !tune().patchall &&
-        (pass == PHX_PASS_FWD || (pass == PHX_PASS_BWD_WEIGHTS && use_f16_mfma(p, PHX_PASS_BWD_WEIGHTS) && wgrad_on_f16_mfma(p))))
+        (pass == PHX_PASS_FWD || (pass == PHX_PASS_BWD_WEIGHTS && fp16_arithmetic(p, PHX_PASS_BWD_WEIGHTS) && wgrad_on_f16_mfma(p))))
         return false;
     const FilterStrides& f = p.fs;
     long si = 0;
@@ -1734,7 +1756,7 @@ static bool wgrad_by_classes(const Problem& p) {
     S2dView v;
     if (s2d_view(p, v)) return false;
     if (tune().wgphase >= 0) return tune().wgphase != 0;
-    if (use_f16_mfma(p, PHX_PASS_BWD_WEIGHTS) && !wgrad_on_f16_mfma(p)) return true;
+    if (fp16_arithmetic(p, PHX_PASS_BWD_WEIGHTS) && !wgrad_on_f16_mfma(p)) return true;
     const double flops = 32.0 * p.n * p.ci * p.co * p.ho * p.wo * p.kh * p.kw;
     return flops >= 200e9;
 }
@@ -1809,8 +1831,8 @@ static int slices_rule(const Problem& p, int pass, const Corr& creal) {
     Corr c;
     FwdPlan pl;
     int pw = 0;
-    const bool f16 = use_f16_mfma(p, pass);
-    if (!plan_corr(creal, p.mode, f16, c, pl, pw)) return 0;
+    const bool f16 = use_f16_mfma(p);
+    if (!plan_corr(creal, pass_mode(p, pass), f16, c, pl, pw)) return 0;
     const int red = creal.Cin;
     const auto fits = [&](int z) { return red % z == 0 && (red / z) % 16 == 0 && red / z >= 32; };
     if (tune().kslices > 1) return fits(tune().kslices) ? tune().kslices : 0;
@@ -1947,7 +1969,7 @@ static size_t workspace_for(const Problem& p, int pass) {
                 Corr c;
                 FwdPlan pl;
                 int pw = 0;
-                if (!plan_corr(phase_corr(sc.q, ah, aw), p.mode, use_f16_mfma(p, pass), c, pl, pw)) return 0;
+                if (!plan_corr(phase_corr(sc.q, ah, aw), pass_mode(p, pass), use_f16_mfma(p), c, pl, pw)) return 0;
                 most = std::max(most, sc.partial_bytes + (size_t)Z * align_up(pl.wpk_bytes, 256));
             }
         return bufs + most;
@@ -2407,7 +2429,7 @@ struct ChannelsLast {
 namespace phx {
 static bool nhwc_window_native(const Problem& p, int pass) {
     if (!p.nhwc || (pass != PHX_PASS_FWD && pass != PHX_PASS_BWD_DATA) || is_empty(p) || is_pointwise_unit(p)) return false;
-    if (p.real_input || p.groups != 1 || tune().nowincl || !use_f16_mfma(p, pass)) return false;
+    if (p.real_input || p.groups != 1 || tune().nowincl || !use_f16_mfma(p)) return false;
     // (a strided forward pass reads its staged window with the stride, whatever the memory order; a strided input
     // gradient runs by phases or on zero-inserted windows, neither of which is staged in chunks)
     if ((p.sh != 1 || p.sw != 1) && pass != PHX_PASS_FWD) return false;
@@ -2419,7 +2441,7 @@ static bool nhwc_window_native(const Problem& p, int pass) {
     Corr c;
     FwdPlan pl;
     int pw = 0;
-    if (!plan_corr(pass == PHX_PASS_FWD ? corr_forward(p) : corr_dgrad(p), p.mode, true, c, pl, pw)) return false;
+    if (!plan_corr(pass == PHX_PASS_FWD ? corr_forward(p) : corr_dgrad(p), pass_mode(p, pass), true, c, pl, pw)) return false;
     if (!(pl.lds_filters && pl.chunks && !pl.pwx && pw == 0)) return false;
     // a small batch on a deep layer gains more from reduction slices (corr_slices), which run on channels-first copies:
     // the copies of so small a problem cost next to nothing; so do dilated windows from their dilation phases
@@ -2488,7 +2510,7 @@ static bool thin_groups(const Problem& p, int pass) {
     // matrix-core rate to lose against, and their filter gradient works on 64 x 64 channel tiles: measured like above,
     // 8 x 8 channels per group 159 / 149 / 206 us here against 194 / 193 / 742 merged, 16 x 16 260 / 254 / 346 against
     // 192 / 193 / 745 -- up to 64 pairs per group run here, the filter gradient up to 256.
-    if (use_f16_mfma(p, pass)) return pairs <= tune().thin_max;
+    if (use_f16_mfma(p)) return pairs <= tune().thin_max;
     return pairs <= (long)tune().thin_max32 * (pass == PHX_PASS_BWD_WEIGHTS ? 4 : 1);
 }
 
@@ -2599,7 +2621,7 @@ static size_t groups_workspace(const Problem& p, int pass) {
 static int merged_groups(const Problem& p, int pass) {
     if (p.groups <= 1 || is_empty(p) || p.real_input || tune().nomerge) return 0;
     // (the filter gradient in fp32 arithmetic works on 64 x 64 channel tiles)
-    const int tile = (pass == PHX_PASS_BWD_WEIGHTS && !wgrad_on_f16_mfma(flatten_pointwise(p))) ? 64 : 32;
+    const int tile = (pass == PHX_PASS_BWD_WEIGHTS && !(fp16_arithmetic(p, pass) && wgrad_on_f16_mfma(flatten_pointwise(p)))) ? 64 : 32;
     const int most = std::min(p.groups, tile / std::max(p.ci, p.co));  // groups that fit a tile
     if (most < 2) return 0;
     int divisor = 1;
