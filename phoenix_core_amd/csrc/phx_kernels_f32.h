@@ -30,6 +30,8 @@ struct ConvArgs {
     int tiles_n, tiles_h, tiles_w, co_tiles;
     int nchunks;        // ceil(Cin / CK) for the kernel's chunk size CK
     int vec;            // output pixels a lane stores at once (4, 2 or 1): divides TW and Wout
+    int even;           // lanes kernel: the window starts at an even column (the staged row holds one column more, or the
+                        // first one behind it, which is zero like the next row's first)
     int nhwc;           // the output is channels-last, out[4][N][Hout][Wout][CoutS] (fp16 chunk-staging kernel only)
     int groups;         // grid rows: the groups of a grouped convolution run by this one launch (1 otherwise)
     long g_in, g_w, g_bias, g_out;  // bytes from one group's input / packed filters / bias / output to the next group's

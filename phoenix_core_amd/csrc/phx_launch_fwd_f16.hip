@@ -64,6 +64,7 @@ static int launch_lds16(const FwdVariant& v, const ConvArgs& a, hipStream_t st) 
 }
 
 int launch_fwd_f16(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
+    if (v.lanes) return launch_fwd_f16_lanes(v, a, st);
     if (v.lds_filters && v.mode == 8) return launch_fwd_f16_lds8(v, a, st);
     // real-valued input (one stored component), several filter groups per chunk: the variant without the absent products
     if (v.lds_filters && v.chunks && a.in.ncomp == 1 && !(v.ngroups == 1 && v.NTW == 1)) return launch_fwd_f16_lds16_real(v, a, st);
@@ -72,6 +73,7 @@ int launch_fwd_f16(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
 }
 
 int launch_pack_filters_f16(const FwdVariant& v, const PackArgs& a, int blocks, hipStream_t st) {
+    if (v.lanes) return launch_pack_filters_lanes(v.map, v.ngroups, a, blocks, st);
     const dim3 g(blocks, grid_rows(a.groups)), b(WG_THREADS);
     if (v.lds_filters) {
         PackLdsArgs la{a, v.WCO, v.ngroups, v.pw};

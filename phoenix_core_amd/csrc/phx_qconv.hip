@@ -29,6 +29,7 @@ namespace phx {
 struct Tuning {
     int tile_wco = 0, tile_ntw = 0;   // PHX_TUNE_TILE="wco,ntw"
     bool flat = false, noflat = false, nopw = false, pw8 = false, zi8 = false, wg8 = false, nos2d = false, noearly = false, norealx = false, nosub = false, oldplan = false;
+    bool nolanes = false;             // PHX_TUNE_NOLANES: factorized fp16 problems form their lanes in front of the products
     bool nopwx = false;               // PHX_TUNE_NOPWX: pointwise fp16 problems stay on the staged-window kernels
     bool nohalf = false;              // PHX_TUNE_NOHALF: the pointwise streaming kernel never cuts items in two
     bool nopwr = false;               // PHX_TUNE_NOPWR: pointwise fp16 problems with small filters stay on the streaming kernel
@@ -72,6 +73,7 @@ struct Tuning {
         nosub = getenv("PHX_TUNE_NOSUB") != nullptr;
         oldplan = getenv("PHX_TUNE_OLDPLAN") != nullptr;
         nopwx = getenv("PHX_TUNE_NOPWX") != nullptr;
+        nolanes = getenv("PHX_TUNE_NOLANES") != nullptr;
         nohalf = getenv("PHX_TUNE_NOHALF") != nullptr;
         nopwr = getenv("PHX_TUNE_NOPWR") != nullptr;
         pwrall = getenv("PHX_TUNE_PWRALL") != nullptr;
@@ -512,6 +514,7 @@ struct FwdPlan {
     int ngroups;             // tap groups per chunk in that case
     bool vstage;             // fp32 MFMA: window rows widened to a multiple of 4, staged as 4-position vectors
     bool pairs;              // fp16 MFMA: window rows widened to even columns, staged as position pairs
+    bool lanes;              // fp16 MFMA, 8-product: product lanes dealt over the waves (phx_kernels_lanes16.h)
     bool chunks;             // fp16 MFMA, filters in LDS: window rows widened to a multiple of 8, staged as chunks
     int NB, TH, TW, HTH, HTW, HP, HPp;
     int tiles_n, tiles_h, tiles_w, co_tiles, nchunks;
@@ -525,7 +528,7 @@ struct FwdPlan {
 
 constexpr int LDS_FLOATS_MAX = 16384;  // 64 KiB: two workgroups per CU
 
-static bool plan_forward(const Corr& c, int mode, bool f16mfma, FwdPlan& best, bool pointwise = false) {
+static bool plan_forward(const Corr& c, int mode, bool large, bool f16mfma, FwdPlan& best, bool pointwise = false) {
     double best_score = -1.0;
     // fp16 MFMA with filters in LDS: stage activations as aligned pairs when rows are even
     // filters through LDS: 16-product always, 8-product where the chunk staging applies
@@ -535,6 +538,11 @@ static bool plan_forward(const Corr& c, int mode, bool f16mfma, FwdPlan& best, b
     const bool chunks = ldsk && dense_window;
     const bool pairs = f16mfma && !chunks && (c.Win % 2 == 0) && dense_window;
     const bool vstage = !f16mfma && dense_window;
+    // product lanes dealt over the waves (phx_kernels_lanes16.h): three tap groups or more per chunk; that kernel addresses
+    // its input with 32-bit byte offsets and divides rows and columns in floating point
+    const bool lanes_ok = chunks && mode == 8 && !pointwise && cdiv(c.Kh * c.Kw, F16_TG) >= 3 && !large && !tune().nolanes &&
+                          std::max(c.Hin + c.Kh * c.dh, c.Wout) < (1 << 19);
+    best.lanes = false;
     best.pairs = pairs; best.chunks = chunks; best.vstage = vstage;
     const int wcos[3] = {1, 2, 4};
     // PHX_TUNE_TILE="wco,ntw" pins the workgroup shape (kernel tuning experiments)
@@ -570,14 +578,23 @@ static bool plan_forward(const Corr& c, int mode, bool f16mfma, FwdPlan& best, b
                     // The factorized LDS kernels hold one workgroup per CU, so their time is counted out: rounds of
                     // workgroups over the CUs (half by the whole rounds the last workgroup waits for, half by the
                     // work there is -- a last round that is partly empty still frees power and memory bandwidth) times
-                    // the tile's area over the shape's throughput (measured at 128 channels, 28x28, per unit of tile
-                    // area: two column tiles per wave 1.0 / 1.04 with two / one filter sub-tile, one column tile
-                    // 0.79 / 0.85).  A small problem then takes the small tile that fills the CUs (64 channels at
-                    // 14x14, N=64: 0.041 -> 0.032 ms per pass).
-                    const double rate = NTW == 2 ? (WCO == 2 ? 1.0 : 1.04) : (WCO == 2 ? 0.79 : 0.85);
+                    // a workgroup's time: clocks per step of 16 channels and one tap, and clocks for its start and
+                    // epilogue.  Measured at 128 channels, 28x28, N=128 (3x3, us a pass; lanes dealt over the waves /
+                    // formed in front of the products): two filter sub-tiles x 128 pixels 284 / 394, x 64 pixels
+                    // 435 / 505, one sub-tile x 256 pixels - / 435, x 128 pixels - / 472; and the phase stamps of the
+                    // two-sub-tile kernel.  A small problem takes the small tile that fills the CUs.  Rows of a tile
+                    // that are neither whole image rows nor multiples of eight pixels are stored in pieces.
+                    const bool dealt = lanes_ok && WCO == 2;
+                    // (the wide dealt kernel is held by the chip's power where it fills the chip: 5x5 on 256 channels at 28x28, N=4,
+                    // 112 workgroups: 122 us, its narrow form with 256 of them 134)
+                    const double busy = std::min(1.0, std::max(0.6, wgs / 256.0));
+                    const double step = dealt ? (NTW == 2 ? 780 * busy : 525) : NTW == 2 ? (WCO == 2 ? 1290 : 1480) : (WCO == 2 ? 750 : 690);
+                    double edges = dealt ? (NTW == 2 ? 26000 : 20000) : NTW == 2 ? 18000 : 17000;
+                    if (dealt && TW != c.Wout && TW % 8) edges += NTW == 2 ? 10000 : 5000;
+                    const double steps = (double)cdiv(c.Cin, F16_CK) * cdiv(c.Kh * c.Kw, F16_TG) * F16_TG;
                     const double cus = 256.0;
-                    const double rounds = 0.5 * std::ceil(wgs / cus) + 0.5 * (wgs / cus);
-                    score = 1e6 * rate / (rounds * BN * 32.0 * WCO) * (0.9 + 0.1 * halo);
+                    const double rounds = std::max(1.0, 0.5 * std::ceil(wgs / cus) + 0.5 * (wgs / cus));
+                    score = 1e12 / (rounds * (steps * step + edges)) * (0.9 + 0.1 * halo);
                 } else if (ldsk && !pointwise && !tune().oldplan) {
                     // the 16-product LDS kernels by the same count (one column tile per wave: two workgroups share a
                     // CU at about half speed each, so the rounds are still rounds over the CUs)
@@ -660,6 +677,11 @@ static bool plan_forward(const Corr& c, int mode, bool f16mfma, FwdPlan& best, b
             const size_t wimg = (size_t)F16_TG * best.WCO * WC * 64 * 16;  // one filter group image
             best.lds_bytes += 2 * wimg;
             best.wpk_bytes = (size_t)best.co_tiles * best.nchunks * best.ngroups * wimg;
+            best.lanes = lanes_ok && best.WCO == 2;
+            if (best.lanes) {
+                best.lds_bytes = lanes_lds_bytes();
+                best.wpk_bytes = lanes_image_bytes(best.co_tiles, best.nchunks, best.ngroups);
+            }
         }
         return true;
     }
@@ -700,6 +722,14 @@ static bool use_f16_mfma(const Problem& p) { return p.dtype == PHX_F16; }
 // which fp16 rounds, so fp32 arithmetic on the fp16 instructions is always the 16-product form.
 static int pass_mode(const Problem& p, int pass) {
     return use_f16_mfma(p) && !fp16_arithmetic(p, pass) ? PHX_PRODUCT_16 : p.mode;
+}
+
+// ... as the planner of the forward / input-gradient kernels takes it: with a flag for tensors that one of its kernels,
+// which addresses them with 32-bit byte offsets, cannot reach (4 components of 2 bytes)
+constexpr int CORR_LARGE = 256;
+static int corr_mode(const Problem& p, int pass) {
+    const long most = (long)p.n * std::max((long)p.ci_mem * p.h * p.w, (long)p.co_mem * p.ho * p.wo);
+    return pass_mode(p, pass) | (most >= (1L << 28) ? CORR_LARGE : 0);
 }
 
 // Kernel labels tell the two apart: f16mfma = fp16 arithmetic allowed, exact16mfma = fp32 arithmetic on fp16 instructions.
@@ -743,7 +773,9 @@ static bool pwx_applies(const Corr& c, bool f16mfma) {
            (long)c.N * ((c.Win + 7) / 8) < (1L << 30) && !tune().nopwx && !tune().pw8;
 }
 
-static bool plan_corr_uncached(const Corr& creal, int mode, bool f16mfma, Corr& c, FwdPlan& pl, int& pw) {
+static bool plan_corr_uncached(const Corr& creal, int corr_mode, bool f16mfma, Corr& c, FwdPlan& pl, int& pw) {
+    const int mode = corr_mode & 255;
+    const bool large = (corr_mode & CORR_LARGE) != 0;
     pl.pwx = 0; pl.pwx_steps = 0;
     if (pwx_applies(creal, f16mfma)) {
         pw = 0;
@@ -761,7 +793,7 @@ static bool plan_corr_uncached(const Corr& creal, int mode, bool f16mfma, Corr& 
     c = virtual_pointwise(creal, f16mfma, pw);
     if (pw) {
         pl.kmode = (mode == 8 && !tune().pw8) ? 16 : mode;
-        if (plan_forward(c, pl.kmode, f16mfma, pl, true) && pl.lds_filters && pl.chunks) return true;
+        if (plan_forward(c, pl.kmode, large, f16mfma, pl, true) && pl.lds_filters && pl.chunks) return true;
     }
     pw = 0;
     c = creal;
@@ -782,7 +814,7 @@ static bool plan_corr_uncached(const Corr& creal, int mode, bool f16mfma, Corr& 
     // 0.029 -> 0.028; from 64 channels on the factorized kernel wins (14x14: 0.032 against 0.033).
     // (with 25 taps the halved products count again: 5x5 on 24 channels 0.031 against 0.034 ms)
     if (f16mfma && mode == 8 && c.Kh * c.Kw > 1 && c.Kh * c.Kw <= 9 && c.Cin <= 32 && !tune().zi8) pl.kmode = 16;
-    return plan_forward(c, pl.kmode, f16mfma, pl);
+    return plan_forward(c, pl.kmode, large, f16mfma, pl);
 }
 
 struct CorrPlan {
@@ -1050,7 +1082,7 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     int pw = 0;
     Corr c;
     FwdPlan pl;
-    if (!plan_corr(creal, pass_mode(p, map_pass(map)), f16, c, pl, pw)) return PHX_ERR_NOT_SUPPORTED;
+    if (!plan_corr(creal, corr_mode(p, map_pass(map)), f16, c, pl, pw)) return PHX_ERR_NOT_SUPPORTED;
     if (pl.pwx) return run_pwx(p, creal, pl, map, st, in, w, bias, out, ws, ws_bytes);
     const GroupBatch gb = g_batch;
     const size_t image = align_up(pl.wpk_bytes, 256);  // (group after group where one launch runs them all)
@@ -1061,7 +1093,7 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     FwdVariant v;
     v.mode = pl.kmode; v.map = map;
     v.WCO = pl.WCO; v.NTW = pl.NTW; v.CK = pl.CK; v.P2LOG = pl.P2LOG; v.wgs = pl.wgs; v.lds_bytes = pl.lds_bytes;
-    v.lds_filters = pl.lds_filters; v.ngroups = pl.ngroups; v.pairs = pl.pairs; v.chunks = pl.chunks; v.pw = pw; v.vstage = pl.vstage;
+    v.lds_filters = pl.lds_filters; v.ngroups = pl.ngroups; v.pairs = pl.pairs; v.chunks = pl.chunks; v.lanes = pl.lanes; v.pw = pw; v.vstage = pl.vstage;
 
     PackArgs pa{};
     pa.groups = gb.n; pa.g_w = (long)gb.w; pa.g_out = (long)image;
@@ -1072,7 +1104,8 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     pa.rows = c.Cout; pa.red = creal.Cin; pa.row_tiles = pl.co_tiles * pl.WCO;
     pa.nchunks = f16 ? pl.nchunks : pl.nchunks * (pl.CK / F32_CK);
     // (LDS images: one thread per packed half, in 8-product form one thread per element of eight lane vectors)
-    const long pack_items = pl.lds_filters ? (long)(pl.wpk_bytes / 2) / (pl.kmode == 8 ? 8 : 1)
+    // (lanes dealt over the waves: one thread per channel element of a (tap, sub-tile, lane) slot)
+    const long pack_items = pl.lanes ? (long)pl.co_tiles * pl.nchunks * pl.ngroups * F16_TG * 2 * 64 * 8 : pl.lds_filters ? (long)(pl.wpk_bytes / 2) / (pl.kmode == 8 ? 8 : 1)
                                             : (long)pa.row_tiles * pa.nchunks * creal.Kh * creal.Kw * (f16 ? 1 : 4) * 64;
     if (pl.lds_filters) pa.row_tiles = pl.co_tiles;  // packed per workgroup tile of WCO*32 channels
     const int pack_blocks = (int)std::min<long>((pack_items + WG_THREADS - 1) / WG_THREADS, 4096);
@@ -1098,6 +1131,12 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     a.tiles_n = pl.tiles_n; a.tiles_h = pl.tiles_h; a.tiles_w = pl.tiles_w; a.co_tiles = pl.co_tiles;
     a.nchunks = pl.nchunks;
     // pixels a lane may store as one word: the groups must not straddle tile rows or the image edge
+    if (pl.lanes && !cl && c.Win % 2 == 0) {
+        // The staged window may start one column earlier where its rows have room for that column, or where the column
+        // they lose at the end is padding: it is then read as the first column of the next row, which lies before the image.
+        const int need = (pl.TW - 1) * c.sw + (c.Kw - 1) * c.dw + 1;
+        a.even = pl.HTW > need || (pl.tiles_w == 1 && c.pl > 0 && need - 1 - c.pl >= c.Win);
+    }
     a.vec = (pl.TW % 4 == 0 && c.Wout % 4 == 0) ? 4 : (pl.TW % 2 == 0 && c.Wout % 2 == 0) ? 2 : 1;
     if (tune().vec > 0) a.vec = std::min(a.vec, tune().vec);
 
@@ -1110,7 +1149,7 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
             j.a = pa; j.a.groups = 1;
             j.a.w = at_bytes(pa.w, g * gb.w);
             j.a.out = at_bytes(pa.out, g * image);
-            j.kind = !f16 ? PACK_F32 : pl.lds_filters ? PACK_F16_LDS : PACK_F16;
+            j.kind = !f16 ? PACK_F32 : pl.lanes ? PACK_F16_LANES : pl.lds_filters ? PACK_F16_LDS : PACK_F16;
             j.mode = pl.kmode; j.map = map; j.WCO = pl.WCO; j.ngroups = pl.ngroups; j.pw = pw;
             if (const int rrc = record_pack_job(j, pack_items)) return rrc;
         }
@@ -1122,9 +1161,9 @@ static int run_corr(const Problem& p, const Corr& creal, int map, hipStream_t st
     }
     if (rc != 0) return PHX_ERR_NOT_SUPPORTED;
     PHX_HIP(hipGetLastError());
-    snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_%smfma%s%s_p%d_%s_wco%d_ntw%d_ck%d_%s%dx%dx%d", g_name_prefix,
+    snprintf(g_name_buf, sizeof(g_name_buf), "%sqconv_%s_%smfma%s%s_p%d_%s_wco%d_ntw%d_ck%d_%s%dx%dx%d%s", g_name_prefix,
              map == MAP_FWD ? "fwd" : "dgrad", f16 ? f16_tag(p, map_pass(map)) : "f32", pl.lds_filters ? (pw ? "ldspw" : pl.chunks ? "ldsc" : "lds") : "",
-             cl ? "cl" : "", pl.kmode, p.dtype == PHX_F32 ? "f32" : "f16", pl.WCO, pl.NTW, pl.CK, pl.tall ? "flat" : "tile", pl.NB, pl.TH, pl.TW);
+             cl ? "cl" : "", pl.kmode, p.dtype == PHX_F32 ? "f32" : "f16", pl.WCO, pl.NTW, pl.CK, pl.tall ? "flat" : "tile", pl.NB, pl.TH, pl.TW, pl.lanes ? "_lanes" : "");
     label_groups(gb.n);
     g_last_kernel = g_name_buf;
     say(p, map == MAP_FWD ? "forward" : "input gradient");
@@ -1541,12 +1580,12 @@ static size_t workspace_plain(const Problem& p, int pass) {
                 const PhaseAxis ah = phase_axis(a, p.h, p.kh, p.dh, p.sh, p.pt), aw = phase_axis(b, p.w, p.kw, p.dw, p.sw, p.pl);
                 if (!ah.taps || !aw.taps || !ah.size || !aw.size) continue;
                 bufs += align_up((size_t)4 * p.n * p.ci * ah.size * aw.size * esize, 256);
-                if (!plan_corr(phase_corr(p, ah, aw), pass_mode(p, pass), use_f16_mfma(p), c, pl, pw)) return 0;
+                if (!plan_corr(phase_corr(p, ah, aw), corr_mode(p, pass), use_f16_mfma(p), c, pl, pw)) return 0;
                 wpk = std::max(wpk, align_up(pl.wpk_bytes, 256));
             }
         return bufs + wpk;
     }
-    return plan_corr((pass == PHX_PASS_FWD) ? corr_forward(p) : corr_dgrad(p), pass_mode(p, pass), use_f16_mfma(p), c, pl, pw)
+    return plan_corr((pass == PHX_PASS_FWD) ? corr_forward(p) : corr_dgrad(p), corr_mode(p, pass), use_f16_mfma(p), c, pl, pw)
                ? align_up(pl.wpk_bytes, 256)
                : 0;
 }
@@ -1832,7 +1871,7 @@ static int slices_rule(const Problem& p, int pass, const Corr& creal) {
     FwdPlan pl;
     int pw = 0;
     const bool f16 = use_f16_mfma(p);
-    if (!plan_corr(creal, pass_mode(p, pass), f16, c, pl, pw)) return 0;
+    if (!plan_corr(creal, corr_mode(p, pass), f16, c, pl, pw)) return 0;
     const int red = creal.Cin;
     const auto fits = [&](int z) { return red % z == 0 && (red / z) % 16 == 0 && red / z >= 32; };
     if (tune().kslices > 1) return fits(tune().kslices) ? tune().kslices : 0;
@@ -1841,9 +1880,12 @@ static int slices_rule(const Problem& p, int pass, const Corr& creal) {
     // reduction steps of the unsliced pass
     const long wgs = pl.pwx ? (long)cdiv(creal.N * cdiv(creal.Hin * creal.Win, 8), 8 * (4 / pl.pwx)) * pl.co_tiles : pl.wgs;
     const long steps = pl.pwx ? pl.pwx_steps : (long)pl.nchunks * c.Kh * c.Kw;  // (c: a pointwise problem may run as a column of virtual taps)
-    const long most = pl.pwx ? cus : 2L * cus;
+    // (product lanes dealt over the waves: one workgroup per CU, unless the slices come down to the 32 channels that run in
+    // 16-product form.  8 images of 256 channels at 14x14, 128 workgroups: two slices 47 us, four 51, none 67; 16 images of 512
+    // at 7x7 86 / 95 / 137; 4 images, 32 workgroups: 16 slices 34, 8 slices 37)
     int Z = 1;
-    while (fits(2 * Z) && wgs * 2 * Z <= most && steps / (2 * Z) >= 8) Z *= 2;
+    const auto most = [&](int z) { return pl.pwx || (pl.lanes && red / z > 32) ? (long)cus : 2L * cus; };
+    while (fits(2 * Z) && wgs * 2 * Z <= most(2 * Z) && steps / (2 * Z) >= 8) Z *= 2;
     // (on the fp16 matrix cores two slices pay for the extra pass over the result only where the unsliced pass leaves
     // half of the CUs without a workgroup: 64 -> 64 3x3 at 14x14, N=32, 128 workgroups 27 -> 23 us, at 56x56, N=1
     // 31 -> 24; but 256 -> 256 at 14x14, N=16, 256 workgroups 107 -> 115, 64 -> 64 at 56x56, N=4, 200 workgroups
@@ -1969,7 +2011,7 @@ static size_t workspace_for(const Problem& p, int pass) {
                 Corr c;
                 FwdPlan pl;
                 int pw = 0;
-                if (!plan_corr(phase_corr(sc.q, ah, aw), pass_mode(p, pass), use_f16_mfma(p), c, pl, pw)) return 0;
+                if (!plan_corr(phase_corr(sc.q, ah, aw), corr_mode(p, pass), use_f16_mfma(p), c, pl, pw)) return 0;
                 most = std::max(most, sc.partial_bytes + (size_t)Z * align_up(pl.wpk_bytes, 256));
             }
         return bufs + most;
@@ -2441,7 +2483,7 @@ static bool nhwc_window_native(const Problem& p, int pass) {
     Corr c;
     FwdPlan pl;
     int pw = 0;
-    if (!plan_corr(pass == PHX_PASS_FWD ? corr_forward(p) : corr_dgrad(p), pass_mode(p, pass), true, c, pl, pw)) return false;
+    if (!plan_corr(pass == PHX_PASS_FWD ? corr_forward(p) : corr_dgrad(p), corr_mode(p, pass), true, c, pl, pw)) return false;
     if (!(pl.lds_filters && pl.chunks && !pl.pwx && pw == 0)) return false;
     // a small batch on a deep layer gains more from reduction slices (corr_slices), which run on channels-first copies:
     // the copies of so small a problem cost next to nothing; so do dilated windows from their dilation phases
