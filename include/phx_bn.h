@@ -1,4 +1,4 @@
-/* Training-mode batch normalisation (+ optional ReLU) for activations in the engine's layout.
+/* Batch normalisation (+ optional residual and ReLU), training and evaluation, for activations in the engine's layout.
  *
  * No counterpart in the reference engine, which holds no model code: these entry points serve the
  * quaternion ResNet-50 harness that the images/s figure is quoted on (phoenix_core_amd/nn.py,
@@ -40,6 +40,11 @@ size_t phx_bn_workspace_bytes(const phx_bn_desc* desc);
 int phx_bn_fwd_train(const phx_bn_desc* desc, phx_stream_t stream, const void* x, const void* residual_or_null,
                      const float* gamma, const float* beta, void* y, float* save_mean, float* save_invstd,
                      float* running_mean_or_null, float* running_var_or_null, void* workspace, size_t workspace_bytes);
+
+/* Evaluation: the same with the running statistics in place of the batch's, y = gamma * (x - running_mean) /
+ * sqrt(running_var + eps) + beta (+ residual), then the optional ReLU, in one pass; desc->momentum is not read. */
+int phx_bn_fwd_eval(const phx_bn_desc* desc, phx_stream_t stream, const void* x, const void* residual_or_null,
+                    const float* gamma, const float* beta, const float* running_mean, const float* running_var, void* y);
 
 /* dx, dgamma, dbeta from x, dy and the saved statistics (beta and the residual are read for the ReLU mask
  * only); with a residual (relu must be set), dresidual receives its gradient, dy behind the ReLU. */

@@ -37,7 +37,7 @@ EXPORTS = (
 
 
 # every symbol include/phx_bn.h declares (batch normalisation for the ResNet harness)
-EXPORTS_BN = ("phx_bn_workspace_bytes", "phx_bn_fwd_train", "phx_bn_bwd")
+EXPORTS_BN = ("phx_bn_workspace_bytes", "phx_bn_fwd_train", "phx_bn_fwd_eval", "phx_bn_bwd")
 
 
 # every symbol include/phx_pool.h declares (max pooling for the same harness)
@@ -104,6 +104,7 @@ def lib():
         L.phx_bn_workspace_bytes.restype = sz
         L.phx_bn_workspace_bytes.argtypes = [bd]
         L.phx_bn_fwd_train.argtypes = [bd, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz]
+        L.phx_bn_fwd_eval.argtypes = [bd, vp, vp, vp, vp, vp, vp, vp, vp]
         L.phx_bn_bwd.argtypes = [bd, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz]
         L.phx_maxpool3x3s2_fwd.argtypes = [ctypes.c_int32, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, vp, vp, vp, vp]
         L.phx_maxpool3x3s2_bwd.argtypes = [ctypes.c_int32, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, vp, vp, vp, vp]

@@ -315,7 +315,8 @@ class QBatchNorm2d(nn.Module):
     statistics of their channel), optionally followed by ReLU, on the library's streaming kernels in
     training mode: a channel is spread over many workgroups, where one-workgroup-per-channel library kernels
     leave a 16-channel layer on 16 of 256 CUs.  Parameters and statistics are fp32 whatever the tensor type.
-    Evaluation mode uses torch.nn.functional.batch_norm with the running statistics."""
+    Evaluation mode (running statistics) is one pass of the library's, with the residual and the ReLU in it, where no
+    gradient is asked for and the tensors are ones the kernel reads; torch.nn.functional.batch_norm otherwise."""
 
     def __init__(self, num_features, eps=1e-5, momentum=0.1, relu=False):
         super().__init__()
@@ -333,10 +334,24 @@ class QBatchNorm2d(nn.Module):
         if self.training:
             return _QBatchNormFn.apply(x.contiguous(), None if residual is None else residual.contiguous(), self.weight,
                                        self.bias, self.running_mean, self.running_var, self.eps, self.momentum, self.relu)
+        if self._eval_on_kernel(x, residual):
+            return ops.batch_norm_eval(x, self.weight, self.bias, self.running_mean, self.running_var, self.eps, self.relu,
+                                       residual)
         y = nn.functional.batch_norm(x, self.running_mean, self.running_var, self.weight, self.bias, False, 0.0, self.eps)
         if residual is not None:
             y = y + residual
         return torch.relu(y) if self.relu else y
+
+
+    def _eval_on_kernel(self, x, residual):
+        own = (self.weight, self.bias, self.running_mean, self.running_var)
+        if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, residual, self.weight, self.bias)):
+            return False
+        if not (x.is_cuda and x.is_contiguous() and x.dim() >= 2 and x.shape[1] == self.weight.numel() and
+                x.dtype in (torch.float32, torch.float16) and all(t.dtype == torch.float32 and t.device == x.device for t in own)):
+            return False
+        return residual is None or (residual.shape == x.shape and residual.dtype == x.dtype and residual.device == x.device and
+                                    residual.is_contiguous())
 
 
 class _QMaxPoolFn(torch.autograd.Function):

@@ -490,6 +490,24 @@ def batch_norm_fwd(x, gamma, beta, running_mean, running_var, eps, momentum, rel
     return y, mean, invstd
 
 
+def batch_norm_eval(x, gamma, beta, running_mean, running_var, eps, relu, residual=None):
+    """Evaluation-mode batch normalisation (+ residual, + ReLU) of [rows, C, H, W]: the running statistics in place of
+    the batch's, one pass over the tensor (include/phx_bn.h)."""
+    dev = _dev_check(x, gamma, beta, running_mean, running_var, residual)
+    rows, c = x.shape[0], x.shape[1]
+    if x.dtype not in _DTYPES:
+        raise ValueError("batch normalisation takes float32 or float16 activations")
+    if residual is not None:
+        _expect(residual, x.shape, x.dtype, "residual")
+    for t, what in ((gamma, "gamma"), (beta, "beta"), (running_mean, "running_mean"), (running_var, "running_var")):
+        _expect(t, (c,), torch.float32, what)
+    desc = capi.BnDesc(_DTYPES[x.dtype], rows, c, x.numel() // max(rows * c, 1), eps, 0.0, int(relu))
+    y = torch.empty_like(x)
+    capi.check(capi.lib().phx_bn_fwd_eval(ctypes.byref(desc), _stream(dev), _ptr(x), _ptr(residual), _ptr(gamma), _ptr(beta),
+                                          _ptr(running_mean), _ptr(running_var), _ptr(y)), "phx_bn_fwd_eval")
+    return y
+
+
 def batch_norm_bwd(x, dy, gamma, beta, mean, invstd, eps, relu, residual=None):
     """Returns (dx, dgamma, dbeta, dresidual) of batch_norm_fwd; dresidual is None without a residual."""
     dev = _dev_check(x, dy, gamma, beta, mean, invstd, residual)

@@ -101,3 +101,37 @@ def test_statistics_of_a_channel_with_a_large_mean(dtype):
     n = shape[0] * shape[2] * shape[3]
     close(mod.running_var, 0.9 + 0.1 * var * n / (n - 1), 1e-3, "running var")
     close(y, want, 1e-3 if dtype == torch.float32 else 4e-3, "y")
+
+
+@pytest.mark.parametrize("relu,residual", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (3, 130, 1, 1), (5, 7, 1, 3), (4, 6, 2, 3), (9, 33, 7, 1), (2, 3, 2, 4),
+                                   (12, 65, 7, 7), (1, 2, 64, 32), (3, 5, 45, 91)], ids=lambda s: "x".join(map(str, s)))
+def test_evaluation_pass(shape, dtype, relu, residual):
+    """The one-pass evaluation kernel at the edges of its runs (planes smaller than a 16-byte chunk, of exactly one, of
+    a whole run; a ragged end) against fp64.  Five fp32 operations: 8 * 2^-24 of the largest term, and half a unit in
+    the last place of the result type."""
+    gen = torch.Generator().manual_seed(sum(shape))
+    c = shape[1]
+    mod = phx.QBatchNorm2d(c, relu=relu).cuda().eval()
+    x = (torch.randn(shape, generator=gen) * 1.5 + 20.0).to(dtype)
+    res = torch.randn(shape, generator=gen).to(dtype) if residual else None
+    with torch.no_grad():
+        mod.weight.copy_(torch.rand(c, generator=gen) + 0.5)
+        mod.bias.copy_(torch.randn(c, generator=gen))
+        mod.running_mean.copy_(torch.randn(c, generator=gen) + 20.0)
+        mod.running_var.copy_(torch.rand(c, generator=gen) + 0.5)
+        y = mod(x.cuda(), res.cuda()) if residual else mod(x.cuda())
+    d = [t.detach().double().cpu().view(1, c, 1, 1) for t in (mod.weight, mod.bias, mod.running_mean, mod.running_var)]
+    term = d[0] * (x.double() - d[2]) / (d[3] + mod.eps).sqrt()
+    want = term + d[1] + (res.double() if residual else 0.0)
+    if relu:
+        want = torch.relu(want)
+    size = term.abs().max() + d[1].abs().max() + (res.double().abs().max() if residual else 0.0)
+    bound = 8 * 2.0 ** -24 * size + (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -24) * want.abs()
+    assert ((y.double().cpu() - want).abs() <= bound).all()
+    if shape != (1, 1, 1, 1):  # a gradient through the evaluation mode takes torch's way and agrees
+        xg = x.cuda().requires_grad_(True)
+        yg = mod(xg, res.cuda()) if residual else mod(xg)
+        yg.sum().backward()
+        assert torch.isfinite(xg.grad).all()
