@@ -222,8 +222,8 @@ int launch_slice_sum(bool half_storage, const void* partial, int slices, long co
 }
 
 int launch_transpose(bool half_storage, const TransposeArgs& a, hipStream_t st) {
-    const int T = half_storage ? 64 : 32;  // tile edge of one wave
-    const long tiles = a.batch * ((a.R + T - 1) / T) * ((a.Cc + T - 1) / T);
+    const int V = half_storage ? 8 : 4;  // block edge of one lane
+    const long tiles = a.batch * transpose_tiles((a.R + V - 1) / V, (a.Cc + V - 1) / V);
     if (tiles == 0) return 0;
     const int blocks = (int)std::min<long>((tiles + 3) / 4, 1 << 16);
     if (half_storage) hipLaunchKernelGGL((transpose_kernel<_Float16>), dim3(blocks), dim3(WG_THREADS), 0, st, a);
