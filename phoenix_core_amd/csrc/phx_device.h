@@ -336,4 +336,9 @@ __device__ __forceinline__ void stage_store(TD* dst, const float (&v)[(4 * NCH) 
     }
 }
 
+// a workgroup barrier that waits for LDS alone: loads from memory stay in flight
+__device__ __forceinline__ void wg_barrier_no_vmem_wait() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 }  // namespace phx

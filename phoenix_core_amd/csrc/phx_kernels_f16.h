@@ -316,9 +316,6 @@ __device__ __forceinline__ void lds_dma_16_untracked(const void* gsrc, void* lds
                  : "v"(gsrc), "s"(lds_addr)
                  : "memory");  // (m0 is a reserved register: it cannot be named as clobbered, and nothing else here uses it)
 }
-__device__ __forceinline__ void wg_barrier_no_vmem_wait() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
 
 
 // Chunk staging of the activation window (CHUNKS): the window is NB*HTH rows of HTW positions, HTW a

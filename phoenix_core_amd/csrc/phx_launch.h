@@ -133,6 +133,10 @@ struct ThinArgs {
     int tile_R, tile_J, tile_rows, tile_cols, tile_bands;
     int tile_row0, tile_col0;  // strided input gradient by phases: the tile's first row / column relative to its first output block
     ThinDiv d_cols, d_rows, d_wout, d_R;
+    // fp16 tiles whose window rows are copied as whole image rows (thin_rows_plan): divisions by the image's width and by
+    // the chunks of an image; 0 chunks: element by element
+    ThinDiv d_win, d_chunks;
+    int row_chunks;
 };
 // < 0: not launched; 1: ran on the kernel that stages window tiles in LDS, 2: the strided input gradient by phases from
 // such tiles; 0 otherwise

@@ -204,6 +204,87 @@ __device__ __forceinline__ void thin_store(__amdgpu_buffer_rsrc_t buffer, unsign
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), buffer, bytes, 0, 0);
 }
 
+// fp16 window tiles by whole image rows.  The rows of a band that lie inside the image are one run of the plane: a thread
+// takes four positions of all four components (8-byte loads), pairs the components with byte permutes and writes the four
+// entries -- at most one row ends inside the four, image rows being at least that long; the last chunk ends where the run
+// ends (and writes some entries of its neighbour once more).  The columns outside the image are cleared once, ahead of the
+// first tile (thin_clear), the rows outside it per tile.  Element by element, with some 45 instructions and four 2-byte
+// loads per entry, depthwise 3x3 on 128 channels of 28x28, N=32 took 28 / 27 / 47 us (forward, input and filter gradient),
+// by rows it takes 26 / 26 / 32 (25.7 MB in, 25.7 MB out).  Bound: the vector ALU, which the eight dot products per tap and output
+// fill a third of.  Requesting the first rows ahead of the filter, or a tile ahead in the filter gradient, costs registers,
+// hence waves in flight, and measured slower (28 / 28 / 38); so did registers capped for more waves (26 / 28 / 34, spills).
+struct ThinRows {
+    int lo, hi, run;  // image rows of the window inside the image, and their elements
+    __device__ __forceinline__ ThinRows(int ih0, int tile_rows, int H, int W) {
+        lo = max(ih0, 0);
+        hi = min(ih0 + tile_rows, H);
+        run = (hi - lo) * W;
+    }
+};
+typedef unsigned int thin_u32x2 __attribute__((ext_vector_type(2)));
+constexpr int THIN_BATCH = 2;  // chunks per thread whose loads are in flight together
+
+// chunk `c` of the tile's images (P.row_chunks each, or what the band's run holds): its image and first element in the run
+__device__ __forceinline__ bool thin_chunk(const ThinArgs& P, const ThinRows& rows, int images, int c, int& j, int& start) {
+    j = P.tile_J > 1 ? thin_div(c, P.d_chunks) : 0;
+    start = (P.tile_J > 1 ? c - j * P.row_chunks : c) * 4;
+    if (j >= images || start >= rows.run) return false;
+    start = min(start, rows.run - 4);
+    return true;
+}
+
+__device__ __forceinline__ void thin_load_rows(const ThinArgs& P, const ThinRows& rows, const __amdgpu_buffer_rsrc_t (&planes)[4], int images,
+                                               int image_elems, int W, int c0, thin_u32x2 (&v)[THIN_BATCH][4]) {
+#pragma unroll
+    for (int b = 0; b < THIN_BATCH; ++b) {
+        int j, start;
+        const bool ok = thin_chunk(P, rows, images, c0 + b * WG_THREADS, j, start);
+        const unsigned int at = ok ? (unsigned int)(j * image_elems + rows.lo * W + start) * 2u : THIN_NOWHERE;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[b][p] = __builtin_bit_cast(thin_u32x2, __builtin_amdgcn_raw_buffer_load_b64(planes[p], at, 0, 0));
+    }
+}
+
+template <bool CONJ>
+__device__ __forceinline__ void thin_write_rows(const ThinArgs& P, const ThinRows& rows, int images, int ih0, int iw0, int W, int c0,
+                                                thin_u32x2 (&v)[THIN_BATCH][4], unsigned char* tile) {
+#pragma unroll
+    for (int b = 0; b < THIN_BATCH; ++b) {
+        int j, start;
+        if (!thin_chunk(P, rows, images, c0 + b * WG_THREADS, j, start)) continue;
+        const int r = thin_div(start, P.d_win), col = start - r * W;
+        thin_u32x2* at = reinterpret_cast<thin_u32x2*>(tile) + (j * P.tile_rows + rows.lo - ih0 + r) * P.tile_cols + col - iw0;
+        thin_u32x2* wrapped = at + (P.tile_cols - W);  // elements behind the end of the row
+        if (CONJ) {
+#pragma unroll
+            for (int p = 1; p < 4; ++p) v[b][p] ^= 0x80008000u;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned int sel = (i & 1) ? 0x07060302u : 0x05040100u;
+            const thin_u32x2 e = {__builtin_amdgcn_perm(v[b][1][i >> 1], v[b][0][i >> 1], sel), __builtin_amdgcn_perm(v[b][3][i >> 1], v[b][2][i >> 1], sel)};
+            (col + i < W ? at : wrapped)[i] = e;
+        }
+    }
+}
+
+// zeros in the rows of the tile outside the image, and in all rows of images past the last
+__device__ __forceinline__ void thin_clear_rows(const ThinArgs& P, const ThinRows& rows, int images, int ih0, unsigned char* tile) {
+    const int top = (rows.hi > rows.lo ? rows.lo - ih0 : P.tile_rows) * P.tile_cols, bottom = (rows.hi > rows.lo ? rows.hi - ih0 : P.tile_rows) * P.tile_cols;
+    const int image = P.tile_rows * P.tile_cols;
+    thin_u32x2* t = reinterpret_cast<thin_u32x2*>(tile);
+    for (int j = 0; j < P.tile_J; ++j, t += image) {
+        const int t_end = j < images ? top : image, b_start = j < images ? bottom : image;
+        for (int e = threadIdx.x; e < t_end; e += WG_THREADS) t[e] = thin_u32x2{0u, 0u};
+        for (int e = b_start + threadIdx.x; e < image; e += WG_THREADS) t[e] = thin_u32x2{0u, 0u};
+    }
+}
+
+__device__ __forceinline__ void thin_clear(const ThinArgs& P, unsigned char* tile) {
+    for (int e = threadIdx.x; e < P.tile_J * P.tile_rows * P.tile_cols; e += WG_THREADS) reinterpret_cast<thin_u32x2*>(tile)[e] = thin_u32x2{0u, 0u};
+    __syncthreads();
+}
+
 // body(integral_constant<N>) for N == slots, 0 <= slots <= MAX
 template <int MAX, typename Body>
 __device__ __forceinline__ void thin_dispatch_slots(int slots, const Body& body) {
@@ -215,7 +296,7 @@ __device__ __forceinline__ void thin_dispatch_slots(int slots, const Body& body)
     }
 }
 
-template <typename TS, bool DGRAD>
+template <typename TS, bool DGRAD, bool ROWS>
 __global__ void __launch_bounds__(THIN_TILE_THREADS) qconv_thin_tile_kernel(const ThinArgs P) {
     using T = ThinTile<TS>;
     using Entry = typename T::Entry;
@@ -225,6 +306,23 @@ __global__ void __launch_bounds__(THIN_TILE_THREADS) qconv_thin_tile_kernel(cons
     const int c = blockIdx.y;  // channel of the written tensor, over all groups
     const int cside = DGRAD ? P.cig : P.cog, K = DGRAD ? P.cog : P.cig;
     const int g = c / cside, c_in_group = c - g * cside;
+    const int Hin = DGRAD ? P.Ho : P.H, Win = DGRAD ? P.Wo : P.W;    // the tensor read
+    const int Hout = DGRAD ? P.H : P.Ho, Wout = DGRAD ? P.W : P.Wo;  // the tensor written
+    const int rstep = DGRAD ? 1 : P.sh, cstep = DGRAD ? 1 : P.sw;    // window rows / columns per output row / column
+    const long opix = (long)Hout * Wout, ipix = (long)Hin * Win;
+    const long Cin_all = (long)P.groups * K, Cout_all = (long)P.groups * cside;
+    const bool real_x = !DGRAD && P.real_x;  // real-valued input: one stored component, the others read as zero
+    const long in_cs = real_x ? 0 : P.N * Cin_all * ipix, out_cs = P.N * Cout_all * opix;
+    const int ng = blockIdx.x / P.tile_bands, band = blockIdx.x - ng * P.tile_bands;
+    const int n0 = ng * P.tile_J, r0 = band * P.tile_R;
+    // the tile's first row and column in the tensor read
+    const int ih0 = DGRAD ? r0 + P.pt - (P.Kh - 1) * P.dh : r0 * P.sh - P.pt;
+    const int iw0 = DGRAD ? P.pl - (P.Kw - 1) * P.dw : -P.pl;
+    const int entries = P.tile_J * P.tile_rows * P.tile_cols;
+    const int image_in = (int)(Cin_all * ipix), image_out = (int)(Cout_all * opix);  // elements from an image to the next
+    const TS* in = static_cast<const TS*>(P.in) + ((long)n0 * Cin_all + (long)g * K) * ipix;
+    const ThinRows rows(ih0, P.tile_rows, Hin, Win);
+    const int images = min(P.tile_J, P.N - n0), chunks = P.tile_J > 1 ? images * P.row_chunks : (rows.run + 3) >> 2;
     Filter* filt = reinterpret_cast<Filter*>(thin_lds);                          // [other-side channel][tap]
     Entry* tile = reinterpret_cast<Entry*>(thin_lds + (size_t)K * taps * sizeof(Filter));  // [image][window row][window column]
     const TS* W = static_cast<const TS*>(P.w);
@@ -240,20 +338,6 @@ __global__ void __launch_bounds__(THIN_TILE_THREADS) qconv_thin_tile_kernel(cons
         }
         filt[e] = T::filter(w);
     }
-    const int Hin = DGRAD ? P.Ho : P.H, Win = DGRAD ? P.Wo : P.W;    // the tensor read
-    const int Hout = DGRAD ? P.H : P.Ho, Wout = DGRAD ? P.W : P.Wo;  // the tensor written
-    const int rstep = DGRAD ? 1 : P.sh, cstep = DGRAD ? 1 : P.sw;    // window rows / columns per output row / column
-    const long opix = (long)Hout * Wout, ipix = (long)Hin * Win;
-    const long Cin_all = (long)P.groups * K, Cout_all = (long)P.groups * cside;
-    const bool real_x = !DGRAD && P.real_x;  // real-valued input: one stored component, the others read as zero
-    const long in_cs = real_x ? 0 : P.N * Cin_all * ipix, out_cs = P.N * Cout_all * opix;
-    const int ng = blockIdx.x / P.tile_bands, band = blockIdx.x - ng * P.tile_bands;
-    const int n0 = ng * P.tile_J, r0 = band * P.tile_R;
-    // the tile's first row and column in the tensor read
-    const int ih0 = DGRAD ? r0 + P.pt - (P.Kh - 1) * P.dh : r0 * P.sh - P.pt;
-    const int iw0 = DGRAD ? P.pl - (P.Kw - 1) * P.dw : -P.pl;
-    const int entries = P.tile_J * P.tile_rows * P.tile_cols;
-    const int image_in = (int)(Cin_all * ipix), image_out = (int)(Cout_all * opix);  // elements from an image to the next
 
     // this thread's outputs: numbers tid, tid + 256, .. of the workgroup's J x R x Wout
     int tbase[THIN_PXT];
@@ -278,22 +362,33 @@ __global__ void __launch_bounds__(THIN_TILE_THREADS) qconv_thin_tile_kernel(cons
     const int total = P.tile_J * P.tile_R * Wout;
     const int wave_slots = total <= wave_first ? 0 : std::min(THIN_PXT, (total - wave_first + THIN_TILE_THREADS - 1) / THIN_TILE_THREADS);
 
-    const TS* in = static_cast<const TS*>(P.in) + ((long)n0 * Cin_all + (long)g * K) * ipix;
     for (int k = 0; k < K; ++k, in += ipix) {
         if (k) __syncthreads();  // (everyone has read the previous channel's tile)
         const __amdgpu_buffer_rsrc_t planes[4] = {thin_buffer(in), thin_buffer(in + in_cs), thin_buffer(in + 2 * in_cs),
                                                   thin_buffer(in + 3 * in_cs)};
+        if constexpr (ROWS) {
+            unsigned char* const bytes = reinterpret_cast<unsigned char*>(tile);
+            thin_u32x2 v[THIN_BATCH][4];
+            thin_load_rows(P, rows, planes, images, image_in, Win, threadIdx.x, v);
+            if (k == 0) thin_clear(P, bytes);  // (while the first loads are on their way)
+            thin_write_rows<false>(P, rows, images, ih0, iw0, Win, threadIdx.x, v, bytes);
+            for (int c0 = THIN_BATCH * WG_THREADS; c0 < chunks; c0 += THIN_BATCH * WG_THREADS) {
+                thin_load_rows(P, rows, planes, images, image_in, Win, c0 + threadIdx.x, v);
+                thin_write_rows<false>(P, rows, images, ih0, iw0, Win, c0 + threadIdx.x, v, bytes);
+            }
+        } else {
 #pragma unroll 2
-        for (int e = threadIdx.x; e < entries; e += THIN_TILE_THREADS) {
-            const int row = thin_div(e, P.d_cols), tc = e - row * P.tile_cols;
-            const int j = thin_div(row, P.d_rows), tr = row - j * P.tile_rows;
-            const int ih = ih0 + tr, iw = iw0 + tc;
-            const bool ok = n0 + j < P.N && (unsigned)ih < (unsigned)Hin && (unsigned)iw < (unsigned)Win;
-            const unsigned int at = ok ? (unsigned int)(j * image_in + ih * Win + iw) * (unsigned int)sizeof(TS) : THIN_NOWHERE;
-            float v[4];
+            for (int e = threadIdx.x; e < entries; e += THIN_TILE_THREADS) {
+                const int row = thin_div(e, P.d_cols), tc = e - row * P.tile_cols;
+                const int j = thin_div(row, P.d_rows), tr = row - j * P.tile_rows;
+                const int ih = ih0 + tr, iw = iw0 + tc;
+                const bool ok = n0 + j < P.N && (unsigned)ih < (unsigned)Hin && (unsigned)iw < (unsigned)Win;
+                const unsigned int at = ok ? (unsigned int)(j * image_in + ih * Win + iw) * (unsigned int)sizeof(TS) : THIN_NOWHERE;
+                float v[4];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) v[p] = thin_load<TS>(planes[p], (p && real_x) ? THIN_NOWHERE : at);
-            tile[e] = T::entry(v);
+                for (int p = 0; p < 4; ++p) v[p] = thin_load<TS>(planes[p], (p && real_x) ? THIN_NOWHERE : at);
+                tile[e] = T::entry(v);
+            }
         }
         __syncthreads();
         // (one instance of the tap loop per number of slots, so that a tap's reads are issued together)
@@ -464,6 +559,21 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_dgrad_phase_kernel(cons
 
 static ThinDiv thin_magic(int d) { return d > 1 ? ThinDiv{(unsigned int)(((1ULL << 32) + d - 1) / d), 0u} : ThinDiv{0u, ~0u}; }
 
+// Window rows by whole image rows (ThinRows): fp16, all four components stored, rows of at least one chunk, and tiles that
+// hold every column of the image (an unpadded window with a stride may leave the last ones out).
+static void thin_rows_plan(bool half_storage, bool dgrad, ThinArgs& a) {
+    const int H = dgrad ? a.Ho : a.H, W = dgrad ? a.Wo : a.W;
+    const int iw0 = dgrad ? a.pl - (a.Kw - 1) * a.dw : -a.pl, ih0 = dgrad ? a.pt - (a.Kh - 1) * a.dh : -a.pt;
+    a.row_chunks = 0;
+    if (!half_storage || (!dgrad && a.real_x) || W < 4 || iw0 > 0 || iw0 + a.tile_cols < W) return;
+    // (more than one image in a tile: whole images, whose window the first row's padding starts)
+    const int run = (std::min(ih0 + a.tile_rows, H) - std::max(ih0, 0)) * W;
+    if (a.tile_J > 1 && run < 4) return;
+    a.row_chunks = a.tile_J > 1 ? (run + 3) / 4 : 1;
+    a.d_win = thin_magic(W);
+    a.d_chunks = thin_magic(a.row_chunks);
+}
+
 // Fills the tile fields of `a` for the forward pass / unit-stride input gradient; false where the tiled kernel does not
 // apply (a strided input gradient, rows wider than a workgroup's outputs, a window that does not fit LDS).
 static bool thin_tile_plan(bool half_storage, bool dgrad, int filter_entries, int tile_pixels, ThinArgs& a, size_t& lds) {
@@ -487,6 +597,7 @@ static bool thin_tile_plan(bool half_storage, bool dgrad, int filter_entries, in
     a.tile_bands = (Hout + R - 1) / R;
     a.d_cols = thin_magic(a.tile_cols); a.d_rows = thin_magic(a.tile_rows); a.d_wout = thin_magic(Wout); a.d_R = thin_magic(R);
     lds = bytes_of(R, J);
+    thin_rows_plan(half_storage, dgrad, a);
     return true;
 }
 
@@ -565,6 +676,18 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_kernel(const Thin
     }
 }
 
+// the sum over the sixteen threads of a DPP row (through the vector ALU alone, four instructions; the exchanges of whole
+// waves go through LDS)
+__device__ __forceinline__ float thin_row_sum(float v) {
+    const auto add = [](float a, auto ctrl) {
+        return a + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, a), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    v = add(v, std::integral_constant<int, 0xB1>());   // quad_perm: neighbours
+    v = add(v, std::integral_constant<int, 0x4E>());   // quad_perm: pairs
+    v = add(v, std::integral_constant<int, 0x141>());  // row_half_mirror: quads
+    return add(v, std::integral_constant<int, 0x140>());  // row_mirror: halves
+}
+
 // The filter gradient from the same window tiles (forward geometry): a workgroup walks over its share of the
 // (image group, row band) tiles of one channel pair; per tile it copies the CONJUGATED window of x into LDS, each
 // thread takes its (up to four) output positions' gradient values straight from global memory, turns them into the
@@ -572,13 +695,13 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_kernel(const Thin
 // place -- and accumulates TB taps from LDS.  Partial sums per slice of the tiles, as in the kernel above.
 constexpr int THIN_WG_PXT = 2;  // output positions per thread and tile of the tiled filter gradient
 
-template <typename TS, int TB>
+template <typename TS, int TB, bool ROWS>
 __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_tile_kernel(const ThinArgs P) {
     using T = ThinTile<TS>;
     using Entry = typename T::Entry;
     using Filter = typename T::Filter;
     extern __shared__ __align__(16) unsigned char thin_lds[];
-    __shared__ float red[WG_THREADS / 64][TB * 4];
+    __shared__ float red[WG_THREADS / 16][TB * 4];
     Entry* tile = reinterpret_cast<Entry*>(thin_lds);
     const int pair = blockIdx.x;
     const int co = pair / P.cig, i = pair - co * P.cig, g = co / P.cog;
@@ -621,13 +744,12 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_tile_kernel(const
 
     const auto run_tiles = [&](auto slots) {
         constexpr int NS = decltype(slots)::value;
-        int ng = t0 / P.tile_bands, band = t0 - ng * P.tile_bands;
-        for (int tile_idx = t0; tile_idx < t1; ++tile_idx) {
-            const int n0 = ng * P.tile_J, r0 = band * P.tile_R;
+        float gv[NS > 0 ? NS : 1][4];
+        thin_u32x2 v[THIN_BATCH][4];
+        const auto load_grad = [&](int n0, int r0) {
             const TS* gtile = gr + (long)n0 * Co_all * gpix + (long)r0 * P.Wo;
             const __amdgpu_buffer_rsrc_t gplanes[4] = {thin_buffer(gtile), thin_buffer(gtile + g_cs), thin_buffer(gtile + 2 * g_cs),
                                                        thin_buffer(gtile + 3 * g_cs)};
-            float gv[NS > 0 ? NS : 1][4];
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 const bool live = pj[s] < P.tile_J && n0 + pj[s] < P.N && r0 + pr[s] < P.Ho;
@@ -635,37 +757,70 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_tile_kernel(const
 #pragma unroll
                 for (int q = 0; q < 4; ++q) gv[s][q] = thin_load<TS>(gplanes[q], at);
             }
-            if (tile_idx != t0) __syncthreads();  // (everyone has read the previous tile)
-            const int ih0 = r0 * P.sh - P.pt, iw0 = -P.pl;
+        };
+        const auto load_window = [&](int n0, int ih0, int c0) {
             const TS* xin = x + (long)n0 * Ci_all * xpix;
             const __amdgpu_buffer_rsrc_t xplanes[4] = {thin_buffer(xin), thin_buffer(xin + x_cs), thin_buffer(xin + 2 * x_cs),
                                                        thin_buffer(xin + 3 * x_cs)};
-#pragma unroll 2
-            for (int e = threadIdx.x; e < entries; e += WG_THREADS) {
-                const int row = thin_div(e, P.d_cols), tc = e - row * P.tile_cols;
-                const int j = thin_div(row, P.d_rows), tr = row - j * P.tile_rows;
-                const int ih = ih0 + tr, iw = iw0 + tc;
-                const bool ok = n0 + j < P.N && (unsigned)ih < (unsigned)P.H && (unsigned)iw < (unsigned)P.W;
-                const unsigned int at = ok ? (unsigned int)(j * image_x + ih * P.W + iw) * (unsigned int)sizeof(TS) : THIN_NOWHERE;
-                float v[4];
-#pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    const float f = thin_load<TS>(xplanes[p], (p && P.real_x) ? THIN_NOWHERE : at);
-                    v[p] = p ? -f : f;  // conjugate
+            const ThinRows rows(ih0, P.tile_rows, P.H, P.W);
+            const int images = min(P.tile_J, P.N - n0), chunks = P.tile_J > 1 ? images * P.row_chunks : (rows.run + 3) >> 2;
+            thin_load_rows(P, rows, xplanes, images, image_x, P.W, c0, v);
+        };
+        const int iw0 = -P.pl;
+        int ng = t0 / P.tile_bands, band = t0 - ng * P.tile_bands;
+        for (int tile_idx = t0; tile_idx < t1; ++tile_idx) {
+            const int n0 = ng * P.tile_J, r0 = band * P.tile_R, ih0 = r0 * P.sh - P.pt;
+            if (++band == P.tile_bands) { band = 0; ++ng; }
+            Filter f[NS > 0 ? NS : 1];
+            if constexpr (ROWS) {
+                const ThinRows rows(ih0, P.tile_rows, P.H, P.W);
+                const int images = min(P.tile_J, P.N - n0), chunks = P.tile_J > 1 ? images * P.row_chunks : (rows.run + 3) >> 2;
+                load_grad(n0, r0);
+                load_window(n0, ih0, threadIdx.x);
+                if (tile_idx == t0) thin_clear(P, thin_lds);
+                else wg_barrier_no_vmem_wait();  // (everyone has read the previous tile)
+                thin_clear_rows(P, rows, images, ih0, thin_lds);
+                thin_write_rows<true>(P, rows, images, ih0, iw0, P.W, threadIdx.x, v, thin_lds);
+                for (int c0 = THIN_BATCH * WG_THREADS; c0 < chunks; c0 += THIN_BATCH * WG_THREADS) {
+                    load_window(n0, ih0, c0 + threadIdx.x);
+                    thin_write_rows<true>(P, rows, images, ih0, iw0, P.W, c0 + threadIdx.x, v, thin_lds);
                 }
-                tile[e] = T::entry(v);
+#pragma unroll
+                for (int s = 0; s < NS; ++s) f[s] = T::filter(gv[s]);
+                wg_barrier_no_vmem_wait();
+            } else {
+                load_grad(n0, r0);
+                if (tile_idx != t0) __syncthreads();  // (everyone has read the previous tile)
+                const TS* xin = x + (long)n0 * Ci_all * xpix;
+                const __amdgpu_buffer_rsrc_t xplanes[4] = {thin_buffer(xin), thin_buffer(xin + x_cs), thin_buffer(xin + 2 * x_cs),
+                                                           thin_buffer(xin + 3 * x_cs)};
+#pragma unroll 2
+                for (int e = threadIdx.x; e < entries; e += WG_THREADS) {
+                    const int row = thin_div(e, P.d_cols), tc = e - row * P.tile_cols;
+                    const int j = thin_div(row, P.d_rows), tr = row - j * P.tile_rows;
+                    const int ih = ih0 + tr, iw = iw0 + tc;
+                    const bool ok = n0 + j < P.N && (unsigned)ih < (unsigned)P.H && (unsigned)iw < (unsigned)P.W;
+                    const unsigned int at = ok ? (unsigned int)(j * image_x + ih * P.W + iw) * (unsigned int)sizeof(TS) : THIN_NOWHERE;
+                    float c[4];
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        const float e1 = thin_load<TS>(xplanes[p], (p && P.real_x) ? THIN_NOWHERE : at);
+                        c[p] = p ? -e1 : e1;  // conjugate
+                    }
+                    tile[e] = T::entry(c);
+                }
+#pragma unroll
+                for (int s = 0; s < NS; ++s) f[s] = T::filter(gv[s]);
+                __syncthreads();
             }
-            __syncthreads();
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                const Filter f = T::filter(gv[s]);
                 Entry xv[TB];
 #pragma unroll
                 for (int j = 0; j < TB; ++j) xv[j] = tile[tbase[s] + toff[j]];
 #pragma unroll
-                for (int j = 0; j < TB; ++j) T::mac(acc[j], xv[j], f);
+                for (int j = 0; j < TB; ++j) T::mac(acc[j], xv[j], f[s]);
             }
-            if (++band == P.tile_bands) { band = 0; ++ng; }
         }
     };
     thin_dispatch_slots<THIN_WG_PXT>(wave_slots, run_tiles);  // (a wave without outputs still fills and meets the barriers)
@@ -674,10 +829,8 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_tile_kernel(const
     for (int j = 0; j < TB; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            float v = acc[j][q];
-#pragma unroll
-            for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s, 64);
-            if (lane == 0) red[wave][j * 4 + q] = v;
+            const float v = thin_row_sum(acc[j][q]);
+            if ((lane & 15) == 0) red[wave * 4 + (lane >> 4)][j * 4 + q] = v;
         }
     __syncthreads();
     if (threadIdx.x < TB * 4) {
@@ -685,7 +838,7 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_wgrad_tile_kernel(const
         if (tap0 + j < taps) {
             float sum = 0.f;
 #pragma unroll
-            for (int w = 0; w < WG_THREADS / 64; ++w) sum += red[w][threadIdx.x];
+            for (int w = 0; w < WG_THREADS / 16; ++w) sum += red[w][threadIdx.x];
             P.partial[(((long)blockIdx.z * gridDim.x + pair) * taps + tap0 + j) * 4 + q] = sum;
         }
     }
@@ -780,11 +933,13 @@ int launch_thin(bool half_storage, int pass, const ThinArgs& a, hipStream_t st) 
         const dim3 grid((unsigned int)pairs, (unsigned int)((taps + TB - 1) / TB), (unsigned int)t.Z), block(WG_THREADS);
         if (tiled) {
             if (TB == 1) {
-                if (half_storage) hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<_Float16, 1>), grid, block, lds, st, t);
-                else hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<float, 1>), grid, block, lds, st, t);
+                if (half_storage && t.row_chunks) hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<_Float16, 1, true>), grid, block, lds, st, t);
+                else if (half_storage) hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<_Float16, 1, false>), grid, block, lds, st, t);
+                else hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<float, 1, false>), grid, block, lds, st, t);
             } else {
-                if (half_storage) hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<_Float16, 9>), grid, block, lds, st, t);
-                else hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<float, 9>), grid, block, lds, st, t);
+                if (half_storage && t.row_chunks) hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<_Float16, 9, true>), grid, block, lds, st, t);
+                else if (half_storage) hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<_Float16, 9, false>), grid, block, lds, st, t);
+                else hipLaunchKernelGGL((qconv_thin_wgrad_tile_kernel<float, 9, false>), grid, block, lds, st, t);
             }
         } else if (TB == 1) {
             if (half_storage) hipLaunchKernelGGL((qconv_thin_wgrad_kernel<_Float16, 1>), grid, block, 0, st, t);
@@ -809,11 +964,13 @@ int launch_thin(bool half_storage, int pass, const ThinArgs& a, hipStream_t st) 
         if (blocks >= (1L << 31)) return -1;
         const dim3 grid((unsigned int)blocks, (unsigned int)channels), block(THIN_TILE_THREADS);
         if (dgrad) {
-            if (half_storage) hipLaunchKernelGGL((qconv_thin_tile_kernel<_Float16, true>), grid, block, tile_lds, st, t);
-            else hipLaunchKernelGGL((qconv_thin_tile_kernel<float, true>), grid, block, tile_lds, st, t);
+            if (half_storage && t.row_chunks) hipLaunchKernelGGL((qconv_thin_tile_kernel<_Float16, true, true>), grid, block, tile_lds, st, t);
+            else if (half_storage) hipLaunchKernelGGL((qconv_thin_tile_kernel<_Float16, true, false>), grid, block, tile_lds, st, t);
+            else hipLaunchKernelGGL((qconv_thin_tile_kernel<float, true, false>), grid, block, tile_lds, st, t);
         } else {
-            if (half_storage) hipLaunchKernelGGL((qconv_thin_tile_kernel<_Float16, false>), grid, block, tile_lds, st, t);
-            else hipLaunchKernelGGL((qconv_thin_tile_kernel<float, false>), grid, block, tile_lds, st, t);
+            if (half_storage && t.row_chunks) hipLaunchKernelGGL((qconv_thin_tile_kernel<_Float16, false, true>), grid, block, tile_lds, st, t);
+            else if (half_storage) hipLaunchKernelGGL((qconv_thin_tile_kernel<_Float16, false, false>), grid, block, tile_lds, st, t);
+            else hipLaunchKernelGGL((qconv_thin_tile_kernel<float, false, false>), grid, block, tile_lds, st, t);
         }
         return 1;
     }
