@@ -106,7 +106,8 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
     const int row = small_div(ch, __builtin_amdgcn_rcpf(cpr)), cc = ch - row * cpr;
     const bool task = ch < P.NB * P.HTH * cpr;
     unsigned int bits = 0;   // positions of the task inside the image
-    bool careful = false;    // a load would leave the tensor
+    bool careful = false;    // the tensor is too small for loads of eight positions
+    int rot = 0;             // the loads start this many positions (modulo 8) behind the task's first one (see StageChunk)
     long element = 0;        // the task's first position, channel 0
     {
         const int nb = tall ? 0 : small_div(row, __builtin_amdgcn_rcpf(P.HTH)), hr = row - nb * P.HTH;
@@ -126,46 +127,55 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
             }
         }
         const long comp = ((0x78 >> (2 * p)) & 3) * P.in.comp_stride;
-        const long size = 3 * P.in.comp_stride + (CL ? (long)P.in.N * P.in.Hd * P.in.Wd * P.in.Cs
-                                                     : ((long)(P.in.N - 1) * P.in.Cs + P.in.C) * P.in.Hd * P.in.Wd);
+        const long size = 3 * P.in.comp_stride + ((long)(P.in.N - 1) * P.in.Cs + P.in.C) * P.in.Hd * P.in.Wd;  // (planes)
         if constexpr (CL) {
             element = comp + (((long)img * P.in.Hd + vh) * P.in.Wd + vw) * P.in.Cs;
-            careful = bits && (element < 0 || element + 7L * cpr * P.in.Cs + ((P.in.C + 15) & ~15) > size);
         } else {
             element = comp + ((long)img * P.in.Cs * P.in.Hd + vh) * P.in.Wd + vw;
-            careful = bits && (element < 0 || element + (long)(P.in.C - 1) * P.in.Hd * P.in.Wd + 8 > size);
+            if (bits) {
+                const long sh = inside_shift(element, (long)(P.in.C - 1) * P.in.Hd * P.in.Wd, size);
+                careful = sh == NO_SHIFT;
+                if (!careful) {
+                    element += sh;
+                    rot = (int)sh & 7;
+                }
+            }
         }
     }
     // (32-bit byte offsets: the host keeps larger tensors off this kernel; tasks that load nothing read the tensor's start)
     const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(P.in.base), 0, -1, 0x00020000);
-    const unsigned int xoff = bits && !careful ? (unsigned int)(element * 2) : 0u;
+    const unsigned int xoff = CL || (bits && !careful) ? (unsigned int)(element * 2) : 0u;  // (channels-last: added up modulo 2^32)
     const unsigned int xstep = (CL ? cpr * P.in.Cs : P.in.Hd * P.in.Wd) * 2;  // CL: to the next position, else to the next channel
     const int first = (CL && task) ? row * P.HTW + cc : ch * 8;  // first position and distance of the task's positions
     const int pstep = (CL && task) ? cpr : 1;                    // (threads without a task clear positions behind the window)
-    const bool any_careful = __any(careful);
+    const bool any_careful = !CL && __any(careful || rot);
     u32x4 stage[8];
     auto load_stage = [&](int chan, int i) {  // (channels past the tensor meet zero filters, any finite value will do)
         unsigned int off;
         if constexpr (CL) {
-            const unsigned int o = bits && !careful && chan + pack * 8 < P.in.C ? xoff + (chan + pack * 8) * 2 + i * xstep : 0u;
+            const unsigned int o = ((bits >> i) & 1u) && chan + pack * 8 < P.in.C ? xoff + (chan + pack * 8) * 2 + i * xstep : 0u;
             stage[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, o, 0, 0));
         } else {
             const int c = chan + pack * 8 + i;
             stage[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, xoff, c < P.in.C ? c * xstep : 0u, 0));
         }
     };
-    // Threads whose loads would leave the tensor (its first and last rows) fill their values one by one.
+    // Threads whose loads were moved to stay inside the tensor (its first and last rows) rotate their values into place,
+    // or fill them one by one.
     auto fill_careful = [&](int chan) {
+        if (rot) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) stage[i] = rotate_halves(stage[i], rot);
+        }
         if (!careful) return;
         const _Float16* src = static_cast<const _Float16*>(P.in.base) + element;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             _Float16 e[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {  // channels-last: position i, channel k; planes: channel i, position k
-                const int c = chan + pack * 8 + (CL ? k : i);
-                const bool ok = c < P.in.C && ((bits >> (CL ? i : k)) & 1);
-                e[k] = ok ? (CL ? src[(long)i * cpr * P.in.Cs + c] : src[(long)c * P.in.Hd * P.in.Wd + k]) : (_Float16)0;
+            for (int k = 0; k < 8; ++k) {  // channel i, position k
+                const int c = chan + pack * 8 + i;
+                e[k] = c < P.in.C && ((bits >> k) & 1) ? src[(long)c * P.in.Hd * P.in.Wd + k] : (_Float16)0;
             }
 #pragma unroll
             for (int m = 0; m < 4; ++m) stage[i][m] = __builtin_bit_cast(unsigned int, f16x2{e[2 * m], e[2 * m + 1]});
