@@ -123,10 +123,19 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_kernel(const ThinArgs P
 // and first copies the window of those rows -- every element once, zeros where the window leaves the image -- into
 // LDS, four components side by side per position.  A tap is then one LDS read per output (and one broadcast read of
 // the filter entry per four outputs) with no address arithmetic beyond an add, against four global loads before.
-// fp16 tensors keep their halves in LDS, paired (x0,x1) (x2,x3), and the filter entry as the eight pairs
-// (s(0,q) w[q], s(1,q) w[1^q]), (s(2,q) w[2^q], s(3,q) w[3^q]): a tap is eight v_dot2_f32_f16 -- two products and
-// their sum into an fp32 accumulator each -- instead of sixteen FMAs and four conversions.
+// fp16 tensors keep their halves in LDS, (x0, x1, x2, x3) side by side, and the filter entry as the 4 x 4 matrix of its
+// product, row q = (s(0,q) w[q], s(1,q) w[1^q], s(2,q) w[2^q], s(3,q) w[3^q]).  A tap of 64 outputs is then ONE matrix
+// instruction, v_mfma_f32_4x4x4_16b_f16: sixteen products of a 4x4 by a 4x4 matrix, in which a lane supplies one column of
+// the right matrices (the entry of its own pixel) and one row of the left ones (row lane % 4 of the filter, the same in all
+// sixteen), and receives its column of the products: its own four output components, in fp32.  (Columns never meet: what
+// a lane without an output holds stays in that lane.  The instruction runs in all lanes, whatever the mask: whole waves
+// come here.)  The filter gradient has a left matrix per pixel and takes eight v_dot2_f32_f16 (two products and their sum
+// into an fp32 accumulator each) in its place, as all passes did before: depthwise 3x3 on 128 channels of 28x28, N=32, forward
+// and input gradient 26 us each then, 19 and 20 now; 5x5 on 96 channels of 56x56, N=8, 46 / 40 (windows copied by element, too)
+// -> 27 / 24.  The registers are held to six waves a SIMD: left alone, the compiler spreads the accumulators over both
+// register files, three waves are left, and the first case takes 28.
 typedef _Float16 thin_half2 __attribute__((ext_vector_type(2)));
+typedef _Float16 thin_half4 __attribute__((ext_vector_type(4)));
 
 template <typename TS>
 struct ThinTile;
@@ -134,6 +143,8 @@ template <>
 struct ThinTile<float> {
     using Entry = float4;
     using Filter = float4;
+    using Operand = float4;  // what a lane reads of a filter entry
+    static __device__ __forceinline__ Operand operand(const Filter* f) { return *f; }
     static __device__ __forceinline__ Entry entry(const float v[4]) { return make_float4(v[0], v[1], v[2], v[3]); }
     static __device__ __forceinline__ Filter filter(const float w[4]) { return make_float4(w[0], w[1], w[2], w[3]); }
     static __device__ __forceinline__ void mac(float acc[4], const Entry& x, const Filter& f) {
@@ -147,7 +158,11 @@ struct ThinTile<float> {
 template <>
 struct ThinTile<_Float16> {
     struct __align__(8) Entry { thin_half2 lo, hi; };
-    struct __align__(16) Filter { thin_half2 lo[4], hi[4]; };
+    struct __align__(16) Filter { thin_half2 row[4][2]; };
+    using Operand = thin_half4;
+    static __device__ __forceinline__ Operand operand(const Filter* f) {
+        return *reinterpret_cast<const thin_half4*>(f->row[threadIdx.x & 3]);
+    }
     static __device__ __forceinline__ Entry entry(const float v[4]) {
         Entry e;
         e.lo = thin_half2{(_Float16)v[0], (_Float16)v[1]};  // (values that came from halves: exact)
@@ -158,17 +173,22 @@ struct ThinTile<_Float16> {
         Filter f;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            f.lo[q] = thin_half2{(_Float16)(qneg(0, q) ? -w[q] : w[q]), (_Float16)(qneg(1, q) ? -w[1 ^ q] : w[1 ^ q])};
-            f.hi[q] = thin_half2{(_Float16)(qneg(2, q) ? -w[2 ^ q] : w[2 ^ q]), (_Float16)(qneg(3, q) ? -w[3 ^ q] : w[3 ^ q])};
+            f.row[q][0] = thin_half2{(_Float16)(qneg(0, q) ? -w[q] : w[q]), (_Float16)(qneg(1, q) ? -w[1 ^ q] : w[1 ^ q])};
+            f.row[q][1] = thin_half2{(_Float16)(qneg(2, q) ? -w[2 ^ q] : w[2 ^ q]), (_Float16)(qneg(3, q) ? -w[3 ^ q] : w[3 ^ q])};
         }
         return f;
     }
     static __device__ __forceinline__ void mac(float acc[4], const Entry& x, const Filter& f) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            acc[q] = __builtin_amdgcn_fdot2(x.lo, f.lo[q], acc[q], false);
-            acc[q] = __builtin_amdgcn_fdot2(x.hi, f.hi[q], acc[q], false);
+            acc[q] = __builtin_amdgcn_fdot2(x.lo, f.row[q][0], acc[q], false);
+            acc[q] = __builtin_amdgcn_fdot2(x.hi, f.row[q][1], acc[q], false);
         }
+    }
+    static __device__ __forceinline__ void mac(float acc[4], const Entry& x, const Operand& row) {
+        const f32x4 sum = __builtin_amdgcn_mfma_f32_4x4x4f16(row, __builtin_bit_cast(thin_half4, x), f32x4{acc[0], acc[1], acc[2], acc[3]}, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = sum[q];
     }
 };
 
@@ -210,8 +230,8 @@ __device__ __forceinline__ void thin_store(__amdgpu_buffer_rsrc_t buffer, unsign
 // ends (and writes some entries of its neighbour once more).  The columns outside the image are cleared once, ahead of the
 // first tile (thin_clear), the rows outside it per tile.  Element by element, with some 45 instructions and four 2-byte
 // loads per entry, depthwise 3x3 on 128 channels of 28x28, N=32 took 28 / 27 / 47 us (forward, input and filter gradient),
-// by rows it takes 26 / 26 / 32 (25.7 MB in, 25.7 MB out).  Bound: the vector ALU, which the eight dot products per tap and output
-// fill a third of.  Requesting the first rows ahead of the filter, or a tile ahead in the filter gradient, costs registers,
+// by rows 26 / 26 / 32, with the products on the matrix cores 19 / 20 / 31 (25.7 MB in, 25.7 MB out: 10 us).  Bound: the vector
+// ALU, with addresses and stores around the products, in the filter gradient its dot products.  Requesting the first rows ahead of the filter, or a tile ahead in the filter gradient, costs registers,
 // hence waves in flight, and measured slower (28 / 28 / 38); so did registers capped for more waves (26 / 28 / 34, spills).
 struct ThinRows {
     int lo, hi, run;  // image rows of the window inside the image, and their elements
@@ -222,7 +242,7 @@ struct ThinRows {
     }
 };
 typedef unsigned int thin_u32x2 __attribute__((ext_vector_type(2)));
-constexpr int THIN_BATCH = 2;  // chunks per thread whose loads are in flight together
+constexpr int THIN_BATCH = 1;  // chunks per thread whose loads are in flight together
 
 // chunk `c` of the tile's images (P.row_chunks each, or what the band's run holds): its image and first element in the run
 __device__ __forceinline__ bool thin_chunk(const ThinArgs& P, const ThinRows& rows, int images, int c, int& j, int& start) {
@@ -297,7 +317,7 @@ __device__ __forceinline__ void thin_dispatch_slots(int slots, const Body& body)
 }
 
 template <typename TS, bool DGRAD, bool ROWS>
-__global__ void __launch_bounds__(THIN_TILE_THREADS) qconv_thin_tile_kernel(const ThinArgs P) {
+__global__ void __launch_bounds__(THIN_TILE_THREADS, sizeof(TS) == 2 ? 6 : 1) qconv_thin_tile_kernel(const ThinArgs P) {
     using T = ThinTile<TS>;
     using Entry = typename T::Entry;
     using Filter = typename T::Filter;
@@ -399,7 +419,7 @@ __global__ void __launch_bounds__(THIN_TILE_THREADS) qconv_thin_tile_kernel(cons
             for (int t = 0; t < taps; ++t) {
                 const int toff = DGRAD ? (P.Kh - 1 - kh) * P.dh * P.tile_cols + (P.Kw - 1 - kw) * P.dw
                                        : kh * P.dh * P.tile_cols + kw * P.dw;
-                const Filter f = filt[k * taps + t];
+                const typename T::Operand f = T::operand(filt + k * taps + t);
                 Entry x[NS > 0 ? NS : 1];
 #pragma unroll
                 for (int s = 0; s < NS; ++s) x[s] = tile[tbase[s] + toff];
@@ -440,7 +460,7 @@ __device__ __forceinline__ void thin_dispatch_phase(int phase, const Body& body)
 }
 
 template <typename TS, int SH, int SW>
-__global__ void __launch_bounds__(WG_THREADS) qconv_thin_dgrad_phase_kernel(const ThinArgs P) {
+__global__ void __launch_bounds__(WG_THREADS, sizeof(TS) == 2 ? 5 : 1) qconv_thin_dgrad_phase_kernel(const ThinArgs P) {
     using T = ThinTile<TS>;
     using Entry = typename T::Entry;
     using Filter = typename T::Filter;
@@ -525,7 +545,7 @@ __global__ void __launch_bounds__(WG_THREADS) qconv_thin_dgrad_phase_kernel(cons
             for (int t = 0; t < taps; ++t) {
                 const int2 where = table[t];
                 const int toff = __builtin_amdgcn_readfirstlane(where.x), phase = __builtin_amdgcn_readfirstlane(where.y);
-                const Filter f = filt[k * taps + t];
+                const typename T::Operand f = T::operand(filt + k * taps + t);
                 Entry x[NS > 0 ? NS : 1];
 #pragma unroll
                 for (int s = 0; s < NS; ++s) x[s] = tile[tbase[s] + toff];
