@@ -942,4 +942,46 @@ __global__ void __launch_bounds__(WG_THREADS) reduce_wgrad_kernel(const ReduceAr
     }
 }
 
+// The same for filters whose output channels lie side by side in memory (Dense "IO", HWIO): a workgroup sums a tile of 64
+// output x 16 input channels, reading runs of input channels, and turns it over in LDS, so that it writes runs of output
+// channels.  Bound: bytes.  Dense 1024 -> 1024, two partials (33.6 MB in, 8.4 MB out): 12.6 us against 29.9 with two-byte stores a
+// row apart.
+constexpr int REDUCE_CO = 64, REDUCE_CI = 16;
+
+template <typename TS>
+__global__ void __launch_bounds__(WG_THREADS) reduce_wgrad_turned_kernel(const ReduceArgs P0) {
+    const ReduceArgs P = group_view(P0);
+    __shared__ __align__(16) float turned[REDUCE_CI][REDUCE_CO + 4];
+    const int co_tiles = (P.Co + REDUCE_CO - 1) / REDUCE_CO, ci_tiles = (P.Ci + REDUCE_CI - 1) / REDUCE_CI;
+    int t = blockIdx.x;
+    const int ci0 = (t % ci_tiles) * REDUCE_CI;
+    t /= ci_tiles;
+    const int co0 = (t % co_tiles) * REDUCE_CO;
+    t /= co_tiles;
+    const int r = t & 3, tap = t >> 2;
+    const long zstride = 4L * P.Kh * P.Kw * P.CoP * P.CiP;
+    const int co_l = threadIdx.x >> 2, ci_l = (threadIdx.x & 3) * 4;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    if (co0 + co_l < P.Co && ci0 + ci_l < P.Ci) {
+        const float* src = P.partial + (((long)tap * 4 + r) * P.CoP + co0 + co_l) * P.CiP + ci0 + ci_l;
+#pragma unroll 4
+        for (int z = 0; z < P.Z; ++z) sum += *reinterpret_cast<const f32x4*>(src + z * zstride);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) turned[ci_l + e][co_l] = sum[e];
+    __syncthreads();
+    const int row = threadIdx.x >> 4, col = (threadIdx.x & 15) * 4;
+    const int ci = ci0 + row, co = co0 + col;
+    if (ci >= P.Ci || co >= P.Co) return;
+    const f32x4 v = *reinterpret_cast<const f32x4*>(&turned[row][col]);
+    const float out[4] = {v[0], v[1], v[2], v[3]};
+    const int kh = tap / P.Kw, kw = tap - kh * P.Kw;
+    TS* dst = static_cast<TS*>(P.dw) + r * P.wcs + co + ci * P.si + kh * P.skh + kw * P.skw;
+    if (co + 4 <= P.Co) {
+        store_pixels<TS, 4>(dst, out);
+    } else {
+        for (int e = 0; co + e < P.Co; ++e) stf<TS>(dst + e, out[e]);
+    }
+}
+
 }  // namespace phx

@@ -26,6 +26,14 @@ int launch_wgrad_f32(bool half_storage, bool vec, int mode, const WgradArgs& a, 
 }
 
 int launch_reduce_wgrad(bool half_storage, const ReduceArgs& a, hipStream_t st) {
+    // (a thread of this form adds all partials of its outputs: it needs workgroups of its own for every CU, which few outputs
+    // with many partials do not give it)
+    const long tiles = 4L * a.Kh * a.Kw * ((a.Co + REDUCE_CO - 1) / REDUCE_CO) * ((a.Ci + REDUCE_CI - 1) / REDUCE_CI);
+    if (a.so == 1 && a.si != 1 && tiles >= 512 && tiles < (1L << 31)) {
+        if (half_storage) hipLaunchKernelGGL((reduce_wgrad_turned_kernel<_Float16>), dim3((unsigned int)tiles, grid_rows(a.groups)), dim3(WG_THREADS), 0, st, a);
+        else hipLaunchKernelGGL((reduce_wgrad_turned_kernel<float>), dim3((unsigned int)tiles, grid_rows(a.groups)), dim3(WG_THREADS), 0, st, a);
+        return 0;
+    }
     const long groups = 4L * a.Kh * a.Kw * a.Co * ((a.Ci + 3) / 4);
     const int per_wg = WG_THREADS / reduce_slices(a.Z);
     const int blocks = (int)((groups + per_wg - 1) / per_wg);
