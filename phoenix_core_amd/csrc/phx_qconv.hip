@@ -984,6 +984,7 @@ static bool nhwc_native(const Problem& p, int pass) {
 // reduction -- Dense layers on a few hundred rows, deep pointwise layers on small batches -- run as Z slices of the
 // reduced channels in one launch and a pass that adds the partial tensors.  Z = the largest power of two that keeps at
 // least 32 channels (a multiple of 16) and 8 steps of 16 channels per slice and at most one item per CU; at least 4.
+static bool fp32_sliced(const Problem& p, const Corr& creal);
 static int nhwc_slices(const Problem& p, int map) {
     if (tune().kslices == 0) return 0;
     const int cin = map == MAP_FWD ? p.ci : p.co, cout = map == MAP_FWD ? p.co : p.ci;
@@ -994,6 +995,7 @@ static int nhwc_slices(const Problem& p, int map) {
     const int steps = cdiv(cin, 16);
     int Z = 1;
     while (fits(2 * Z) && items * 2 * Z <= 256 && steps / (2 * Z) >= 8) Z *= 2;
+    if (!fp16_arithmetic(p, map_pass(map)) && !fp32_sliced(p, map == MAP_FWD ? corr_forward(p) : corr_dgrad(p))) return 0;
     return Z >= 4 ? Z : 0;
 }
 
@@ -1866,12 +1868,11 @@ static Problem band_problem(const Problem& p, const TapBand& t, long& tap_offset
 // and at most two workgroups per CU in flight; 0 = the pass runs unsliced (enough workgroups already; groups and
 // real-valued input are never sliced).  The unit-stride problem on a subsampled copy (strided pointwise forward) and
 // the phases of a strided input gradient are passes of their own and sliced as such (do_fwd, phase_slices).
-static int slices_rule(const Problem& p, int pass, const Corr& creal) {
+static int slices_on(int mode, bool f16, const Corr& creal) {
     Corr c;
     FwdPlan pl;
     int pw = 0;
-    const bool f16 = use_f16_mfma(p);
-    if (!plan_corr(creal, corr_mode(p, pass), f16, c, pl, pw)) return 0;
+    if (!plan_corr(creal, mode, f16, c, pl, pw)) return 0;
     const int red = creal.Cin;
     const auto fits = [&](int z) { return red % z == 0 && (red / z) % 16 == 0 && red / z >= 32; };
     if (tune().kslices > 1) return fits(tune().kslices) ? tune().kslices : 0;
@@ -1892,6 +1893,16 @@ static int slices_rule(const Problem& p, int pass, const Corr& creal) {
     // 35 -> 43; in fp32 arithmetic they always do: 570 -> 410)
     if (f16 && !pl.pwx && Z == 2 && wgs <= cus / 2) return 2;
     return Z >= (f16 ? 4 : 2) ? Z : 0;
+}
+
+// The partial tensors have the caller's type, so a sliced fp16 pass is rounded twice: with N(0,1) operands the 2-norm error
+// against fp64 is 1.41 times that of an unsliced pass, however many the slices.  fp32 arithmetic on fp16 tensors is therefore
+// sliced only where its plan for the fp32 matrix instructions would be: the faster unit brings no rounding with it.
+static bool fp32_sliced(const Problem& p, const Corr& creal) { return slices_on(p.mode, false, creal) != 0; }
+
+static int slices_rule(const Problem& p, int pass, const Corr& creal) {
+    if (use_f16_mfma(p) && !fp16_arithmetic(p, pass) && !fp32_sliced(p, creal)) return 0;
+    return slices_on(corr_mode(p, pass), use_f16_mfma(p), creal);
 }
 
 static bool nhwc_window_native(const Problem& p, int pass);
