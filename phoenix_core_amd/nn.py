@@ -334,24 +334,34 @@ class QBatchNorm2d(nn.Module):
         if self.training:
             return _QBatchNormFn.apply(x.contiguous(), None if residual is None else residual.contiguous(), self.weight,
                                        self.bias, self.running_mean, self.running_var, self.eps, self.momentum, self.relu)
-        if self._eval_on_kernel(x, residual):
-            return ops.batch_norm_eval(x, self.weight, self.bias, self.running_mean, self.running_var, self.eps, self.relu,
-                                       residual)
-        y = nn.functional.batch_norm(x, self.running_mean, self.running_var, self.weight, self.bias, False, 0.0, self.eps)
+        own = (self.weight, self.bias, self.running_mean, self.running_var)
+        if self._eval_on_kernel(x, residual, own):
+            return ops.batch_norm_eval(x, *own, self.eps, self.relu, residual)
+        y = nn.functional.batch_norm(x, own[2], own[3], own[0], own[1], False, 0.0, self.eps)
         if residual is not None:
             y = y + residual
         return torch.relu(y) if self.relu else y
 
-
-    def _eval_on_kernel(self, x, residual):
-        own = (self.weight, self.bias, self.running_mean, self.running_var)
-        if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, residual, self.weight, self.bias)):
+    @staticmethod
+    def _eval_on_kernel(x, residual, own):
+        # The kernel reads plain tensors' memory: what traces, batches or differentiates through operators (graph
+        # capture by fx, jit or compile, vmap, forward mode, dispatch modes and tensor subclasses) sees torch's own.
+        if type(x) is not torch.Tensor or not x.is_cuda or x.dtype not in (torch.float32, torch.float16):
             return False
-        if not (x.is_cuda and x.is_contiguous() and x.dim() >= 2 and x.shape[1] == self.weight.numel() and
-                x.dtype in (torch.float32, torch.float16) and all(t.dtype == torch.float32 and t.device == x.device for t in own)):
+        if (torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None or
+                torch._C._is_tracing() or torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0):
             return False
-        return residual is None or (residual.shape == x.shape and residual.dtype == x.dtype and residual.device == x.device and
-                                    residual.is_contiguous())
+        grad, device = torch.is_grad_enabled(), x.device
+        if x.dim() < 2 or not x.is_contiguous() or (grad and x.requires_grad):
+            return False
+        c = x.shape[1]
+        for t in own:
+            if (type(t) not in (torch.Tensor, nn.Parameter) or t.dtype != torch.float32 or t.device != device or
+                    t.numel() != c or not t.is_contiguous() or (grad and t.requires_grad)):
+                return False
+        return residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape and residual.dtype == x.dtype and
+                                    residual.device == device and residual.is_contiguous() and
+                                    not (grad and residual.requires_grad))
 
 
 class _QMaxPoolFn(torch.autograd.Function):

@@ -135,3 +135,20 @@ def test_evaluation_pass(shape, dtype, relu, residual):
         yg = mod(xg, res.cuda()) if residual else mod(xg)
         yg.sum().backward()
         assert torch.isfinite(xg.grad).all()
+
+
+def test_evaluation_under_transforms():
+    """What batches, differentiates forward or traces through the evaluation mode sees torch's operators: the kernel,
+    which reads memory, would drop tangents and freeze a trace."""
+    gen = torch.Generator().manual_seed(5)
+    mod = phx.QBatchNorm2d(3, relu=False).cuda().eval().requires_grad_(False)
+    mod.running_mean.copy_(torch.randn(3, generator=gen))
+    mod.running_var.copy_(torch.rand(3, generator=gen) + 0.5)
+    x, t = (torch.randn((2, 5, 3, 4, 4), generator=gen).cuda() for _ in range(2))
+    want = torch.stack([mod(v) for v in x])
+    scale = (mod.weight / (mod.running_var + mod.eps).sqrt()).view(1, 3, 1, 1)
+    assert torch.allclose(torch.func.vmap(mod)(x), want, rtol=1e-5, atol=1e-6)
+    y, dy = torch.func.jvp(mod, (x[0],), (t[0],))
+    assert torch.allclose(y, want[0], rtol=1e-5, atol=1e-6) and torch.allclose(dy, scale * t[0], rtol=1e-5, atol=1e-6)
+    assert torch.allclose(torch.jit.trace(mod, x[0])(x[1]), want[1], rtol=1e-5, atol=1e-6)
+    assert torch.allclose(torch.fx.symbolic_trace(mod, {"residual": None})(x[1]), want[1], rtol=1e-5, atol=1e-6)
