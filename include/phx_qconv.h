@@ -230,6 +230,23 @@ int phx_qconv2d_bwd_data_add(const phx_qconv_desc* desc, phx_stream_t stream, co
                              const void* packed_bwd_data_or_null, size_t packed_bwd_data_bytes, const void* addend, void* dx,
                              void* workspace, size_t workspace_bytes);
 
+/* Forward pass with an evaluation-mode batch norm, a residual and a ReLU behind it:
+ * y = gamma * (conv(x, w) (+ bias) - mean) / sqrt(var + eps) + beta (+ residual), then the optional ReLU; the parameters are
+ * per output channel (the four components share them), the residual is laid out like y and is not y itself.  No counterpart
+ * in the reference's interface; it is what a network in evaluation mode does next with a convolution's result, and saves that
+ * pass over it: the fp16 kernels normalise in fp32 what they store, every other path is followed by the pass of
+ * phx_bn_fwd_eval.  NCHW quaternion descriptors; packed_fwd_or_null, workspace as phx_qconv2d_fwd_prepacked /
+ * phx_qconv2d_fwd; limits of phx_bn_fwd_eval. */
+typedef struct phx_output_norm {
+    const float *gamma, *beta, *mean, *var;
+    const void* residual_or_null;
+    float eps;
+    int32_t relu;
+} phx_output_norm;
+int phx_qconv2d_fwd_norm(const phx_qconv_desc* desc, phx_stream_t stream, const void* x, const void* w,
+                         const void* packed_fwd_or_null, size_t packed_fwd_bytes, const void* bias_or_null,
+                         const phx_output_norm* norm, void* y, void* workspace, size_t workspace_bytes);
+
 /* Dense trio.  Replaces UpstrideDenseFunctor / UpstrideDenseGradFunctor for the quaternion
  * algebra (src/dense.hpp:52-62, 77-180, 223-237, 252-377). */
 int phx_qdense_fwd(const phx_qdense_desc* desc, phx_stream_t stream, const void* x, const void* w,

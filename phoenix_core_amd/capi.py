@@ -32,7 +32,7 @@ EXPORTS = (
     "phx_init", "phx_tuning_reload", "phx_plan_cache_stats", "phx_qconv2d_fwd_noalloc",
     "phx_qconv2d_packed_filter_bytes", "phx_qconv2d_pack_filters", "phx_qconv2d_fwd_prepacked",
     "phx_qconv2d_bwd_data_prepacked",
-    "phx_qconv2d_bwd_data_add",
+    "phx_qconv2d_bwd_data_add", "phx_qconv2d_fwd_norm",
 )
 
 
@@ -47,6 +47,10 @@ EXPORTS_POOL = ("phx_maxpool3x3s2_fwd", "phx_maxpool3x3s2_bwd")
 class BnDesc(ctypes.Structure):
     _fields_ = [("dtype", ctypes.c_int32), ("rows", ctypes.c_int32), ("c", ctypes.c_int32), ("hw", ctypes.c_int32),
                 ("eps", ctypes.c_float), ("momentum", ctypes.c_float), ("relu", ctypes.c_int32)]
+
+
+class OutputNorm(ctypes.Structure):
+    _fields_ = [(k, ctypes.c_void_p) for k in ("gamma", "beta", "mean", "var", "residual")] + [("eps", ctypes.c_float), ("relu", ctypes.c_int32)]
 
 
 class QConvDesc(ctypes.Structure):
@@ -96,6 +100,7 @@ def lib():
         L.phx_qconv2d_fwd_prepacked.argtypes = [cd, vp, vp, vp, sz, vp, vp, vp, sz]
         L.phx_qconv2d_bwd_data_prepacked.argtypes = [cd, vp, vp, vp, sz, vp, vp, sz]
         L.phx_qconv2d_bwd_data_add.argtypes = [cd, vp, vp, vp, vp, sz, vp, vp, vp, sz]
+        L.phx_qconv2d_fwd_norm.argtypes = [cd, vp, vp, vp, vp, sz, vp, ctypes.POINTER(OutputNorm), vp, vp, sz]
         L.phx_qconv2d_bwd_weights.argtypes = [cd, vp, vp, vp, vp, vp, sz]
         L.phx_qdense_fwd.argtypes = [dd, vp, vp, vp, vp, vp, vp, sz]
         L.phx_qdense_bwd_data.argtypes = [dd, vp, vp, vp, vp, vp, sz]

@@ -338,6 +338,16 @@ static void launch_eval(const BnEvalArgs& a, hipStream_t st) {
     else hipLaunchKernelGGL((bn_eval_kernel<TS, false>), grid, dim3(256), lds, st, a);
 }
 
+int bn_eval_status(const phx_bn_desc* d) {
+    if ((d->dtype != PHX_F32 && d->dtype != PHX_F16) || d->rows < 0 || d->c <= 0 || d->hw < 0 || !(d->eps >= 0.f))
+        return PHX_ERR_INVALID_ARGUMENT;
+    if (d->rows == 0 || d->hw == 0) return PHX_OK;
+    // (the kernel multiplies a run's plane numbers by hw in 32 bits; a launch has fewer than 2^32 threads)
+    const long run = 256L * BN_EVAL_CHUNKS * (d->dtype == PHX_F16 ? Vec<_Float16>::N : Vec<float>::N);
+    if (d->hw >= 1 << 30 || (long)d->rows * d->c > (run << 24) / d->hw - 1) return PHX_ERR_NOT_SUPPORTED;
+    return PHX_OK;
+}
+
 static int plan(const phx_bn_desc* d, BnArgs& a) {
     if (!d || (d->dtype != PHX_F32 && d->dtype != PHX_F16) || d->rows < 0 || d->c <= 0 || d->hw < 0 || !(d->eps > 0.f))
         return PHX_ERR_INVALID_ARGUMENT;
@@ -398,13 +408,10 @@ int phx_bn_fwd_train(const phx_bn_desc* desc, phx_stream_t stream, const void* x
 
 int phx_bn_fwd_eval(const phx_bn_desc* desc, phx_stream_t stream, const void* x, const void* residual_or_null,
                     const float* gamma, const float* beta, const float* running_mean, const float* running_var, void* y) {
-    if (!desc || (desc->dtype != PHX_F32 && desc->dtype != PHX_F16) || desc->rows < 0 || desc->c <= 0 || desc->hw < 0 || !(desc->eps >= 0.f))
-        return PHX_ERR_INVALID_ARGUMENT;
-    if (desc->rows == 0 || desc->hw == 0) return PHX_OK;
+    if (!desc) return PHX_ERR_INVALID_ARGUMENT;
+    if (desc->rows >= 0 && desc->c > 0 && (desc->rows == 0 || desc->hw == 0)) return bn_eval_status(desc);
     if (!x || !gamma || !beta || !running_mean || !running_var || !y) return PHX_ERR_INVALID_ARGUMENT;
-    // (the kernel multiplies a run's plane numbers by hw in 32 bits; a launch has fewer than 2^32 threads)
-    const long run = 256L * BN_EVAL_CHUNKS * (desc->dtype == PHX_F16 ? Vec<_Float16>::N : Vec<float>::N);
-    if (desc->hw >= 1 << 30 || (long)desc->rows * desc->c > (run << 24) / desc->hw - 1) return PHX_ERR_NOT_SUPPORTED;
+    if (const int rc = bn_eval_status(desc)) return rc;
     BnEvalArgs a{x, residual_or_null, y, gamma, beta, running_mean, running_var, (long)desc->rows * desc->c * desc->hw,
                  desc->c, desc->hw, desc->eps, desc->relu};
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -575,7 +575,8 @@ __device__ __forceinline__ void lane_step(const f16x8 (&x)[4], f16x8 (&L)[8], in
 // start of the group, ahead of the filter copy (which the same wait then covers).
 // XREAL (16-product, chunk staging): the input holds its real component only (P.in.ncomp == 1); the twelve
 // products with the absent components and their operand reads are left out at compile time.
-template <int MODE, int WCO, int NTW, int P2LOG, bool CHUNKS, bool EARLY = false, bool XREAL = false>
+// NORM (planes only): P.norm is applied to what is stored.
+template <int MODE, int WCO, int NTW, int P2LOG, bool CHUNKS, bool EARLY = false, bool XREAL = false, bool NORM = false>
 __global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) qconv_fwd_f16_lds_kernel(const ConvArgs P0) {
     const ConvArgs P = group_view(P0);
     static_assert(!EARLY || CHUNKS, "early activation requests belong to chunk staging");
@@ -607,6 +608,11 @@ __global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) 
     bid /= P.tiles_w;
     const int th = bid % P.tiles_h;
     const int tn = bid / P.tiles_h;
+    f32x4 channel_factors = {};  // of channel tid of the tile: formed under the first loads, shared in front of the epilogue
+    if constexpr (NORM) {
+        const int co = ct * WCO * 32 + tid;
+        if (tid < 32 * WCO && co < P.Cout) channel_factors = norm_factors(P.norm, co);
+    }
     const int n0 = tn * P.NB, ho0 = th * P.TH, wo0 = tw * P.TW;
     int h0 = ho0 * P.sh - P.pt;
     const int w0 = wo0 * P.sw - P.pl;
@@ -860,7 +866,13 @@ __global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) 
         if (++g == ngroups) { g = 0; ++chunk; }
     }
 
-    if (CHUNKS && P.nhwc) conv_epilogue_cl<MODE, NTW, NW>(P, acc, (ct * WCO + wco) * 32, oaddr, pvalid);
+    if constexpr (NORM) {
+        f32x4* const factors = reinterpret_cast<f32x4*>(xl);  // (the staged window, which nobody reads any more)
+        __syncthreads();
+        if (tid < 32 * WCO) factors[tid] = channel_factors;
+        __syncthreads();
+        conv_epilogue<_Float16, MODE, NTW, NW, true>(P, acc, (ct * WCO + wco) * 32 + 4 * kk, oaddr, pvalid, factors + wco * 32 + 4 * kk);
+    } else if (CHUNKS && P.nhwc) conv_epilogue_cl<MODE, NTW, NW>(P, acc, (ct * WCO + wco) * 32, oaddr, pvalid);
     else conv_epilogue<_Float16, MODE, NTW, NW>(P, acc, (ct * WCO + wco) * 32 + 4 * kk, oaddr, pvalid);
 #ifdef PHX_PHASE_TIMING
     __builtin_amdgcn_s_waitcnt(0x0F70);  // (charge the stores to the epilogue; otherwise the wave ends with them in flight)

@@ -14,6 +14,23 @@ constexpr int F16_CK = 16;  // fp16 MFMA: input channels per K chunk = one MFMA 
 constexpr int F16_TG = 3;   // fp16 MFMA, LDS-staged filters: taps per filter group
 constexpr int F16_XPITCH = 256;  // fp16 LDS kernels with chunk staging: entries per unit of the staged window
 
+// Evaluation-mode batch norm (+ residual, ReLU) of what a pass stores: y = gamma / sqrt(var + eps) * (y - mean) + beta
+// per output channel, then + residual (a tensor laid out like the output), then the ReLU.  gamma null: none.
+struct NormArgs {
+    const float *gamma, *beta, *mean, *var;  // [output channels]
+    const void* res;                         // or null
+    float eps;
+    int relu;
+};
+
+// a channel's factors, in the form in which the evaluation pass of its own (bn_eval_kernel) applies them
+__device__ __forceinline__ f32x4 norm_factors(const NormArgs& n, int c) {
+    return f32x4{n.gamma[c] / sqrtf(n.var[c] + n.eps), n.mean[c], n.beta[c], 0.f};
+}
+// (the mean is taken off first: a scaled mean folded into beta would cancel against a large x)
+__device__ __forceinline__ float norm_apply(const f32x4& f, float v) { return f[0] * (v - f[1]) + f[2]; }
+__device__ __forceinline__ float relu_if(int relu, float v) { return (relu && v < 0.f) ? 0.f : v; }  // (NaN stays)
+
 struct ConvArgs {
     TileSrc in;         // x (forward) or the output gradient (input-gradient pass)
     const void* wpk;    // packed filters (see the pack_filters kernels), in the MFMA operand type
@@ -35,6 +52,7 @@ struct ConvArgs {
     int nhwc;           // the output is channels-last, out[4][N][Hout][Wout][CoutS] (fp16 chunk-staging kernel only)
     int groups;         // grid rows: the groups of a grouped convolution run by this one launch (1 otherwise)
     long g_in, g_w, g_bias, g_out;  // bytes from one group's input / packed filters / bias / output to the next group's
+    NormArgs norm;      // NORM instances only
 };
 
 // the arguments as group blockIdx.y sees them
@@ -98,9 +116,23 @@ __device__ __forceinline__ void store_pixels(TS* ptr, const float (&v)[V]) {
     }
 }
 
-template <typename TS, int MODE, int NTW, int NACC>
+// what follows the normalisation of V consecutive elements of the output at element offset `at`: residual and ReLU
+template <typename TS, int V>
+__device__ __forceinline__ void norm_tail(const ConvArgs& P, long at, float (&o)[V]) {
+    if (P.norm.res) {
+        typedef TS tv __attribute__((ext_vector_type(V), aligned(sizeof(TS))));
+        const tv r = *reinterpret_cast<const tv*>(static_cast<const TS*>(P.norm.res) + at);
+#pragma unroll
+        for (int i = 0; i < V; ++i) o[i] += (float)r[i];
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) o[i] = relu_if(P.norm.relu, o[i]);
+}
+
+// NORM: P.norm is applied in fp32, in front of the one rounding; factors[i] belongs to channel co_base + i.
+template <typename TS, int MODE, int NTW, int NACC, bool NORM = false>
 __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&acc)[NTW][NACC], int co_base,
-                                              const long (&oaddr)[NTW], const bool (&pvalid)[NTW]) {
+                                              const long (&oaddr)[NTW], const bool (&pvalid)[NTW], const f32x4* factors = nullptr) {
     TS* out = static_cast<TS*>(P.out);
     const TS* bias = static_cast<const TS*>(P.bias);
     const long plane = (long)P.Hout * P.Wout;
@@ -130,6 +162,11 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
 #pragma unroll
                     for (int q = 0; q < 4; ++q) y[k][q] += ldf<TS>(bias + q * P.CoutS + co);
                 }
+                if constexpr (NORM) {
+                    const f32x4 f = factors[8 * rq + k];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) y[k][q] = norm_apply(f, y[k][q]);
+                }
             }
             if (P.vec == 4) {
                 const int co = co_base + 8 * rq + ql;
@@ -138,6 +175,9 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
                     const float a[4] = {y[0][q], y[1][q], y[2][q], y[3][q]};
                     float o[4];
                     quad_transpose(a, o, ql);
+                    if constexpr (NORM) {
+                        if (co < P.Cout) norm_tail<TS, 4>(P, q * P.out_cs + (oaddr[t] - ql) + co * plane, o);
+                    }
                     if (co < P.Cout) store_pixels<TS, 4>(out + q * P.out_cs + (oaddr[t] - ql) + co * plane, o);
                 }
             } else if (P.vec == 2) {
@@ -149,6 +189,10 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
                     pair_transpose(a, b, d, odd);
                     const int co = co_base + 8 * rq + odd;
                     TS* dst = out + q * P.out_cs + (oaddr[t] - odd);
+                    if constexpr (NORM) {
+                        if (co < P.Cout) norm_tail<TS, 2>(P, dst - out + co * plane, b);
+                        if (co + 2 < P.Cout) norm_tail<TS, 2>(P, dst - out + (co + 2) * plane, d);
+                    }
                     if (co < P.Cout) store_pixels<TS, 2>(dst + co * plane, b);
                     if (co + 2 < P.Cout) store_pixels<TS, 2>(dst + (co + 2) * plane, d);
                 }
@@ -158,8 +202,11 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
                     const int co = co_base + 8 * rq + k;
                     if (co < P.Cout) {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            stf<TS>(out + q * P.out_cs + oaddr[t] + co * plane, y[k][q]);
+                        for (int q = 0; q < 4; ++q) {
+                            float o[1] = {y[k][q]};
+                            if constexpr (NORM) norm_tail<TS, 1>(P, q * P.out_cs + oaddr[t] + co * plane, o);
+                            stf<TS>(out + q * P.out_cs + oaddr[t] + co * plane, o[0]);
+                        }
                     }
                 }
             }

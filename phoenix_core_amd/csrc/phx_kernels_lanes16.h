@@ -35,6 +35,7 @@ namespace phx {
 constexpr int LANES_UPITCH = 265;             // 16-byte entries
 constexpr int LANES_BUF = 16 * LANES_UPITCH;  // one chunk: 4 waves x 2 lanes x 2 packs of 8 channels
 constexpr int LANES_LDS_BYTES = 8 * 128 * 36 * 4;  // the epilogue's exchange (channels-last) is larger than the two buffers
+constexpr int LANES_NORM_BYTES = 64 * 16;      // behind it: the factors of the tile's channels (NORM)
 static_assert(2 * LANES_BUF * 16 <= LANES_LDS_BYTES && 8 * 32 * (128 + 4) * 4 <= LANES_LDS_BYTES, "LDS of the lanes kernel");
 constexpr int LANES_STEP = 256;               // 16-byte vectors of one wave's filter operands per tap: [lane][sub-tile][64]
 constexpr int LANES_GROUP = 3;                // taps per group = taps in a filter register ring
@@ -51,7 +52,8 @@ inline size_t lanes_packed_bytes(int co_tiles, int nchunks, int taps3) {
 // a / b for 0 <= a < 2^20 and the reciprocal of 1 <= b < 2^20
 __device__ __forceinline__ int small_div(int a, float rcp_b) { return (int)(((float)a + 0.5f) * rcp_b); }
 
-template <int NPT, bool CL>
+// NORM (planes only): P.norm is applied to what is stored.
+template <int NPT, bool CL, bool NORM = false>
 __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(const ConvArgs P0) {
     const ConvArgs P = group_view(P0);
     constexpr int TG = LANES_GROUP;
@@ -73,6 +75,10 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
     const int tn = bid / P.tiles_h;
     // Origin of the tile; flat tiling (P.in.tall, see qconv_fwd_f16_lds_kernel): position q0 of the tall image is column
     // c0 of row y0 of image n0.
+    f32x4* const factors = reinterpret_cast<f32x4*>(lds16 + LANES_LDS_BYTES / 16);  // (formed in front of the first barrier, read in the epilogue)
+    if constexpr (NORM) {
+        if (tid < 64) factors[tid] = ct * 64 + tid < P.Cout ? norm_factors(P.norm, ct * 64 + tid) : f32x4{};
+    }
     const bool tall = P.in.tall != 0;
     const int q0 = th * PX, R0 = tall ? q0 / P.Wout : 0;
     const int n0 = tall ? R0 / P.in.tall : tn * P.NB;
@@ -470,6 +476,33 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
                     for (int e = 0; e < 8; ++e) c[e][q] += (float)bias[q * P.CoutS + co + (CL ? e : 0)];
+            }
+            if constexpr (NORM && !CL) {
+                const f32x4 f = factors[s * 32 + r];
+                const _Float16* const res = static_cast<const _Float16*>(P.norm.res);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) c[e][q] = norm_apply(f, c[e][q]);
+                    if (res) {
+                        f16x8 rv = {};
+                        const long at = q * P.out_cs + co * plane_out;
+                        if (run8) {
+                            rv = __builtin_bit_cast(f16x8, load16_a2(res + at + o8[0]));
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) {
+                                int off;
+                                long o;
+                                if (decode(g8 * 8 + e, off, o)) rv[e] = res[at + o];
+                            }
+                        }
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) c[e][q] += (float)rv[e];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) c[e][q] = relu_if(P.norm.relu, c[e][q]);
+                }
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q)

@@ -45,11 +45,11 @@ __device__ __forceinline__ float agpr_value(float a) {
     return r;
 }
 
-// ADD: the instance that adds P.addend (a tensor laid out like the output; an fp16 addition to the rounded result)
-// to what it stores.
-template <int WCO, bool ADD = false>
+// TAIL: what is done to the results on their way out (PWX_PLAIN ...); P.addend is a tensor laid out like the output.
+template <int WCO, int TAIL = PWX_PLAIN>
 __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxArgs P0) {
     const PwxArgs P = group_view(P0);
+    constexpr bool ADD = TAIL == PWX_ADD || TAIL == PWX_NORM_ADD, NORM = TAIL >= PWX_NORM;
     extern __shared__ f16x8 lds16[];  // filters [K step][sub-tile][component][lane], then the waves' rings
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -188,6 +188,8 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
         for (int wc = 0; wc < NCO; ++wc) {
             const int co = (w0 + wc) * 32 + j;
             const bool co_ok = co < P.Cout;
+            f32x4 factors;
+            if constexpr (NORM) factors = norm_factors(P.norm, co_ok ? co : 0);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 __builtin_amdgcn_sched_barrier(0);  // (one tile at a time leaves the accumulator file)
@@ -206,8 +208,13 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
                         f16x2 h;
-                        h[0] = (_Float16)(agpr_value(acc[wc][q][4 * g + 2 * i]) + bv);
-                        h[1] = (_Float16)(agpr_value(acc[wc][q][4 * g + 2 * i + 1]) + bv);
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            float v = agpr_value(acc[wc][q][4 * g + 2 * i + e]) + bv;
+                            if constexpr (NORM) v = norm_apply(factors, v);
+                            if constexpr (NORM && !ADD) v = relu_if(P.norm.relu, v);
+                            h[e] = (_Float16)v;
+                        }
                         d[g][i] = __builtin_bit_cast(unsigned int, h);
                     }
 #pragma unroll
@@ -220,6 +227,9 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
                         v[2 + i] = s[1];
                     }
                     if constexpr (ADD) v = add_halves(v, ad[a]);
+                    if constexpr (ADD && NORM) {
+                        if (P.norm.relu) v = u32x4{relu_pair(v[0]), relu_pair(v[1]), relu_pair(v[2]), relu_pair(v[3])};
+                    }
                     if (ovalid[a] && co_ok) *reinterpret_cast<u32x4_a2*>(dst + oaddr[a]) = v;
                 }
             }

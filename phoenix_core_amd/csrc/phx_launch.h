@@ -2,6 +2,7 @@
 // instantiate the kernel templates (split so that they compile in parallel).
 #pragma once
 
+#include "../../include/phx_bn.h"
 #include "../../include/phx_qconv.h"
 #include "phx_kernels_f32.h"
 #include "phx_kernels_realx.h"
@@ -43,6 +44,8 @@ struct FwdVariant {
 int launch_pack_filters(const FwdVariant& v, const PackArgs& a, int blocks, hipStream_t st);
 int launch_fwd_f32(const FwdVariant& v, const ConvArgs& a, hipStream_t st);
 int launch_fwd_f16(const FwdVariant& v, const ConvArgs& a, hipStream_t st);
+bool fwd_f16_takes_norm(const FwdVariant& v, const ConvArgs& a);  // whether launch_fwd_f16_norm has an instance
+int launch_fwd_f16_norm(const FwdVariant& v, const ConvArgs& a, hipStream_t st);
 int launch_fwd_f16_lds8(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // 8-product, filters through LDS
 int launch_fwd_f16_lanes(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // 8-product, lanes dealt over the waves
 size_t lanes_lds_bytes();
@@ -143,6 +146,9 @@ struct ThinArgs {
 int launch_thin(bool half_storage, int pass, const ThinArgs& a, hipStream_t st);
 int thin_wgrad_slices(bool half_storage, const ThinArgs& a);  // Z of the filter gradient (sizes `partial`)
 
+// whether phx_bn_fwd_eval takes the descriptor (phx_bn.hip)
+int bn_eval_status(const phx_bn_desc* d);
+
 // space-to-depth rearrangements (stride-2 convolutions with very few input channels)
 int launch_s2d_input(bool half_storage, const S2dArgs& a, hipStream_t st);
 int launch_subsample(bool half_storage, const SubsampleArgs& a, hipStream_t st);
@@ -157,9 +163,9 @@ int launch_transpose(bool half_storage, const TransposeArgs& a, hipStream_t st);
 int launch_fill_zero(void* dst, size_t bytes, hipStream_t st);  // a kernel, so that it can be captured in a graph
 int launch_add_inplace(bool half_storage, void* dst, const void* src, long count, hipStream_t st);  // dst += src
 // dst = the sum of `slices` partial tensors of `count` elements (+ bias of the element's channel, + addend); partial results
-// of a pass whose channel reduction was cut into slices
+// of a pass whose channel reduction was cut into slices; then norm, where its gamma is not null
 int launch_slice_sum(bool half_storage, const void* partial, int slices, long count, void* dst, const void* bias, const void* addend,
-                     int plane, int channels, long comp_count, hipStream_t st);
+                     int plane, int channels, long comp_count, const NormArgs& norm, hipStream_t st);
 
 // REAL / COMPLEX / GA_300 as compositions on the quaternion entry points (phx_algebra.hip); pass = phx_pass,
 // (a, b) = (x, w) forward, (grad, w) input gradient, (x, grad) filter gradient

@@ -192,32 +192,38 @@ int launch_add_inplace(bool half_storage, void* dst, const void* src, long count
 // belongs to channel (e / plane) % channels of component e / comp_count; then + addend, element by element, in the storage
 // type): what closes a forward / input-gradient pass whose reduction over the channels was cut into slices.  fp32 sums,
 // one rounding.
-template <typename TS>
+template <typename TS, bool NORM>
 __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial, int slices, long count, TS* dst, const TS* bias,
-                                                               const TS* addend, int plane, int channels, long comp_count) {
+                                                               const TS* addend, int plane, int channels, long comp_count,
+                                                               const NormArgs norm) {
     const long stride = (long)gridDim.x * blockDim.x;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += stride) {
         float acc = 0.0f;
         for (int z = 0; z < slices; ++z) acc += (float)partial[z * count + e];
         if (bias) acc += (float)bias[(e / comp_count) * channels + (e / plane) % channels];
+        if constexpr (NORM) {
+            acc = norm_apply(norm_factors(norm, (int)((e / plane) % channels)), acc);
+            if (norm.res) acc += (float)static_cast<const TS*>(norm.res)[e];
+            acc = relu_if(norm.relu, acc);
+        }
         TS r = (TS)acc;
         if (addend) r = (TS)((float)r + (float)addend[e]);  // (as the separate in-place pass would: the rounded result plus the addend)
         dst[e] = r;
     }
 }
 
+template <typename TS>
+static void slice_sum(const void* partial, int slices, long count, void* dst, const void* bias, const void* addend, int plane, int channels,
+                      long comp_count, const NormArgs& norm, hipStream_t st) {
+    const auto kernel = norm.gamma ? slice_sum_kernel<TS, true> : slice_sum_kernel<TS, false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks_for(count)), dim3(WG_THREADS), 0, st, static_cast<const TS*>(partial), slices, count,
+                       static_cast<TS*>(dst), static_cast<const TS*>(bias), static_cast<const TS*>(addend), plane, channels, comp_count, norm);
+}
+
 int launch_slice_sum(bool half_storage, const void* partial, int slices, long count, void* dst, const void* bias, const void* addend,
-                     int plane, int channels, long comp_count, hipStream_t st) {
+                     int plane, int channels, long comp_count, const NormArgs& norm, hipStream_t st) {
     if (count <= 0) return 0;
-    const int blocks = blocks_for(count);
-    if (half_storage)
-        hipLaunchKernelGGL((slice_sum_kernel<_Float16>), dim3(blocks), dim3(WG_THREADS), 0, st, static_cast<const _Float16*>(partial),
-                           slices, count, static_cast<_Float16*>(dst), static_cast<const _Float16*>(bias),
-                           static_cast<const _Float16*>(addend), plane, channels, comp_count);
-    else
-        hipLaunchKernelGGL((slice_sum_kernel<float>), dim3(blocks), dim3(WG_THREADS), 0, st, static_cast<const float*>(partial), slices,
-                           count, static_cast<float*>(dst), static_cast<const float*>(bias), static_cast<const float*>(addend), plane,
-                           channels, comp_count);
+    (half_storage ? slice_sum<_Float16> : slice_sum<float>)(partial, slices, count, dst, bias, addend, plane, channels, comp_count, norm, st);
     return 0;
 }
 

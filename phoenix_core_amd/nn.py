@@ -349,7 +349,7 @@ class QBatchNorm2d(nn.Module):
         return torch.relu(y) if self.relu else y
 
     @staticmethod
-    def _eval_on_kernel(x, residual, own):
+    def _eval_on_kernel(x, residual, own, channels=None):
         # The kernel reads plain tensors' memory: what traces, batches or differentiates through operators (graph
         # capture by fx, jit or compile, vmap, forward mode, function and dispatch modes, tensor subclasses) sees torch's
         # own.  (is_compiling first: what torch.compile traces must not reach the queries behind it, which it refuses.)
@@ -361,7 +361,8 @@ class QBatchNorm2d(nn.Module):
         grad, device = torch.is_grad_enabled(), x.device
         if x.dim() < 2 or not x.is_contiguous() or (grad and x.requires_grad):
             return False
-        rows, c = x.shape[0], x.shape[1]
+        # (channels: those of the tensor that is normalised where it is not x itself, see _conv_norm)
+        rows, c = x.shape[0], x.shape[1] if channels is None else channels
         # (what its descriptor and its 32-bit indices hold: include/phx_bn.h; an empty tensor is torch's as well)
         if not 0 < x.numel() < min(rows * c << 30, 1 << 34) or rows >= 1 << 31:
             return False
@@ -372,6 +373,42 @@ class QBatchNorm2d(nn.Module):
         return residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape and residual.dtype == x.dtype and
                                     residual.device == device and residual.is_contiguous() and
                                     not (grad and residual.requires_grad))
+
+
+def _hooked(module):
+    d = module.__dict__
+    return d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d
+
+
+def _conv_norm(conv, norm, x, residual=None):
+    """norm(conv(x), residual), as one operator where that can be told from the two by nothing but its rounding: both
+    modules are this file's and unhooked, norm is in evaluation mode, and no gradient is recorded.  (A network in evaluation
+    mode is bound by the host: parameters are taken from the modules' dictionaries, not through Module.__getattr__.)"""
+    if (type(conv) is QConv2d and type(norm) is QBatchNorm2d and not norm.training and not torch.is_grad_enabled() and
+            conv.data_format == "NCHW" and not (_hooked(conv) or _hooked(norm) or torch.nn.modules.module._has_any_global_hook())):
+        cp, np, buffers = conv._parameters, norm._parameters, norm._buffers
+        w, bias = cp.get("weight"), cp.get("bias")
+        own = (np.get("weight"), np.get("bias"), buffers.get("running_mean"), buffers.get("running_var"))
+        if type(w) is nn.Parameter and norm._eval_on_kernel(x, None, own, w.shape[1]):
+            device, dtype = x.device, x.dtype
+            fwd, _ = conv._descriptors(x)
+            shape = fwd.output_shape
+            n4, c, h, wd = shape
+            # (what the operators ask of these tensors, and what the pass behind a convolution that does not normalise what it
+            # stores asks of their sizes)
+            if (x.shape == fwd.input_shape and w.shape == fwd.filter_shape and w.dtype == dtype and w.device == device and
+                    w.is_contiguous() and 0 < n4 * c * h * wd < min(n4 * c << 30, 1 << 34) and
+                    (bias is None or (fwd.use_bias and not fwd.real_valued_input and type(bias) is nn.Parameter and
+                                      bias.shape == fwd.bias_shape and bias.dtype == dtype and bias.device == device and
+                                      bias.is_contiguous())) and
+                    (residual is None or (norm.relu and type(residual) is torch.Tensor and residual.shape == shape and
+                                          residual.dtype == dtype and residual.device == device and residual.is_contiguous()))):
+                packed = conv._packed_filters((tuple(x.shape), dtype), fwd)
+                if packed is not None and packed.fwd is not None:
+                    packed.check(fwd)
+                return ops._conv2d_fwd_norm(device, x, w, bias, fwd, own, norm.eps, norm.relu, residual, packed)
+    y = conv(x)
+    return norm(y) if residual is None else norm(y, residual)
 
 
 class _QMaxPoolFn(torch.autograd.Function):
@@ -412,6 +449,11 @@ class _Bottleneck(nn.Module):
         self.relu = nn.ReLU(inplace=True)
 
     def forward(self, x):
+        if self.fused_bn and not self.training and not torch.is_grad_enabled():
+            m = self._modules
+            y = _conv_norm(m["conv1"], m["bn1"], x)
+            idt = x if m.get("down") is None else self._down(x)
+            return _conv_norm(m["conv3"], m["bn3"], _conv_norm(m["conv2"], m["bn2"], y), idt)
         if self.fused_bn:
             # (conv1 hands x on to the identity branch, see QConv2d.forward: one elementwise pass less per block)
             y, x = self.conv1(x, passthrough=True) if FUSE_BRANCH_GRADIENT else (self.conv1(x), x)
@@ -424,6 +466,13 @@ class _Bottleneck(nn.Module):
         y = self.relu(self.bn2(self.conv2(y)))
         y = self.bn3(self.conv3(y))
         return self.relu(y + idt)
+
+    def _down(self, x):
+        # (a Sequential of other modules, or one with hooks, is called as one)
+        down = self.down
+        if type(down) is not nn.Sequential or len(down._modules) != 2 or _hooked(down) or torch.nn.modules.module._has_any_global_hook():
+            return down(x)
+        return _conv_norm(*down._modules.values(), x)
 
 
 class QResNet50(nn.Module):
@@ -457,7 +506,7 @@ class QResNet50(nn.Module):
         return torch.cat([images, z, z, z], dim=0)
 
     def forward(self, x):
-        y = self.bn(self.stem(x))
+        y = _conv_norm(self.stem, self.bn, x) if self.fused_bn else self.bn(self.stem(x))
         y = self.pool(y if self.fused_bn else self.relu(y))
         y = self.blocks(y)
         y = y.float().mean(dim=(2, 3)).to(x.dtype)            # [4N, 512]

@@ -304,12 +304,14 @@ class PackedFilters:
             raise ValueError("these packed filters belong to another descriptor")
 
 
+_HAS_BIAS = capi.QConvDesc.has_bias
+
+
 def _layout_key(desc):
     """Everything of a descriptor that a packed image depends on: its C struct without the bias flag (the forward
     and backward descriptors of one layer differ in it and share their images) + the tuning generation."""
-    c = capi.QConvDesc.from_buffer_copy(bytes(desc.c))
-    c.has_bias = 0
-    return bytes(c), capi.tuning_generation
+    whole = bytes(desc.c)
+    return whole[:_HAS_BIAS.offset] + whole[_HAS_BIAS.offset + _HAS_BIAS.size:], capi.tuning_generation
 
 
 def conv2d_packed_filter_bytes(desc, which):
@@ -365,6 +367,45 @@ def conv2d_fwd(x, w, bias, desc, out=None, packed=None):
     capi.check(capi.lib().phx_qconv2d_fwd(ctypes.byref(desc.c), _stream(dev), _ptr(x), _ptr(w),
                                           _ptr(bias if desc.use_bias else None), _ptr(y), _ptr(ws), nbytes),
                "phx_qconv2d_fwd")
+    return y
+
+
+def conv2d_fwd_norm(x, w, bias, desc, gamma, beta, running_mean, running_var, eps, relu, residual=None, packed=None):
+    """conv2d_fwd followed by batch_norm_eval of its result (phx_qconv2d_fwd_norm: in the convolution's kernel where it can
+    normalise what it stores, a pass behind it otherwise).  NCHW quaternion descriptors."""
+    dev = _dev_check(x, w, bias, gamma, beta, running_mean, running_var, residual)
+    dtype, shape = desc.dtype, desc.output_shape
+    _expect(x, desc.input_shape, dtype, "input")
+    _expect(w, desc.filter_shape, dtype, "filter")
+    if desc.use_bias:
+        if desc.real_valued_input:
+            raise RuntimeError("Bias addition is not supported for type0 inputs")
+        _expect(bias, desc.bias_shape, dtype, "bias")
+    if residual is not None:
+        _expect(residual, shape, dtype, "residual")
+    for t in (gamma, beta, running_mean, running_var):
+        _expect(t, shape[1:2], torch.float32, "normalisation parameter")
+    if packed is not None and packed.fwd is not None:
+        packed.check(desc)
+    return _conv2d_fwd_norm(dev, x, w, bias, desc, (gamma, beta, running_mean, running_var), eps, relu, residual, packed)
+
+
+def _conv2d_fwd_norm(dev, x, w, bias, desc, own, eps, relu, residual, packed):
+    """conv2d_fwd_norm of tensors that the caller has checked (a network in evaluation mode is bound by these calls)."""
+    y = torch.empty(desc.output_shape, dtype=desc.dtype, device=dev)
+    nbytes = desc.workspace_bytes(capi.PHX_PASS_FWD)
+    stream = current_stream_handle(dev)
+    ws = _workspace.get(dev, nbytes, stream)
+    gamma, beta, mean, var = own
+    norm = capi.OutputNorm(gamma.data_ptr(), beta.data_ptr(), mean.data_ptr(), var.data_ptr(),
+                           None if residual is None else residual.data_ptr(), eps, relu)
+    image = None if packed is None else packed.fwd
+    status = capi.lib().phx_qconv2d_fwd_norm(ctypes.byref(desc.c), stream, x.data_ptr(), w.data_ptr(),
+                                             None if image is None else image.data_ptr(), 0 if image is None else image.numel(),
+                                             bias.data_ptr() if desc.use_bias else None, ctypes.byref(norm), y.data_ptr(),
+                                             ws.data_ptr(), nbytes)
+    if status:
+        raise capi.PhxError(status, "phx_qconv2d_fwd_norm")
     return y
 
 
