@@ -1,0 +1,93 @@
+"""fp32 passes on bf16 instructions (phx_kernels_x3.h) against fp64, beside the fp32 instructions."""
+import ctypes
+
+import pytest
+import torch
+
+import phoenix_core_amd as phx
+from phoenix_core_amd import capi, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _hamilton(x, w, f):
+    xs, out = x.chunk(4), [0, 0, 0, 0]
+    for p in range(4):
+        for q in range(4):
+            out[q] = out[q] + f(xs[p], w[p ^ q]) * (-1 if (0x3950 >> (p * 4 + q)) & 1 else 1)
+    return torch.cat(out)
+
+
+def _gap(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+# n, ci, co, h, w, k, stride, dilation, groups: sub-tiles of 32 and 64 output channels, wide and narrow tiles, flat and
+# rectangular tilings, ragged channels, planes that are one partial group of four, tensors whose ends every load meets
+CASES = [
+    (3, 8, 40, 9, 13, 3, 1, 1, 1), (1, 9, 33, 3, 3, 3, 1, 1, 1), (1, 1, 1, 1, 2, 3, 1, 1, 1), (40, 16, 64, 14, 14, 3, 1, 1, 1),
+    (2, 24, 20, 30, 7, 5, 1, 1, 1), (4, 130, 70, 21, 18, 3, 2, 1, 1), (2, 17, 65, 20, 20, 3, 1, 2, 1), (1, 64, 96, 7, 7, 3, 1, 1, 1),
+    (2, 80, 96, 12, 10, 3, 1, 1, 2), (64, 72, 64, 16, 16, 3, 1, 1, 1), (1, 5, 7, 70, 3, 7, 1, 1, 1),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_error_against_fp64(case, tune_env):
+    n, ci, co, h, w, k, stride, dilation, groups = case
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(4 * n, ci, h, w, generator=gen, device="cuda")
+    wt = torch.randn(4, co, ci // groups, k, k, generator=gen, device="cuda")
+    bias = torch.randn(4, co, generator=gen, device="cuda")
+    args = dict(stride=stride, dilation=dilation, padding="SAME", groups=groups, dtype=torch.float32, context=phx.Context({}))
+    desc, back = ops.Conv2DDescriptor(x.shape, wt.shape, use_bias=True, **args), ops.Conv2DDescriptor(x.shape, wt.shape, **args)
+    grad = torch.randn(desc.output_shape, generator=gen, device="cuda")
+    (pt, pl), (pb, pr) = desc.pad_before, desc.pad_after
+    xr = x.double().requires_grad_()
+    yr = _hamilton(torch.nn.functional.pad(xr, (pl, pr, pt, pb)), wt.double(),
+                   lambda a, b: torch.nn.functional.conv2d(a, b, stride=stride, dilation=dilation, groups=groups))
+    dxr, = torch.autograd.grad(yr, xr, grad.double())
+    yr = yr.detach() + bias.double().view(4, 1, co, 1, 1).expand(4, n, co, 1, 1).reshape(4 * n, co, 1, 1)
+    gaps = {}
+    for nox3 in (None, "1"):
+        tune_env(PHX_TUNE_NOX3=nox3)
+        y = phx.conv2d_fwd(x, wt, bias, desc)
+        names = [capi.last_kernel_name()]
+        dx = ops.conv2d_bwd_data(wt, grad, back)
+        names.append(capi.last_kernel_name())
+        assert ("f32mfmax3" in names[0]) == (nox3 is None), names
+        assert stride > 1 or ("f32mfmax3" in names[1]) == (nox3 is None), names
+        packed = ops.conv2d_pack_filters(wt, desc)
+        if packed is not None:
+            assert torch.equal(y, phx.conv2d_fwd(x, torch.zeros_like(wt), bias, desc, packed=packed))
+            assert torch.equal(dx, ops.conv2d_bwd_data(torch.zeros_like(wt), grad, back, packed=packed))
+        gaps[nox3] = _gap(y, yr), _gap(dx, dxr)
+    # each error is a sum of many roundings of like size: their 2-norms over hundreds of results lie within a tenth of their
+    # expectation; a dozen results, of a dozen roundings of 2^-25 in the mean each, are bounded by those
+    few = min(yr.numel(), xr.numel()) < 500
+    for ours, fp32 in zip(gaps[None], gaps["1"]):
+        assert ours <= 1.1 * fp32 + (2.0 ** -23 if few else 0.0), gaps
+
+
+def test_whole_numbers_are_exact():
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(-300, 301, (8, 16, 12, 12), generator=gen, device="cuda").float()
+    wt = torch.randint(-40, 41, (4, 40, 16, 3, 3), generator=gen, device="cuda").float()
+    desc = ops.Conv2DDescriptor(x.shape, wt.shape, padding="VALID", dtype=torch.float32, context=phx.Context({}))
+    y = phx.conv2d_fwd(x, wt, None, desc)
+    assert "f32mfmax3" in capi.last_kernel_name()
+    assert torch.equal(y.double(), _hamilton(x.double(), wt.double(), torch.nn.functional.conv2d))
+
+
+def test_fixed_scratch_keeps_the_fp32_instructions_where_the_parts_do_not_fit(tune_env):
+    """192 x 192 x 9 filter values: 10.6 MB packed for the fp32 instructions, twice that as three parts."""
+    x, wt = torch.randn(4, 192, 6, 6, device="cuda"), torch.randn(4, 192, 192, 3, 3, device="cuda")
+    desc = ops.Conv2DDescriptor(x.shape, wt.shape, padding="SAME", dtype=torch.float32, context=phx.Context({}))
+    assert desc.workspace_bytes(capi.PHX_PASS_FWD) > capi.PHX_NOALLOC_SCRATCH_BYTES
+    y = torch.empty(desc.output_shape, device="cuda")
+    stream = ops.current_stream_handle(x.device)
+    capi.check(capi.lib().phx_qconv2d_fwd_noalloc(ctypes.byref(desc.c), stream, x.data_ptr(), wt.data_ptr(), None, y.data_ptr()), "noalloc")
+    assert "f32mfmax3" not in capi.last_kernel_name()
+    phx.conv2d_fwd(x, wt, None, desc)
+    assert "f32mfmax3" in capi.last_kernel_name()
+    tune_env(PHX_TUNE_NOX3="1")
+    assert torch.equal(y, phx.conv2d_fwd(x, wt, None, desc))
