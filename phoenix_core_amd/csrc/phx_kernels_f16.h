@@ -575,9 +575,9 @@ __device__ __forceinline__ void lane_step(const f16x8 (&x)[4], f16x8 (&L)[8], in
 // start of the group, ahead of the filter copy (which the same wait then covers).
 // XREAL (16-product, chunk staging): the input holds its real component only (P.in.ncomp == 1); the twelve
 // products with the absent components and their operand reads are left out at compile time.
-// NORM (planes only): P.norm is applied to what is stored.
+// NORM (planes only): P0.norm is applied to what is stored.
 template <int MODE, int WCO, int NTW, int P2LOG, bool CHUNKS, bool EARLY = false, bool XREAL = false, bool NORM = false>
-__global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) qconv_fwd_f16_lds_kernel(const ConvArgs P0) {
+__global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) qconv_fwd_f16_lds_kernel(const ConvArgsOf<NORM> P0) {
     const ConvArgs P = group_view(P0);
     static_assert(!EARLY || CHUNKS, "early activation requests belong to chunk staging");
     static_assert(!XREAL || (MODE == 16 && CHUNKS), "the real-input variant is a 16-product kernel with chunk staging");
@@ -611,7 +611,7 @@ __global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) 
     f32x4 channel_factors = {};  // of channel tid of the tile: formed under the first loads, shared in front of the epilogue
     if constexpr (NORM) {
         const int co = ct * WCO * 32 + tid;
-        if (tid < 32 * WCO && co < P.Cout) channel_factors = norm_factors(P.norm, co);
+        if (tid < 32 * WCO && co < P.Cout) channel_factors = norm_factors(P0.norm, co);
     }
     const int n0 = tn * P.NB, ho0 = th * P.TH, wo0 = tw * P.TW;
     int h0 = ho0 * P.sh - P.pt;
@@ -871,7 +871,7 @@ __global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) 
         __syncthreads();
         if (tid < 32 * WCO) factors[tid] = channel_factors;
         __syncthreads();
-        conv_epilogue<_Float16, MODE, NTW, NW, true>(P, acc, (ct * WCO + wco) * 32 + 4 * kk, oaddr, pvalid, factors + wco * 32 + 4 * kk);
+        conv_epilogue<_Float16, MODE, NTW, NW, true>(P, acc, (ct * WCO + wco) * 32 + 4 * kk, oaddr, pvalid, factors + wco * 32 + 4 * kk, &P0.norm);
     } else if (CHUNKS && P.nhwc) conv_epilogue_cl<MODE, NTW, NW>(P, acc, (ct * WCO + wco) * 32, oaddr, pvalid);
     else conv_epilogue<_Float16, MODE, NTW, NW>(P, acc, (ct * WCO + wco) * 32 + 4 * kk, oaddr, pvalid);
 #ifdef PHX_PHASE_TIMING

@@ -3,6 +3,8 @@
 // formulation.  Storage type TS is float or _Float16 (operands widened while staged into LDS).
 #pragma once
 
+#include <type_traits>
+
 #include "phx_device.h"
 
 namespace phx {
@@ -52,8 +54,13 @@ struct ConvArgs {
     int nhwc;           // the output is channels-last, out[4][N][Hout][Wout][CoutS] (fp16 chunk-staging kernel only)
     int groups;         // grid rows: the groups of a grouped convolution run by this one launch (1 otherwise)
     long g_in, g_w, g_bias, g_out;  // bytes from one group's input / packed filters / bias / output to the next group's
-    NormArgs norm;      // NORM instances only
 };
+
+struct ConvNormArgs : ConvArgs {  // of the NORM instances (the others' calls carry no bytes they do not read: 0.2 us a launch)
+    NormArgs norm;
+};
+template <bool NORM>
+using ConvArgsOf = std::conditional_t<NORM, ConvNormArgs, ConvArgs>;
 
 // the arguments as group blockIdx.y sees them
 __device__ __forceinline__ ConvArgs group_view(const ConvArgs& P0) {
@@ -118,21 +125,22 @@ __device__ __forceinline__ void store_pixels(TS* ptr, const float (&v)[V]) {
 
 // what follows the normalisation of V consecutive elements of the output at element offset `at`: residual and ReLU
 template <typename TS, int V>
-__device__ __forceinline__ void norm_tail(const ConvArgs& P, long at, float (&o)[V]) {
-    if (P.norm.res) {
+__device__ __forceinline__ void norm_tail(const NormArgs& norm, long at, float (&o)[V]) {
+    if (norm.res) {
         typedef TS tv __attribute__((ext_vector_type(V), aligned(sizeof(TS))));
-        const tv r = *reinterpret_cast<const tv*>(static_cast<const TS*>(P.norm.res) + at);
+        const tv r = *reinterpret_cast<const tv*>(static_cast<const TS*>(norm.res) + at);
 #pragma unroll
         for (int i = 0; i < V; ++i) o[i] += (float)r[i];
     }
 #pragma unroll
-    for (int i = 0; i < V; ++i) o[i] = relu_if(P.norm.relu, o[i]);
+    for (int i = 0; i < V; ++i) o[i] = relu_if(norm.relu, o[i]);
 }
 
-// NORM: P.norm is applied in fp32, in front of the one rounding; factors[i] belongs to channel co_base + i.
+// NORM: norm is applied in fp32, in front of the one rounding; factors[i] belongs to channel co_base + i.
 template <typename TS, int MODE, int NTW, int NACC, bool NORM = false>
 __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&acc)[NTW][NACC], int co_base,
-                                              const long (&oaddr)[NTW], const bool (&pvalid)[NTW], const f32x4* factors = nullptr) {
+                                              const long (&oaddr)[NTW], const bool (&pvalid)[NTW], const f32x4* factors = nullptr,
+                                              const NormArgs* norm = nullptr) {
     TS* out = static_cast<TS*>(P.out);
     const TS* bias = static_cast<const TS*>(P.bias);
     const long plane = (long)P.Hout * P.Wout;
@@ -176,7 +184,7 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
                     float o[4];
                     quad_transpose(a, o, ql);
                     if constexpr (NORM) {
-                        if (co < P.Cout) norm_tail<TS, 4>(P, q * P.out_cs + (oaddr[t] - ql) + co * plane, o);
+                        if (co < P.Cout) norm_tail<TS, 4>(*norm, q * P.out_cs + (oaddr[t] - ql) + co * plane, o);
                     }
                     if (co < P.Cout) store_pixels<TS, 4>(out + q * P.out_cs + (oaddr[t] - ql) + co * plane, o);
                 }
@@ -190,8 +198,8 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
                     const int co = co_base + 8 * rq + odd;
                     TS* dst = out + q * P.out_cs + (oaddr[t] - odd);
                     if constexpr (NORM) {
-                        if (co < P.Cout) norm_tail<TS, 2>(P, dst - out + co * plane, b);
-                        if (co + 2 < P.Cout) norm_tail<TS, 2>(P, dst - out + (co + 2) * plane, d);
+                        if (co < P.Cout) norm_tail<TS, 2>(*norm, dst - out + co * plane, b);
+                        if (co + 2 < P.Cout) norm_tail<TS, 2>(*norm, dst - out + (co + 2) * plane, d);
                     }
                     if (co < P.Cout) store_pixels<TS, 2>(dst + co * plane, b);
                     if (co + 2 < P.Cout) store_pixels<TS, 2>(dst + (co + 2) * plane, d);
@@ -204,7 +212,7 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
                             float o[1] = {y[k][q]};
-                            if constexpr (NORM) norm_tail<TS, 1>(P, q * P.out_cs + oaddr[t] + co * plane, o);
+                            if constexpr (NORM) norm_tail<TS, 1>(*norm, q * P.out_cs + oaddr[t] + co * plane, o);
                             stf<TS>(out + q * P.out_cs + oaddr[t] + co * plane, o[0]);
                         }
                     }

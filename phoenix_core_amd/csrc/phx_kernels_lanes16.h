@@ -52,9 +52,9 @@ inline size_t lanes_packed_bytes(int co_tiles, int nchunks, int taps3) {
 // a / b for 0 <= a < 2^20 and the reciprocal of 1 <= b < 2^20
 __device__ __forceinline__ int small_div(int a, float rcp_b) { return (int)(((float)a + 0.5f) * rcp_b); }
 
-// NORM (planes only): P.norm is applied to what is stored.
+// NORM (planes only): P0.norm is applied to what is stored.
 template <int NPT, bool CL, bool NORM = false>
-__global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(const ConvArgs P0) {
+__global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(const ConvArgsOf<NORM> P0) {
     const ConvArgs P = group_view(P0);
     constexpr int TG = LANES_GROUP;
     constexpr int CK = F16_CK;
@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
     // c0 of row y0 of image n0.
     f32x4* const factors = reinterpret_cast<f32x4*>(lds16 + LANES_LDS_BYTES / 16);  // (formed in front of the first barrier, read in the epilogue)
     if constexpr (NORM) {
-        if (tid < 64) factors[tid] = ct * 64 + tid < P.Cout ? norm_factors(P.norm, ct * 64 + tid) : f32x4{};
+        if (tid < 64) factors[tid] = ct * 64 + tid < P.Cout ? norm_factors(P0.norm, ct * 64 + tid) : f32x4{};
     }
     const bool tall = P.in.tall != 0;
     const int q0 = th * PX, R0 = tall ? q0 / P.Wout : 0;
@@ -479,7 +479,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
             }
             if constexpr (NORM && !CL) {
                 const f32x4 f = factors[s * 32 + r];
-                const _Float16* const res = static_cast<const _Float16*>(P.norm.res);
+                const _Float16* const res = static_cast<const _Float16*>(P0.norm.res);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -501,7 +501,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
                         for (int e = 0; e < 8; ++e) c[e][q] += (float)rv[e];
                     }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) c[e][q] = relu_if(P.norm.relu, c[e][q]);
+                    for (int e = 0; e < 8; ++e) c[e][q] = relu_if(P0.norm.relu, c[e][q]);
                 }
             }
 #pragma unroll

@@ -77,13 +77,18 @@ struct PwxArgs {
     int NP;                 // channels-last kernel: pixels in all, N * HW
     int groups;             // grid rows: the groups of a grouped convolution run by this one launch (1 otherwise)
     long g_in, g_w, g_bias, g_out;  // bytes from one group's input / packed filters / bias / output (and addend) to the next group's
-    NormArgs norm;          // NCHW kernels, instances PWX_NORM and PWX_NORM_ADD
+};
+
+struct PwxNormArgs : PwxArgs {  // of the instances PWX_NORM and PWX_NORM_ADD
+    NormArgs norm;
 };
 
 // What is done to a result on its way out: nothing; addend added (fp16, to the rounded result); evaluation-mode batch norm
 // and ReLU; the same with the addend as the residual between the two (the normalised value is rounded in front of the
 // addition, where a pass of its own rounds the convolution's result: the same number of roundings).
 enum { PWX_PLAIN = 0, PWX_ADD = 1, PWX_NORM = 2, PWX_NORM_ADD = 3 };
+template <int TAIL>
+using PwxArgsOf = std::conditional_t<(TAIL >= 2), PwxNormArgs, PwxArgs>;  // (a literal: the name of an unnamed enum's value differs between host and device symbols)
 
 // the ReLU on packed halves; NaN stays
 __device__ __forceinline__ unsigned int relu_pair(unsigned int v) {
@@ -135,7 +140,7 @@ struct PwxShape {
 // TAIL: what is done to the results (the plain instance carries none of that code: the extra
 // registers of the addend's prefetch cost the plain kernel 4 % where both were one)
 template <int WCO, int TAIL = PWX_PLAIN>
-__global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxArgs P0) {
+__global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxArgsOf<TAIL> P0) {
     const PwxArgs P = group_view(P0);
     constexpr bool ADD = TAIL == PWX_ADD || TAIL == PWX_NORM_ADD, NORM = TAIL >= PWX_NORM;
     using S = PwxShape<WCO>;
@@ -349,7 +354,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
         const int co = co0 + j;
         const bool co_ok = co < P.Cout;
         f32x4 factors;
-        if constexpr (NORM) factors = norm_factors(P.norm, co_ok ? co : 0);
+        if constexpr (NORM) factors = norm_factors(P0.norm, co_ok ? co : 0);
         wait_vmem_all();  // this wave's copies of the steps ahead: landed
         PHX_STAMP(2)
         char* scr = reinterpret_cast<char*>(lds16 + RF * WV + RA * XV) + wave * (S::SCRV * 16);  // (TSTORE) this wave's own
@@ -371,7 +376,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
 #pragma unroll
                             for (int e = 0; e < 2; ++e) {
                                 const float v = norm_apply(factors, acc[q][m][g4 * 4 + 2 * k2 + e] + bv);
-                                h[e] = (_Float16)(ADD ? v : relu_if(P.norm.relu, v));
+                                h[e] = (_Float16)(ADD ? v : relu_if(P0.norm.relu, v));
                             }
                         } else if constexpr (BIAS) {
                             h[0] = (_Float16)(acc[q][m][g4 * 4 + 2 * k2] + bv);
@@ -395,7 +400,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
                         if (ov && co_ok) {
                             if constexpr (ADD) v = add_halves4(v, load8_a2(P.addend + q * P.out_cs + (long)co * HW + oa + 4 * kk));
                             if constexpr (ADD && NORM) {
-                                if (P.norm.relu) v = u32x2{relu_pair(v[0]), relu_pair(v[1])};
+                                if (P0.norm.relu) v = u32x2{relu_pair(v[0]), relu_pair(v[1])};
                             }
                             *reinterpret_cast<u32x2_a2*>(dst + oa + 4 * kk) = v;
                         }
@@ -412,7 +417,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
                     t[i] = *reinterpret_cast<const u32x4*>(scr + ((8 * i + (lane >> 3)) * 9 + (lane & 7)) * 16);
                     if constexpr (ADD) t[i] = add_halves(t[i], ad[i]);
                     if constexpr (ADD && NORM) {
-                        if (P.norm.relu) t[i] = u32x4{relu_pair(t[i][0]), relu_pair(t[i][1]), relu_pair(t[i][2]), relu_pair(t[i][3])};
+                        if (P0.norm.relu) t[i] = u32x4{relu_pair(t[i][0]), relu_pair(t[i][1]), relu_pair(t[i][2]), relu_pair(t[i][3])};
                     }
                 }
                 if constexpr (ADD) {

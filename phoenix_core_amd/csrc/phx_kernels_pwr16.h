@@ -47,7 +47,7 @@ __device__ __forceinline__ float agpr_value(float a) {
 
 // TAIL: what is done to the results on their way out (PWX_PLAIN ...); P.addend is a tensor laid out like the output.
 template <int WCO, int TAIL = PWX_PLAIN>
-__global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxArgs P0) {
+__global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxArgsOf<TAIL> P0) {
     const PwxArgs P = group_view(P0);
     constexpr bool ADD = TAIL == PWX_ADD || TAIL == PWX_NORM_ADD, NORM = TAIL >= PWX_NORM;
     extern __shared__ f16x8 lds16[];  // filters [K step][sub-tile][component][lane], then the waves' rings
@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
             const int co = (w0 + wc) * 32 + j;
             const bool co_ok = co < P.Cout;
             f32x4 factors;
-            if constexpr (NORM) factors = norm_factors(P.norm, co_ok ? co : 0);
+            if constexpr (NORM) factors = norm_factors(P0.norm, co_ok ? co : 0);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 __builtin_amdgcn_sched_barrier(0);  // (one tile at a time leaves the accumulator file)
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
                         for (int e = 0; e < 2; ++e) {
                             float v = agpr_value(acc[wc][q][4 * g + 2 * i + e]) + bv;
                             if constexpr (NORM) v = norm_apply(factors, v);
-                            if constexpr (NORM && !ADD) v = relu_if(P.norm.relu, v);
+                            if constexpr (NORM && !ADD) v = relu_if(P0.norm.relu, v);
                             h[e] = (_Float16)v;
                         }
                         d[g][i] = __builtin_bit_cast(unsigned int, h);
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
                     }
                     if constexpr (ADD) v = add_halves(v, ad[a]);
                     if constexpr (ADD && NORM) {
-                        if (P.norm.relu) v = u32x4{relu_pair(v[0]), relu_pair(v[1]), relu_pair(v[2]), relu_pair(v[3])};
+                        if (P0.norm.relu) v = u32x4{relu_pair(v[0]), relu_pair(v[1]), relu_pair(v[2]), relu_pair(v[3])};
                     }
                     if (ovalid[a] && co_ok) *reinterpret_cast<u32x4_a2*>(dst + oaddr[a]) = v;
                 }

@@ -46,7 +46,7 @@ int launch_pack_filters(const FwdVariant& v, const PackArgs& a, int blocks, hipS
 int launch_fwd_f32(const FwdVariant& v, const ConvArgs& a, hipStream_t st);
 int launch_fwd_f16(const FwdVariant& v, const ConvArgs& a, hipStream_t st);
 bool fwd_f16_takes_norm(const FwdVariant& v, const ConvArgs& a);  // whether launch_fwd_f16_norm has an instance
-int launch_fwd_f16_norm(const FwdVariant& v, const ConvArgs& a, hipStream_t st);
+int launch_fwd_f16_norm(const FwdVariant& v, const ConvArgs& a, const NormArgs& norm, hipStream_t st);
 int launch_fwd_f16_lds8(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // 8-product, filters through LDS
 int launch_fwd_f16_lanes(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // 8-product, lanes dealt over the waves
 int launch_fwd_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // fp32 on bf16 instructions
@@ -61,8 +61,8 @@ int launch_pack_filters_f16(const FwdVariant& v, const PackArgs& a, int blocks, 
 
 // pointwise fp16-MFMA kernels with raw operand copies (phx_kernels_pw16.h); WCO = 32-channel sub-tiles per workgroup
 struct PwxArgs;
-int launch_pwx_f16(int WCO, const PwxArgs& a, int blocks, hipStream_t st);
-int launch_pwr_f16(int WCO, const PwxArgs& a, int blocks, hipStream_t st);  // packed filter resident in LDS
+int launch_pwx_f16(int WCO, const PwxArgs& a, const NormArgs& norm, int blocks, hipStream_t st);
+int launch_pwr_f16(int WCO, const PwxArgs& a, const NormArgs& norm, int blocks, hipStream_t st);  // packed filter resident in LDS
 size_t pwr_lds_bytes(int WCO, int nsteps);
 int launch_pwx_nhwc_f16(int WCO, const PwxArgs& a, int blocks, hipStream_t st);  // channels-last tensors
 size_t pwx_packed_bytes(int WCO, int co_tiles, int nsteps);

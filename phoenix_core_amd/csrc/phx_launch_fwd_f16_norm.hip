@@ -11,14 +11,15 @@ namespace phx {
 bool fwd_f16_takes_norm(const FwdVariant& v, const ConvArgs& a) { return !a.nhwc && (v.lanes || (v.lds_filters && v.chunks)); }
 
 template <auto kernel>
-static int launch_one(const FwdVariant& v, const ConvArgs& a, hipStream_t st, size_t more_lds = 0) {
+static int launch_one(const FwdVariant& v, const ConvNormArgs& a, hipStream_t st, size_t more_lds = 0) {
     if (!BigLds<kernel>::registered) return -1;  // dynamic LDS opt-in at set-up, see BigLds
     hipLaunchKernelGGL(kernel, dim3(v.wgs, grid_rows(a.groups)), dim3(WG_THREADS), v.lds_bytes + more_lds, st, a);
     return 0;
 }
 
 // (the instance that the same variant takes without NORM: launch_fwd_f16)
-int launch_fwd_f16_norm(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
+int launch_fwd_f16_norm(const FwdVariant& v, const ConvArgs& plain, const NormArgs& norm, hipStream_t st) {
+    const ConvNormArgs a{plain, norm};
     if (v.lanes) return v.NTW == 1 ? launch_one<qconv_fwd_f16_lanes_kernel<2, false, true>>(v, a, st, LANES_NORM_BYTES) :
                         v.NTW == 2 ? launch_one<qconv_fwd_f16_lanes_kernel<4, false, true>>(v, a, st, LANES_NORM_BYTES) : -1;
 #define PHX_CASE(MODE_, WCO_, NTW_, EARLY_, XREAL_) \

@@ -5,7 +5,7 @@
 namespace phx {
 
 template <int WCO, int TAIL>
-static int launch_pwx_one(const PwxArgs& a, int blocks, hipStream_t st) {
+static int launch_pwx_one(const PwxArgsOf<TAIL>& a, int blocks, hipStream_t st) {
     constexpr auto kernel = qconv_pwx_f16_kernel<WCO, TAIL>;
     if (!BigLds<kernel>::registered) return -1;  // more than 64 KiB of dynamic LDS: opted in per device at set-up, see BigLds
     hipLaunchKernelGGL(kernel, dim3(blocks, grid_rows(a.groups)), dim3(WG_THREADS), PwxShape<WCO>::lds_bytes_nchw, st, a);
@@ -13,15 +13,16 @@ static int launch_pwx_one(const PwxArgs& a, int blocks, hipStream_t st) {
 }
 
 template <int WCO>
-static int launch_pwx_tail(const PwxArgs& a, int blocks, hipStream_t st) {
-    if (a.norm.gamma) return a.addend ? launch_pwx_one<WCO, PWX_NORM_ADD>(a, blocks, st) : launch_pwx_one<WCO, PWX_NORM>(a, blocks, st);
+static int launch_pwx_tail(const PwxArgs& a, const NormArgs& norm, int blocks, hipStream_t st) {
+    const PwxNormArgs na{a, norm};
+    if (norm.gamma) return a.addend ? launch_pwx_one<WCO, PWX_NORM_ADD>(na, blocks, st) : launch_pwx_one<WCO, PWX_NORM>(na, blocks, st);
     return a.addend ? launch_pwx_one<WCO, PWX_ADD>(a, blocks, st) : launch_pwx_one<WCO, PWX_PLAIN>(a, blocks, st);
 }
 
-int launch_pwx_f16(int WCO, const PwxArgs& a, int blocks, hipStream_t st) {
-    if (WCO == 4) return launch_pwx_tail<4>(a, blocks, st);
-    if (WCO == 2) return launch_pwx_tail<2>(a, blocks, st);
-    if (WCO == 1) return launch_pwx_tail<1>(a, blocks, st);
+int launch_pwx_f16(int WCO, const PwxArgs& a, const NormArgs& norm, int blocks, hipStream_t st) {
+    if (WCO == 4) return launch_pwx_tail<4>(a, norm, blocks, st);
+    if (WCO == 2) return launch_pwx_tail<2>(a, norm, blocks, st);
+    if (WCO == 1) return launch_pwx_tail<1>(a, norm, blocks, st);
     return -1;
 }
 

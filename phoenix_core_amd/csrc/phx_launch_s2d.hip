@@ -192,10 +192,11 @@ int launch_add_inplace(bool half_storage, void* dst, const void* src, long count
 // belongs to channel (e / plane) % channels of component e / comp_count; then + addend, element by element, in the storage
 // type): what closes a forward / input-gradient pass whose reduction over the channels was cut into slices.  fp32 sums,
 // one rounding.
+struct NoNorm {};
 template <typename TS, bool NORM>
 __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial, int slices, long count, TS* dst, const TS* bias,
                                                                const TS* addend, int plane, int channels, long comp_count,
-                                                               const NormArgs norm) {
+                                                               const std::conditional_t<NORM, NormArgs, NoNorm> norm) {
     const long stride = (long)gridDim.x * blockDim.x;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += stride) {
         float acc = 0.0f;
@@ -215,9 +216,12 @@ __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial
 template <typename TS>
 static void slice_sum(const void* partial, int slices, long count, void* dst, const void* bias, const void* addend, int plane, int channels,
                       long comp_count, const NormArgs& norm, hipStream_t st) {
-    const auto kernel = norm.gamma ? slice_sum_kernel<TS, true> : slice_sum_kernel<TS, false>;
-    hipLaunchKernelGGL(kernel, dim3(blocks_for(count)), dim3(WG_THREADS), 0, st, static_cast<const TS*>(partial), slices, count,
-                       static_cast<TS*>(dst), static_cast<const TS*>(bias), static_cast<const TS*>(addend), plane, channels, comp_count, norm);
+    const auto launch = [&](auto kernel, const auto& last) {
+        hipLaunchKernelGGL(kernel, dim3(blocks_for(count)), dim3(WG_THREADS), 0, st, static_cast<const TS*>(partial), slices, count,
+                           static_cast<TS*>(dst), static_cast<const TS*>(bias), static_cast<const TS*>(addend), plane, channels, comp_count, last);
+    };
+    if (norm.gamma) launch(slice_sum_kernel<TS, true>, norm);
+    else launch(slice_sum_kernel<TS, false>, NoNorm{});
 }
 
 int launch_slice_sum(bool half_storage, const void* partial, int slices, long count, void* dst, const void* bias, const void* addend,
