@@ -114,6 +114,21 @@ struct DenseSmallArgs {
 };
 int launch_dense_small(bool half_storage, int pass, const DenseSmallArgs& a, hipStream_t st);
 
+// Dense as matrix products (phx_launch_dense_gemm.hip): rows m of a, columns n of b, reduction over k; element
+// (component, m, k) of a at component * acs + m * ars + k * aks, of b likewise, output (q, m, n) at q * ocs + m * ors + n * ons.
+// Forward (x, w, k = inputs), input gradient (g, w, k = outputs), filter gradient (x, g, k = rows).
+struct DenseGemmArgs {
+    const void *a, *b;
+    const void* bias;  // forward: [4][N] or null
+    void* out;
+    float* partial;    // [Z][4][M][N] where Z > 1, else null
+    long acs, ars, aks, bcs, brs, bks, ocs, ors, ons;
+    int M, N, K;       // units at least 8
+    int MT, tiles_m, tiles_n, Z, kper;  // dense_gemm_plan
+};
+void dense_gemm_plan(bool half_storage, DenseGemmArgs& a);  // fills in the last line from M, N, K
+int launch_dense_gemm(bool half_storage, int pass, const DenseGemmArgs& a, hipStream_t st);
+
 // Grouped convolutions with very few channels per group (depthwise and the like) on fp32 FMA threads, on the caller's
 // channels-first tensors and filter (phx_launch_thin.hip).  in = x (forward, filter gradient) or the output gradient
 // (input gradient); out = y, dx or dw.  Filter element (r, co, i, kh, kw), co over all groups and i inside its group,
