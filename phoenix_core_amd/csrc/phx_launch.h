@@ -124,10 +124,18 @@ struct DenseGemmArgs {
     float* partial;    // [Z][4][M][N] where Z > 1, else null
     long acs, ars, aks, bcs, brs, bks, ocs, ors, ons;
     int M, N, K;       // units at least 8
-    int MT, tiles_m, tiles_n, Z, kper;  // dense_gemm_plan
+    int MT, tiles_m, tiles_n, chunks, Z, kper;  // dense_gemm_plan (chunks of reduced indices, of a slice)
 };
-void dense_gemm_plan(bool half_storage, DenseGemmArgs& a);  // fills in the last line from M, N, K
+// The filter gradient of a pointwise fp32 convolution on image planes is the same product with k running over the pixels of the
+// images, which lie at these distances.
+struct GemmPlanes {
+    int images;
+    int chunks;  // of an image (dense_gemm_plan)
+    long aimg, bimg;
+};
+void dense_gemm_plan(bool half_storage, DenseGemmArgs& a, GemmPlanes* planes = nullptr);  // fills in the last line from M, N, K
 int launch_dense_gemm(bool half_storage, int pass, const DenseGemmArgs& a, hipStream_t st);
+int launch_planes_gemm(const DenseGemmArgs& a, const GemmPlanes& planes, hipStream_t st);
 
 // Grouped convolutions with very few channels per group (depthwise and the like) on fp32 FMA threads, on the caller's
 // channels-first tensors and filter (phx_launch_thin.hip).  in = x (forward, filter gradient) or the output gradient

@@ -169,12 +169,21 @@ constexpr bool dense_negative(int pass, int p, int q) {
     return qneg(p, q) != (pass == PHX_PASS_BWD_DATA && (p ^ q) > 0) != (pass == PHX_PASS_BWD_WEIGHTS && p > 0);
 }
 
-// COLTURN: the column operand is contiguous along its rows (the filter gradient's operands both are)
-template <typename T, int PASS, bool COLTURN, int MT>
-__global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const DenseGemmArgs P) {
+struct GemmArgsPlanes : DenseGemmArgs {
+    GemmPlanes planes;
+};
+template <bool PLANES>
+using GemmArgsOf = std::conditional_t<PLANES, GemmArgsPlanes, DenseGemmArgs>;
+
+// ROWTURN, COLTURN: the operand is contiguous along its rows, not along the reduction.  PLANES: the filter gradient of a pointwise
+// convolution on image planes: the reduction runs over the pixels of one image after the other, and results are contiguous along
+// m, so the matrix instructions take their operands the other way round.
+template <typename T, int PASS, bool ROWTURN, bool COLTURN, bool PLANES, int MT>
+__global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArgsOf<PLANES> P) {
     using S = DenseTile<T>;
     constexpr bool F32 = sizeof(T) == 4;
-    using Rows = DenseOperand<T, PASS == PHX_PASS_BWD_WEIGHTS, 64 * MT>;
+    static_assert(!PLANES || PASS == PHX_PASS_BWD_WEIGHTS, "planes: the filter gradient");
+    using Rows = DenseOperand<T, ROWTURN, 64 * MT>;
     using Cols = DenseOperand<T, COLTURN, 64>;
     extern __shared__ u32x4 ldsd[];
     u32x4* const rl = ldsd;
@@ -186,15 +195,31 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const DenseGe
     const int n0 = bid % P.tiles_n * 64;
     bid /= P.tiles_n;
     const int m0 = bid % P.tiles_m * (64 * MT), z = bid / P.tiles_m;
-    const int k_first = z * P.kper, k_end = min(P.K, k_first + P.kper);
+    const T* a = static_cast<const T*>(P.a);
+    const T* b = static_cast<const T*>(P.b);
+    // the slice's chunks; planes: chunk c is one of image c / planes.chunks
+    const int first = z * P.kper, end = min(P.chunks, first + P.kper);
+    int load_img = 0, load_k = first * S::KC;
+    if constexpr (PLANES) {
+        load_img = first / P.planes.chunks;
+        load_k = (first - load_img * P.planes.chunks) * S::KC;
+    }
 
     Rows rows;
     Cols cols;
-    const T* const a = static_cast<const T*>(P.a);
-    const T* const b = static_cast<const T*>(P.b);
-    auto load = [&](int k) {
-        rows.load(a, P.acs, P.ars, P.aks, m0, P.M, k, P.K);
-        cols.load(b, P.bcs, P.brs, P.bks, n0, P.N, k, P.K);
+    auto load = [&] {  // the next chunk; the cursor moves on
+        const T *la = a, *lb = b;
+        if constexpr (PLANES) {
+            la += load_img * P.planes.aimg;
+            lb += load_img * P.planes.bimg;
+        }
+        rows.load(la, P.acs, P.ars, P.aks, m0, P.M, load_k, P.K);
+        cols.load(lb, P.bcs, P.brs, P.bks, n0, P.N, load_k, P.K);
+        load_k += S::KC;
+        if (PLANES && load_k >= P.K) {
+            load_k = 0;
+            ++load_img;
+        }
     };
     f32x16 acc[MT][4], low[F32 ? 4 : 1];
 #pragma unroll
@@ -210,20 +235,22 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const DenseGe
     const u32x4* const ca = cl + kk * Cols::PITCH + wn * 32 + j;
     auto negated = [](const u32x4 v) { return v ^ u32x4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u}; };
 
-    load(k_first);
-    for (int k = k_first; k < k_end; k += S::KC) {
+    int k = load_k;  // of the chunk being stored and multiplied
+    load();
+    for (int c = first; c < end; ++c) {
         const bool tail = k + S::KC > P.K;
-        if (k > k_first) __syncthreads();
+        if (c > first) __syncthreads();
         rows.store(rl, m0, P.M, k, P.K, tail);
         cols.store(cl, n0, P.N, k, P.K, tail);
         __syncthreads();
-        if (k + S::KC < k_end) load(k + S::KC);
+        k = load_k;
+        if (c + 1 < end) load();
 #pragma unroll
         for (int ks = 0; ks < S::KP / 2; ++ks) {
             if constexpr (!F32) {
                 f16x8 w[4];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) w[c] = __builtin_bit_cast(f16x8, ca[(c * S::KP + 2 * ks) * Cols::PITCH]);
+                for (int i = 0; i < 4; ++i) w[i] = __builtin_bit_cast(f16x8, ca[(i * S::KP + 2 * ks) * Cols::PITCH]);
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -231,16 +258,19 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const DenseGe
                         const u32x4 v = ra[(p * S::KP + 2 * ks) * Rows::PITCH + t * 32];
                         const f16x8 x = __builtin_bit_cast(f16x8, v), nx = __builtin_bit_cast(f16x8, negated(v));
 #pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            acc[t][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[p ^ q], dense_negative(PASS, p, q) ? nx : x, acc[t][q], 0, 0, 0);
+                        for (int q = 0; q < 4; ++q) {
+                            const f16x8 xs = dense_negative(PASS, p, q) ? nx : x;
+                            acc[t][q] = PLANES ? __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, w[p ^ q], acc[t][q], 0, 0, 0)
+                                               : __builtin_amdgcn_mfma_f32_32x32x16_f16(w[p ^ q], xs, acc[t][q], 0, 0, 0);
+                        }
                     }
             } else {
                 bf16x8 w[3][4];
 #pragma unroll
                 for (int part = 0; part < 3; ++part)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        w[part][c] = __builtin_bit_cast(bf16x8, ca[((part * 4 + c) * S::KP + 2 * ks) * Cols::PITCH]);
+                    for (int i = 0; i < 4; ++i)
+                        w[part][i] = __builtin_bit_cast(bf16x8, ca[((part * 4 + i) * S::KP + 2 * ks) * Cols::PITCH]);
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
                     bf16x8 x[3], nx[3];
@@ -255,8 +285,10 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const DenseGe
                         constexpr int wp[6] = {2, 0, 1, 1, 0, 0}, xp[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
+                            const bf16x8 xs = dense_negative(PASS, p, q) ? nx[xp[term]] : x[xp[term]];
                             f32x16& sum = term < 5 ? low[q] : acc[0][q];
-                            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[wp[term]][p ^ q], dense_negative(PASS, p, q) ? nx[xp[term]] : x[xp[term]], sum, 0, 0, 0);
+                            sum = PLANES ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, w[wp[term]][p ^ q], sum, 0, 0, 0)
+                                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[wp[term]][p ^ q], xs, sum, 0, 0, 0);
                         }
                     }
                 }
@@ -264,45 +296,54 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const DenseGe
         }
     }
 
-    // accumulator register 4 g + e: column 8 g + 4 kk + e of the wave's 32, row j
+    // accumulator register 4 g + e: column 8 g + 4 kk + e of the wave's 32 at row j (PLANES: row 8 g + 4 kk + e at column j)
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        const int m = m0 + (wm * MT + t) * 32 + j;
-        if (m >= P.M) continue;
+        const int lane_index = PLANES ? n0 + wn * 32 + j : m0 + (wm * MT + t) * 32 + j;
+        if (lane_index >= (PLANES ? P.N : P.M)) continue;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int n = n0 + wn * 32 + 8 * g + 4 * kk;
+                const int run = (PLANES ? m0 + (wm * MT + t) * 32 : n0 + wn * 32) + 8 * g + 4 * kk, length = PLANES ? P.M : P.N;
+                const int m = PLANES ? run : lane_index, n = PLANES ? lane_index : run;
+                const bool whole = run + 3 < length;
                 f32x4 y = {acc[t][q][4 * g], acc[t][q][4 * g + 1], acc[t][q][4 * g + 2], acc[t][q][4 * g + 3]};
                 if constexpr (F32) y += f32x4{low[q][4 * g], low[q][4 * g + 1], low[q][4 * g + 2], low[q][4 * g + 3]};
-                if (P.partial) {
-                    float* dst = P.partial + (((long)z * 4 + q) * P.M + m) * P.N + n;
-                    if (n + 3 < P.N) *reinterpret_cast<f32x4_a4*>(dst) = y;
+                if (P.partial) {  // [slice][component][m][n], PLANES [n][m]
+                    float* dst = P.partial + (((long)z * 4 + q) * (PLANES ? P.N : P.M) + lane_index) * length + run;
+                    if (whole) *reinterpret_cast<f32x4_a4*>(dst) = y;
                     else
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            if (n + e < P.N) dst[e] = y[e];
+                            if (run + e < length) dst[e] = y[e];
                     continue;
                 }
-                T* dst = static_cast<T*>(P.out) + q * P.ocs + m * P.ors + n * P.ons;
-                const T* bias = static_cast<const T*>(P.bias) + q * P.N + n;
+                const long step = PLANES ? P.ors : P.ons;
                 typedef T t4 __attribute__((ext_vector_type(4)));
+                if constexpr (PASS == PHX_PASS_FWD) {
+                    if (P.bias) {
+                        const T* bias = static_cast<const T*>(P.bias) + q * P.N + n;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) y[e] += n + e < P.N ? (float)bias[e] : 0.f;
+                    }
+                }
                 t4 o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = (T)(y[e] + (P.bias && n + e < P.N ? (float)bias[e] : 0.f));
-                if (P.ons == 1 && n + 3 < P.N)
+                for (int e = 0; e < 4; ++e) o[e] = (T)y[e];
+                T* dst = static_cast<T*>(P.out) + q * P.ocs + m * P.ors + n * P.ons;
+                if (step == 1 && whole)
                     *reinterpret_cast<std::conditional_t<F32, u32x4_a4, u32x2_a2>*>(dst) = __builtin_bit_cast(std::conditional_t<F32, u32x4, u32x2>, o);
                 else
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (n + e < P.N) dst[e * P.ons] = o[e];
+                        if (run + e < length) dst[e * step] = o[e];
             }
     }
 }
 
 // out = the sum of the slices' partial results (+ bias), one rounding
-template <typename T>
+template <typename T, bool PLANES>
 __global__ void __launch_bounds__(WG_THREADS) dense_gemm_sum_kernel(const DenseGemmArgs P) {
     const long count = 4L * P.M * P.N, stride = (long)gridDim.x * blockDim.x;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += stride) {
@@ -312,9 +353,11 @@ __global__ void __launch_bounds__(WG_THREADS) dense_gemm_sum_kernel(const DenseG
 #pragma unroll
             for (int i = 0; i < 4; ++i) sum[i] += P.partial[(z + i) * count + e];
         for (; z < P.Z; ++z) sum[0] += P.partial[z * count + e];
-        const long row = e / P.N;
-        const int n = (int)(e - row * P.N), q = (int)(row / P.M), m = (int)(row - (long)q * P.M);
         float y = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        const int length = PLANES ? P.M : P.N, lines = PLANES ? P.N : P.M;
+        const long row = e / length;
+        const int run = (int)(e - row * length), q = (int)(row / lines), line = (int)(row - (long)q * lines);
+        const int m = PLANES ? run : line, n = PLANES ? line : run;
         if (P.bias) y += (float)static_cast<const T*>(P.bias)[q * P.N + n];
         static_cast<T*>(P.out)[q * P.ocs + m * P.ors + n * P.ons] = (T)y;
     }
@@ -324,54 +367,73 @@ __global__ void __launch_bounds__(WG_THREADS) dense_gemm_sum_kernel(const DenseG
 // for more than one slice the partial results' way to memory and back in a second kernel.  A chunk of a lone workgroup takes
 // the latency of its loads, those of two or three on one CU overlap.  Times from M, N, K = 64 ... 4096 (us a chunk, one to three
 // workgroups on a CU: fp16 64 rows 1.7 / 2.8 / 3.9, 128 rows 3.9 / 4.8; fp32 3.4 / 5.7).
-void dense_gemm_plan(bool half_storage, DenseGemmArgs& a) {
+void dense_gemm_plan(bool half_storage, DenseGemmArgs& a, GemmPlanes* planes) {
     const int KC = half_storage ? DenseTile<_Float16>::KC : DenseTile<float>::KC;
-    const int chunks = (a.K + KC - 1) / KC;
+    a.chunks = (a.K + KC - 1) / KC;
+    if (planes) {
+        planes->chunks = a.chunks;
+        a.chunks *= planes->images;
+    }
     a.tiles_n = (a.N + 63) / 64;
     double best = 1e30;
     for (int mt = 1; mt <= (half_storage ? 2 : 1); ++mt) {
         const int tiles_m = (a.M + 64 * mt - 1) / (64 * mt), most = half_storage && mt == 1 ? 3 : 2;
         const double first = !half_storage ? 3.4 : mt == 2 ? 3.9 : 1.7, more = !half_storage ? 2.3 : mt == 2 ? 0.9 : 1.1;
-        for (int Z = 1; Z <= std::min(chunks, 64); ++Z) {
-            const int per = (chunks + Z - 1) / Z;
-            if ((chunks + per - 1) / per != Z) continue;
+        for (int Z = 1; Z <= std::min(a.chunks, planes ? 512 : 64); ++Z) {
+            const int per = (a.chunks + Z - 1) / Z;
+            if ((a.chunks + per - 1) / per != Z) continue;
             const double load = std::ceil((double)tiles_m * a.tiles_n * Z / 256.0), full = std::floor(load / most), rest = load - full * most;
             double us = 4.0 + per * (full * (first + (most - 1) * more) + (rest > 0 ? first + (rest - 1) * more : 0.0));
             if (Z > 1) us += 4.0 + (Z + 0.5) * 32.0 * a.M * a.N / 3.0e6;
             if (us < best) {
                 best = us;
-                a.MT = mt; a.tiles_m = tiles_m; a.Z = Z; a.kper = per * KC;
+                a.MT = mt; a.tiles_m = tiles_m; a.Z = Z; a.kper = per;
             }
         }
     }
 }
 
-template <typename T, int PASS, bool COLTURN, int MT>
-static int launch_one(const DenseGemmArgs& a, hipStream_t st) {
-    constexpr size_t lds = (size_t)(DenseOperand<T, PASS == PHX_PASS_BWD_WEIGHTS, 64 * MT>::ENTRIES + DenseOperand<T, COLTURN, 64>::ENTRIES) * 16;
+template <typename T, int PASS, bool ROWTURN, bool COLTURN, bool PLANES, int MT>
+static int launch_one(const GemmArgsOf<PLANES>& a, hipStream_t st) {
+    constexpr size_t lds = (size_t)(DenseOperand<T, ROWTURN, 64 * MT>::ENTRIES + DenseOperand<T, COLTURN, 64>::ENTRIES) * 16;
     static_assert(lds <= 64 * 1024, "no opt-in for dynamic LDS");
-    hipLaunchKernelGGL((dense_gemm_kernel<T, PASS, COLTURN, MT>), dim3((unsigned)((long)a.tiles_m * a.tiles_n * a.Z)), dim3(WG_THREADS), lds, st, a);
+    hipLaunchKernelGGL((dense_gemm_kernel<T, PASS, ROWTURN, COLTURN, PLANES, MT>), dim3((unsigned)((long)a.tiles_m * a.tiles_n * a.Z)),
+                       dim3(WG_THREADS), lds, st, a);
+    return 0;
+}
+
+template <typename T, bool PLANES>
+static int launch_sum(const DenseGemmArgs& a, hipStream_t st) {
+    if (a.Z == 1) return 0;
+    const long count = 4L * a.M * a.N;
+    const dim3 grid((unsigned)std::min<long>((count + WG_THREADS - 1) / WG_THREADS, 1 << 14));
+    hipLaunchKernelGGL((dense_gemm_sum_kernel<T, PLANES>), grid, dim3(WG_THREADS), 0, st, a);
     return 0;
 }
 
 template <typename T, int MT>
 static int launch_pass(int pass, const DenseGemmArgs& a, hipStream_t st) {
     const bool turn = a.bks != 1;
-    if (pass == PHX_PASS_FWD) return turn ? launch_one<T, PHX_PASS_FWD, true, MT>(a, st) : launch_one<T, PHX_PASS_FWD, false, MT>(a, st);
-    if (pass == PHX_PASS_BWD_DATA) return turn ? launch_one<T, PHX_PASS_BWD_DATA, true, MT>(a, st) : launch_one<T, PHX_PASS_BWD_DATA, false, MT>(a, st);
-    return launch_one<T, PHX_PASS_BWD_WEIGHTS, true, MT>(a, st);
+    if (pass == PHX_PASS_FWD)
+        return turn ? launch_one<T, PHX_PASS_FWD, false, true, false, MT>(a, st) : launch_one<T, PHX_PASS_FWD, false, false, false, MT>(a, st);
+    if (pass == PHX_PASS_BWD_DATA)
+        return turn ? launch_one<T, PHX_PASS_BWD_DATA, false, true, false, MT>(a, st) : launch_one<T, PHX_PASS_BWD_DATA, false, false, false, MT>(a, st);
+    return launch_one<T, PHX_PASS_BWD_WEIGHTS, true, true, false, MT>(a, st);
 }
 
 int launch_dense_gemm(bool half_storage, int pass, const DenseGemmArgs& a, hipStream_t st) {
     // (a load's 16 bytes lie inside a row of units, a task's rows inside the units that are contiguous)
     if (a.M < 1 || a.K < 1 || a.N < 8 || (pass == PHX_PASS_BWD_WEIGHTS ? a.M : a.K) < 8 || (a.Z > 1) != (a.partial != nullptr)) return -1;
     const int rc = !half_storage ? launch_pass<float, 1>(pass, a, st) : a.MT == 2 ? launch_pass<_Float16, 2>(pass, a, st) : launch_pass<_Float16, 1>(pass, a, st);
-    if (rc != 0 || a.Z == 1) return rc;
-    const long count = 4L * a.M * a.N;
-    const dim3 grid((unsigned)std::min<long>((count + WG_THREADS - 1) / WG_THREADS, 1 << 14));
-    if (half_storage) hipLaunchKernelGGL((dense_gemm_sum_kernel<_Float16>), grid, dim3(WG_THREADS), 0, st, a);
-    else hipLaunchKernelGGL((dense_gemm_sum_kernel<float>), grid, dim3(WG_THREADS), 0, st, a);
-    return 0;
+    if (rc != 0) return rc;
+    return half_storage ? launch_sum<_Float16, false>(a, st) : launch_sum<float, false>(a, st);
+}
+
+int launch_planes_gemm(const DenseGemmArgs& plain, const GemmPlanes& planes, hipStream_t st) {
+    const GemmArgsPlanes a{plain, planes};
+    if (a.M < 1 || a.K < 4 || a.N < 1 || a.MT != 1 || (a.Z > 1) != (a.partial != nullptr)) return -1;  // (loads of four pixels inside a plane)
+    if (const int rc = launch_one<float, PHX_PASS_BWD_WEIGHTS, false, false, true, 1>(a, st)) return rc;
+    return launch_sum<float, true>(a, st);
 }
 
 }  // namespace phx

@@ -95,3 +95,26 @@ def test_rule_takes_the_sizes_it_was_measured_at(tune_env):
     assert all("mfmagemm" in k for k in names(3707, 95, 408, torch.float16))
     assert all("pwxcl" in k for k in names(4096, 1024, 1024, torch.float16))
     assert "mfmagemm" in names(33, 1672, 416, torch.float16)[0]
+
+
+@pytest.mark.parametrize("case", [
+    (3, 97, 97, 2, 2, 1, "NCHW", torch.float32), (5, 65, 190, 7, 7, 1, "NCHW", torch.float32), (2, 129, 130, 19, 19, 1, "NCHW", torch.float32),
+    (70, 96, 96, 5, 3, 1, "NCHW", torch.float32), (2, 250, 66, 13, 9, 2, "NCHW", torch.float32), (3, 97, 100, 7, 5, 1, "NHWC", torch.float32),
+    (4, 52, 61, 9, 9, 1, "NHWC", torch.float16), (1, 49, 49, 3, 3, 1, "NHWC", torch.float16)], ids=lambda c: "n%d_%dto%d_%dx%d_s%d_%s_%s" % c)
+def test_filter_gradient_of_pointwise_convolutions(case):
+    n, ci, co, h, w, stride, layout, dtype = case
+    gen = torch.Generator(device="cuda").manual_seed(h * w)
+    x = torch.randn(4 * n, ci, h, w, generator=gen, device="cuda").to(dtype)
+    wt = torch.zeros(4, co, ci, 1, 1, device="cuda", dtype=dtype)
+    xs = x[:, :, ::stride, ::stride]
+    grad = torch.randn((4 * n, co) + xs.shape[2:], generator=gen, device="cuda").to(dtype)
+    args = dict(stride=stride, padding="SAME", dtype=dtype, context=phx.Context({"UPSTRIDE_CONV_FP16_POLICY": "full16"}), data_format=layout)
+    last = (lambda t: t.permute(0, 2, 3, 1).contiguous()) if layout == "NHWC" else (lambda t: t)
+    desc = ops.Conv2DDescriptor(last(x).shape, wt.shape, **args)
+    dw = ops.conv2d_bwd_weights(last(x), last(grad), desc)
+    assert "mfmagemm" in capi.last_kernel_name(), capi.last_kernel_name()
+    rows = lambda t: t.permute(0, 2, 3, 1).reshape(-1, t.shape[1])
+    (_, _, want), (_, _, total) = _reference(rows(xs), wt.view(4, co, ci).transpose(1, 2), rows(grad))
+    half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -24
+    got = dw.double().view(4, co, ci).transpose(1, 2)
+    assert bool(((got - want).abs() <= 1.001 * half_ulp * want.abs() + 2.0 ** -19 * total + 2.0 ** -25).all())
