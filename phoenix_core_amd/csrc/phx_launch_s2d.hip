@@ -199,8 +199,13 @@ __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial
                                                                const std::conditional_t<NORM, NormArgs, NoNorm> norm) {
     const long stride = (long)gridDim.x * blockDim.x;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += stride) {
-        float acc = 0.0f;
-        for (int z = 0; z < slices; ++z) acc += (float)partial[z * count + e];
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};  // (four loads in flight)
+        int z = 0;
+        for (; z + 4 <= slices; z += 4)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[i] += (float)partial[(z + i) * count + e];
+        for (; z < slices; ++z) sum[0] += (float)partial[z * count + e];
+        float acc = (sum[0] + sum[1]) + (sum[2] + sum[3]);
         if (bias) acc += (float)bias[(e / comp_count) * channels + (e / plane) % channels];
         if constexpr (NORM) {
             acc = norm_apply(norm_factors(norm, (int)((e / plane) % channels)), acc);
