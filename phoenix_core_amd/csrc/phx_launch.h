@@ -91,6 +91,9 @@ int launch_pack_jobs(const PackJobs& jobs, hipStream_t st);
 constexpr int wgrad_f32_ksets(int mode, bool vec) { return (mode == 8 && vec) ? 2 : 1; }
 int launch_wgrad_f32(bool half_storage, bool vec, int mode, const WgradArgs& a, dim3 grid, size_t lds_bytes,
                      hipStream_t st);  // vec: windows staged as groups of 4 positions
+// fp32 filter gradient on bf16 instructions (phx_kernels_wgx3.h)
+size_t wgrad_x3_lds_bytes();
+int launch_wgrad_x3(const WgradArgs& a, dim3 grid, hipStream_t st);
 // fp16-MFMA filter gradient: channel tile 32*MT x 32*NT, TPW taps per workgroup (1 or 3), stride SW along W (1 or 2)
 int launch_wgrad_f16(int mode, int MT, int NT, int TPW, int SW, const WgradArgs& a, int nblocks, size_t lds_bytes,
                      hipStream_t st);

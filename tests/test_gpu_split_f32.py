@@ -1,4 +1,4 @@
-"""fp32 passes on bf16 instructions (phx_kernels_x3.h) against fp64, beside the fp32 instructions."""
+"""fp32 passes on bf16 instructions (phx_kernels_x3.h, phx_kernels_wgx3.h) against fp64, beside the fp32 instructions."""
 import ctypes
 
 import pytest
@@ -91,3 +91,50 @@ def test_fixed_scratch_keeps_the_fp32_instructions_where_the_parts_do_not_fit(tu
     assert "f32mfmax3" in capi.last_kernel_name()
     tune_env(PHX_TUNE_NOX3="1")
     assert torch.equal(y, phx.conv2d_fwd(x, wt, None, desc))
+
+
+# n, ci, co, h, w, k, stride, groups: one, two and three taps of a filter row and their remainders (5, 7), rows shorter than a
+# segment and with a remainder, an odd number of segments, channels past a tile of either side, one and many reduction slices,
+# tensors whose ends every load meets, groups in one launch, strides by tap classes
+WGRAD_CASES = [
+    (1, 24, 24, 9, 9, 3, 1, 1), (4, 70, 130, 14, 14, 3, 1, 1), (2, 33, 31, 9, 17, 7, 1, 1), (16, 104, 40, 58, 7, 5, 1, 1),
+    (64, 32, 32, 9, 9, 1, 1, 1), (64, 64, 64, 4, 4, 3, 1, 1), (20, 64, 64, 17, 17, 3, 1, 1), (128, 48, 40, 9, 9, 3, 1, 1),
+    (16, 512, 256, 7, 7, 3, 1, 1), (4, 160, 192, 12, 10, 3, 1, 2), (32, 128, 128, 14, 14, 5, 2, 1),
+]
+
+
+def _wgrad(case, x=None, grad=None):
+    n, ci, co, h, w, k, stride, groups = case
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(4 * n, ci, h, w, generator=gen, device="cuda") if x is None else x
+    desc = ops.Conv2DDescriptor(x.shape, (4, co, ci // groups, k, k), stride=stride, padding="SAME", groups=groups,
+                                dtype=torch.float32, context=phx.Context({}))
+    grad = torch.randn(desc.output_shape, generator=gen, device="cuda") if grad is None else grad
+    (pt, pl), (pb, pr) = desc.pad_before, desc.pad_after
+    wr = torch.zeros(4, co, ci // groups, k, k, dtype=torch.float64, device="cuda", requires_grad=True)
+    yr = _hamilton(torch.nn.functional.pad(x.double(), (pl, pr, pt, pb)), wr,
+                   lambda a, b: torch.nn.functional.conv2d(a, b, stride=stride, groups=groups))
+    return x, grad, desc, torch.autograd.grad(yr, wr, grad.double())[0]
+
+
+@pytest.mark.parametrize("case", WGRAD_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_filter_gradient_error_against_fp64(case, tune_env):
+    x, grad, desc, ref = _wgrad(case)
+    gaps = {}
+    for nox3 in (None, "1"):
+        tune_env(PHX_TUNE_NOX3=nox3)
+        dw = ops.conv2d_bwd_weights(x, grad, desc)
+        assert ("f32mfmax3" in capi.last_kernel_name()) == (nox3 is None), capi.last_kernel_name()
+        gaps[nox3] = _gap(dw, ref)
+    assert gaps[None] <= 1.1 * gaps["1"], gaps  # (the norms of thousands of roundings: see above)
+
+
+def test_filter_gradient_of_whole_numbers_is_exact():
+    case = (6, 40, 70, 11, 13, 3, 1, 1)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(-300, 301, (24, 40, 11, 13), generator=gen, device="cuda").float()
+    grad = 2 * torch.randint(-20, 21, (24, 70, 11, 13), generator=gen, device="cuda").float()  # (four of the lanes are halved)
+    x, grad, desc, ref = _wgrad(case, x, grad)
+    dw = ops.conv2d_bwd_weights(x, grad, desc)
+    assert "f32mfmax3" in capi.last_kernel_name()
+    assert torch.equal(dw.double(), ref)
