@@ -37,6 +37,7 @@ struct FwdVariant {
     bool chunks;        // fp16 MFMA, filters in LDS: activations staged as 8-position chunks
     bool lanes;         // fp16 MFMA, 8-product: product lanes dealt over the waves (phx_kernels_lanes16.h)
     bool x3;            // fp32 tensors, 8-product: on bf16 instructions (phx_kernels_x3.h)
+    bool pwx3;          // ... its pointwise kernel (phx_kernels_pwx3.h)
     int pw;             // pointwise convolution run as a column of pw virtual taps over 16-channel sub-chunks (0 = off)
     int wgs;
     size_t lds_bytes;
@@ -52,6 +53,11 @@ int launch_fwd_f16_lanes(const FwdVariant& v, const ConvArgs& a, hipStream_t st)
 int launch_fwd_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // fp32 on bf16 instructions
 size_t x3_lds_bytes();
 size_t x3_image_bytes(int WCO, int co_tiles, int nchunks, int ngroups);
+int launch_pw_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // ... pointwise
+int pw_x3_pixels();
+size_t pw_x3_lds_bytes();
+size_t pw_x3_image_bytes(int WCO, int co_tiles, int nsteps);
+int launch_pack_filters_pw_x3(int map, int WCO, const PackArgs& a, int blocks, hipStream_t st);
 int launch_pack_filters_x3(int map, int WCO, int ngroups, const PackArgs& a, int blocks, hipStream_t st);
 size_t lanes_lds_bytes();
 size_t lanes_image_bytes(int co_tiles, int nchunks, int ngroups);
@@ -71,12 +77,12 @@ int launch_pack_filters_pwx(int map, int WCO, int nsteps, const PackArgs& a, hip
 // Several filter images packed by one launch (phx_launch_pack.hip): a convolution's forward and input-gradient
 // images, the sub-filters of a strided input gradient's phases, the groups of a grouped convolution.  A job is one
 // call of one of the packing kernels above; the workgroups of the launch are dealt to the jobs in order.
-enum PackKind { PACK_F32 = 0, PACK_F16 = 1, PACK_F16_LDS = 2, PACK_PWX = 3, PACK_F16_LANES = 4, PACK_F32_X3 = 5 };
+enum PackKind { PACK_F32 = 0, PACK_F16 = 1, PACK_F16_LDS = 2, PACK_PWX = 3, PACK_F16_LANES = 4, PACK_F32_X3 = 5, PACK_F32_PWX3 = 6 };
 struct PackJob {
     PackArgs a;
     int kind;                    // PackKind
     int mode, map;               // 16 / 8, MAP_FWD / MAP_DGRAD
-    int WCO, ngroups, pw;        // PACK_F16_LDS (PackLdsArgs), PACK_PWX (WCO), PACK_F16_LANES (ngroups), PACK_F32_X3 (WCO, ngroups)
+    int WCO, ngroups, pw;        // PACK_F16_LDS (PackLdsArgs), PACK_PWX (WCO), PACK_F16_LANES (ngroups), PACK_F32_X3 (WCO, ngroups), PACK_F32_PWX3 (WCO)
     int nsteps;                  // PACK_PWX
     int block0, nblocks;         // this job's workgroups: [block0, block0 + nblocks)
 };

@@ -27,11 +27,13 @@ static int launch_variant(const FwdVariant& v, const ConvArgs& a, hipStream_t st
 // (fp32 tensors only: fp16 tensors run on the fp16 matrix instructions under every policy)
 int launch_fwd_f32(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
     // one kernel for both passes: the input gradient differs only in how its filters are packed
+    if (v.pwx3) return launch_pw_x3(v, a, st);
     if (v.x3) return launch_fwd_x3(v, a, st);
     return v.mode == 16 ? launch_variant<16>(v, a, st) : launch_variant<8>(v, a, st);
 }
 
 int launch_pack_filters(const FwdVariant& v, const PackArgs& a, int blocks, hipStream_t st) {
+    if (v.pwx3) return launch_pack_filters_pw_x3(v.map, v.WCO, a, blocks, st);
     if (v.x3) return launch_pack_filters_x3(v.map, v.WCO, v.ngroups, a, blocks, st);
     const dim3 g(blocks, grid_rows(a.groups)), b(WG_THREADS);
     if (v.mode == 16 && v.map == MAP_FWD) hipLaunchKernelGGL((pack_filters_f32_kernel<float, 16, MAP_FWD>), g, b, 0, st, a);

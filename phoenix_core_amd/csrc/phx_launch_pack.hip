@@ -1,6 +1,6 @@
 // One launch that packs several filter images (PackJobs in phx_launch.h): every workgroup finds the job its index
 // falls into and runs that packing kernel's body over the job's own index range.
-#include "phx_kernels_x3.h"
+#include "phx_kernels_pwx3.h"
 #include "phx_kernels_pw16.h"
 #include "phx_launch.h"
 
@@ -17,6 +17,8 @@ static __device__ __forceinline__ void pack_job_as(const PackJob& j, long first,
         pack_filters_f16_lds_body<MODE, MAP>(la, first, stride);
     } else if (j.kind == PACK_F32_X3) {
         if constexpr (MODE == 8) pack_filters_x3_body<MAP>(PackLanesArgs{j.a, j.ngroups * X3_GROUP}, j.WCO, first, stride);
+    } else if (j.kind == PACK_F32_PWX3) {
+        if constexpr (MODE == 8) pack_filters_pwx3_body<MAP>(j.a, j.WCO, first, stride);
     } else if (j.kind == PACK_F16_LANES) {
         if constexpr (MODE == 8) pack_filters_lanes_body<MAP>(PackLanesArgs{j.a, j.ngroups * LANES_GROUP}, first, stride);
     } else if (MODE == 16) {  // PACK_PWX (16-product form only)

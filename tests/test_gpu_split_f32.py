@@ -23,11 +23,14 @@ def _gap(a, b):
 
 
 # n, ci, co, h, w, k, stride, dilation, groups: sub-tiles of 32 and 64 output channels, wide and narrow tiles, flat and
-# rectangular tilings, ragged channels, planes that are one partial group of four, tensors whose ends every load meets
+# rectangular tilings, ragged channels, planes that are one partial group of four, tensors whose ends every load meets;
+# pointwise: odd planes, a plane of one pair, tiles over several images, a remainder of a K step, slices, groups, a stride
 CASES = [
     (3, 8, 40, 9, 13, 3, 1, 1, 1), (1, 9, 33, 3, 3, 3, 1, 1, 1), (1, 1, 1, 1, 2, 3, 1, 1, 1), (40, 16, 64, 14, 14, 3, 1, 1, 1),
     (2, 24, 20, 30, 7, 5, 1, 1, 1), (4, 130, 70, 21, 18, 3, 2, 1, 1), (2, 17, 65, 20, 20, 3, 1, 2, 1), (1, 64, 96, 7, 7, 3, 1, 1, 1),
     (2, 80, 96, 12, 10, 3, 1, 1, 2), (64, 72, 64, 16, 16, 3, 1, 1, 1), (1, 5, 7, 70, 3, 7, 1, 1, 1),
+    (2, 20, 33, 5, 7, 1, 1, 1, 1), (1, 16, 16, 1, 2, 1, 1, 1, 1), (1, 3, 1, 3, 1, 1, 1, 1, 1), (13, 40, 24, 9, 9, 1, 1, 1, 1),
+    (2, 512, 128, 7, 7, 1, 1, 1, 1), (3, 80, 96, 12, 10, 1, 1, 1, 2), (4, 40, 72, 15, 14, 1, 2, 1, 1),
 ]
 
 
