@@ -575,9 +575,10 @@ __device__ __forceinline__ void lane_step(const f16x8 (&x)[4], f16x8 (&L)[8], in
 // start of the group, ahead of the filter copy (which the same wait then covers).
 // XREAL (16-product, chunk staging): the input holds its real component only (P.in.ncomp == 1); the twelve
 // products with the absent components and their operand reads are left out at compile time.
-// NORM (planes only): P0.norm is applied to what is stored.
-template <int MODE, int WCO, int NTW, int P2LOG, bool CHUNKS, bool EARLY = false, bool XREAL = false, bool NORM = false>
-__global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) qconv_fwd_f16_lds_kernel(const ConvArgsOf<NORM> P0) {
+// NORM (planes only): P0.norm is applied to what is stored.  PHASES: the correlations of a ConvPhases, one to a grid row.
+template <int MODE, int WCO, int NTW, int P2LOG, bool CHUNKS, bool EARLY = false, bool XREAL = false, bool NORM = false, bool PHASES = false>
+__global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1)
+qconv_fwd_f16_lds_kernel(const std::conditional_t<PHASES, ConvPhases, ConvArgsOf<NORM>> P0) {
     const ConvArgs P = group_view(P0);
     static_assert(!EARLY || CHUNKS, "early activation requests belong to chunk staging");
     static_assert(!XREAL || (MODE == 16 && CHUNKS), "the real-input variant is a 16-product kernel with chunk staging");
@@ -602,6 +603,9 @@ __global__ void __launch_bounds__(WG_THREADS, (MODE == 16 && NTW == 1) ? 2 : 1) 
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // (a scalar the compiler can address LDS copies with)
 
     int bid = xcd_remap(blockIdx.x, gridDim.x);
+    if constexpr (PHASES) {
+        if (bid >= conv_tiles(P)) return;  // (a phase smaller than the largest)
+    }
     const int ct = bid % P.co_tiles;
     bid /= P.co_tiles;
     const int tw = bid % P.tiles_w;

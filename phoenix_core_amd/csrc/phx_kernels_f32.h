@@ -72,6 +72,15 @@ __device__ __forceinline__ ConvArgs group_view(const ConvArgs& P0) {
     return P;
 }
 
+// Up to four correlations of one kernel instance in one launch (grid rows), each with arguments of its own: the phases of a
+// strided input gradient.  The grid is as wide as the largest one.
+constexpr int CONV_PHASES_MAX = 4;
+struct ConvPhases {
+    ConvArgs phase[CONV_PHASES_MAX];
+};
+__device__ __forceinline__ ConvArgs group_view(const ConvPhases& P0) { return P0.phase[blockIdx.y]; }
+__host__ __device__ inline int conv_tiles(const ConvArgs& a) { return a.co_tiles * a.tiles_w * a.tiles_h * a.tiles_n; }
+
 // ---------------------------------------------------------------------------------------------
 // Epilogue shared by the forward / input-gradient kernels (32x32 MFMA tiles: a lane holds one pixel
 // column, register e the channel row 8*(e/4) + 4*(lane/32) + e%4).  Vector memory instructions are

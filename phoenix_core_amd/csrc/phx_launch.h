@@ -50,6 +50,7 @@ bool fwd_f16_takes_norm(const FwdVariant& v, const ConvArgs& a);  // whether lau
 int launch_fwd_f16_norm(const FwdVariant& v, const ConvArgs& a, const NormArgs& norm, hipStream_t st);
 int launch_fwd_f16_lds8(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // 8-product, filters through LDS
 int launch_fwd_f16_lanes(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // 8-product, lanes dealt over the waves
+int launch_fwd_f16_phases(const FwdVariant& v, const ConvPhases& a, int phases, hipStream_t st);  // WCO 1 or 2
 int launch_fwd_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // fp32 on bf16 instructions
 size_t x3_lds_bytes();
 size_t x3_image_bytes(int WCO, int co_tiles, int nchunks, int ngroups);

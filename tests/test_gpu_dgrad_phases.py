@@ -1,0 +1,51 @@
+"""Strided fp16 input gradients whose phases run in one launch, against the zero-inserted form of the same kernel."""
+import pytest
+import torch
+
+import phoenix_core_amd as phx
+from phoenix_core_amd import capi, ops
+
+pytestmark = pytest.mark.gpu
+
+# n, ci, co, h, w, k, stride, dilation, padding: one and two filter sub-tiles, phases of different sizes and tap counts, a phase
+# without taps, a whole plane as one row, odd rows, channels past a chunk, strides along one axis
+CASES = [
+    (3, 36, 52, 13, 11, 3, 2, 1, "SAME"), (2, 16, 20, 9, 9, 3, 2, 1, "SAME"), (1, 70, 33, 33, 21, 4, 2, 1, "SAME"),
+    (2, 64, 64, 12, 40, 5, 2, 1, "SAME"), (4, 24, 16, 9, 9, 2, 2, 2, "VALID"), (2, 33, 17, 15, 16, 3, 2, 2, "SAME"),
+    (2, 20, 40, 10, 12, 3, (1, 2), 1, "SAME"), (2, 20, 40, 12, 10, 3, (2, 1), 1, "SAME"), (1, 8, 8, 9, 30, 3, (1, 3), 1, "SAME"),
+    (1, 40, 24, 2, 3, 3, 2, 1, "SAME"), (2, 24, 24, 17, 17, 7, 2, 1, "SAME"), (9, 130, 48, 14, 14, 3, 2, 1, "SAME"),
+]
+
+
+@pytest.mark.parametrize("policy", ["full16", ""])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_one_launch_equals_zero_insertion(case, policy, tune_env):
+    n, ci, co, h, w, k, stride, dilation, padding = case
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    wt = torch.randn(4, co, ci, k, k, generator=gen, device="cuda").half()
+    desc = ops.Conv2DDescriptor((4 * n, ci, h, w), wt.shape, stride=stride, dilation=dilation, padding=padding, dtype=torch.float16,
+                                context=phx.Context({"UPSTRIDE_CONV_FP16_POLICY": policy}))
+    grad = torch.randn(desc.output_shape, generator=gen, device="cuda").half()
+    tune_env(PHX_TUNE_PHASE="0", PHX_TUNE_KSLICES="0")
+    ref = ops.conv2d_bwd_data(wt, grad, desc)
+    assert "p16" in capi.last_kernel_name() and "phase" not in capi.last_kernel_name(), capi.last_kernel_name()
+    tune_env(PHX_TUNE_PHASE="2", PHX_TUNE_KSLICES="0")
+    dx = ops.conv2d_bwd_data(wt, grad, desc)
+    assert capi.last_kernel_name().startswith("phases"), capi.last_kernel_name()
+    assert torch.equal(dx, ref)  # (the same products, added in the same order: channels by chunks, taps by groups of them)
+    packed = ops.conv2d_pack_filters(wt, desc)
+    assert torch.equal(dx, ops.conv2d_bwd_data(torch.zeros_like(wt), grad, desc, packed=packed))
+
+
+def test_an_infinite_gradient_stays_within_its_taps(tune_env):
+    """A phase multiplies its own taps only: what one infinite gradient value reaches is what the filter reaches."""
+    wt = torch.ones(4, 64, 64, 3, 3, device="cuda").half()
+    desc = ops.Conv2DDescriptor((32, 64, 56, 56), wt.shape, stride=2, padding="SAME", dtype=torch.float16,
+                                context=phx.Context({"UPSTRIDE_CONV_FP16_POLICY": "full16"}))
+    grad = torch.ones(desc.output_shape, device="cuda").half()
+    grad[0, 0, 10, 10] = float("inf")
+    dx = ops.conv2d_bwd_data(wt, grad, desc)
+    assert capi.last_kernel_name().startswith("phases")
+    (pt, pl), _ = desc.pad_before, desc.pad_after
+    bad = ~torch.isfinite(dx[0, 0])
+    assert bad[20 - pt:23 - pt, 20 - pl:23 - pl].all() and bad.sum() == 9
