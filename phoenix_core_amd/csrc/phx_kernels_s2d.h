@@ -411,8 +411,10 @@ __host__ __device__ inline int transpose_tiles(int br, int bc) {
 // CU's address unit (16-byte accesses at odd multiples of 2 bytes take it four times as long).  Measured, 36 channels of
 // 57x43, 44 images (7.8 MB) 7.7 us, 52 channels of 29x22 (2.9 MB) 5.0; both took 11.4 while the cut
 // blocks went element by element, 64 loads and stores one after the other.
-template <typename TS>
-__global__ void __launch_bounds__(WG_THREADS) transpose_kernel(const TransposeArgs A) {
+// The matrices of A, each from src to a destination d_step elements behind the last one's, whose column c becomes row
+// row_of(c).
+template <typename TS, typename RowOf>
+__device__ __forceinline__ void transpose_body(const TransposeArgs& A, long d_step, RowOf row_of) {
     constexpr int V = 16 / sizeof(TS);
     typedef const __attribute__((address_space(1))) u32x4_a2* gload;
     typedef __attribute__((address_space(1))) u32x4_a2* gstore;
@@ -442,7 +444,7 @@ __global__ void __launch_bounds__(WG_THREADS) transpose_kernel(const TransposeAr
         if (rb >= br || cb >= bc) continue;
         int r0 = rb * V, c0 = cb * V;
         const TS* s = src + b * A.R * (long)A.Cc;
-        TS* d = dst + b * A.R * (long)A.Cc;
+        TS* d = dst + b * d_step;
         if (A.R >= V && A.Cc >= V) {
             r0 = min(r0, A.R - V);
             c0 = min(c0, A.Cc - V);
@@ -464,12 +466,42 @@ __global__ void __launch_bounds__(WG_THREADS) transpose_kernel(const TransposeAr
                                                           (j & 1) ? 0x07060302u : 0x05040100u);
             }
 #pragma unroll
-            for (int j = 0; j < V; ++j) *(gstore)(d + (long)(c0 + j) * A.R + r0) = out[j];
+            for (int j = 0; j < V; ++j) *(gstore)(d + row_of(c0 + j) * A.R + r0) = out[j];
         } else {
             for (int i = 0; i < V && r0 + i < A.R; ++i)
-                for (int j = 0; j < V && c0 + j < A.Cc; ++j) d[(long)(c0 + j) * A.R + r0 + i] = s[(long)(r0 + i) * A.Cc + c0 + j];
+                for (int j = 0; j < V && c0 + j < A.Cc; ++j) d[row_of(c0 + j) * A.R + r0 + i] = s[(long)(r0 + i) * A.Cc + c0 + j];
         }
     }
+}
+
+template <typename TS>
+__global__ void __launch_bounds__(WG_THREADS) transpose_kernel(const TransposeArgs A) {
+    transpose_body<TS>(A, A.R * (long)A.Cc, [](int c) { return (long)c; });
+}
+
+// two tensors in one launch, one to a grid row (a filter gradient's: 36 channels of 57x43 and 52 of 29x22, 44 images, 9.6 us for
+// 12.7 in two)
+struct TransposePair {
+    TransposeArgs a[2];
+};
+template <typename TS>
+__global__ void __launch_bounds__(WG_THREADS) transpose_pair_kernel(const TransposePair P) {
+    const TransposeArgs A = P.a[blockIdx.y];
+    transpose_body<TS>(A, A.R * (long)A.Cc, [](int c) { return (long)c; });
+}
+
+// phase_merge_kernel into a channels-last tensor: phase blockIdx.y of every image, [C][rows x columns of the phase], straight
+// to its pixels of [H][W][C].  11 images of 36 channels, 57x43, fp16: 7.1 us, where the merge into planes takes 8.1 and their
+// transpose 7.7.
+template <typename TS>
+__global__ void __launch_bounds__(WG_THREADS) phase_transpose_kernel(const PhaseMergeArgs M, int C) {
+    const int a = blockIdx.y / M.sw, b = blockIdx.y - a * M.sw;
+    const int Hq = (M.H - a + M.sh - 1) / M.sh, Wq = (M.W - b + M.sw - 1) / M.sw;
+    const TransposeArgs A{static_cast<const TS*>(M.buf) + M.off[blockIdx.y], M.dx, M.planes / C, C, Hq * Wq};
+    transpose_body<TS>(A, (long)C * M.H * M.W, [&](int c) {
+        const int i = c / Wq;
+        return (long)(M.sh * i + a) * M.W + M.sw * (c - i * Wq) + b;
+    });
 }
 
 // Merged groups (see merged_groups in phx_qconv.hip): m consecutive groups of a grouped convolution run as one group of

@@ -197,6 +197,8 @@ int launch_s2d_filter(bool half_storage, const S2dFilterArgs& a, bool to_caller,
 int launch_phase_merge(bool half_storage, const PhaseMergeArgs& a, hipStream_t st);
 int launch_merge_filter(bool half_storage, const MergeFilterArgs& a, bool to_caller, hipStream_t st);  // block-diagonal filters of merged groups
 // batched matrix transposes between channels-last tensors and the kernels' channels-first layout
+int launch_transpose_pair(bool half_storage, const TransposeArgs& a, const TransposeArgs& b, hipStream_t st);
+int launch_phase_transpose(bool half_storage, const PhaseMergeArgs& a, int C, hipStream_t st);  // every phase exists
 int launch_transpose(bool half_storage, const TransposeArgs& a, hipStream_t st);
 int launch_fill_zero(void* dst, size_t bytes, hipStream_t st);  // a kernel, so that it can be captured in a graph
 int launch_add_inplace(bool half_storage, void* dst, const void* src, long count, hipStream_t st);  // dst += src

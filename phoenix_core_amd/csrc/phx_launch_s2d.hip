@@ -236,11 +236,33 @@ int launch_slice_sum(bool half_storage, const void* partial, int slices, long co
     return 0;
 }
 
-int launch_transpose(bool half_storage, const TransposeArgs& a, hipStream_t st) {
-    const int V = half_storage ? 8 : 4;  // block edge of one lane
-    const long tiles = a.batch * transpose_tiles((a.R + V - 1) / V, (a.Cc + V - 1) / V);
+int launch_phase_transpose(bool half_storage, const PhaseMergeArgs& a, int C, hipStream_t st) {
+    const int V = half_storage ? 8 : 4;
+    const int most = ((a.H + a.sh - 1) / a.sh) * ((a.W + a.sw - 1) / a.sw);  // pixels of the largest phase
+    const long tiles = (a.planes / C) * transpose_tiles((C + V - 1) / V, (most + V - 1) / V);
     if (tiles == 0) return 0;
-    const int blocks = (int)std::min<long>((tiles + 3) / 4, 1 << 16);
+    const dim3 grid((unsigned int)std::min<long>((tiles + 3) / 4, 1 << 16), (unsigned int)(a.sh * a.sw));
+    if (half_storage) hipLaunchKernelGGL((phase_transpose_kernel<_Float16>), grid, dim3(WG_THREADS), 0, st, a, C);
+    else hipLaunchKernelGGL((phase_transpose_kernel<float>), grid, dim3(WG_THREADS), 0, st, a, C);
+    return 0;
+}
+
+static int transpose_blocks(const TransposeArgs& a, int V) {
+    return (int)std::min<long>((a.batch * transpose_tiles((a.R + V - 1) / V, (a.Cc + V - 1) / V) + 3) / 4, 1 << 16);
+}
+
+int launch_transpose_pair(bool half_storage, const TransposeArgs& a, const TransposeArgs& b, hipStream_t st) {
+    const int V = half_storage ? 8 : 4;
+    const dim3 grid(std::max(transpose_blocks(a, V), transpose_blocks(b, V)), 2);
+    if (grid.x == 0) return 0;
+    if (half_storage) hipLaunchKernelGGL((transpose_pair_kernel<_Float16>), grid, dim3(WG_THREADS), 0, st, TransposePair{{a, b}});
+    else hipLaunchKernelGGL((transpose_pair_kernel<float>), grid, dim3(WG_THREADS), 0, st, TransposePair{{a, b}});
+    return 0;
+}
+
+int launch_transpose(bool half_storage, const TransposeArgs& a, hipStream_t st) {
+    const int blocks = transpose_blocks(a, half_storage ? 8 : 4);  // (the block edge of one lane)
+    if (blocks == 0) return 0;
     if (half_storage) hipLaunchKernelGGL((transpose_kernel<_Float16>), dim3(blocks), dim3(WG_THREADS), 0, st, a);
     else hipLaunchKernelGGL((transpose_kernel<float>), dim3(blocks), dim3(WG_THREADS), 0, st, a);
     return 0;

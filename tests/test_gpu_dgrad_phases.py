@@ -49,3 +49,22 @@ def test_an_infinite_gradient_stays_within_its_taps(tune_env):
     (pt, pl), _ = desc.pad_before, desc.pad_after
     bad = ~torch.isfinite(dx[0, 0])
     assert bad[20 - pt:23 - pt, 20 - pl:23 - pl].all() and bad.sum() == 9
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [(3, 36, 52, 57, 43, 3, 2), (2, 70, 9, 13, 14, 3, 2), (2, 5, 16, 9, 8, 3, 2), (1, 24, 16, 3, 4, 3, 2),
+                                  (2, 16, 12, 8, 15, 5, (1, 2)), (1, 16, 8, 1, 9, 3, 2), (2, 24, 40, 10, 12, 4, 3)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_channels_last_result_is_written_by_the_phases(case, dtype, tune_env):
+    n, ci, co, h, w, k, stride = case
+    tune_env(PHX_TUNE_PHASE="2")
+    wt = torch.randn(4, co, ci, k, k, device="cuda").to(dtype)
+    args = dict(stride=stride, padding="SAME", dtype=dtype, context=phx.Context({"UPSTRIDE_CONV_FP16_POLICY": "full16"}))
+    planes = ops.Conv2DDescriptor((4 * n, ci, h, w), wt.shape, **args)
+    grad = torch.randn(planes.output_shape, device="cuda").to(dtype)
+    ref = ops.conv2d_bwd_data(wt, grad, planes)
+    assert "phase" in capi.last_kernel_name(), capi.last_kernel_name()
+    last = ops.Conv2DDescriptor((4 * n, h, w, ci), wt.shape, data_format="NHWC", **args)
+    dx = ops.conv2d_bwd_data(wt, grad.permute(0, 2, 3, 1).contiguous(), last)
+    assert "phase" in capi.last_kernel_name(), capi.last_kernel_name()
+    assert torch.equal(dx.permute(0, 3, 1, 2), ref)
