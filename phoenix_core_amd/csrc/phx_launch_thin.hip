@@ -927,14 +927,19 @@ static int thin_wgrad_taps_per_block(int taps) { return taps == 1 ? 1 : 9; }
 static bool thin_wgrad_plan(bool half_storage, ThinArgs& a, size_t& lds) {
     const int taps = a.Kh * a.Kw, TB = thin_wgrad_taps_per_block(taps);
     const long columns = (long)a.groups * a.cog * a.cig * ((taps + TB - 1) / TB);
-    const long want = (2048 + columns - 1) / columns;
+    // Tiles: one round of four workgroups a CU where a workgroup has all taps -- each ends in a sum over its threads, and a few
+    // workgroups beyond the round would be a second one (depthwise 3x3, us with 2048 workgroups / these: N=32, 128 channels at
+    // 28x28 37 / 33, 64 at 56x56 53 / 49, 48 at 112x112 131 / 121, N=8, 32 at 112x112 46 / 35, N=16, 100 at 33x21 29 / 22); twice
+    // that where nine taps of more share it (5x5, N=16, 96 at 40x30 46 / 48), and for fp32 tensors, whose sums would grow longer
+    // (128 channels at 28x28 42 / 37 us, but 2-norm error against fp64 1.5e-7 / 1.7e-7; fp16 results round to 2e-4 either way).
+    const long want = TB < taps || !half_storage ? (2048 + columns - 1) / columns : std::max(1L, 1024 / columns);
     if (!tuning_thin_notile() && thin_tile_plan(half_storage, false, 0, THIN_WG_PXT * WG_THREADS, THIN_TILE_LDS - thin_wgrad_sums_bytes(TB), a, lds)) {
         const long ntiles = (long)((a.N + a.tile_J - 1) / a.tile_J) * a.tile_bands;
         a.Z = (int)std::max(1L, std::min({want, ntiles, 65535L}));
         return true;
     }
     const long fit = std::max(1L, (long)a.N * a.Ho * a.Wo / (4 * WG_THREADS));
-    a.Z = (int)std::max(1L, std::min({want, fit, (long)a.N, 65535L}));
+    a.Z = (int)std::max(1L, std::min({(2048 + columns - 1) / columns, fit, (long)a.N, 65535L}));
     return false;
 }
 
