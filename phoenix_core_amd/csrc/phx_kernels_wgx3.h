@@ -15,8 +15,8 @@ namespace phx {
 //   once for three taps.
 // A thread makes the eight lanes and their three parts of one component quadruple of four pixels (waves 0-3: gradient, 4-6:
 // input), some 260 instructions, from values loaded a step ahead, into the other half of a double buffer.  The two waves of a
-// SIMD take turns: one starts a step with its products, the other with its staging, so that one's products run beside the
-// other's arithmetic.
+// SIMD take turns: one starts a step with its staging (the gradient's), the other with its products, so that one's products run
+// beside the other's arithmetic.
 //
 // Rounding: the instructions' sums drop their lowest bits downwards, the same way whatever the sign, which over thousands of
 // steps adds up.  Every K step's six products therefore start from zero and are added to the accumulator by an ordinary
@@ -24,10 +24,10 @@ namespace phx {
 // values, here / fp32 instructions): 3x3, 128 x 48 channels at 9x9 1.8e-7 / 3.4e-7, 16 x 512 at 7x7 2.4e-7 / 4.7e-7, 4 x 256 at
 // 14x14 1.6e-7 / 2.9e-7; without the negation 6.3e-7, 2.4e-7, 2.0e-7; accumulated by the instructions 1.5-2 times as much again.
 //
-// Bound: the two pipes of a SIMD together.  64 channels at 56x56, N=64 (1399 us on fp32 instructions, 790 here): a step of
-// 2.6 us holds 72 products of 32 clocks and 700 vector instructions of 4, which overlap in part: 610 us without the staging,
-// 450 without the products.  (Tried: the additions dealt between the products 850, subtracting parts by dot2 instructions 868,
-// other pairings of the waves 858.)
+// Bound: the two pipes of a SIMD together.  64 channels at 56x56, N=64 (1399 us on fp32 instructions, 770 here): a step of
+// 2.5 us holds 72 products of 32 clocks and 700 vector instructions of 4, which overlap in part: 610 us without the staging,
+// 450 without the products.  (Tried, against 800 with the gradient's products first: the additions dealt between the products 850,
+// subtracting parts by dot2 instructions 868, neighbouring waves in turn 858.)
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
 
 constexpr int WGX3_TPW = 3;                              // taps of a filter row
@@ -206,11 +206,16 @@ __global__ void __launch_bounds__(WGX3_THREADS, 1) qconv_wgrad_x3_kernel(const W
         wg_barrier_no_vmem_wait();
         int buf = 0;
         for (int tile = zi; tile < P.ntiles; tile += P.zsplit, buf ^= 1) {
+            const auto turn = [&] {  // (ahead of the other wave's arithmetic)
+                __builtin_amdgcn_s_setprio(2);
+                products(buf);
+                __builtin_amdgcn_s_setprio(0);
+            };
             const bool more = tile + P.zsplit < P.ntiles, more2 = more && tile + 2 * P.zsplit < P.ntiles;
-            if (wave < 4) { __builtin_amdgcn_s_setprio(2); products(buf); __builtin_amdgcn_s_setprio(0); }
+            if (wave >= 4) turn();
             if (more) convert(buf ^ 1);
             if (more2) issue();
-            if (wave >= 4) { __builtin_amdgcn_s_setprio(2); products(buf); __builtin_amdgcn_s_setprio(0); }
+            if (wave < 4) turn();
             wg_barrier_no_vmem_wait();
         }
     }
