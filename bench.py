@@ -12,8 +12,8 @@ short JSON line of the contract (under 1800 characters): headline (`value`, `roo
 = the ResNet-50's images/s.  `--workload NAME` runs one configuration alone (used for profiling).
 
 Throughput is real-equivalent: 16 real multiply-adds per quaternion multiply-add whichever product
-formulation runs; the factorized (8-product) kernels execute half of them, which `executed_frac`
-reports next to the real-equivalent `frac`.
+formulation runs; the factorized (8-product) kernels execute half of them and the kernels on bf16 parts six times as many
+(on instructions of sixteen times the rate), which `executed_frac` reports next to the real-equivalent `frac`.
 """
 import argparse
 import ctypes
@@ -60,8 +60,14 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.md")
 def executed_share(kernel_name):
     """Executed / real-equivalent arithmetic of a kernel: the factorized (8-product) kernels run half the
     multiplications.  The product mode asks for a formulation; where the 16-product kernel is the faster one
-    the library runs that in either mode, so the share is read off the kernel that actually ran."""
-    return 0.5 if "_p8_" in kernel_name else 1.0
+    the library runs that in either mode, so the share is read off the kernel that actually ran.  Kernels on three bf16
+    parts a value run six products for one."""
+    return (0.5 if "_p8_" in kernel_name else 1.0) * (6.0 if on_bf16_parts(kernel_name) else 1.0)
+
+
+def on_bf16_parts(kernel_name):
+    """fp32 passes whose products are made by the bf16 matrix instructions: their roof is those instructions' peak."""
+    return "f32mfmax3" in kernel_name or "f32mfmagemm" in kernel_name
 
 
 def measured_traffic():
@@ -312,7 +318,7 @@ def roofline_of(pass_name, kernel, flops, nbytes, kernel_ms, compute, counters):
     run of this kernel variant say it is held by: "mfma" when the matrix pipe is busy at least half the
     time, "hbm" when the measured traffic moves at half of peak bandwidth or more, otherwise "issue/latency";
     null when the variant has no counter row."""
-    peak = PEAK_TFLOPS[compute]
+    peak = PEAK_TFLOPS["f16" if on_bf16_parts(kernel) else compute]  # (bf16 instructions run at the fp16 rate)
     tflops = flops / (kernel_ms * 1e-3) / 1e12
     gbs = nbytes / (kernel_ms * 1e-3) / 1e9
     share = executed_share(kernel)
