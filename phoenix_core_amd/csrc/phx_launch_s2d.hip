@@ -199,13 +199,16 @@ __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial
                                                                const std::conditional_t<NORM, NormArgs, NoNorm> norm) {
     const long stride = (long)gridDim.x * blockDim.x;
     for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += stride) {
-        float sum[4] = {0.f, 0.f, 0.f, 0.f};  // (four loads in flight)
+        float acc = 0.0f;
         int z = 0;
-        for (; z + 4 <= slices; z += 4)
+        for (; z + 4 <= slices; z += 4) {  // (four loads in flight; added one after the other, the order of a plain loop)
+            TS v[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sum[i] += (float)partial[(z + i) * count + e];
-        for (; z < slices; ++z) sum[0] += (float)partial[z * count + e];
-        float acc = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            for (int i = 0; i < 4; ++i) v[i] = partial[(z + i) * count + e];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc += (float)v[i];
+        }
+        for (; z < slices; ++z) acc += (float)partial[z * count + e];
         if (bias) acc += (float)bias[(e / comp_count) * channels + (e / plane) % channels];
         if constexpr (NORM) {
             acc = norm_apply(norm_factors(norm, (int)((e / plane) % channels)), acc);

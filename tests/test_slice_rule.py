@@ -60,3 +60,16 @@ def test_passes_that_run_in_slices(case, which, slices, tune_env):
     n, ci, co, h, w, k, stride = case[:7]
     outputs = 4 * n * co * -(-h // stride) * -(-w // stride) if which == FWD else 4 * n * ci * h * w
     assert planned >= slices * outputs * 2 and planned != whole  # (that many partial tensors at least)
+
+
+@pytest.mark.parametrize("case,which", [(c, w) for c, w, _ in SLICED], ids=str)
+def test_slices_keep_32_channels(case, which, tune_env):
+    """A slice's sums are rounded to the tensors' type: one per 32 reduced channels at most, also where slices are asked for."""
+    _, whole = workspaces(case, which, tune_env)
+    n, ci, co, h, w, k, stride, policy = case
+    desc = phx.Conv2DDescriptor((4 * n, ci, h, w), (4, co, ci, k, k), stride, 1, "SAME", dtype=torch.float16, context=Ctx(policy))
+    red = ci if which == FWD else co
+    tune_env(PHX_TUNE_KSLICES=str(red // 16))
+    assert desc.workspace_bytes(which) == whole
+    tune_env(PHX_TUNE_KSLICES=str(red // 32))
+    assert desc.workspace_bytes(which) != whole
