@@ -234,8 +234,8 @@ int phx_qconv2d_bwd_data_add(const phx_qconv_desc* desc, phx_stream_t stream, co
  * y = gamma * (conv(x, w) (+ bias) - mean) / sqrt(var + eps) + beta (+ residual), then the optional ReLU; the parameters are
  * per output channel (the four components share them), the residual is laid out like y and is not y itself.  No counterpart
  * in the reference's interface; it is what a network in evaluation mode does next with a convolution's result, and saves that
- * pass over it: the fp16 kernels normalise in fp32 what they store, every other path is followed by the pass of
- * phx_bn_fwd_eval.  NCHW quaternion descriptors; packed_fwd_or_null, workspace as phx_qconv2d_fwd_prepacked /
+ * pass over it: the fp16 kernels normalise in fp32 the rounded results that they would store, every other path is followed by
+ * the pass of phx_bn_fwd_eval.  The result is bit for bit that of phx_qconv2d_fwd and phx_bn_fwd_eval one after the other.  NCHW quaternion descriptors; packed_fwd_or_null, workspace as phx_qconv2d_fwd_prepacked /
  * phx_qconv2d_fwd; limits of phx_bn_fwd_eval. */
 typedef struct phx_output_norm {
     const float *gamma, *beta, *mean, *var;

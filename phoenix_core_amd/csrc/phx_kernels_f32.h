@@ -31,6 +31,10 @@ __device__ __forceinline__ f32x4 norm_factors(const NormArgs& n, int c) {
 }
 // (the mean is taken off first: a scaled mean folded into beta would cancel against a large x)
 __device__ __forceinline__ float norm_apply(const f32x4& f, float v) { return f[0] * (v - f[1]) + f[2]; }
+// A convolution's result v on its way out: rounded to TS, as the pass of its own would read it, so that the two ways give the
+// same bits.
+template <typename TS>
+__device__ __forceinline__ float norm_result(const f32x4& f, float v) { return norm_apply(f, (float)(TS)v); }
 __device__ __forceinline__ float relu_if(int relu, float v) { return (relu && v < 0.f) ? 0.f : v; }  // (NaN stays)
 
 struct ConvArgs {
@@ -145,7 +149,7 @@ __device__ __forceinline__ void norm_tail(const NormArgs& norm, long at, float (
     for (int i = 0; i < V; ++i) o[i] = relu_if(norm.relu, o[i]);
 }
 
-// NORM: norm is applied in fp32, in front of the one rounding; factors[i] belongs to channel co_base + i.
+// NORM: norm is applied to the rounded results, in fp32; factors[i] belongs to channel co_base + i.
 template <typename TS, int MODE, int NTW, int NACC, bool NORM = false>
 __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&acc)[NTW][NACC], int co_base,
                                               const long (&oaddr)[NTW], const bool (&pvalid)[NTW], const f32x4* factors = nullptr,
@@ -182,7 +186,7 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& P, const f32x16 (&
                 if constexpr (NORM) {
                     const f32x4 f = factors[8 * rq + k];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) y[k][q] = norm_apply(f, y[k][q]);
+                    for (int q = 0; q < 4; ++q) y[k][q] = norm_result<TS>(f, y[k][q]);
                 }
             }
             if (P.vec == 4) {

@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_f16_lanes_kernel(cons
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) c[e][q] = norm_apply(f, c[e][q]);
+                    for (int e = 0; e < 8; ++e) c[e][q] = norm_result<_Float16>(f, c[e][q]);
                     if (res) {
                         f16x8 rv = {};
                         const long at = q * P.out_cs + co * plane_out;

@@ -83,21 +83,30 @@ struct PwxNormArgs : PwxArgs {  // of the instances PWX_NORM and PWX_NORM_ADD
     NormArgs norm;
 };
 
-// What is done to a result on its way out: nothing; addend added (fp16, to the rounded result); evaluation-mode batch norm
-// and ReLU; the same with the addend as the residual between the two (the normalised value is rounded in front of the
-// addition, where a pass of its own rounds the convolution's result: the same number of roundings).
+// What is done to a result, rounded to fp16, on its way out: nothing; addend added (fp16); evaluation-mode batch norm and
+// ReLU in fp32, rounded once more; the same with the addend as the residual between the two.
 enum { PWX_PLAIN = 0, PWX_ADD = 1, PWX_NORM = 2, PWX_NORM_ADD = 3 };
 template <int TAIL>
 using PwxArgsOf = std::conditional_t<(TAIL >= 2), PwxNormArgs, PwxArgs>;  // (a literal: the name of an unnamed enum's value differs between host and device symbols)
 
-// the ReLU on packed halves; NaN stays
-__device__ __forceinline__ unsigned int relu_pair(unsigned int v) {
-    const f16x2 h = __builtin_bit_cast(f16x2, v);
-    f16x2 r;
-    const _Float16 a = h[0], b = h[1];
-    r[0] = a < (_Float16)0 ? (_Float16)0 : a;
-    r[1] = b < (_Float16)0 ? (_Float16)0 : b;
-    return __builtin_bit_cast(unsigned int, r);
+// rounded results of one channel through norm, residual (RES) and ReLU, as bn_eval_kernel takes them
+template <bool RES, typename W>
+__device__ __forceinline__ W norm_words(const f32x4& factors, const W& y, const W& res, int relu) {
+    W out;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(W) / 4); ++i) {
+        const f16x2 h = __builtin_bit_cast(f16x2, (unsigned int)y[i]), r = __builtin_bit_cast(f16x2, (unsigned int)res[i]);
+        f16x2 o;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            float v = norm_apply(factors, (float)h[e]);
+            asm("" : "+v"(v));  // (an fp32 value: v_fma_mixlo_f16 would round the product and sum to fp16 at once)
+            if constexpr (RES) v += (float)r[e];
+            o[e] = (_Float16)relu_if(relu, v);
+        }
+        out[i] = __builtin_bit_cast(unsigned int, o);
+    }
+    return out;
 }
 
 // the arguments as group blockIdx.y sees them
@@ -353,8 +362,14 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
         if constexpr (TSTORE && ADD) request_addend(0, ad);
         const int co = co0 + j;
         const bool co_ok = co < P.Cout;
-        f32x4 factors;
-        if constexpr (NORM) factors = norm_factors(P0.norm, co_ok ? co : 0);
+        f32x4 factors[4];  // TSTORE: of the channels that this lane stores; else of its own
+        if constexpr (NORM) {
+#pragma unroll
+            for (int i = 0; i < (TSTORE ? 4 : 1); ++i) {
+                const int c = co0 + (TSTORE ? 8 * i + (lane >> 3) : j);
+                factors[i] = norm_factors(P0.norm, c < P.Cout ? c : 0);
+            }
+        }
         wait_vmem_all();  // this wave's copies of the steps ahead: landed
         PHX_STAMP(2)
         char* scr = reinterpret_cast<char*>(lds16 + RF * WV + RA * XV) + wave * (S::SCRV * 16);  // (TSTORE) this wave's own
@@ -372,13 +387,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
 #pragma unroll
                     for (int k2 = 0; k2 < 2; ++k2) {
                         f16x2 h;
-                        if constexpr (NORM) {
-#pragma unroll
-                            for (int e = 0; e < 2; ++e) {
-                                const float v = norm_apply(factors, acc[q][m][g4 * 4 + 2 * k2 + e] + bv);
-                                h[e] = (_Float16)(ADD ? v : relu_if(P0.norm.relu, v));
-                            }
-                        } else if constexpr (BIAS) {
+                        if constexpr (BIAS) {
                             h[0] = (_Float16)(acc[q][m][g4 * 4 + 2 * k2] + bv);
                             h[1] = (_Float16)(acc[q][m][g4 * 4 + 2 * k2 + 1] + bv);
                         } else {
@@ -398,10 +407,10 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
                         for (int a = 0; a < NOA; ++a)
                             if (a == 4 * mt + g4) { oa = oaddr[a]; ov = ovalid[a]; }
                         if (ov && co_ok) {
-                            if constexpr (ADD) v = add_halves4(v, load8_a2(P.addend + q * P.out_cs + (long)co * HW + oa + 4 * kk));
-                            if constexpr (ADD && NORM) {
-                                if (P0.norm.relu) v = u32x2{relu_pair(v[0]), relu_pair(v[1])};
-                            }
+                            u32x2 a = v;
+                            if constexpr (ADD) a = load8_a2(P.addend + q * P.out_cs + (long)co * HW + oa + 4 * kk);
+                            if constexpr (NORM) v = norm_words<ADD>(factors[0], v, a, P0.norm.relu);
+                            else if constexpr (ADD) v = add_halves4(v, a);
                             *reinterpret_cast<u32x2_a2*>(dst + oa + 4 * kk) = v;
                         }
                     }
@@ -415,10 +424,8 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     t[i] = *reinterpret_cast<const u32x4*>(scr + ((8 * i + (lane >> 3)) * 9 + (lane & 7)) * 16);
-                    if constexpr (ADD) t[i] = add_halves(t[i], ad[i]);
-                    if constexpr (ADD && NORM) {
-                        if (P0.norm.relu) t[i] = u32x4{relu_pair(t[i][0]), relu_pair(t[i][1]), relu_pair(t[i][2]), relu_pair(t[i][3])};
-                    }
+                    if constexpr (NORM) t[i] = norm_words<ADD>(factors[i], t[i], ADD ? ad[i] : t[i], P0.norm.relu);
+                    else if constexpr (ADD) t[i] = add_halves(t[i], ad[i]);
                 }
                 if constexpr (ADD) {
                     if (q < 3) request_addend(q + 1, ad);  // (in front of this component's stores)

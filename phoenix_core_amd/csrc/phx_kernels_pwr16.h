@@ -210,10 +210,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
                         f16x2 h;
 #pragma unroll
                         for (int e = 0; e < 2; ++e) {
-                            float v = agpr_value(acc[wc][q][4 * g + 2 * i + e]) + bv;
-                            if constexpr (NORM) v = norm_apply(factors, v);
-                            if constexpr (NORM && !ADD) v = relu_if(P0.norm.relu, v);
-                            h[e] = (_Float16)v;
+                            h[e] = (_Float16)(agpr_value(acc[wc][q][4 * g + 2 * i + e]) + bv);
                         }
                         d[g][i] = __builtin_bit_cast(unsigned int, h);
                     }
@@ -226,10 +223,8 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
                         v[i] = s[0];
                         v[2 + i] = s[1];
                     }
-                    if constexpr (ADD) v = add_halves(v, ad[a]);
-                    if constexpr (ADD && NORM) {
-                        if (P0.norm.relu) v = u32x4{relu_pair(v[0]), relu_pair(v[1]), relu_pair(v[2]), relu_pair(v[3])};
-                    }
+                    if constexpr (NORM) v = norm_words<ADD>(factors, v, ADD ? ad[a] : v, P0.norm.relu);
+                    else if constexpr (ADD) v = add_halves(v, ad[a]);
                     if (ovalid[a] && co_ok) *reinterpret_cast<u32x4_a2*>(dst + oaddr[a]) = v;
                 }
             }

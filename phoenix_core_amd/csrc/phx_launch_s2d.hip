@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial
         for (; z < slices; ++z) acc += (float)partial[z * count + e];
         if (bias) acc += (float)bias[(e / comp_count) * channels + (e / plane) % channels];
         if constexpr (NORM) {
-            acc = norm_apply(norm_factors(norm, (int)((e / plane) % channels)), acc);
+            acc = norm_result<TS>(norm_factors(norm, (int)((e / plane) % channels)), acc);
             if (norm.res) acc += (float)static_cast<const TS*>(norm.res)[e];
             acc = relu_if(norm.relu, acc);
         }

@@ -381,7 +381,7 @@ def _hooked(module):
 
 
 def _conv_norm(conv, norm, x, residual=None):
-    """norm(conv(x), residual), as one operator where that can be told from the two by nothing but its rounding: both
+    """norm(conv(x), residual), as one operator (the same bits) where that can be told from the two by nothing: both
     modules are this file's and unhooked, norm is in evaluation mode, and no gradient is recorded.  (A network in evaluation
     mode is bound by the host: parameters are taken from the modules' dictionaries, not through Module.__getattr__.)"""
     if (type(conv) is QConv2d and type(norm) is QBatchNorm2d and not norm.training and not torch.is_grad_enabled() and

@@ -68,6 +68,46 @@ def test_normalised_on_the_way_out(case, residual, relu):
         assert bool(((got.double() - want.double()).abs() <= eps * 1.01 * _gap(want, conv, own, res) + 1e-7).all())
 
 
+# (more of the pointwise kernels: half items, several items a workgroup, odd planes behind four sub-tiles)
+@pytest.mark.parametrize("residual,relu", [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize("case", CASES + [(64, 64, 128, 14, 14, 1, 1, FACTORIZED, {"bias": True}, "mfmapw"),
+                                          (5, 128, 96, 7, 9, 1, 1, FACTORIZED, {}, ""), (32, 16, 64, 28, 28, 1, 1, FACTORIZED, {}, "mfmapw")],
+                         ids=lambda c: "%dx%d-%d_%dx%d_k%ds%d_%s" % (c[:7] + (c[9] or "-".join(c[8]),)))
+def test_the_bits_of_the_two_operators(case, residual, relu):
+    n, ci, co, h, w, k, stride, env, opt, path = case
+    dtype = torch.float32 if opt.get("f32") else torch.float16
+    groups, real = opt.get("groups", 1), opt.get("real", False)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")
+    x, wt = rnd((n if real else 4 * n), ci, h, w).to(dtype), (rnd(4, co, ci // groups, k, k) * (ci * k * k) ** -0.5).to(dtype)
+    bias = rnd(4, co).to(dtype) if opt.get("bias") else None
+    desc = ops.Conv2DDescriptor(x.shape, wt.shape, stride=stride, padding="SAME", use_bias=bias is not None, dtype=dtype,
+                                context=phx.Context(env), groups=groups, real_valued_input=real)
+    # (normalised values beyond fp16's range, which the residual brings back into it)
+    own = (rnd(co) * 4e4, rnd(co), rnd(co), rnd(co).abs() + 0.2)
+    res = (rnd(*desc.output_shape) * 4e4).to(dtype) if residual else None
+    got = ops.conv2d_fwd_norm(x, wt, bias, desc, *own, 1e-5, relu, res)
+    assert path in capi.last_kernel_name()
+    assert torch.equal(got, ops.batch_norm_eval(phx.conv2d_fwd(x, wt, bias, desc), *own, 1e-5, relu, res))
+
+
+@pytest.mark.parametrize("env", [FACTORIZED, PRODUCTS, MIXED], ids=["factorized", "products", "mixed"])
+def test_a_network_gives_the_bits_of_its_operators(env):
+    torch.manual_seed(4)
+    model = qnn.QResNet50(dtype=torch.float16, context=phx.Context(env)).cuda()
+    images = torch.randn(2, 3, 96, 80, device="cuda").half()
+    for m in model.modules():
+        m.momentum = 1.0  # (statistics that fit the activations)
+    with torch.no_grad():
+        model(images)
+        one = model.eval()(images)
+        assert bool(torch.isfinite(one).all())
+        for m in model.modules():  # (a module with a hook is called by itself)
+            if isinstance(m, qnn.QBatchNorm2d):
+                m.register_forward_hook(lambda m, i, o: None)
+        assert torch.equal(one, model(images))
+
+
 def test_not_a_number_passes_the_relu():
     desc = ops.Conv2DDescriptor((8, 16, 8, 8), (4, 64, 16, 1, 1), dtype=torch.float16, context=phx.Context(FACTORIZED))
     x, wt = torch.zeros(8, 16, 8, 8, device="cuda").half(), torch.ones(4, 64, 16, 1, 1, device="cuda").half()
