@@ -26,7 +26,7 @@ constexpr int PWX3_PX = 64;
 constexpr int PWX3_LDS_BYTES = 8 * 32 * PWX3_PX * 4;  // the epilogue's exchange of the product lanes
 constexpr int pwx3_vectors(int S) { return 2 * 3 * S * 64; }  // 16-byte vectors of a wave's filters per K step: [lane][part][sub-tile][64]
 
-inline size_t pwx3_packed_bytes(int S, int co_tiles, int nsteps) { return (size_t)co_tiles * 4 * nsteps * pwx3_vectors(S) * 16; }
+__host__ __device__ inline size_t pwx3_packed_bytes(int S, int co_tiles, int nsteps) { return (size_t)co_tiles * 4 * nsteps * pwx3_vectors(S) * 16; }
 
 typedef u32x2 u32x2_a4 __attribute__((aligned(4)));
 
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvAr
                     for (int i = 0; i < 2; ++i) {
                         const unsigned int ua = xa[2 * q + i][t], ub = xb[2 * q + i][t];
                         const float a = __builtin_bit_cast(float, ua), b = __builtin_bit_cast(float, ub);
-                        v[i] = l ? a - b : a + b;
+                        v[i] = fmaf(a, SPLIT_SCALE, l ? -SPLIT_SCALE * b : SPLIT_SCALE * b);
                     }
 #pragma unroll
                     for (int u = 0; u < 3; ++u) {
@@ -157,6 +157,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvAr
         o[h] = (long)img[h] * P.CoutS * plane + p[h];
     }
     const bool joined = ok[1] && o[1] == o[0] + 2;
+    float bad = 0.f;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         if (s > 0) wg_barrier_no_vmem_wait();  // the previous round has been read
@@ -178,6 +179,9 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvAr
             merge_output(in, y);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
+                y[q] *= SPLIT_RESULT;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) split_check(bad, y[q][k]);
                 if (bias) y[q] += bias[q * P.CoutS + co];
                 float* const d = out + q * P.out_cs + (long)co * plane;
                 if (joined) {
@@ -190,15 +194,24 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvAr
             }
         }
     }
+    if (bad != bad) {  // (rare; see phx_kernels_x3.h)
+        const f32x4* const copy = reinterpret_cast<const f32x4*>(static_cast<const char*>(P.wpk) + pwx3_packed_bytes(S, P.co_tiles, P.nchunks));
+#pragma unroll 1
+        for (int i = 0; i < 4 * 2 * S; ++i) {
+            const int co = ct * S * 32 + row0 + 16 * (i >> 2), h = (i >> 1) & 1, pixel = p[h] + (i & 1), y = pixel / P.in.Wd;
+            if (co < P.Cout && ok[h]) conv_again(P, copy, img[h], y, pixel - y * P.in.Wd, co);
+        }
+    }
 }
 
-// Filter packing: [filter tile of S * 32][wave][K step][lane][part][sub-tile][64] x 8 bf16 (conjugated / transposed for MAP_DGRAD).
-// One thread per (tile, K step, sub-tile, row, channel of the step): eight product lanes from the same four filter values.
+// Filter packing: [filter tile of S * 32][wave][K step][lane][part][sub-tile][64] x 8 bf16 (conjugated / transposed for MAP_DGRAD),
+// then the fp32 copy (phx_kernels_x3.h).  One thread per (tile, K step, sub-tile, row, channel of the step): eight product lanes from the same four filter values.
 template <int MAP>
 __device__ __forceinline__ void pack_filters_pwx3_body(const PackArgs& P, int S, long first, long stride) {
     const long total = (long)P.row_tiles * P.nchunks * S * 32 * PWX3_STEP;
     const float* w = static_cast<const float*>(P.w);
     __bf16* outh = static_cast<__bf16*>(P.out);
+    f32x4* const copy = reinterpret_cast<f32x4*>(static_cast<char*>(P.out) + pwx3_packed_bytes(S, P.row_tiles, P.nchunks));
     for (long idx = first; idx < total; idx += stride) {
         const int i = idx & 7, r = (idx >> 3) & 31, k8 = (idx >> 8) & 1;
         long s = idx >> 9;
@@ -214,6 +227,9 @@ __device__ __forceinline__ void pack_filters_pwx3_body(const PackArgs& P, int S,
             float wv[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) wv[c] = ((MAP == MAP_DGRAD && c > 0) ? -1.f : 1.f) * w[c * P.wcs + off];
+            copy[(long)red * P.rows + row] = f32x4{wv[0], wv[1], wv[2], wv[3]};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) wv[c] *= SPLIT_SCALE;
             lanes_right(wv, R);
         }
 #pragma unroll

@@ -41,6 +41,37 @@ constexpr int WGX3_LDS_BYTES = 2 * WGX3_BUF;
 constexpr int WGX3_PITCH = WGX3_CI + 1;                  // epilogue: [lane][co][ci]
 static_assert(8 * WGX3_CO * WGX3_PITCH * 4 <= WGX3_LDS_BYTES && WGX3_LDS_BYTES <= 160 * 1024, "LDS of the split filter gradient");
 
+// tap (kh, kw) of channels (co, ci), over the segments of reduction slice zi, in fp32
+__device__ __forceinline__ void wgrad_fp32(const WgradArgs& P, int zi, int kh, int kw, int co, int ci, float (&y)[4]) {
+    const long xplane = (long)P.x.Hd * P.x.Wd, gplane = (long)P.g.Hd * P.g.Wd;
+    const int rows = P.g.Hd;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = 0.f;
+    for (int tile = zi; tile < P.ntiles; tile += P.zsplit)
+        for (int seg = 2 * tile; seg < 2 * tile + 2; ++seg) {
+            const int line = seg / P.cpr, img = line / rows, ho = line - img * rows, h = ho * P.sh + kh * P.dh - P.pt;
+            if (img >= P.g.N || h < 0 || h >= P.x.Hd) continue;
+            const float* const x = static_cast<const float*>(P.x.base) + ((long)img * P.x.Cs + ci) * xplane + (long)h * P.x.Wd;
+            const float* const g = static_cast<const float*>(P.g.base) + ((long)img * P.g.Cs + co) * gplane + (long)ho * P.g.Wd;
+            const int c0 = (seg - line * P.cpr) * 8;
+            for (int c = c0; c < min(c0 + 8, P.g.Wd); ++c) {
+                const int w = c + kw - P.pl;
+                if (w < 0 || w >= P.x.Wd) continue;
+                float xv[4], gv[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    xv[i] = x[i * P.x.comp_stride + w];
+                    gv[i] = g[i * P.g.comp_stride + c];
+                }
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) y[r] = fmaf(qneg(p, p ^ r) ? -xv[p] : xv[p], gv[p ^ r], y[r]);
+            }
+            if (all_nan(y)) return;
+        }
+}
+
 __global__ void __launch_bounds__(WGX3_THREADS, 1) qconv_wgrad_x3_kernel(const WgradArgs P0) {
     const WgradArgs P = group_view(P0);
     extern __shared__ u32x4 ldswgx3[];
@@ -84,7 +115,7 @@ __global__ void __launch_bounds__(WGX3_THREADS, 1) qconv_wgrad_x3_kernel(const W
     const int step_c = step % P.cpr, step_h = (step / P.cpr) % rows, step_n = step / (P.cpr * rows);
 
     const unsigned int sign = (unsigned int)zi << 31;  // odd slices: on the negated gradient
-    u32x4 v[4];
+    u32x4 v[4] = {};        // (finite where nothing is loaded: multiplied by zero)
     unsigned int keep = 0;  // pixels of the task inside the image
     auto issue = [&]() {    // requests the values of the current tile; steps to the workgroup's next one
         const int r = ho * row_step + row0, c = cc * 8 + col0;
@@ -117,10 +148,10 @@ __global__ void __launch_bounds__(WGX3_THREADS, 1) qconv_wgrad_x3_kernel(const W
         float lanes[PX][8];
 #pragma unroll
         for (int k = 0; k < PX; ++k) {
-            const unsigned int m = (unsigned int)((int)(keep << (31 - k)) >> 31);
+            const float m = ((keep >> k) & 1) ? (ROLE == 0 && sign ? -SPLIT_SCALE : SPLIT_SCALE) : 0.f;
             float e[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) e[q] = __builtin_bit_cast(float, ROLE == 0 ? (v[q][k] & m) ^ sign : v[q][k] & m);
+            for (int q = 0; q < 4; ++q) e[q] = __builtin_bit_cast(float, (unsigned int)v[q][k]) * m;
             if constexpr (ROLE == 0) lanes_grad(e, lanes[k], 0.5f);
             else lanes_left(e, lanes[k]);
         }
@@ -224,6 +255,7 @@ __global__ void __launch_bounds__(WGX3_THREADS, 1) qconv_wgrad_x3_kernel(const W
     const long tap_stride = 4L * P.CoP * P.CiP, comp = (long)P.CoP * P.CiP;
     float* const dst = P.partial + ((long)zi * P.Kh * P.Kw + kh * P.Kw + kw0) * tap_stride;
     float* const xch = reinterpret_cast<float*>(lds);
+    float bad = 0.f;
 #pragma unroll
     for (int t = 0; t < WGX3_TPW; ++t) {
         if (t >= nkw) continue;
@@ -243,6 +275,27 @@ __global__ void __launch_bounds__(WGX3_THREADS, 1) qconv_wgrad_x3_kernel(const W
                 l[i] = __builtin_bit_cast(float, __builtin_bit_cast(unsigned int, xch[(i * WGX3_CO + co) * WGX3_PITCH + j]) ^ sign);
             merge_right_grad(l, y);
             float* const d = dst + t * tap_stride + (long)(cot * WGX3_CO + co) * P.CiP + cit * WGX3_CI + j;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                y[r] *= SPLIT_RESULT;
+                split_check(bad, y[r]);
+                d[r * comp] = y[r];
+            }
+        }
+    }
+    if (bad != bad) {  // (rare; see phx_kernels_x3.h) sums that are not finite, once more in fp32
+        constexpr int ROUNDS = WGX3_CO * WGX3_CI / WGX3_THREADS;
+#pragma unroll 1
+        for (int i = 0; i < ROUNDS * nkw; ++i) {
+            const int t = i / ROUNDS, row = cot * WGX3_CO + (tid >> 5) + (i - t * ROUNDS) * (WGX3_THREADS / 32), column = cit * WGX3_CI + j;
+            if (row >= P.g.C || column >= P.x.C) continue;
+            float* const d = dst + t * tap_stride + (long)row * P.CiP + column;
+            bool again = false;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) again = again || split_bad(d[r * comp]);
+            if (!again) continue;
+            float y[4];
+            wgrad_fp32(P, zi, kh, kw0 + t, row, column, y);
 #pragma unroll
             for (int r = 0; r < 4; ++r) d[r * comp] = y[r];
         }

@@ -13,8 +13,15 @@ namespace phx {
 // each as one 32x32x16 instruction over 8 channels of two parts (K halves | ), whose products are exact and whose sums are
 // fp32.  Three instructions of 32 clocks take the place of four fp32 instructions of 64.  Error of a K-long sum against fp64,
 // standard normal operands, relative 2-norm: K = 64 1.34e-7 (fp32 instructions 1.42e-7), 256 2.4e-7 (3.0e-7), 2304 7.9e-7
-// (8.3e-7): it rounds a fraction as often.  An infinite operand gives NaN (inf - inf in its parts; the factorized form gives
-// NaN in three components of four anyway).
+// (8.3e-7): it rounds a fraction as often.
+//
+// Range.  The parts have fp32's exponents, so m and l of a value below 2^-109 would end in bf16's subnormals, an infinity (or a
+// value that rounds to one) leaves inf - inf in m, and m * inf may have the other sign than h * inf.  So
+//   - operands are scaled by 2^24 ahead of the split, results by 2^-48: every fp32 value below 2^104, subnormals too, is then the
+//     sum of its parts;
+//   - whatever lies beyond (infinities, operands of 2^104 or more, sums of 2^80 or more) makes the results that it reaches
+//     infinite or not a number, and no others: those are formed once more, in fp32 FMA, by the threads that stored them
+//     (split_bad; the packed filters carry an fp32 copy for it).  NaN is what remains where the operands say so.
 //
 // The tile and the lanes are those of qconv_fwd_f16_lanes_kernel: S * 32 output channels x NPT * 32 pixels, wave v owns the two
 // product lanes made from one pair of components.  A chunk is 8 channels, and its three parts of eight lanes do not fit LDS
@@ -33,7 +40,7 @@ static_assert(2 * X3_BUF * 16 <= X3_LDS_BYTES, "LDS of the split kernel");
 constexpr int x3_step(int S) { return 128 * S; }  // 16-byte vectors of a wave's filter operands per phase and tap: [2 operands][sub-tile][64]
 constexpr int X3_GROUP = 3;                      // taps per group = taps in the filter register ring
 
-inline size_t x3_packed_bytes(int S, int co_tiles, int nchunks, int taps3) {
+__host__ __device__ inline size_t x3_packed_bytes(int S, int co_tiles, int nchunks, int taps3) {  // (in front of the fp32 copy)
     return ((size_t)co_tiles * 4 * nchunks * 2 * taps3 + X3_GROUP) * x3_step(S) * 16;
 }
 
@@ -47,6 +54,57 @@ __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
 }
 __device__ __forceinline__ float bf16_low(unsigned int v) { return __builtin_bit_cast(float, v << 16); }
 __device__ __forceinline__ float bf16_high(unsigned int v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
+
+constexpr float SPLIT_SCALE = 0x1p24f, SPLIT_RESULT = 0x1p-48f;
+
+// bad stays zero as long as every y is finite, and is NaN from the first one on that is not
+__device__ __forceinline__ void split_check(float& bad, float y) { bad = fmaf(y, 0.f, bad); }
+__device__ __forceinline__ bool split_bad(float y) { return !(fabsf(y) < __builtin_inff()); }
+__device__ __forceinline__ bool all_nan(const float (&y)[4]) { return y[0] != y[0] && y[1] != y[1] && y[2] != y[2] && y[3] != y[3]; }
+
+// y += x (x) w, in fp32
+__device__ __forceinline__ void add_product(const float (&x)[4], const f32x4& w, float (&y)[4]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[q] = fmaf(qneg(p, q) ? -x[p] : x[p], w[p ^ q], y[q]);
+}
+
+// The packed image's fp32 copy of the filter, [tap][reduced channel][output channel] x 4 components (conjugated / mirrored /
+// transposed for MAP_DGRAD), and the four components of one output from it
+inline size_t split_copy_bytes(int taps, int red, int rows) { return (size_t)taps * red * rows * 16; }
+__device__ __forceinline__ void conv_fp32(const ConvArgs& P, const f32x4* copy, int n, int ho, int wo, int co, float (&y)[4]) {
+    const long plane = (long)P.in.Hd * P.in.Wd;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) y[q] = 0.f;
+    for (int tap = 0; tap < P.taps; ++tap) {
+        const int kh = tap / P.Kw, h = ho * P.sh - P.pt + kh * P.dh, w = wo * P.sw - P.pl + (tap - kh * P.Kw) * P.dw;
+        if (h < 0 || h >= P.in.Hd || w < 0 || w >= P.in.Wd) continue;
+        const float* src = static_cast<const float*>(P.in.base) + (long)n * P.in.Cs * plane + (long)h * P.in.Wd + w;
+        const f32x4* f = copy + (long)tap * P.in.C * P.Cout + co;
+        for (int c = 0; c < P.in.C; ++c, src += plane, f += P.Cout) {
+            const float x[4] = {src[0], src[P.in.comp_stride], src[2 * P.in.comp_stride], src[3 * P.in.comp_stride]};
+            add_product(x, *f, y);
+        }
+        if (all_nan(y)) return;
+    }
+}
+
+// output (n, ho, wo, co) once more if what has been stored is not finite
+__device__ __forceinline__ void conv_again(const ConvArgs& P, const f32x4* copy, int n, int ho, int wo, int co) {
+    float* const out = static_cast<float*>(P.out) + (((long)n * P.CoutS + co) * P.Hout + ho) * P.Wout + wo;
+    bool bad = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) bad = bad || split_bad(out[q * P.out_cs]);
+    if (!bad) return;
+    float y[4];
+    conv_fp32(P, copy, n, ho, wo, co, y);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (P.bias) y[q] += static_cast<const float*>(P.bias)[q * P.CoutS + co];
+        out[q * P.out_cs] = y[q];
+    }
+}
 
 template <int S, int NPT>
 __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvArgs P0) {
@@ -131,11 +189,11 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
                 stage[i][k] = ((bits >> k) & 1) ? src[(long)c * plane_in + k] : 0u;
             }
     };
-    unsigned int keep[4];
+    float keep[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) keep[k] = (unsigned int)((int)(bits << (31 - k)) >> 31);
+    for (int k = 0; k < 4; ++k) keep[k] = ((bits >> k) & 1) ? SPLIT_SCALE : 0.f;
     // Position k of the task, channels 2q and 2q + 1, in nine steps of one to three instructions, which go between the
-    // products: cleared outside the image, the partner's, sum (l = 0) or difference, the three parts; behind the last pair
+    // products: scaled, or cleared outside the image (a value there that is not finite is one more reason for conv_again), the partner's, sum (l = 0) or difference, the three parts; behind the last pair
     // the parts' eight channels go to LDS.
     float e[2], f[2];
     unsigned int part[3][4];
@@ -143,7 +201,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
     auto slice = [&](int l, int k, int q, int u) {
         if (u == 0) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) e[i] = __builtin_bit_cast(float, stage[2 * q + i][k] & keep[k]);
+            for (int i = 0; i < 2; ++i) e[i] = __builtin_bit_cast(float, (unsigned int)stage[2 * q + i][k]) * keep[k];
         } else if (u == 1) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)  // row_ror:12 = from four threads on
@@ -176,8 +234,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
 
     // window offset, output offset and validity of a pixel of the tile
     const float rcp_w = __builtin_amdgcn_rcpf(tall ? P.Wout : P.TW), rcp_h = __builtin_amdgcn_rcpf(tall ? P.in.tall : P.TH * P.TW);
-    auto decode = [&](int pix, int& off, long& oaddr) -> bool {
-        int n, ho, wo;
+    auto decode_at = [&](int pix, int& off, int& n, int& ho, int& wo) -> bool {
         bool valid;
         if (tall) {
             const int x = c0 + pix, r = small_div(x, rcp_w), y = y0 + r, d = small_div(y, rcp_h);
@@ -190,6 +247,11 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
             valid = nb < P.NB && n < P.in.N && ho < P.Hout && wo < P.Wout;
             off = valid ? (nb * P.HTH + r * P.sh) * P.HTW + c * P.sw : 0;
         }
+        return valid;
+    };
+    auto decode = [&](int pix, int& off, long& oaddr) -> bool {
+        int n, ho, wo;
+        const bool valid = decode_at(pix, off, n, ho, wo);
         oaddr = ((long)n * P.CoutS * P.Hout + ho) * P.Wout + wo;
         return valid;
     };
@@ -337,6 +399,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
         const bool a = decode(g8 * 8 + 4 * h, off, o8[h]), b = decode(g8 * 8 + 4 * h + 3, off, end);
         run4[h] = a && b && end == o8[h] + 3;
     }
+    float bad = 0.f;  // (pixels behind the tile's last one count as well: conv_again looks)
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         if (s > 0) wg_barrier_no_vmem_wait();  // the previous round has been read
@@ -374,7 +437,10 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
                     for (int i = 0; i < 8; ++i) in[i] = lanes[i][h][k];
                     merge_output(in, c);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) y[q][k] = c[q];
+                    for (int q = 0; q < 4; ++q) {
+                        y[q][k] = c[q] * SPLIT_RESULT;
+                        split_check(bad, y[q][k]);
+                    }
                 }
                 if (bias) {
 #pragma unroll
@@ -397,11 +463,20 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
             }
         }
     }
+    if (bad != bad) {  // (rare)
+        const f32x4* const copy = reinterpret_cast<const f32x4*>(static_cast<const char*>(P.wpk) + x3_packed_bytes(S, P.co_tiles, P.nchunks, ngroups * TG));
+#pragma unroll 1
+        for (int i = 0; i < 8 * S * (32 / ROWS); ++i) {
+            const int co = ct * S * 32 + row0 + (i >> 3) * ROWS;
+            int off, n, ho, wo;
+            if (co < P.Cout && decode_at(g8 * 8 + (i & 7), off, n, ho, wo)) conv_again(P, copy, n, ho, wo, co);
+        }
+    }
 }
 
 // Filter packing: [filter tile of S * 32][wave][chunk][phase][tap, padded to whole groups][operand (h | m), (l | h)][sub-tile][64] x 8
-// bf16 (conjugated / mirrored / transposed for MAP_DGRAD).  One thread per (tile, chunk, tap, sub-tile, row, channel of the
-// chunk): eight product lanes from the same four filter values.
+// bf16 (conjugated / mirrored / transposed for MAP_DGRAD), then the fp32 copy.  One thread per (tile, chunk, tap, sub-tile, row,
+// channel of the chunk): eight product lanes from the same four filter values.
 template <int MAP>
 __device__ __forceinline__ void pack_filters_x3_body(const PackLanesArgs& A, int S, long first, long stride) {
     const PackArgs& P = A.base;
@@ -409,6 +484,7 @@ __device__ __forceinline__ void pack_filters_x3_body(const PackLanesArgs& A, int
     const long total = (long)P.row_tiles * P.nchunks * A.taps3 * S * 32 * 8;
     const float* w = static_cast<const float*>(P.w);
     __bf16* outh = static_cast<__bf16*>(P.out);
+    f32x4* const copy = reinterpret_cast<f32x4*>(static_cast<char*>(P.out) + x3_packed_bytes(S, P.row_tiles, P.nchunks, A.taps3));
     for (long idx = first; idx < total; idx += stride) {
         const int i = idx & 7, r = (idx >> 3) & 31;
         long s = idx >> 8;
@@ -428,6 +504,9 @@ __device__ __forceinline__ void pack_filters_x3_body(const PackLanesArgs& A, int
             float wv[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) wv[c] = ((MAP == MAP_DGRAD && c > 0) ? -1.f : 1.f) * w[c * P.wcs + off];
+            copy[((long)tap * P.red + red) * P.rows + row] = f32x4{wv[0], wv[1], wv[2], wv[3]};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) wv[c] *= SPLIT_SCALE;
             lanes_right(wv, R);
         }
 #pragma unroll

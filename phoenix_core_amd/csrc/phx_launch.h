@@ -53,11 +53,11 @@ int launch_fwd_f16_lanes(const FwdVariant& v, const ConvArgs& a, hipStream_t st)
 int launch_fwd_f16_phases(const FwdVariant& v, const ConvPhases& a, int phases, hipStream_t st);  // WCO 1 or 2
 int launch_fwd_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // fp32 on bf16 instructions
 size_t x3_lds_bytes();
-size_t x3_image_bytes(int WCO, int co_tiles, int nchunks, int ngroups);
+size_t x3_image_bytes(int WCO, int co_tiles, int nchunks, int ngroups, int taps, int red, int rows);
 int launch_pw_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st);  // ... pointwise
 int pw_x3_pixels();
 size_t pw_x3_lds_bytes();
-size_t pw_x3_image_bytes(int WCO, int co_tiles, int nsteps);
+size_t pw_x3_image_bytes(int WCO, int co_tiles, int nsteps, int red, int rows);
 int launch_pack_filters_pw_x3(int map, int WCO, const PackArgs& a, int blocks, hipStream_t st);
 int launch_pack_filters_x3(int map, int WCO, int ngroups, const PackArgs& a, int blocks, hipStream_t st);
 size_t lanes_lds_bytes();

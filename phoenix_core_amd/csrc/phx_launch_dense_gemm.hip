@@ -20,7 +20,8 @@
 // 64 rows the launches.  Error against fp64 in fp32: 1.3e-7 where the fp32 instructions had 2.9e-7 (512 units).
 //
 // fp32 operands are split into three bf16 parts on their way into LDS and multiplied as six products (see phx_kernels_x3.h for
-// the arithmetic), in 16-product form whatever the mode asks for; the five small products have accumulators of their own.
+// the arithmetic and for what becomes of values that have no three parts), in 16-product form whatever the mode asks for; the
+// five small products have accumulators of their own.
 #include <algorithm>
 
 #include "phx_kernels_x3.h"
@@ -146,6 +147,8 @@ struct DenseOperand {
                         for (int i = 0; i < 8; ++i) x[i] = i < left ? x[i] : 0.f;
                     }
 #pragma unroll
+                    for (int i = 0; i < 8; ++i) x[i] *= SPLIT_SCALE;
+#pragma unroll
                     for (int part = 0; part < 3; ++part) {
                         u32x4 w;
 #pragma unroll
@@ -174,6 +177,39 @@ struct GemmArgsPlanes : DenseGemmArgs {
 };
 template <bool PLANES>
 using GemmArgsOf = std::conditional_t<PLANES, GemmArgsPlanes, DenseGemmArgs>;
+
+// fp32: the four components of result (m, n), without the bias, over the chunks [first, end) in fp32 FMA (see split_bad in
+// phx_kernels_x3.h)
+template <int PASS, bool PLANES>
+__device__ __forceinline__ void dense_fp32(const GemmArgsOf<PLANES>& P, int first, int end, int m, int n, float (&y)[4]) {
+    constexpr int KC = DenseTile<float>::KC;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) y[q] = 0.f;
+    for (int c = first; c < end; ++c) {
+        const float* a = static_cast<const float*>(P.a) + m * P.ars;
+        const float* b = static_cast<const float*>(P.b) + n * P.brs;
+        int k0 = c * KC;
+        if constexpr (PLANES) {
+            const int img = c / P.planes.chunks;
+            a += img * P.planes.aimg;
+            b += img * P.planes.bimg;
+            k0 = (c - img * P.planes.chunks) * KC;
+        }
+        for (int k = k0; k < min(k0 + KC, P.K); ++k) {
+            float x[4], w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[i] = a[i * P.acs + k * P.aks];
+                w[i] = b[i * P.bcs + k * P.bks];
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) y[q] = fmaf(dense_negative(PASS, p, q) ? -x[p] : x[p], w[p ^ q], y[q]);
+        }
+        if (all_nan(y)) return;
+    }
+}
 
 // ROWTURN, COLTURN: the operand is contiguous along its rows, not along the reduction.  PLANES: the filter gradient of a pointwise
 // convolution on image planes: the reduction runs over the pixels of one image after the other, and results are contiguous along
@@ -296,6 +332,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArg
         }
     }
 
+    float bad = 0.f;
     // accumulator register 4 g + e: column 8 g + 4 kk + e of the wave's 32 at row j (PLANES: row 8 g + 4 kk + e at column j)
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
@@ -309,7 +346,11 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArg
                 const int m = PLANES ? run : lane_index, n = PLANES ? lane_index : run;
                 const bool whole = run + 3 < length;
                 f32x4 y = {acc[t][q][4 * g], acc[t][q][4 * g + 1], acc[t][q][4 * g + 2], acc[t][q][4 * g + 3]};
-                if constexpr (F32) y += f32x4{low[q][4 * g], low[q][4 * g + 1], low[q][4 * g + 2], low[q][4 * g + 3]};
+                if constexpr (F32) {
+                    y = (y + f32x4{low[q][4 * g], low[q][4 * g + 1], low[q][4 * g + 2], low[q][4 * g + 3]}) * SPLIT_RESULT;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) split_check(bad, y[e]);
+                }
                 if (P.partial) {  // [slice][component][m][n], PLANES [n][m]
                     float* dst = P.partial + (((long)z * 4 + q) * (PLANES ? P.N : P.M) + lane_index) * length + run;
                     if (whole) *reinterpret_cast<f32x4_a4*>(dst) = y;
@@ -339,6 +380,31 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArg
                     for (int e = 0; e < 4; ++e)
                         if (run + e < length) dst[e * step] = o[e];
             }
+    }
+    if constexpr (F32) {
+        if (bad != bad) {  // (rare) results that are not finite, once more
+            const int lane_index = PLANES ? n0 + wn * 32 + j : m0 + wm * 32 + j, length = PLANES ? P.M : P.N;
+#pragma unroll 1
+            for (int i = 0; i < 16; ++i) {
+                const int run = (PLANES ? m0 + wm * 32 : n0 + wn * 32) + 8 * (i >> 2) + 4 * kk + (i & 3);
+                if (run >= length) break;
+                const int m = PLANES ? run : lane_index, n = PLANES ? lane_index : run;
+                float* const dst = P.partial ? P.partial + ((long)z * 4 * (PLANES ? P.N : P.M) + lane_index) * length + run
+                                             : static_cast<float*>(P.out) + m * P.ors + n * P.ons;
+                const long cs = P.partial ? (long)(PLANES ? P.N : P.M) * length : P.ocs;
+                bool again = false;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) again = again || split_bad(dst[q * cs]);
+                if (!again) continue;
+                float y[4];
+                dense_fp32<PASS, PLANES>(P, first, end, m, n, y);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (PASS == PHX_PASS_FWD && !P.partial && P.bias) y[q] += static_cast<const float*>(P.bias)[q * P.N + n];
+                    dst[q * cs] = y[q];
+                }
+            }
+        }
     }
 }
 

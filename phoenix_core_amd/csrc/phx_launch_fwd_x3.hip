@@ -5,7 +5,9 @@
 namespace phx {
 
 size_t x3_lds_bytes() { return X3_LDS_BYTES; }
-size_t x3_image_bytes(int WCO, int co_tiles, int nchunks, int ngroups) { return x3_packed_bytes(WCO, co_tiles, nchunks, ngroups * X3_GROUP); }
+size_t x3_image_bytes(int WCO, int co_tiles, int nchunks, int ngroups, int taps, int red, int rows) {
+    return x3_packed_bytes(WCO, co_tiles, nchunks, ngroups * X3_GROUP) + split_copy_bytes(taps, red, rows);
+}
 
 template <int S, int NPT>
 static int launch_one(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {

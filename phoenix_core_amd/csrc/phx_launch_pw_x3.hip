@@ -6,7 +6,9 @@ namespace phx {
 
 int pw_x3_pixels() { return PWX3_PX; }
 size_t pw_x3_lds_bytes() { return PWX3_LDS_BYTES; }
-size_t pw_x3_image_bytes(int WCO, int co_tiles, int nsteps) { return pwx3_packed_bytes(WCO, co_tiles, nsteps); }
+size_t pw_x3_image_bytes(int WCO, int co_tiles, int nsteps, int red, int rows) {
+    return pwx3_packed_bytes(WCO, co_tiles, nsteps) + split_copy_bytes(1, red, rows);
+}
 
 int launch_pw_x3(const FwdVariant& v, const ConvArgs& a, hipStream_t st) {
     const dim3 grid(v.wgs, grid_rows(a.groups));
