@@ -23,6 +23,7 @@ namespace phx {
 // clocks and 230 vector instructions of 4 a wave.
 constexpr int PWX3_STEP = 16;
 constexpr int PWX3_PX = 64;
+constexpr int PWX3_STRETCH = SPLIT_STRETCH / PWX3_STEP;  // K steps between two changes of sign
 constexpr int PWX3_LDS_BYTES = 8 * 32 * PWX3_PX * 4;  // the epilogue's exchange of the product lanes
 constexpr int pwx3_vectors(int S) { return 2 * 3 * S * 64; }  // 16-byte vectors of a wave's filters per K step: [lane][part][sub-tile][64]
 
@@ -102,7 +103,17 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvAr
 
     load_x(0);
     constexpr int FP[6] = {2, 0, 1, 1, 0, 0}, XP[6] = {0, 2, 1, 0, 1, 0};  // parts of filter and input: the largest product last
+    float result = SPLIT_RESULT;
     for (int step = 0; step < P.nchunks; ++step) {
+        if (step > 0 && step % PWX3_STRETCH == 0) {  // (see Drift in phx_kernels_x3.h)
+            result = -result;
+#pragma unroll
+            for (int l = 0; l < 2; ++l)
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) acc[l][s][t] = -acc[l][s][t];
+        }
         const bool more = step + 1 < P.nchunks;
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
@@ -179,7 +190,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvAr
             merge_output(in, y);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                y[q] *= SPLIT_RESULT;
+                y[q] *= result;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) split_check(bad, y[q][k]);
                 if (bias) y[q] += bias[q * P.CoutS + co];
@@ -229,7 +240,7 @@ __device__ __forceinline__ void pack_filters_pwx3_body(const PackArgs& P, int S,
             for (int c = 0; c < 4; ++c) wv[c] = ((MAP == MAP_DGRAD && c > 0) ? -1.f : 1.f) * w[c * P.wcs + off];
             copy[(long)red * P.rows + row] = f32x4{wv[0], wv[1], wv[2], wv[3]};
 #pragma unroll
-            for (int c = 0; c < 4; ++c) wv[c] *= SPLIT_SCALE;
+            for (int c = 0; c < 4; ++c) wv[c] *= ((step / PWX3_STRETCH) & 1) ? -SPLIT_SCALE : SPLIT_SCALE;
             lanes_right(wv, R);
         }
 #pragma unroll

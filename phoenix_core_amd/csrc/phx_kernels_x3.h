@@ -23,6 +23,12 @@ namespace phx {
 //     infinite or not a number, and no others: those are formed once more, in fp32 FMA, by the threads that stored them
 //     (split_bad; the packed filters carry an fp32 copy for it).  NaN is what remains where the operands say so.
 //
+// Drift.  The instructions' sums drop what lies 2^-30 or so below them downwards, whatever their sign: in a chain of n of them
+// n * 2^-31 of the whole beside the sqrt(n) * 2^-25 of its roundings (error against fp64 / that of the fp32 instructions, zero-mean
+// operands: 4608 products 0.89, 12800 0.92, 25088 0.96, 51200 1.03).  So every 2304 products the accumulators change their sign,
+// and the filters of every other such stretch are packed negated: what one stretch loses the next one gains
+// (0.86, 0.83, 0.82, 0.78).  A change takes 3 k clocks of the 440 k of a stretch.
+//
 // The tile and the lanes are those of qconv_fwd_f16_lanes_kernel: S * 32 output channels x NPT * 32 pixels, wave v owns the two
 // product lanes made from one pair of components.  A chunk is 8 channels, and its three parts of eight lanes do not fit LDS
 // twice, so a chunk is worked on in two phases, the waves' sum lanes and then their difference lanes, each with a buffer of
@@ -39,6 +45,9 @@ constexpr int X3_LDS_BYTES = 8 * 32 * (128 + 4) * 4;  // the epilogue's exchange
 static_assert(2 * X3_BUF * 16 <= X3_LDS_BYTES, "LDS of the split kernel");
 constexpr int x3_step(int S) { return 128 * S; }  // 16-byte vectors of a wave's filter operands per phase and tap: [2 operands][sub-tile][64]
 constexpr int X3_GROUP = 3;                      // taps per group = taps in the filter register ring
+
+constexpr int SPLIT_STRETCH = 2304;               // products between two changes of sign
+__host__ __device__ constexpr int x3_stretch(int taps3) { return taps3 * X3_CK < SPLIT_STRETCH ? SPLIT_STRETCH / (taps3 * X3_CK) : 1; }  // in chunks
 
 __host__ __device__ inline size_t x3_packed_bytes(int S, int co_tiles, int nchunks, int taps3) {  // (in front of the fp32 copy)
     return ((size_t)co_tiles * 4 * nchunks * 2 * taps3 + X3_GROUP) * x3_step(S) * 16;
@@ -361,7 +370,25 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
     using I3 = std::integral_constant<int, 3>;
+    const int stretch = x3_stretch(ngroups * TG);
+    int left = stretch;
+    float result = SPLIT_RESULT;
     for (int chunk = 0; chunk < P.nchunks; ++chunk) {
+        if (left-- == 0) {
+            left = stretch - 1;
+            result = -result;
+#pragma unroll
+            for (int l = 0; l < 2; ++l)
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int t = 0; t < NPT; ++t) {
+                        asm volatile("" : "+a"(acc[l][s][t]));
+                        acc[l][s][t] = -acc[l][s][t];
+                        asm volatile("" : "+a"(acc[l][s][t]));
+                        __builtin_amdgcn_sched_barrier(0);  // (a tile at a time leaves the accumulator file)
+                    }
+        }
         const int chan_next = (chunk + 1) * X3_CK;  // (behind the last chunk: loads of channel 0, into a buffer nobody reads)
         start_phase(0);
         for (int g = 2; g < ngroups; ++g) group(I0{}, I0{}, 0);
@@ -438,7 +465,7 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvA
                     merge_output(in, c);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        y[q][k] = c[q] * SPLIT_RESULT;
+                        y[q][k] = c[q] * result;
                         split_check(bad, y[q][k]);
                     }
                 }
@@ -485,6 +512,7 @@ __device__ __forceinline__ void pack_filters_x3_body(const PackLanesArgs& A, int
     const float* w = static_cast<const float*>(P.w);
     __bf16* outh = static_cast<__bf16*>(P.out);
     f32x4* const copy = reinterpret_cast<f32x4*>(static_cast<char*>(P.out) + x3_packed_bytes(S, P.row_tiles, P.nchunks, A.taps3));
+    const int stretch = x3_stretch(A.taps3);
     for (long idx = first; idx < total; idx += stride) {
         const int i = idx & 7, r = (idx >> 3) & 31;
         long s = idx >> 8;
@@ -506,7 +534,7 @@ __device__ __forceinline__ void pack_filters_x3_body(const PackLanesArgs& A, int
             for (int c = 0; c < 4; ++c) wv[c] = ((MAP == MAP_DGRAD && c > 0) ? -1.f : 1.f) * w[c * P.wcs + off];
             copy[((long)tap * P.red + red) * P.rows + row] = f32x4{wv[0], wv[1], wv[2], wv[3]};
 #pragma unroll
-            for (int c = 0; c < 4; ++c) wv[c] *= SPLIT_SCALE;
+            for (int c = 0; c < 4; ++c) wv[c] *= ((chunk / stretch) & 1) ? -SPLIT_SCALE : SPLIT_SCALE;
             lanes_right(wv, R);
         }
 #pragma unroll

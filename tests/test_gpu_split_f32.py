@@ -71,6 +71,32 @@ def test_error_against_fp64(case, tune_env):
         assert ours <= 1.1 * fp32 + (2.0 ** -23 if few else 0.0), gaps
 
 
+@pytest.mark.parametrize("case", [(2, 512, 64, 14, 5), (1, 600, 40, 14, 7), (1, 1024, 30, 21, 5), (4, 8192, 64, 14, 1), (2, 9250, 30, 9, 1)],
+                         ids=lambda c: "n%d_%dto%d_%dx_k%d" % c)
+def test_long_reductions_do_not_drift(case, tune_env):
+    """One chain of all products: the instructions drop low bits downwards, which would take 0.3 of the root mean square error
+    and more off every result at 12800 products and 8192 single ones.  What remains is at most half a stretch of 2304 products'
+    own, a sixth of the error there and less behind longer sums."""
+    tune_env(PHX_TUNE_KSLICES="0")
+    n, ci, co, h, k = case
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, wt, grad = (torch.randn(s, generator=gen, device="cuda") for s in ((4 * n, ci, h, h), (4, co, ci, k, k), (4 * n, ci, h, h)))
+    conv = lambda a, b: torch.nn.functional.conv2d(a, b, padding=k // 2)
+    desc = ops.Conv2DDescriptor(x.shape, wt.shape, padding="SAME", dtype=torch.float32, context=phx.Context({}))
+    y = phx.conv2d_fwd(x, wt, None, desc)
+    assert "f32mfmax3" in capi.last_kernel_name() and "kslices" not in capi.last_kernel_name()
+    # (the input gradient of the layer whose filter is the other way round)
+    back = wt.transpose(1, 2).contiguous()
+    desc = ops.Conv2DDescriptor((4 * n, co, h, h), back.shape, padding="SAME", dtype=torch.float32, context=phx.Context({}))
+    dx = ops.conv2d_bwd_data(back, grad, desc)
+    assert "f32mfmax3" in capi.last_kernel_name() and "kslices" not in capi.last_kernel_name()
+    z = torch.zeros(4 * n, co, h, h, dtype=torch.float64, device="cuda", requires_grad=True)
+    dxr, = torch.autograd.grad(_hamilton(z, back.double(), conv), z, grad.double())
+    for got, want in ((y, _hamilton(x.double(), wt.double(), conv)), (dx, dxr)):
+        error = got.double() - want
+        assert abs(float(error.mean())) <= 0.15 * float(error.square().mean().sqrt())
+
+
 def test_whole_numbers_are_exact():
     gen = torch.Generator(device="cuda").manual_seed(1)
     x = torch.randint(-300, 301, (8, 16, 12, 12), generator=gen, device="cuda").float()
