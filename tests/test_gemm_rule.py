@@ -1,0 +1,37 @@
+"""Which passes run as matrix products (phx_launch_dense_gemm.hip), read from the workspace they ask for (no device)."""
+import pytest
+import torch
+
+import phoenix_core_amd as phx
+from phoenix_core_amd import capi
+from test_slice_rule import Ctx
+
+WGRAD = capi.PHX_PASS_BWD_WEIGHTS
+
+
+def _dense(n, ci, co, dtype):
+    return phx.DenseDescriptor((4 * n, ci), (4, ci, co), dtype=dtype, context=Ctx("full16"))
+
+
+def _pointwise(n, ci, co, h, w, layout):
+    shape = (4 * n, ci, h, w) if layout == "NCHW" else (4 * n, h, w, ci)
+    return phx.Conv2DDescriptor(shape, (4, co, ci, 1, 1), dtype=torch.float32, context=Ctx("fp32"), data_format=layout)
+
+
+@pytest.mark.parametrize("desc,which", [(_dense(300, 700, 500, torch.float32), capi.PHX_PASS_FWD), (_dense(768, 512, 512, torch.float32), capi.PHX_PASS_BWD_DATA),
+                                        (_dense(768, 512, 512, torch.float32), WGRAD), (_pointwise(32, 96, 96, 56, 56, "NCHW"), WGRAD),
+                                        (_pointwise(32, 96, 96, 56, 56, "NHWC"), WGRAD)], ids=["fwd", "dgrad", "wgrad", "planes", "channels_last"])
+def test_the_fp32_instructions_on_request(desc, which, tune_env):
+    """PHX_TUNE_NOX3 keeps everything in fp32 off the bf16 instructions, these products too."""
+    sizes = []
+    for variables in ({}, {"PHX_TUNE_NOX3": "1"}, {"PHX_TUNE_NOX3": "1", "PHX_TUNE_NODENSEGEMM": "1"}):
+        tune_env(**{"PHX_TUNE_NOX3": None, "PHX_TUNE_NODENSEGEMM": None, **variables})
+        sizes.append(desc.workspace_bytes(which))
+    assert sizes[1] == sizes[2] != sizes[0]
+
+
+def test_fp16_products_are_not_concerned(tune_env):
+    desc = _dense(300, 700, 500, torch.float16)
+    planned = desc.workspace_bytes(capi.PHX_PASS_FWD)
+    tune_env(PHX_TUNE_NOX3="1")
+    assert desc.workspace_bytes(capi.PHX_PASS_FWD) == planned
