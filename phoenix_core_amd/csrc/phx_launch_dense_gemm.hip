@@ -445,16 +445,17 @@ void dense_gemm_plan(bool half_storage, DenseGemmArgs& a, GemmPlanes* planes) {
     for (int mt = 1; mt <= (half_storage ? 2 : 1); ++mt) {
         const int tiles_m = (a.M + 64 * mt - 1) / (64 * mt), most = half_storage && mt == 1 ? 3 : 2;
         const double first = !half_storage ? 3.4 : mt == 2 ? 3.9 : 1.7, more = !half_storage ? 2.3 : mt == 2 ? 0.9 : 1.1;
-        for (int Z = 1; Z <= std::min(a.chunks, planes ? 512 : 64); ++Z) {
-            const int per = (a.chunks + Z - 1) / Z;
-            if ((a.chunks + per - 1) / per != Z) continue;
-            const double load = std::ceil((double)tiles_m * a.tiles_n * Z / 256.0), full = std::floor(load / most), rest = load - full * most;
+        const int limit = std::min(a.chunks, planes ? 512 : 64);
+        for (int Z = 1, per = a.chunks; Z <= limit; Z = (a.chunks + per - 2) / (per - 1)) {  // (the slice counts that leave no slice empty)
+            per = (a.chunks + Z - 1) / Z;
+            const long load = ((long)tiles_m * a.tiles_n * Z + 255) / 256, full = load / most, rest = load % most;
             double us = 4.0 + per * (full * (first + (most - 1) * more) + (rest > 0 ? first + (rest - 1) * more : 0.0));
             if (Z > 1) us += 4.0 + (Z + 0.5) * 32.0 * a.M * a.N / 3.0e6;
             if (us < best) {
                 best = us;
                 a.MT = mt; a.tiles_m = tiles_m; a.Z = Z; a.kper = per;
             }
+            if (per == 1) break;
         }
     }
 }

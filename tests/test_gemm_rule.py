@@ -35,3 +35,27 @@ def test_fp16_products_are_not_concerned(tune_env):
     planned = desc.workspace_bytes(capi.PHX_PASS_FWD)
     tune_env(PHX_TUNE_NOX3="1")
     assert desc.workspace_bytes(capi.PHX_PASS_FWD) == planned
+
+
+def _searched(rows, columns, reduced, images):
+    """The slices of an fp32 filter gradient, by the planner's estimate over every slice count."""
+    chunks, best, slices = -(-reduced // 16) * max(images, 1), float("inf"), 1
+    tiles = -(-rows // 64) * -(-columns // 64)
+    for z in range(1, min(chunks, 512 if images else 64) + 1):
+        per = -(-chunks // z)
+        if -(-chunks // per) != z:
+            continue
+        full, rest = divmod(-(-tiles * z // 256), 2)
+        us = 4.0 + per * (full * 5.7 + (3.4 + (rest - 1) * 2.3 if rest else 0.0))
+        us += 4.0 + (z + 0.5) * 32.0 * rows * columns / 3.0e6 if z > 1 else 0.0
+        if us < best:
+            best, slices = us, z
+    return slices
+
+
+@pytest.mark.parametrize("n,ci,co,h,w", [(32, 96, 96, 56, 56), (4, 256, 64, 56, 56), (1, 100, 97, 2, 2), (64, 256, 256, 14, 14), (7, 512, 130, 13, 9)])
+def test_slices_are_those_of_the_whole_search(n, ci, co, h, w):
+    z = _searched(ci, co, h * w, n)
+    assert _pointwise(n, ci, co, h, w, "NCHW").workspace_bytes(WGRAD) == (z * 16 * ci * co if z > 1 else 0)
+    z = _searched(ci, co, n * h * w, 0)
+    assert _dense(n * h * w, ci, co, torch.float32).workspace_bytes(WGRAD) == (z * 16 * ci * co if z > 1 else 0)
