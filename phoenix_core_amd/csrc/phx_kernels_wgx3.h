@@ -54,13 +54,13 @@ __device__ __forceinline__ void wgrad_fp32(const WgradArgs& P, int zi, int kh, i
             const float* const x = static_cast<const float*>(P.x.base) + ((long)img * P.x.Cs + ci) * xplane + (long)h * P.x.Wd;
             const float* const g = static_cast<const float*>(P.g.base) + ((long)img * P.g.Cs + co) * gplane + (long)ho * P.g.Wd;
             const int c0 = (seg - line * P.cpr) * 8;
-            for (int c = c0; c < min(c0 + 8, P.g.Wd); ++c) {
-                const int w = c + kw - P.pl;
-                if (w < 0 || w >= P.x.Wd) continue;
+            const int shift = kw - P.pl, end = min(min(c0 + 8, P.g.Wd), P.x.Wd - shift);  // (columns whose input lies in the image)
+#pragma unroll 4
+            for (int c = max(c0, -shift); c < end; ++c) {
                 float xv[4], gv[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    xv[i] = x[i * P.x.comp_stride + w];
+                    xv[i] = x[i * P.x.comp_stride + c + shift];
                     gv[i] = g[i * P.g.comp_stride + c];
                 }
 #pragma unroll

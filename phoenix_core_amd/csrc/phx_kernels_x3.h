@@ -91,6 +91,7 @@ __device__ __forceinline__ void conv_fp32(const ConvArgs& P, const f32x4* copy, 
         if (h < 0 || h >= P.in.Hd || w < 0 || w >= P.in.Wd) continue;
         const float* src = static_cast<const float*>(P.in.base) + (long)n * P.in.Cs * plane + (long)h * P.in.Wd + w;
         const f32x4* f = copy + (long)tap * P.in.C * P.Cout + co;
+#pragma unroll 4
         for (int c = 0; c < P.in.C; ++c, src += plane, f += P.Cout) {
             const float x[4] = {src[0], src[P.in.comp_stride], src[2 * P.in.comp_stride], src[3 * P.in.comp_stride]};
             add_product(x, *f, y);

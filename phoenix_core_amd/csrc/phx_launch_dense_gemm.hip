@@ -195,6 +195,7 @@ __device__ __forceinline__ void dense_fp32(const GemmArgsOf<PLANES>& P, int firs
             b += img * P.planes.bimg;
             k0 = (c - img * P.planes.chunks) * KC;
         }
+#pragma unroll 4
         for (int k = k0; k < min(k0 + KC, P.K); ++k) {
             float x[4], w[4];
 #pragma unroll
