@@ -17,11 +17,17 @@
 // gradient 715 / 133, filter gradient 1773 / 143 (16 products of 3.1 G quaternion products: 690 TFLOP/s); 3707, 95 -> 408 86 / 22,
 // 64 / 22, 107 / 27; 49, 530 -> 1552 64 / 16, 118 / 15, 46 / 11; fp32 201, 328 -> 264 152 / 20, 103 / 18, 31 / 18.  Bound: the
 // latency of a chunk's loads (1.7 us) until two or three workgroups share a CU, then the matrix pipe and LDS alike; under
-// 64 rows the launches.  Error against fp64 in fp32: 1.3e-7 where the fp32 instructions had 2.9e-7 (512 units).
+// 64 rows the launches.  Errors of fp32 below.
 //
 // fp32 operands are split into three bf16 parts on their way into LDS and multiplied as six products (see phx_kernels_x3.h for
 // the arithmetic and for what becomes of values that have no three parts), in 16-product form whatever the mode asks for; the
-// five small products have accumulators of their own.
+// five small products have accumulators of their own.  The largest ones have 16 bits and lose nothing under an accumulator, so
+// they do not drift as the sums of phx_kernels_x3.h do (1e-9 of the mean result).  Error against fp64, 2-norm, fp32 instructions /
+// here: zero-mean values, 4096 rows, 1024 units 8.1e-7 / 4.0e-7; of one sign, forward 8.5e-7 / 3.5e-7.  Filter gradients of one
+// sign, which the fp32 instructions sum in more slices, start a chunk's largest products from zero, with one rounding of the
+// whole a chunk instead of four: 512 rows, 512 units 7.0e-8 / 7.7e-8 without, 4.9e-8 with; channels-last 96 -> 96 at 56x56, N=32
+// 5.4e-8 / 6.2e-8, 4.2e-8 (and 3 % slower).  On planes they are the closer ones without (256 -> 256 at 28x28, N=64 10.4e-8 / 7.5e-8;
+// 256 -> 64 at 56x56, N=16 4.9e-8 / 5.0e-8), and it would cost 2-8 %.
 #include <algorithm>
 
 #include "phx_kernels_x3.h"
@@ -308,6 +314,11 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArg
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         w[part][i] = __builtin_bit_cast(bf16x8, ca[((part * 4 + i) * S::KP + 2 * ks) * Cols::PITCH]);
+                // (the filter gradient's largest products below; not on planes, see above)
+                constexpr int TERMS = PASS == PHX_PASS_BWD_WEIGHTS && !PLANES ? 5 : 6;
+                const auto product = [](const bf16x8& x, const bf16x8& y, const f32x16& sum) {
+                    return PLANES ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(y, x, sum, 0, 0, 0);
+                };
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
                     bf16x8 x[3], nx[3];
@@ -318,15 +329,32 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArg
                         nx[part] = __builtin_bit_cast(bf16x8, negated(v));
                     }
 #pragma unroll
-                    for (int term = 0; term < 6; ++term) {
+                    for (int term = 0; term < TERMS; ++term) {
                         constexpr int wp[6] = {2, 0, 1, 1, 0, 0}, xp[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
-                            const bf16x8 xs = dense_negative(PASS, p, q) ? nx[xp[term]] : x[xp[term]];
                             f32x16& sum = term < 5 ? low[q] : acc[0][q];
-                            sum = PLANES ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, w[wp[term]][p ^ q], sum, 0, 0, 0)
-                                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[wp[term]][p ^ q], xs, sum, 0, 0, 0);
+                            sum = product(dense_negative(PASS, p, q) ? nx[xp[term]] : x[xp[term]], w[wp[term]][p ^ q], sum);
                         }
+                    }
+                }
+                if constexpr (TERMS == 5) {  // summed from zero: one rounding of the whole a chunk
+                    __builtin_amdgcn_sched_barrier(0);  // (the other parts' registers come free)
+                    u32x4 h[4];
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) h[p] = ra[(p * S::KP + 2 * ks) * Rows::PITCH];
+#pragma unroll
+                    for (int q = 0; q < 4; q += 2) {
+                        f32x16 sum[2];
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) sum[0][r] = sum[1][r] = 0.f;
+#pragma unroll
+                        for (int p = 0; p < 4; ++p)
+#pragma unroll
+                            for (int i = 0; i < 2; ++i)
+                                sum[i] = product(__builtin_bit_cast(bf16x8, dense_negative(PASS, p, q + i) ? negated(h[p]) : h[p]), w[0][p ^ (q + i)], sum[i]);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) acc[0][q + i] += sum[i];
                     }
                 }
             }

@@ -97,6 +97,64 @@ def test_long_reductions_do_not_drift(case, tune_env):
         assert abs(float(error.mean())) <= 0.15 * float(error.square().mean().sqrt())
 
 
+SIGNS = ["mean_zero", "one_sign"]
+
+
+def _values(signs, gen, *shape):
+    """Normal values, or positive ones (activations behind a ReLU, say), whose sums grow with every product."""
+    return torch.randn(shape, generator=gen, device="cuda") if signs == "mean_zero" else torch.rand(shape, generator=gen, device="cuda") + 0.05
+
+
+@pytest.mark.parametrize("signs", SIGNS)
+@pytest.mark.parametrize("case", [(8, 64, 64, 28, 3), (2, 512, 64, 14, 5), (16, 64, 64, 28, 1), (4, 2048, 64, 14, 1)], ids=lambda c: "n%d_%dto%d_%d_k%d" % c)
+def test_error_of_either_kind_of_sums(case, signs, tune_env):
+    n, ci, co, h, k = case
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, wt = _values(signs, gen, 4 * n, ci, h, h), _values(signs, gen, 4, co, ci, k, k)
+    if signs == "one_sign":
+        wt[1:] *= -1  # (a component of four products of one sign)
+    desc = ops.Conv2DDescriptor(x.shape, wt.shape, padding="SAME", dtype=torch.float32, context=phx.Context({}))
+    want = _hamilton(x.double(), wt.double(), lambda a, b: torch.nn.functional.conv2d(a, b, padding=k // 2))
+    gaps = []
+    for nox3 in (None, "1"):
+        tune_env(PHX_TUNE_NOX3=nox3)
+        gaps.append(_gap(phx.conv2d_fwd(x, wt, None, desc), want))
+        assert ("f32mfmax3" in capi.last_kernel_name()) == (nox3 is None)
+    assert gaps[0] <= 1.1 * gaps[1], gaps  # (see test_error_against_fp64)
+
+
+@pytest.mark.parametrize("signs", SIGNS)
+@pytest.mark.parametrize("case", [(32, 96, 96, 56, 56, "NCHW"), (32, 96, 96, 56, 56, "NHWC"), (16, 256, 128, 28, 28, "NCHW"), (4096, 256, 256, 1, 1, ""),
+                                  (20000, 64, 64, 1, 1, ""), (1000, 2048, 100, 1, 1, "")], ids=lambda c: "n%d_%dto%d_%dx%d%s" % c)
+def test_filter_gradients_as_matrix_products_of_long_sums(case, signs, tune_env):
+    """Reductions over thousands of pixels or rows, in up to a hundred slices, beside the fp32 instructions."""
+    n, ci, co, h, w, layout = case
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, grad = _values(signs, gen, 4 * n, h, w, ci), _values(signs, gen, 4 * n, h, w, co)
+    rows = lambda t: t.reshape(4, -1, t.shape[-1]).double()
+    xs, gs, want = rows(x), rows(grad), torch.zeros(4, ci, co, dtype=torch.float64, device="cuda")
+    for p in range(4):
+        for q in range(4):
+            want[p ^ q] += (xs[p].t().contiguous() @ gs[q]) * (-1 if (0x3950 >> (p * 4 + q)) & 1 else 1)
+    gaps = []
+    for nox3 in (None, "1"):
+        tune_env(PHX_TUNE_NOX3=nox3, PHX_TUNE_NOSMALLDENSE="1")
+        if layout:
+            last = (lambda t: t) if layout == "NHWC" else (lambda t: t.permute(0, 3, 1, 2).contiguous())
+            desc = ops.Conv2DDescriptor(last(x).shape, (4, co, ci, 1, 1), dtype=torch.float32, context=phx.Context({}), data_format=layout)
+            dw = ops.conv2d_bwd_weights(last(x), last(grad), desc).view(4, co, ci).transpose(1, 2)
+            assert ("mfmagemm" in capi.last_kernel_name()) == (nox3 is None), capi.last_kernel_name()
+        else:
+            x2, g2 = x.view(4 * n, ci), grad.view(4 * n, co)
+            wt = torch.zeros(4, ci, co, device="cuda")
+            desc = ops.DenseDescriptor(x2.shape, wt.shape, dtype=torch.float32, context=phx.Context({}))
+            dw, _ = phx.dense_bwd(x2, wt, g2, desc)
+            assert ("mfmagemm" in capi.last_kernel_name()) == (nox3 is None), capi.last_kernel_name()
+        gaps.append(_gap(dw, want))
+    # (of one sign both are little above the last rounding, 2^-25 / sqrt(3) of each value in the mean: it counts for both)
+    assert gaps[0] <= 1.1 * gaps[1], gaps
+
+
 def test_whole_numbers_are_exact():
     gen = torch.Generator(device="cuda").manual_seed(1)
     x = torch.randint(-300, 301, (8, 16, 12, 12), generator=gen, device="cuda").float()
