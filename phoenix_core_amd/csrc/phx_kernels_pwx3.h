@@ -16,7 +16,7 @@ namespace phx {
 //   value to it).
 // Measured (us a pass with its packing, fp32 instructions / here): N=32, 64 -> 64 channels at 56x56 107 / 72, N=16, 256 -> 64 at
 // 28x28 71 / 37, 64 -> 256 57 / 40, 256 -> 256 at 14x14 73 / 41, N=64, 128 -> 128 at 28x28 171 / 102, 16 -> 16 at 56x56 45 / 34,
-// N=8, 512 -> 512 at 7x7 80 / 36, N=2, 20 -> 33 at 5x7 18 / 14.  (With both lanes' filters held a step ahead, 17 registers
+// N=8, 512 -> 512 at 7x7 80 / 36, N=2, 20 -> 33 at 5x7 18 / 14; the scaling of the values 1-2 % more since.  (With both lanes' filters held a step ahead, 17 registers
 // spilled: 85 at 64 -> 64.)  Errors against fp64, relative 2-norm: 256 channels 3.4e-7 (fp32 instructions 4.1e-7), 512 in slices
 // 2.5e-7 (4.1e-7), 64 1.7e-7 (2.2e-7).
 // Bound: memory where channels are few (64 -> 64: 206 MB in 65 us), else the two pipes of a SIMD: a K step is 48 products of 32

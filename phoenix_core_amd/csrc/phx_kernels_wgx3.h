@@ -23,6 +23,8 @@ namespace phx {
 // addition, and every other reduction slice runs on the negated gradient.  Errors against fp64 (relative 2-norm, standard normal
 // values, here / fp32 instructions): 3x3, 128 x 48 channels at 9x9 1.8e-7 / 3.4e-7, 16 x 512 at 7x7 2.4e-7 / 4.7e-7, 4 x 256 at
 // 14x14 1.6e-7 / 2.9e-7; without the negation 6.3e-7, 2.4e-7, 2.0e-7; accumulated by the instructions 1.5-2 times as much again.
+// A pass of one slice has no other to make up for it, and needs none: 512 x 512 at 14x14, N=32 6.2e-7 / 1.36e-6, half of it drift
+// (which grows with the root of the steps, as the roundings do, since each step's sum starts from zero).
 //
 // Bound: the two pipes of a SIMD together.  64 channels at 56x56, N=64 (1399 us on fp32 instructions, 770 here): a step of
 // 2.5 us holds 72 products of 32 clocks and 700 vector instructions of 4, which overlap in part: 610 us without the staging,

@@ -1,8 +1,8 @@
 // fp16-MFMA forward kernels that apply evaluation-mode batch norm (+ residual, ReLU) to what they store: the instances of the
 // chunk-staging and the lane-dealing kernels with NORM (instances of their own: what they add to the epilogue would cost the
-// plain kernels registers).  The quaternion ResNet-50 in evaluation mode, 8 images of 224x224: 1672 us with a normalisation
+// plain kernels registers).  The quaternion ResNet-50 in evaluation mode, 8 images of 224x224: 1717 us with a normalisation
 // pass behind each of its 53 convolutions (265 us of kernel time, and as many operator calls of the host, which bounds it),
-// 875 us with the passes inside the convolutions.
+// 889 us with the passes inside the convolutions; where each pass of the network is waited for, 1815 and 1010.
 #include "phx_kernels_lanes16.h"
 #include "phx_launch.h"
 

@@ -10,18 +10,22 @@ from test_gpu_split_f32 import _hamilton
 
 pytestmark = pytest.mark.gpu
 
-# kind, n, inputs, outputs, h, w, taps, layout, kernels of the forward / input gradient and of the filter gradient
+# kind, n, inputs, outputs, h, w, taps, layout, kernels of the forward / input gradient and of the filter gradient (None: not on these
+# instructions), more of a convolution
 CASES = [
     ("conv", 3, 24, 40, 13, 9, 3, "NCHW", "f32mfmax3_p8", "f32mfmax3_p8"), ("conv", 2, 128, 96, 7, 7, 3, "NCHW", "kslices", "f32mfmax3_p8"),
     ("conv", 64, 64, 64, 28, 28, 3, "NCHW", "flat", "f32mfmax3_p8"), ("conv", 2, 40, 30, 15, 7, 1, "NCHW", "f32mfmax3pw", "f32mfmax3_p8"),
     ("conv", 3, 97, 100, 7, 5, 1, "NCHW", "f32mfmax3pw", "mfmagemm"), ("conv", 9, 128, 128, 14, 11, 1, "NHWC", "f32mfmax3pw", "mfmagemm"),
+    ("conv", 2, 20, 40, 15, 17, 3, "NCHW", "f32mfmax3", None, dict(dilation=2)), ("conv", 2, 24, 40, 21, 18, 7, "NCHW", "f32mfmax3", None, dict(stride=2)),
+    ("conv", 2, 80, 96, 13, 11, 3, "NCHW", "groups2", "groups2", dict(groups=2)),
     ("dense", 70, 130, 90, 1, 1, 1, "", "mfmagemm", "mfmagemm"), ("dense", 33, 1000, 24, 1, 1, 1, "", "mfmagemm", "mfmagemm"),
 ]
 
 
 class _Layer:
     def __init__(self, case):
-        self.kind, n, ci, co, h, w, k, self.layout, self.fwd_kernel, self.wgrad_kernel = case
+        self.kind, n, ci, co, h, w, k, self.layout, self.fwd_kernel, self.wgrad_kernel = case[:10]
+        self.more = dict(case[10]) if len(case) > 10 else {}
         gen = torch.Generator(device="cuda").manual_seed(ci)
 
         def values(*shape):  # magnitudes from 1/8 to 7/8
@@ -32,9 +36,11 @@ class _Layer:
             self.desc = ops.DenseDescriptor(self.x.shape, self.w.shape, dtype=torch.float32, context=phx.Context({}))
         else:
             self.k = k
-            self.x, self.w, self.g = values(4 * n, ci, h, w), values(4, co, ci, k, k), values(4 * n, co, h, w)
+            stride = self.more.get("stride", 1)
+            self.x, self.w = values(4 * n, ci, h, w), values(4, co, ci // self.more.get("groups", 1), k, k)
+            self.g = values(4 * n, co, -(-h // stride), -(-w // stride))
             self.desc = ops.Conv2DDescriptor(self.last(self.x).shape, self.w.shape, padding="SAME", dtype=torch.float32, context=phx.Context({}),
-                                             data_format=self.layout)
+                                             data_format=self.layout, **self.more)
 
     def last(self, t):
         return t.permute(0, 2, 3, 1).contiguous() if self.layout == "NHWC" else t
@@ -47,7 +53,8 @@ class _Layer:
         if self.kind == "dense":
             y = _dense(x, w)
         else:
-            y = _hamilton(x, w, lambda a, b: torch.nn.functional.conv2d(a, b, padding=self.k // 2))
+            (pt, pl), (pb, pr) = self.desc.pad_before, self.desc.pad_after
+            y = _hamilton(torch.nn.functional.pad(x, (pl, pr, pt, pb)), w, lambda a, b: torch.nn.functional.conv2d(a, b, **self.more))
         if which == "fwd":
             return y.detach()
         return torch.autograd.grad(y, x if which == "dgrad" else w, g)[0]
@@ -81,14 +88,9 @@ def _layer(case, tune_env):
     return _Layer(case)
 
 
-_ids = lambda c: "%s_n%d_%dto%d_%dx%d_k%d%s" % c[:8]
-_each = [pytest.mark.parametrize("case", CASES, ids=_ids), pytest.mark.parametrize("which", ["fwd", "dgrad", "wgrad"])]
-
-
-def _everywhere(f):
-    for mark in _each:
-        f = mark(f)
-    return f
+_ids = lambda c: "%s_n%d_%dto%d_%dx%d_k%d%s" % c[:8] + "".join("_%s%d" % m for m in (c[10] if len(c) > 10 else {}).items())
+_everywhere = pytest.mark.parametrize("case,which", [(c, w) for c in CASES for w in ("fwd", "dgrad", "wgrad") if w != "wgrad" or c[9]],
+                                      ids=lambda v: v if isinstance(v, str) else _ids(v))
 
 
 def _middle(t):
