@@ -26,8 +26,8 @@
 // here: zero-mean values, 4096 rows, 1024 units 8.1e-7 / 4.0e-7; of one sign, forward 8.5e-7 / 3.5e-7.  Filter gradients of one
 // sign, which the fp32 instructions sum in more slices, start a chunk's largest products from zero, with one rounding of the
 // whole a chunk instead of four: 512 rows, 512 units 7.0e-8 / 7.7e-8 without, 4.9e-8 with; channels-last 96 -> 96 at 56x56, N=32
-// 5.4e-8 / 6.2e-8, 4.2e-8 (and 3 % slower).  On planes they are the closer ones without (256 -> 256 at 28x28, N=64 10.4e-8 / 7.5e-8;
-// 256 -> 64 at 56x56, N=16 4.9e-8 / 5.0e-8), and it would cost 2-8 %.
+// 5.4e-8 / 6.2e-8, 4.2e-8 (and 3 % slower); on planes 475 -> 475 at 28x27, N=1 6.6e-8 / 7.6e-8, 3.9e-8 (2-8 % slower: 96 -> 96 at
+// 56x56, N=32 260 -> 278 us).
 #include <algorithm>
 
 #include "phx_kernels_x3.h"
@@ -314,8 +314,8 @@ __global__ void __launch_bounds__(WG_THREADS, 2) dense_gemm_kernel(const GemmArg
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         w[part][i] = __builtin_bit_cast(bf16x8, ca[((part * 4 + i) * S::KP + 2 * ks) * Cols::PITCH]);
-                // (the filter gradient's largest products below; not on planes, see above)
-                constexpr int TERMS = PASS == PHX_PASS_BWD_WEIGHTS && !PLANES ? 5 : 6;
+                // (the filter gradient's largest products below)
+                constexpr int TERMS = PASS == PHX_PASS_BWD_WEIGHTS ? 5 : 6;
                 const auto product = [](const bf16x8& x, const bf16x8& y, const f32x16& sum) {
                     return PLANES ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(y, x, sum, 0, 0, 0);
                 };

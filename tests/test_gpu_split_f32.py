@@ -158,7 +158,7 @@ def test_error_of_either_kind_of_sums(case, signs, tune_env):
 
 
 @pytest.mark.parametrize("signs", SIGNS)
-@pytest.mark.parametrize("case", [(32, 96, 96, 56, 56, "NCHW"), (32, 96, 96, 56, 56, "NHWC"), (16, 256, 128, 28, 28, "NCHW"), (4096, 256, 256, 1, 1, ""),
+@pytest.mark.parametrize("case", [(32, 96, 96, 56, 56, "NCHW"), (32, 96, 96, 56, 56, "NHWC"), (16, 256, 128, 28, 28, "NCHW"), (1, 475, 475, 28, 27, "NCHW"), (4096, 256, 256, 1, 1, ""),
                                   (20000, 64, 64, 1, 1, ""), (1000, 2048, 100, 1, 1, "")], ids=lambda c: "n%d_%dto%d_%dx%d%s" % c)
 def test_filter_gradients_as_matrix_products_of_long_sums(case, signs, tune_env):
     """Reductions over thousands of pixels or rows, in up to a hundred slices, beside the fp32 instructions."""
