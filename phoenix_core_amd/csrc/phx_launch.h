@@ -75,10 +75,17 @@ int launch_pwx_nhwc_f16(int WCO, const PwxArgs& a, int blocks, hipStream_t st); 
 size_t pwx_packed_bytes(int WCO, int co_tiles, int nsteps);
 int launch_pack_filters_pwx(int map, int WCO, int nsteps, const PackArgs& a, hipStream_t st);
 
+// fp16 convolutions of few output tiles, operands straight in registers (phx_kernels_reg16.h); cl = channels-last tensors;
+// norm.gamma null: none; waves of a workgroup
+struct RegArgs;
+int launch_reg_f16(int kw, int dw, int sw, bool cl, const RegArgs& a, const NormArgs& norm, int waves, int blocks, hipStream_t st);  // < 0: no such instance
+bool reg_row_shape(int kw, int dw, int sw);  // whether there are instances for filter rows of this shape
+int launch_pack_filters_reg(int map, const PackArgs& a, int blocks, hipStream_t st);
+
 // Several filter images packed by one launch (phx_launch_pack.hip): a convolution's forward and input-gradient
 // images, the sub-filters of a strided input gradient's phases, the groups of a grouped convolution.  A job is one
 // call of one of the packing kernels above; the workgroups of the launch are dealt to the jobs in order.
-enum PackKind { PACK_F32 = 0, PACK_F16 = 1, PACK_F16_LDS = 2, PACK_PWX = 3, PACK_F16_LANES = 4, PACK_F32_X3 = 5, PACK_F32_PWX3 = 6 };
+enum PackKind { PACK_F32 = 0, PACK_F16 = 1, PACK_F16_LDS = 2, PACK_PWX = 3, PACK_F16_LANES = 4, PACK_F32_X3 = 5, PACK_F32_PWX3 = 6, PACK_REG = 7 };
 struct PackJob {
     PackArgs a;
     int kind;                    // PackKind
@@ -203,9 +210,9 @@ int launch_transpose(bool half_storage, const TransposeArgs& a, hipStream_t st);
 int launch_fill_zero(void* dst, size_t bytes, hipStream_t st);  // a kernel, so that it can be captured in a graph
 int launch_add_inplace(bool half_storage, void* dst, const void* src, long count, hipStream_t st);  // dst += src
 // dst = the sum of `slices` partial tensors of `count` elements (+ bias of the element's channel, + addend); partial results
-// of a pass whose channel reduction was cut into slices; then norm, where its gamma is not null
+// of a pass whose channel reduction was cut into slices (partial_f32: fp32 ones of an fp16 result); then norm, where its gamma is not null
 int launch_slice_sum(bool half_storage, const void* partial, int slices, long count, void* dst, const void* bias, const void* addend,
-                     int plane, int channels, long comp_count, const NormArgs& norm, hipStream_t st);
+                     int plane, int channels, long comp_count, const NormArgs& norm, hipStream_t st, bool partial_f32 = false);
 
 // REAL / COMPLEX / GA_300 as compositions on the quaternion entry points (phx_algebra.hip); pass = phx_pass,
 // (a, b) = (x, w) forward, (grad, w) input gradient, (x, grad) filter gradient

@@ -2,6 +2,7 @@
 // falls into and runs that packing kernel's body over the job's own index range.
 #include "phx_kernels_pwx3.h"
 #include "phx_kernels_pw16.h"
+#include "phx_kernels_reg16.h"
 #include "phx_launch.h"
 
 namespace phx {
@@ -21,6 +22,8 @@ static __device__ __forceinline__ void pack_job_as(const PackJob& j, long first,
         if constexpr (MODE == 8) pack_filters_pwx3_body<MAP>(j.a, j.WCO, first, stride);
     } else if (j.kind == PACK_F16_LANES) {
         if constexpr (MODE == 8) pack_filters_lanes_body<MAP>(PackLanesArgs{j.a, j.ngroups * LANES_GROUP}, first, stride);
+    } else if (j.kind == PACK_REG) {
+        if constexpr (MODE == 16) pack_filters_reg_body<MAP>(j.a, first, stride);
     } else if (MODE == 16) {  // PACK_PWX (16-product form only)
         const PackPwxArgs pa{j.a, j.WCO, j.nsteps};
         pack_filters_pwx_body<MAP>(pa, first, stride);
@@ -30,7 +33,7 @@ static __device__ __forceinline__ void pack_job_as(const PackJob& j, long first,
 __global__ void __launch_bounds__(WG_THREADS) pack_jobs_kernel(const PackJobs J) {
     int k = 0;
     while (k + 1 < J.n && (int)blockIdx.x >= J.job[k + 1].block0) ++k;
-    const PackJob& j = J.job[k];
+    const PackJob j = J.job[k];  // (by value: through a reference with this many users the compiler copies all jobs to scratch memory)
     const long first = (long)((int)blockIdx.x - j.block0) * WG_THREADS + threadIdx.x;
     const long stride = (long)j.nblocks * WG_THREADS;
     if (j.mode == 16) {

@@ -1,0 +1,10 @@
+// The kernel on registers for filter rows of 1 tap, dilation 1, stride 1.
+#include "phx_launch_reg16.h"
+
+namespace phx {
+
+int launch_reg_k1d1s1(bool cl, const RegArgs& a, const NormArgs& norm, int waves, int blocks, hipStream_t st) {
+    return launch_reg_row<1, 1, 1>(cl, a, norm, waves, blocks, st);
+}
+
+}  // namespace phx

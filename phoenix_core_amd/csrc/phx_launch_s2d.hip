@@ -193,8 +193,8 @@ int launch_add_inplace(bool half_storage, void* dst, const void* src, long count
 // type): what closes a forward / input-gradient pass whose reduction over the channels was cut into slices.  fp32 sums,
 // one rounding.
 struct NoNorm {};
-template <typename TS, bool NORM>
-__global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial, int slices, long count, TS* dst, const TS* bias,
+template <typename TS, typename TP, bool NORM>
+__global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TP* partial, int slices, long count, TS* dst, const TS* bias,
                                                                const TS* addend, int plane, int channels, long comp_count,
                                                                const std::conditional_t<NORM, NormArgs, NoNorm> norm) {
     const long stride = (long)gridDim.x * blockDim.x;
@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial
         float acc = 0.0f;
         int z = 0;
         for (; z + 4 <= slices; z += 4) {  // (four loads in flight; added one after the other, the order of a plain loop)
-            TS v[4];
+            TP v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = partial[(z + i) * count + e];
 #pragma unroll
@@ -221,21 +221,21 @@ __global__ void __launch_bounds__(WG_THREADS) slice_sum_kernel(const TS* partial
     }
 }
 
-template <typename TS>
+template <typename TS, typename TP>
 static void slice_sum(const void* partial, int slices, long count, void* dst, const void* bias, const void* addend, int plane, int channels,
                       long comp_count, const NormArgs& norm, hipStream_t st) {
     const auto launch = [&](auto kernel, const auto& last) {
-        hipLaunchKernelGGL(kernel, dim3(blocks_for(count)), dim3(WG_THREADS), 0, st, static_cast<const TS*>(partial), slices, count,
+        hipLaunchKernelGGL(kernel, dim3(blocks_for(count)), dim3(WG_THREADS), 0, st, static_cast<const TP*>(partial), slices, count,
                            static_cast<TS*>(dst), static_cast<const TS*>(bias), static_cast<const TS*>(addend), plane, channels, comp_count, last);
     };
-    if (norm.gamma) launch(slice_sum_kernel<TS, true>, norm);
-    else launch(slice_sum_kernel<TS, false>, NoNorm{});
+    if (norm.gamma) launch(slice_sum_kernel<TS, TP, true>, norm);
+    else launch(slice_sum_kernel<TS, TP, false>, NoNorm{});
 }
 
 int launch_slice_sum(bool half_storage, const void* partial, int slices, long count, void* dst, const void* bias, const void* addend,
-                     int plane, int channels, long comp_count, const NormArgs& norm, hipStream_t st) {
+                     int plane, int channels, long comp_count, const NormArgs& norm, hipStream_t st, bool partial_f32) {
     if (count <= 0) return 0;
-    (half_storage ? slice_sum<_Float16> : slice_sum<float>)(partial, slices, count, dst, bias, addend, plane, channels, comp_count, norm, st);
+    (!half_storage ? slice_sum<float, float> : partial_f32 ? slice_sum<_Float16, float> : slice_sum<_Float16, _Float16>)(partial, slices, count, dst, bias, addend, plane, channels, comp_count, norm, st);
     return 0;
 }
 
