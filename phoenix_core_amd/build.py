@@ -1,4 +1,5 @@
-"""Compiles the HIP sources of the engine for gfx950 into phoenix_core_amd/lib/libphx_qconv.so.
+"""Compiles the HIP sources of the engine for gfx950 into phoenix_core_amd/lib/libphx_qconv.so, and the host path of its
+operators on torch tensors into phoenix_core_amd/lib/_phx_host.so (a Python extension module, no device code).
 
 Run as `python -m phoenix_core_amd.build`; hipcc cross-compiles without a GPU present."""
 import os
@@ -17,6 +18,22 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]
+
+
+HOST_SOURCE = os.path.join(HERE, "host", "phx_host.cc")
+HOST_PATH = os.path.join(LIB_DIR, "_phx_host.so")
+
+
+def _host_command():
+    import sysconfig
+    import torch
+    base = os.path.dirname(torch.__file__)
+    # (the HIP headers that torch's own headers of streams include want their platform named where hipcc does not)
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + os.path.join(base, "include"),
+            "-I" + os.path.join(base, "include", "torch", "csrc", "api", "include"), "-I/opt/rocm/include",
+            "-I" + sysconfig.get_paths()["include"], HOST_SOURCE, "-o", HOST_PATH, "-L" + os.path.join(base, "lib"),
+            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
 
 def sources():
@@ -41,8 +58,15 @@ def build(verbose=True, extra_flags=()):
     jobs = [(src, os.path.join(objdir, os.path.basename(src)[:-4] + ".o"), flags) for src in sources()]
     if verbose:
         print("+ %s %s -c {%s}" % (HIPCC, " ".join(flags), ", ".join(os.path.basename(j[0]) for j in jobs)), flush=True)
+    host = _host_command()
+    if verbose:
+        print("+", " ".join(host), flush=True)
     with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as pool:
+        host_result = pool.submit(subprocess.run, host, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         results = list(pool.map(_compile_one, jobs))
+    host_done = host_result.result()
+    if host_done.returncode != 0:
+        raise RuntimeError("%s failed on %s:\n%s" % (host[0], HOST_SOURCE, host_done.stdout))
     for src, rc, out in results:
         if verbose and out.strip():
             print(out, flush=True)

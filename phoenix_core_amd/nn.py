@@ -384,6 +384,12 @@ def _conv_norm(conv, norm, x, residual=None):
     """norm(conv(x), residual), as one operator (the same bits) where that can be told from the two by nothing: both
     modules are this file's and unhooked, norm is in evaluation mode, and no gradient is recorded.  (A network in evaluation
     mode is bound by the host: parameters are taken from the modules' dictionaries, not through Module.__getattr__.)"""
+    if (type(conv) is QConv2d and type(norm) is QBatchNorm2d and PREPACK_FILTERS and not torch.compiler.is_compiling() and
+            not torch.nn.modules.module._has_any_global_hook()):
+        # (from the second call of a shape on: the same checks and the same call)
+        y = ops._host.conv_norm(conv.__dict__, norm.__dict__, x, residual)
+        if y is not NotImplemented:
+            return y
     if (type(conv) is QConv2d and type(norm) is QBatchNorm2d and not norm.training and not torch.is_grad_enabled() and
             conv.data_format == "NCHW" and not (_hooked(conv) or _hooked(norm) or torch.nn.modules.module._has_any_global_hook())):
         cp, np, buffers = conv._parameters, norm._parameters, norm._buffers

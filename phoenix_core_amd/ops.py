@@ -9,6 +9,8 @@ C ABI; nothing here computes on the CPU.  The algebras other than the quaternion
 the same kernels by rearrangement kernels inside the library (csrc/phx_algebra.hip).
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -16,6 +18,30 @@ import torch
 from . import capi
 
 REAL, COMPLEX, QUATERNION, GA_300 = 0, 1, 2, 3  # src/algebras.hpp:17-22
+
+HOST_PATH = os.path.join(os.path.dirname(capi.__file__), "lib", "_phx_host.so")
+
+
+class _Unloaded:
+    """Stands for the extension module (host/phx_host.cc) until its first use; there is no path without it."""
+
+    def __getattr__(self, name):
+        global _host
+        if not os.path.isfile(HOST_PATH):
+            raise ImportError("%s is missing: build it with `python -m phoenix_core_amd.build`" % HOST_PATH)
+        lib = capi.lib()
+        loader = importlib.machinery.ExtensionFileLoader("_phx_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_phx_host", loader))
+        loader.exec_module(module)
+        addresses = {f: ctypes.cast(getattr(lib, f), ctypes.c_void_p).value for f in capi.EXPORTS + capi.EXPORTS_BN}
+        module.bind(addresses, vars(capi), capi.check, torch.nn.Parameter, vars(torch.autograd.forward_ad))
+        _host = module
+        return getattr(module, name)
+
+
+# The operators below hand a plain call to this module, which answers NotImplemented for any other; what follows in each of
+# them is the operator's definition and serves the rest.
+_host = _Unloaded()
 
 
 class Context:
@@ -157,6 +183,9 @@ class Conv2DDescriptor:
             self.context.product_mode, self.context.fp16_policy, int(self.use_bias and not self.real_valued_input),
             int(self.real_valued_input), groups, capi.PHX_NCHW if data_format == "NCHW" else capi.PHX_NHWC)
 
+    def __getstate__(self):  # (copies and pickles make what the host path keeps of a descriptor anew)
+        return {k: v for k, v in self.__dict__.items() if k != "_host"}
+
     def workspace_bytes(self, which):
         return capi.lib().phx_qconv2d_workspace_bytes(ctypes.byref(self.c), which)
 
@@ -192,6 +221,9 @@ class DenseDescriptor:
                                  self.context.product_mode, self.context.fp16_policy, int(self.use_bias),
                                  capi.PHX_IO if filter_layout == "IO" else capi.PHX_OI)
 
+    def __getstate__(self):  # (copies and pickles make what the host path keeps of a descriptor anew)
+        return {k: v for k, v in self.__dict__.items() if k != "_host"}
+
     def workspace_bytes(self, which):
         return capi.lib().phx_qdense_workspace_bytes(ctypes.byref(self.c), which)
 
@@ -205,31 +237,6 @@ def default_context():
         _default_context = Context()
     return _default_context
 
-
-class _Workspace:
-    """Grow-only scratch buffer per device and stream, shared by the operations enqueued there (the reference's
-    Device keeps one workspace for all its operations, src/backend/device.hpp:75-84, and serializes them with a
-    mutex; here the stream's own order serializes them, and calls on different streams get different buffers)."""
-
-    def __init__(self):
-        self.buffers = {}
-
-    def get(self, device, nbytes, stream=None):
-        key = (device, current_stream_handle(device) if stream is None else stream)
-        buf = self.buffers.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-            self.buffers[key] = buf
-        return buf
-
-
-    def holds(self, device, stream, nbytes):
-        """Whether the buffer of that stream is already large enough (no allocation would happen)."""
-        buf = self.buffers.get((device, stream))
-        return buf is not None and buf.numel() >= nbytes
-
-
-_workspace = _Workspace()
 
 # torch.cuda.current_stream() builds a Stream object through several Python layers (6-7 us per call, twice per
 # operator call); the raw handle is all the library needs
@@ -270,16 +277,27 @@ def _ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def _scratch(device, nbytes, stream=None):
+    """Grow-only scratch buffer per device and stream, shared by the operations enqueued there (the reference's
+    Device keeps one workspace for all its operations, src/backend/device.hpp:75-84, and serializes them with a
+    mutex; here the stream's own order serializes them, and calls on different streams get different buffers)."""
+    return _host.workspace(_index(device), current_stream_handle(device) if stream is None else stream, nbytes)
+
+
+def _index(device):
+    return torch.cuda.current_device() if device.index is None else device.index
+
+
 def workspace_holds(device, stream, nbytes):
     """Whether the scratch buffer of that stream (a handle) already has nbytes: a call on it then allocates nothing."""
-    return _workspace.holds(device, stream, int(nbytes))
+    return _host.workspace_holds(_index(device), stream, int(nbytes))
 
 
 def reserve_workspace(nbytes, device=None):
     """Grows the scratch buffer of the current stream to at least nbytes ahead of time -- in front of a stream
     capture, inside which the buffer must not be reallocated."""
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
-    return _workspace.get(device, int(nbytes))
+    return _scratch(device, int(nbytes))
 
 
 def _stream(device, stream=None):
@@ -325,6 +343,10 @@ def conv2d_pack_filters(w, desc, bwd_data=True, into=None):
     """Packs w for the forward pass and (bwd_data) the input gradient of desc with one kernel launch; `into`: a
     PackedFilters of the same descriptor to overwrite (no allocation).  Returns None when neither pass has a
     prepacked form."""
+    if into is not None:
+        done = _host.conv_pack(desc, w, into)
+        if done is not NotImplemented:
+            return done
     dev = _dev_check(w)
     _expect(w, desc.filter_shape, desc.dtype, "filter")
     if into is None:
@@ -346,6 +368,9 @@ def conv2d_pack_filters(w, desc, bwd_data=True, into=None):
 def conv2d_fwd(x, w, bias, desc, out=None, packed=None):
     """conv2DFwd (src/upstride.hpp:18-33): y = x (x) w (+ bias).  packed: PackedFilters of (w, desc) -- the call
     then reads the packed image and not w."""
+    y = _host.conv_fwd(desc, x, w, bias, out, packed)
+    if y is not NotImplemented:
+        return y
     dev = _dev_check(x, w, bias, out)
     _expect(x, desc.input_shape, desc.dtype, "input")
     _expect(w, desc.filter_shape, desc.dtype, "filter")
@@ -357,7 +382,7 @@ def conv2d_fwd(x, w, bias, desc, out=None, packed=None):
         _expect(out, desc.output_shape, desc.dtype, "output")
     y = out if out is not None else torch.empty(desc.output_shape, dtype=desc.dtype, device=dev)
     nbytes = desc.workspace_bytes(capi.PHX_PASS_FWD)
-    ws = _workspace.get(dev, nbytes)
+    ws = _scratch(dev, nbytes)
     if packed is not None and packed.fwd is not None:
         packed.check(desc)
         capi.check(capi.lib().phx_qconv2d_fwd_prepacked(ctypes.byref(desc.c), _stream(dev), _ptr(x), _ptr(packed.fwd),
@@ -395,7 +420,7 @@ def _conv2d_fwd_norm(dev, x, w, bias, desc, own, eps, relu, residual, packed):
     y = torch.empty(desc.output_shape, dtype=desc.dtype, device=dev)
     nbytes = desc.workspace_bytes(capi.PHX_PASS_FWD)
     stream = current_stream_handle(dev)
-    ws = _workspace.get(dev, nbytes, stream)
+    ws = _scratch(dev, nbytes, stream)
     gamma, beta, mean, var = own
     norm = capi.OutputNorm(gamma.data_ptr(), beta.data_ptr(), mean.data_ptr(), var.data_ptr(),
                            None if residual is None else residual.data_ptr(), eps, relu)
@@ -413,12 +438,15 @@ def conv2d_bwd_weights(x, grad, desc, stream=None):
     """The filter-gradient half of conv2DBwd (src/conv2d.hpp:330-440): dw.  stream: the handle of a stream to enqueue
     on instead of the device's current one; the caller then orders that stream behind the producers of x and grad
     and the consumers of dw behind it (dw itself is allocated on the current stream)."""
+    dw = _host.conv_bwd_weights(desc, x, grad, stream)
+    if dw is not NotImplemented:
+        return dw
     dev = _dev_check(x, grad)
     _expect(x, desc.input_shape, desc.dtype, "input")
     _expect(grad, desc.output_shape, desc.dtype, "output gradient")
     dw = torch.empty(desc.filter_shape, dtype=desc.dtype, device=dev)
     nbytes = desc.workspace_bytes(capi.PHX_PASS_BWD_WEIGHTS)
-    ws = _workspace.get(dev, nbytes, stream)
+    ws = _scratch(dev, nbytes, stream)
     capi.check(capi.lib().phx_qconv2d_bwd_weights(ctypes.byref(desc.c), _stream(dev, stream), _ptr(x), _ptr(grad), _ptr(dw),
                                                   _ptr(ws), nbytes), "phx_qconv2d_bwd_weights")
     return dw
@@ -428,6 +456,9 @@ def conv2d_bwd_data(w, grad, desc, packed=None, addend=None):
     """The input-gradient half of conv2DBwd: dx (the descriptor must ask for it).  packed: as in conv2d_fwd.
     addend: a tensor like dx that is added to it (phx_qconv2d_bwd_data_add: in the kernel's epilogue where it can,
     the same values as dx + addend either way); quaternion descriptors only."""
+    dx = _host.conv_bwd_data(desc, w, grad, packed, addend)
+    if dx is not NotImplemented:
+        return dx
     dev = _dev_check(w, grad, addend)
     _expect(w, desc.filter_shape, desc.dtype, "filter")
     _expect(grad, desc.output_shape, desc.dtype, "output gradient")
@@ -435,7 +466,7 @@ def conv2d_bwd_data(w, grad, desc, packed=None, addend=None):
         raise RuntimeError("Input gradient required for type0 input tensor")
     dx = torch.empty(desc.input_shape, dtype=desc.dtype, device=dev)
     nbytes = desc.workspace_bytes(capi.PHX_PASS_BWD_DATA)
-    ws = _workspace.get(dev, nbytes)
+    ws = _scratch(dev, nbytes)
     if addend is not None:
         _expect(addend, desc.input_shape, desc.dtype, "addend")
         image = packed.bwd_data if packed is not None else None
@@ -459,6 +490,9 @@ def conv2d_bwd_data(w, grad, desc, packed=None, addend=None):
 def conv2d_bwd(x, w, grad, desc):
     """conv2DBwd (src/upstride.hpp:35-51): returns (dw, dx); dx is None when the descriptor does
     not require the input gradient."""
+    both = _host.conv_bwd(desc, x, w, grad, desc.require_input_grad)
+    if both is not NotImplemented:
+        return both
     _dev_check(x, w, grad)
     _expect(w, desc.filter_shape, desc.dtype, "filter")
     dw = conv2d_bwd_weights(x, grad, desc)
@@ -468,6 +502,9 @@ def conv2d_bwd(x, w, grad, desc):
 
 def dense_fwd(x, w, bias, desc, out=None):
     """denseFwd (src/upstride.hpp:53-68)."""
+    y = _host.dense_fwd(desc, x, w, bias, out)
+    if y is not NotImplemented:
+        return y
     dev = _dev_check(x, w, bias, out)
     _expect(x, desc.input_shape, desc.dtype, "input")
     _expect(w, desc.filter_shape, desc.dtype, "filter")
@@ -477,7 +514,7 @@ def dense_fwd(x, w, bias, desc, out=None):
         _expect(out, desc.output_shape, desc.dtype, "output")
     y = out if out is not None else torch.empty(desc.output_shape, dtype=desc.dtype, device=dev)
     nbytes = desc.workspace_bytes(capi.PHX_PASS_FWD)
-    ws = _workspace.get(dev, nbytes)
+    ws = _scratch(dev, nbytes)
     capi.check(capi.lib().phx_qdense_fwd(ctypes.byref(desc.c), _stream(dev), _ptr(x), _ptr(w),
                                          _ptr(bias if desc.use_bias else None), _ptr(y), _ptr(ws), nbytes),
                "phx_qdense_fwd")
@@ -486,20 +523,23 @@ def dense_fwd(x, w, bias, desc, out=None):
 
 def dense_bwd(x, w, grad, desc):
     """denseBwd (src/upstride.hpp:70-86): returns (dw, dx)."""
+    both = _host.dense_bwd(desc, x, w, grad, desc.require_input_grad)
+    if both is not NotImplemented:
+        return both
     dev = _dev_check(x, w, grad)
     _expect(x, desc.input_shape, desc.dtype, "input")
     _expect(w, desc.filter_shape, desc.dtype, "filter")
     _expect(grad, desc.output_shape, desc.dtype, "output gradient")
     dw = torch.empty(desc.filter_shape, dtype=desc.dtype, device=dev)
     nbytes = desc.workspace_bytes(capi.PHX_PASS_BWD_WEIGHTS)
-    ws = _workspace.get(dev, nbytes)
+    ws = _scratch(dev, nbytes)
     capi.check(capi.lib().phx_qdense_bwd_weights(ctypes.byref(desc.c), _stream(dev), _ptr(x), _ptr(grad), _ptr(dw),
                                                  _ptr(ws), nbytes), "phx_qdense_bwd_weights")
     dx = None
     if desc.require_input_grad:
         dx = torch.empty(desc.input_shape, dtype=desc.dtype, device=dev)
         nbytes = desc.workspace_bytes(capi.PHX_PASS_BWD_DATA)
-        ws = _workspace.get(dev, nbytes)
+        ws = _scratch(dev, nbytes)
         capi.check(capi.lib().phx_qdense_bwd_data(ctypes.byref(desc.c), _stream(dev), _ptr(grad), _ptr(w), _ptr(dx),
                                                   _ptr(ws), nbytes), "phx_qdense_bwd_data")
     return dw, dx
@@ -509,6 +549,9 @@ def batch_norm_fwd(x, gamma, beta, running_mean, running_var, eps, momentum, rel
     """Training-mode batch normalisation (+ residual, + ReLU) of [rows, C, H, W] (include/phx_bn.h; no counterpart in
     the reference, which holds no model code).  Returns (y, save_mean, save_invstd); the running statistics are
     updated in place when given."""
+    done = _host.bn_fwd(x, gamma, beta, running_mean, running_var, eps, momentum, relu, residual)
+    if done is not NotImplemented:
+        return done
     dev = _dev_check(x, gamma, beta, running_mean, running_var, residual)
     if residual is not None and (residual.shape != x.shape or residual.dtype != x.dtype):
         raise ValueError("the residual must have the shape and type of the input")
@@ -524,7 +567,7 @@ def batch_norm_fwd(x, gamma, beta, running_mean, running_var, eps, momentum, rel
     mean = torch.empty(c, dtype=torch.float32, device=dev)
     invstd = torch.empty(c, dtype=torch.float32, device=dev)
     nbytes = capi.lib().phx_bn_workspace_bytes(ctypes.byref(desc))
-    ws = _workspace.get(dev, nbytes)
+    ws = _scratch(dev, nbytes)
     capi.check(capi.lib().phx_bn_fwd_train(ctypes.byref(desc), _stream(dev), _ptr(x), _ptr(residual), _ptr(gamma), _ptr(beta),
                                            _ptr(y), _ptr(mean), _ptr(invstd), _ptr(running_mean), _ptr(running_var),
                                            _ptr(ws), nbytes), "phx_bn_fwd_train")
@@ -551,6 +594,9 @@ def batch_norm_eval(x, gamma, beta, running_mean, running_var, eps, relu, residu
 
 def batch_norm_bwd(x, dy, gamma, beta, mean, invstd, eps, relu, residual=None):
     """Returns (dx, dgamma, dbeta, dresidual) of batch_norm_fwd; dresidual is None without a residual."""
+    done = _host.bn_bwd(x, dy, gamma, beta, mean, invstd, eps, relu, residual)
+    if done is not NotImplemented:
+        return done
     dev = _dev_check(x, dy, gamma, beta, mean, invstd, residual)
     rows, c = x.shape[0], x.shape[1]
     if x.dtype not in _DTYPES:
@@ -568,7 +614,7 @@ def batch_norm_bwd(x, dy, gamma, beta, mean, invstd, eps, relu, residual=None):
     dgamma = (torch.zeros if empty else torch.empty)(c, dtype=torch.float32, device=dev)
     dbeta = (torch.zeros if empty else torch.empty)(c, dtype=torch.float32, device=dev)
     nbytes = capi.lib().phx_bn_workspace_bytes(ctypes.byref(desc))
-    ws = _workspace.get(dev, nbytes)
+    ws = _scratch(dev, nbytes)
     capi.check(capi.lib().phx_bn_bwd(ctypes.byref(desc), _stream(dev), _ptr(x), _ptr(residual), _ptr(dy), _ptr(gamma),
                                      _ptr(beta), _ptr(mean), _ptr(invstd), _ptr(dx), _ptr(dres), _ptr(dgamma), _ptr(dbeta),
                                      _ptr(ws), nbytes), "phx_bn_bwd")
