@@ -89,22 +89,24 @@ enum { PWX_PLAIN = 0, PWX_ADD = 1, PWX_NORM = 2, PWX_NORM_ADD = 3 };
 template <int TAIL>
 using PwxArgsOf = std::conditional_t<(TAIL >= 2), PwxNormArgs, PwxArgs>;  // (a literal: the name of an unnamed enum's value differs between host and device symbols)
 
-// rounded results of one channel through norm, residual (RES) and ReLU, as bn_eval_kernel takes them
+// Rounded results of one channel through norm, residual (RES) and ReLU, as bn_eval_kernel takes them: v - mean and v + residual
+// of halves in one mixed-precision fma each (tail.one: a factor of 1 that the compiler may not fold), the ReLU against
+// tail.lowest, two results rounded by one instruction.  This arithmetic was half of what the norm cost these kernels, 10.5
+// vector instructions a value and now 5.5.
 template <bool RES, typename W>
-__device__ __forceinline__ W norm_words(const f32x4& factors, const W& y, const W& res, int relu) {
+__device__ __forceinline__ W norm_words(const f32x4& factors, const W& y, const W& res, const NormTail& tail) {
     W out;
 #pragma unroll
     for (int i = 0; i < (int)(sizeof(W) / 4); ++i) {
         const f16x2 h = __builtin_bit_cast(f16x2, (unsigned int)y[i]), r = __builtin_bit_cast(f16x2, (unsigned int)res[i]);
-        f16x2 o;
+        f32x2 o;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            float v = norm_apply(factors, (float)h[e]);
-            asm("" : "+v"(v));  // (an fp32 value: v_fma_mixlo_f16 would round the product and sum to fp16 at once)
-            if constexpr (RES) v += (float)r[e];
-            o[e] = (_Float16)relu_if(relu, v);
+            float v = norm_half(factors, h[e], tail);
+            if constexpr (RES) v = __builtin_fmaf((float)r[e], tail.one, v);
+            o[e] = relu_at(tail, v);
         }
-        out[i] = __builtin_bit_cast(unsigned int, o);
+        out[i] = __builtin_bit_cast(unsigned int, __builtin_convertvector(o, f16x2));
     }
     return out;
 }
@@ -270,6 +272,14 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
     };
 
     f32x16 acc[4][2];
+    constexpr int AHEAD = 2;  // components of the addend in flight (what the registers have room for)
+    // NORM: of output channel j of the wave's 32, requested in front of an item's last products; store_item hands them round
+    // through LDS.  With the arithmetic of norm_words, norm and residual cost 64 -> 256 channels at 14x14, 8 images, 3.4 us on
+    // top of 6.9 (with four channels' loads a lane behind the last product and one component in flight, 5.3), 16 -> 64 at 56x56,
+    // 64 images, 19 on top of 24 (25).
+    NormRaw raw;
+    NormTail tail;
+    if constexpr (NORM) tail = norm_tail_of(P0.norm);
     PHX_PHASES_BEGIN(5)
     const int my_items = P.items > wg ? (P.items - wg + (int)gridDim.x - 1) / (int)gridDim.x : 0;
     const int total_steps = my_items * P.nsteps;
@@ -347,10 +357,10 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
     auto store_item = [&](auto bias_tag, auto half_tag) {
         constexpr bool BIAS = decltype(bias_tag)::value, HALF = decltype(half_tag)::value;
         const int co0 = (c_ct * WCO + wco) * 32;
-        // (TSTORE) the addend's vectors of a component are requested a component ahead -- the first here, in
-        // front of the drain, which then covers their latency; the others in front of the stores of the component
+        // (TSTORE) the addend's vectors of a component are requested AHEAD components ahead -- the first here, in
+        // front of the drain, which then covers their latency; the others in front of the stores of a component
         // before -- so that no store waits for a load of its own
-        u32x4 ad[4];
+        u32x4 ad[AHEAD][4];
         auto request_addend = [&](int q, u32x4 (&dst)[4]) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -359,20 +369,27 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
                 dst[i] = ok ? load16_a2(P.addend + q * P.out_cs + (long)(co0 + c) * HW + oaddr[0]) : u32x4{0u, 0u, 0u, 0u};
             }
         };
-        if constexpr (TSTORE && ADD) request_addend(0, ad);
+        if constexpr (TSTORE && ADD) {
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q) request_addend(q, ad[q]);
+        }
         const int co = co0 + j;
         const bool co_ok = co < P.Cout;
-        f32x4 factors[4];  // TSTORE: of the channels that this lane stores; else of its own
-        if constexpr (NORM) {
-#pragma unroll
-            for (int i = 0; i < (TSTORE ? 4 : 1); ++i) {
-                const int c = co0 + (TSTORE ? 8 * i + (lane >> 3) : j);
-                factors[i] = norm_factors(P0.norm, c < P.Cout ? c : 0);
-            }
-        }
         wait_vmem_all();  // this wave's copies of the steps ahead: landed
         PHX_STAMP(2)
         char* scr = reinterpret_cast<char*>(lds16 + RF * WV + RA * XV) + wave * (S::SCRV * 16);  // (TSTORE) this wave's own
+        f32x4 factors[4];  // TSTORE: of the channels that this lane stores; else of its own
+        if constexpr (NORM) {
+            factors[0] = norm_factors(raw, P0.norm.eps);
+            if constexpr (TSTORE) {
+                f32x4* const shared = reinterpret_cast<f32x4*>(scr);
+                shared[j] = factors[0];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+#pragma unroll
+                for (int i = 0; i < 4; ++i) factors[i] = shared[8 * i + (lane >> 3)];
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             float bv = 0.f;
@@ -409,7 +426,7 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
                         if (ov && co_ok) {
                             u32x2 a = v;
                             if constexpr (ADD) a = load8_a2(P.addend + q * P.out_cs + (long)co * HW + oa + 4 * kk);
-                            if constexpr (NORM) v = norm_words<ADD>(factors[0], v, a, P0.norm.relu);
+                            if constexpr (NORM) v = norm_words<ADD>(factors[0], v, a, tail);
                             else if constexpr (ADD) v = add_halves4(v, a);
                             *reinterpret_cast<u32x2_a2*>(dst + oa + 4 * kk) = v;
                         }
@@ -424,11 +441,11 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     t[i] = *reinterpret_cast<const u32x4*>(scr + ((8 * i + (lane >> 3)) * 9 + (lane & 7)) * 16);
-                    if constexpr (NORM) t[i] = norm_words<ADD>(factors[i], t[i], ADD ? ad[i] : t[i], P0.norm.relu);
-                    else if constexpr (ADD) t[i] = add_halves(t[i], ad[i]);
+                    if constexpr (NORM) t[i] = norm_words<ADD>(factors[i], t[i], ADD ? ad[q % AHEAD][i] : t[i], tail);
+                    else if constexpr (ADD) t[i] = add_halves(t[i], ad[q % AHEAD][i]);
                 }
                 if constexpr (ADD) {
-                    if (q < 3) request_addend(q + 1, ad);  // (in front of this component's stores)
+                    if (q + AHEAD < 4) request_addend(q + AHEAD, ad[q % AHEAD]);  // (in front of this component's stores)
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -459,6 +476,9 @@ __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pwx_f16_kernel(const PwxA
             PHX_STAMP(0)
             wg_barrier_no_vmem_wait();  // ... for every wave; and every wave is done with the stages the next copies overwrite
             PHX_STAMP(1)
+            if constexpr (NORM) {
+                if (c_k + 1 == P.nsteps) raw = norm_raw(P0.norm, min((c_ct * WCO + wco) * 32 + j, P.Cout - 1));
+            }
             if (c_k == 0) products(c_half, std::true_type(), half_tag);
             else products(c_half, std::false_type(), half_tag);
             PHX_STAMP(3)

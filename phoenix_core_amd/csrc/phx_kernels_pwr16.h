@@ -125,6 +125,8 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
     };
 
     f32x16 acc[WCO][4];
+    NormTail tail;
+    if constexpr (NORM) tail = norm_tail_of(P0.norm);
     locate_in(l_item);
     locate_out(c_item);
     issue_stage(0);
@@ -181,7 +183,21 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
     auto store_item = [&](int w0, auto nco_tag) {
         constexpr int NCO = decltype(nco_tag)::value;
         // Stores share the counter of the copies and complete in no fixed order relative to them: the copies of the
-        // next step (requested a step ago) are drained first, and the next step then needs no wait of its own.
+        // next step (requested a step ago) are drained first, and the next step then needs no wait of its own.  What the
+        // results meet on their way out is requested in front of that drain, the addend a component ahead from there on.
+        NormRaw raw[NCO];
+        if constexpr (NORM) {
+#pragma unroll
+            for (int wc = 0; wc < NCO; ++wc) raw[wc] = norm_raw(P0.norm, min((w0 + wc) * 32 + j, P.Cout - 1));
+        }
+        u32x4 ad[2][2];
+        auto request_addend = [&](int i) {  // of component i % 4 of sub-tile i / 4
+            const int co = (w0 + i / 4) * 32 + j;
+            const _Float16* asrc = P.addend + (i % 4) * P.out_cs + (long)co * HW;
+#pragma unroll
+            for (int a = 0; a < 2; ++a) ad[i % 2][a] = (ovalid[a] && co < P.Cout) ? load16_a2(asrc + oaddr[a]) : u32x4{0u, 0u, 0u, 0u};
+        };
+        if constexpr (ADD) request_addend(0);
         wait_vmem_all();
         landed = true;
 #pragma unroll
@@ -189,18 +205,15 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
             const int co = (w0 + wc) * 32 + j;
             const bool co_ok = co < P.Cout;
             f32x4 factors;
-            if constexpr (NORM) factors = norm_factors(P0.norm, co_ok ? co : 0);
+            if constexpr (NORM) factors = norm_factors(raw[wc], P0.norm.eps);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 __builtin_amdgcn_sched_barrier(0);  // (one tile at a time leaves the accumulator file)
                 // (an unconditional load -- zeros where there is no bias -- keeps branches out of the epilogue)
                 const float bv = (float)*(P.bias ? P.bias + q * P.CoutS + (co_ok ? co : 0) : zero_ptr<_Float16>());
                 _Float16* dst = P.out + q * P.out_cs + (long)co * HW;
-                u32x4 ad[2];  // (the addend's words are requested before the conversions, which then cover their latency)
                 if constexpr (ADD) {
-                    const _Float16* asrc = P.addend + q * P.out_cs + (long)co * HW;
-#pragma unroll
-                    for (int a = 0; a < 2; ++a) ad[a] = (ovalid[a] && co_ok) ? load16_a2(asrc + oaddr[a]) : u32x4{0u, 0u, 0u, 0u};
+                    if (wc * 4 + q + 1 < NCO * 4) request_addend(wc * 4 + q + 1);
                 }
                 unsigned int d[4][2];  // [quad][pair]: pixels 8 g + 4 kk + 2 i, + 1
 #pragma unroll
@@ -223,8 +236,8 @@ __global__ void __launch_bounds__(WG_THREADS, 1) qconv_pwr_f16_kernel(const PwxA
                         v[i] = s[0];
                         v[2 + i] = s[1];
                     }
-                    if constexpr (NORM) v = norm_words<ADD>(factors, v, ADD ? ad[a] : v, P0.norm.relu);
-                    else if constexpr (ADD) v = add_halves(v, ad[a]);
+                    if constexpr (NORM) v = norm_words<ADD>(factors, v, ADD ? ad[q % 2][a] : v, tail);
+                    else if constexpr (ADD) v = add_halves(v, ad[q % 2][a]);
                     if (ovalid[a] && co_ok) *reinterpret_cast<u32x4_a2*>(dst + oaddr[a]) = v;
                 }
             }

@@ -353,18 +353,19 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
             const long plane = q * P.out_cs + ((long)img * P.Cout + co) * HWout;
             const float b = P.bias ? (float)P.bias[q * P.Cout + co] : 0.f;
             [[maybe_unused]] f32x4 nf;
+            [[maybe_unused]] NormTail tail;
             const _Float16* more = P.addend;
             if constexpr (NORM) {
+                tail = norm_tail_of(P.norm);
                 nf = norm_factors(P.norm, co);
                 more = static_cast<const _Float16*>(P.norm.res);
             }
             auto result = [&](float sum, float other) __attribute__((always_inline)) {
                 float o = sum + b;
                 if constexpr (NORM) {
-                    o = norm_result<_Float16>(nf, o);
-                    asm("" : "+v"(o));  // (an fp32 value: v_fma_mixlo_f16 would round the product and sum to fp16 at once)
-                    if (more) o += other;
-                    return (_Float16)relu_if(P.norm.relu, o);
+                    o = norm_half(nf, (_Float16)o, tail);
+                    if (more) o = __builtin_fmaf((float)other, tail.one, o);
+                    return (_Float16)relu_at(tail, o);
                 } else {
                     const _Float16 h = (_Float16)o;
                     return more ? (_Float16)((float)h + other) : h;

@@ -55,7 +55,6 @@ __host__ __device__ inline size_t x3_packed_bytes(int S, int co_tiles, int nchun
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 
 __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
