@@ -124,7 +124,8 @@ def test_the_rule_takes_small_problems(tune_env):
     """Both sides of the rule's lines (n, ci, co, extent, k, layout, whether the kernel runs)."""
     tune_env(PHX_TUNE_REG=None)
     for n, ci, co, e, k, layout, runs in [(8, 128, 128, 7, 3, "NCHW", True), (128, 128, 128, 28, 3, "NCHW", False), (4, 24, 64, 9, 3, "NCHW", False),
-                                          (8, 512, 128, 7, 1, "NCHW", True), (8, 64, 128, 14, 1, "NCHW", False), (2, 64, 64, 14, 1, "NHWC", False),
+                                          (8, 512, 128, 7, 1, "NCHW", True), (8, 64, 96, 14, 1, "NCHW", False), (8, 64, 256, 14, 1, "NCHW", True),
+                                          (8, 128, 512, 7, 1, "NCHW", True), (64, 64, 256, 14, 1, "NCHW", False), (2, 64, 64, 14, 1, "NHWC", False),
                                           (2, 66, 64, 14, 1, "NHWC", True), (2, 64, 64, 14, 5, "NHWC", True)]:
         shape = (4 * n, ci, e, e) if layout == "NCHW" else (4 * n, e, e, ci)
         x, w = torch.randn(shape, device="cuda").half(), torch.randn(4, co, ci, k, k, device="cuda").half()
