@@ -74,6 +74,7 @@ struct ConvArgs {
     int nhwc;           // the output is channels-last, out[4][N][Hout][Wout][CoutS] (fp16 chunk-staging kernel only)
     int groups;         // grid rows: the groups of a grouped convolution run by this one launch (1 otherwise)
     long g_in, g_w, g_bias, g_out;  // bytes from one group's input / packed filters / bias / output to the next group's
+    int last_c, last_chunks;        // channels and chunks of the last group (reduction slices of fp32 tensors); 0: as the others'
 };
 
 struct ConvNormArgs : ConvArgs {  // of the NORM instances (the others' calls carry no bytes they do not read: 0.2 us a launch)
@@ -89,6 +90,16 @@ __device__ __forceinline__ ConvArgs group_view(const ConvArgs& P0) {
     P.wpk = group_shift(P0.wpk, P0.g_w);
     P.bias = group_shift(P0.bias, P0.g_bias);
     P.out = group_shift(P0.out, P0.g_out);
+    return P;
+}
+
+// the same, the last one of reduction slices possibly shorter than the others
+__device__ __forceinline__ ConvArgs slice_view(const ConvArgs& P0) {
+    ConvArgs P = group_view(P0);
+    if (P0.last_c && (int)blockIdx.y == P0.groups - 1) {
+        P.in.C = P0.last_c;
+        P.nchunks = P0.last_chunks;
+    }
     return P;
 }
 
@@ -363,10 +374,10 @@ __device__ __forceinline__ void stage_vec_load(f32x4 (&v)[stage_loads(NCH, P2LOG
     const long plane = (long)s.Hd * s.Wd;
     // the same for every thread: scalar arithmetic, one 64-bit add per load and thread
     const long uoff = (long)PL::pe(e) * s.comp_stride + (long)(c0 + PL::ce(e)) * plane;
-    // channels past the tensor meet zero filters: any finite value will do, the tensor's first bytes are safe
+    // channels past the tensor meet zero filters and read zeros (the tensor's own first bytes may not be finite)
     // (components a real-valued tensor does not have are masked to zero by the store)
     const bool ok = sv.fast && (c0 + PL::ce(e)) < sv.c_room && PL::pe(e) < sv.p_room;
-    const TS* ptr = ok ? origin + (sv.tbase + uoff) : origin;
+    const TS* ptr = ok ? origin + (sv.tbase + uoff) : zero_ptr<TS>();
     if constexpr (sizeof(TS) == 4) {
         typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
         v[e] = *reinterpret_cast<const f32x4_a4*>(ptr);
@@ -474,7 +485,7 @@ __device__ __forceinline__ void stage_vec_store_scalar(float* lds, const f32x4 (
 //   MODE 8 : acc[i] += R_i * L_i with the 8 lanes L_i formed in registers, 8 MFMAs per K step.
 template <typename TS, int MODE, int WCO, int NTW, int CK, int P2LOG, bool VSTG>
 __global__ void __launch_bounds__(WG_THREADS, (MODE == 8 || NTW == 1) ? 2 : 1) qconv_fwd_f32_kernel(const ConvArgs P0) {
-    const ConvArgs P = group_view(P0);
+    const ConvArgs P = slice_view(P0);
     constexpr int NACC = (MODE == 16) ? 4 : 8;
     constexpr int WC = (MODE == 16) ? 4 : 8;  // packed filter values per lane and K step
     extern __shared__ float lds[];
@@ -633,12 +644,21 @@ struct PackArgs {
     int row_tiles, nchunks;
     int groups;       // grid rows: the groups packed by this one launch (1 otherwise)
     long g_w, g_out;  // bytes from one group's filter / packed image to the next group's
+    int last_red, last_chunks;  // as ConvArgs::last_c, last_chunks
 };
 
 __device__ __forceinline__ PackArgs group_view(const PackArgs& P0) {
     PackArgs P = P0;
     P.w = group_shift(P0.w, P0.g_w);
     P.out = group_shift(P0.out, P0.g_out);
+    return P;
+}
+__device__ __forceinline__ PackArgs slice_view(const PackArgs& P0) {
+    PackArgs P = group_view(P0);
+    if (P0.last_red && (int)blockIdx.y == P0.groups - 1) {
+        P.red = P0.last_red;
+        P.nchunks = P0.last_chunks;
+    }
     return P;
 }
 
@@ -694,7 +714,7 @@ __device__ __forceinline__ void pack_filters_f32_body(const PackArgs& P, long fi
 
 template <typename TS, int MODE, int MAP>
 __global__ void __launch_bounds__(WG_THREADS) pack_filters_f32_kernel(const PackArgs P0) {
-    const PackArgs P = group_view(P0);
+    const PackArgs P = slice_view(P0);
     pack_filters_f32_body<TS, MODE, MAP>(P, (long)blockIdx.x * blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
 }
 
