@@ -273,6 +273,7 @@ struct TileSrc {
     int pw;            // pointwise trick: window row r holds channels (chunk*pw + r)*16.. of the single image row (0 = off)
     int tall;          // flat tiling: the images are rows [n*tall, n*tall + Hd) of one tall image, zero rows between them (0 = off)
     int nhwc;          // channels-last memory, t[4][N][Hd][Wd][Cs] (chunk staging of the fp16 LDS kernels only; 0 = planes)
+    int last;          // reduction slices of fp32 tensors: channels of the last one (0: as many as the others have)
 };
 
 // Window staging, split so that global loads can be in flight while the previous chunk is being

@@ -74,7 +74,6 @@ struct ConvArgs {
     int nhwc;           // the output is channels-last, out[4][N][Hout][Wout][CoutS] (fp16 chunk-staging kernel only)
     int groups;         // grid rows: the groups of a grouped convolution run by this one launch (1 otherwise)
     long g_in, g_w, g_bias, g_out;  // bytes from one group's input / packed filters / bias / output to the next group's
-    int last_c, last_chunks;        // channels and chunks of the last group (reduction slices of fp32 tensors); 0: as the others'
 };
 
 struct ConvNormArgs : ConvArgs {  // of the NORM instances (the others' calls carry no bytes they do not read: 0.2 us a launch)
@@ -93,12 +92,12 @@ __device__ __forceinline__ ConvArgs group_view(const ConvArgs& P0) {
     return P;
 }
 
-// the same, the last one of reduction slices possibly shorter than the others
-__device__ __forceinline__ ConvArgs slice_view(const ConvArgs& P0) {
+// the same, the last one of reduction slices possibly shorter than the others; ck: channels of a chunk
+__device__ __forceinline__ ConvArgs slice_view(const ConvArgs& P0, int ck) {
     ConvArgs P = group_view(P0);
-    if (P0.last_c && (int)blockIdx.y == P0.groups - 1) {
-        P.in.C = P0.last_c;
-        P.nchunks = P0.last_chunks;
+    if (P0.in.last && (int)blockIdx.y == P0.groups - 1) {
+        P.in.C = P0.in.last;
+        P.nchunks = (P0.in.last + ck - 1) / ck;
     }
     return P;
 }
@@ -485,7 +484,7 @@ __device__ __forceinline__ void stage_vec_store_scalar(float* lds, const f32x4 (
 //   MODE 8 : acc[i] += R_i * L_i with the 8 lanes L_i formed in registers, 8 MFMAs per K step.
 template <typename TS, int MODE, int WCO, int NTW, int CK, int P2LOG, bool VSTG>
 __global__ void __launch_bounds__(WG_THREADS, (MODE == 8 || NTW == 1) ? 2 : 1) qconv_fwd_f32_kernel(const ConvArgs P0) {
-    const ConvArgs P = slice_view(P0);
+    const ConvArgs P = slice_view(P0, CK);
     constexpr int NACC = (MODE == 16) ? 4 : 8;
     constexpr int WC = (MODE == 16) ? 4 : 8;  // packed filter values per lane and K step
     extern __shared__ float lds[];
@@ -643,8 +642,8 @@ struct PackArgs {
     int rows, red;    // correlation: output channels (rows) and reduced channels
     int row_tiles, nchunks;
     int groups;       // grid rows: the groups packed by this one launch (1 otherwise)
+    int last;         // as TileSrc::last, | log2 of the packed chunks in one of the kernel's << 28
     long g_w, g_out;  // bytes from one group's filter / packed image to the next group's
-    int last_red, last_chunks;  // as ConvArgs::last_c, last_chunks
 };
 
 __device__ __forceinline__ PackArgs group_view(const PackArgs& P0) {
@@ -653,11 +652,12 @@ __device__ __forceinline__ PackArgs group_view(const PackArgs& P0) {
     P.out = group_shift(P0.out, P0.g_out);
     return P;
 }
-__device__ __forceinline__ PackArgs slice_view(const PackArgs& P0) {
+__device__ __forceinline__ PackArgs slice_view(const PackArgs& P0, int ck) {
     PackArgs P = group_view(P0);
-    if (P0.last_red && (int)blockIdx.y == P0.groups - 1) {
-        P.red = P0.last_red;
-        P.nchunks = P0.last_chunks;
+    if (P0.last && (int)blockIdx.y == P0.groups - 1) {
+        const int several = P0.last >> 28;
+        P.red = P0.last & 0xFFFFFFF;
+        P.nchunks = (((P.red + ck - 1) / ck + (1 << several) - 1) >> several) << several;
     }
     return P;
 }
@@ -714,7 +714,7 @@ __device__ __forceinline__ void pack_filters_f32_body(const PackArgs& P, long fi
 
 template <typename TS, int MODE, int MAP>
 __global__ void __launch_bounds__(WG_THREADS) pack_filters_f32_kernel(const PackArgs P0) {
-    const PackArgs P = slice_view(P0);
+    const PackArgs P = slice_view(P0, F32_CK);
     pack_filters_f32_body<TS, MODE, MAP>(P, (long)blockIdx.x * blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
 }
 

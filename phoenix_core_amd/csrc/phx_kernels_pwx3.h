@@ -33,7 +33,7 @@ typedef u32x2 u32x2_a4 __attribute__((aligned(4)));
 
 template <int S>
 __global__ void __launch_bounds__(WG_THREADS, 2) qconv_pw_x3_kernel(const ConvArgs P0) {
-    const ConvArgs P = slice_view(P0);
+    const ConvArgs P = slice_view(P0, PWX3_STEP);
     extern __shared__ float ldspwx3[];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -259,7 +259,7 @@ __device__ __forceinline__ void pack_filters_pwx3_body(const PackArgs& P, int S,
 
 template <int MAP>
 __global__ void __launch_bounds__(WG_THREADS) pack_filters_pwx3_kernel(const PackArgs A0, int S) {
-    const PackArgs A = slice_view(A0);
+    const PackArgs A = slice_view(A0, PWX3_STEP);
     pack_filters_pwx3_body<MAP>(A, S, (long)blockIdx.x * blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
 }
 

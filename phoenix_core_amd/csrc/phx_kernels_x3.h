@@ -117,7 +117,7 @@ __device__ __forceinline__ void conv_again(const ConvArgs& P, const f32x4* copy,
 
 template <int S, int NPT>
 __global__ void __launch_bounds__(WG_THREADS, 1) qconv_fwd_x3_kernel(const ConvArgs P0) {
-    const ConvArgs P = slice_view(P0);
+    const ConvArgs P = slice_view(P0, X3_CK);
     constexpr int TG = X3_GROUP;
     constexpr int PX = NPT * 32, STEP = x3_step(S);
     extern __shared__ u32x4 ldsx3[];  // [2][X3_BUF]; the epilogue's exchange
@@ -556,7 +556,7 @@ __device__ __forceinline__ void pack_filters_x3_body(const PackLanesArgs& A, int
 template <int MAP>
 __global__ void __launch_bounds__(WG_THREADS) pack_filters_x3_kernel(const PackLanesArgs A0, int S) {
     PackLanesArgs A = A0;
-    A.base = slice_view(A0.base);
+    A.base = slice_view(A0.base, X3_CK);
     pack_filters_x3_body<MAP>(A, S, (long)blockIdx.x * blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
 }
 
