@@ -255,6 +255,9 @@ int phx_qdense_bwd_data(const phx_qdense_desc* desc, phx_stream_t stream, const 
                         void* dx, void* workspace, size_t workspace_bytes);
 int phx_qdense_bwd_weights(const phx_qdense_desc* desc, phx_stream_t stream, const void* x, const void* grad,
                            void* dw, void* workspace, size_t workspace_bytes);
+/* phx_qdense_bwd_weights and phx_qdense_bwd_data behind each other, with a workspace for either; small problems in one launch. */
+int phx_qdense_bwd(const phx_qdense_desc* desc, phx_stream_t stream, const void* x, const void* w, const void* grad,
+                   void* dw, void* dx, void* workspace, size_t workspace_bytes);
 
 /* Device plumbing for hosts that do not link the HIP runtime themselves.  Replaces what
  * device::CUDA does for the reference (src/backend/cudnn/device.hpp:13-229: malloc/free on the

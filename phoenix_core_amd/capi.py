@@ -25,7 +25,7 @@ PHX_PASS_FWD, PHX_PASS_BWD_DATA, PHX_PASS_BWD_WEIGHTS = 0, 1, 2
 EXPORTS = (
     "phx_status_string", "phx_qconv2d_output_hw", "phx_qconv2d_workspace_bytes", "phx_qdense_workspace_bytes",
     "phx_qconv2d_fwd", "phx_qconv2d_bwd_data", "phx_qconv2d_bwd_weights",
-    "phx_qdense_fwd", "phx_qdense_bwd_data", "phx_qdense_bwd_weights",
+    "phx_qdense_fwd", "phx_qdense_bwd_data", "phx_qdense_bwd_weights", "phx_qdense_bwd",
     "phx_device_count", "phx_device_malloc", "phx_device_free", "phx_memcpy_h2d", "phx_memcpy_d2h",
     "phx_memset_zero", "phx_stream_create", "phx_stream_destroy", "phx_stream_synchronize",
     "phx_last_kernel_name", "phx_profile_enable", "phx_profile_collect", "phx_algebra_map",
@@ -105,6 +105,7 @@ def lib():
         L.phx_qdense_fwd.argtypes = [dd, vp, vp, vp, vp, vp, vp, sz]
         L.phx_qdense_bwd_data.argtypes = [dd, vp, vp, vp, vp, vp, sz]
         L.phx_qdense_bwd_weights.argtypes = [dd, vp, vp, vp, vp, vp, sz]
+        L.phx_qdense_bwd.argtypes = [dd, vp, vp, vp, vp, vp, vp, vp, sz]
         bd = ctypes.POINTER(BnDesc)
         L.phx_bn_workspace_bytes.restype = sz
         L.phx_bn_workspace_bytes.argtypes = [bd]

@@ -130,6 +130,7 @@ struct DenseSmallArgs {
     int n, ni, no;
 };
 int launch_dense_small(bool half_storage, int pass, const DenseSmallArgs& a, hipStream_t st);
+int launch_dense_small_bwd(bool half_storage, const DenseSmallArgs& weights, const DenseSmallArgs& data, hipStream_t st);  // both gradients
 
 // Dense as matrix products (phx_launch_dense_gemm.hip): rows m of a, columns n of b, reduction over k; element
 // (component, m, k) of a at component * acs + m * ars + k * aks, of b likewise, output (q, m, n) at q * ocs + m * ors + n * ons.

@@ -39,7 +39,7 @@ namespace {
 #define PHX_HOST_FUNCTIONS(X)                                                                                                   \
     X(phx_qconv2d_workspace_bytes) X(phx_qdense_workspace_bytes) X(phx_qconv2d_fwd) X(phx_qconv2d_fwd_prepacked)               \
     X(phx_qconv2d_fwd_norm) X(phx_qconv2d_bwd_weights) X(phx_qconv2d_bwd_data) X(phx_qconv2d_bwd_data_prepacked)               \
-    X(phx_qconv2d_bwd_data_add) X(phx_qconv2d_pack_filters) X(phx_qdense_fwd) X(phx_qdense_bwd_data) X(phx_qdense_bwd_weights) \
+    X(phx_qconv2d_bwd_data_add) X(phx_qconv2d_pack_filters) X(phx_qdense_fwd) X(phx_qdense_bwd) X(phx_qdense_bwd_weights) \
     X(phx_bn_workspace_bytes) X(phx_bn_fwd_train) X(phx_bn_bwd)
 struct Library {
 #define PHX_FIELD(f) decltype(&::f) f = nullptr;
@@ -411,19 +411,17 @@ PyObject* both_gradients(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const size_t weights_bytes = workspace_bytes(d, PHX_PASS_BWD_WEIGHTS), data_bytes = want ? workspace_bytes(d, PHX_PASS_BWD_DATA) : 0;
     const at::Tensor ws = scratch(device, stream, std::max(weights_bytes, data_bytes));
     void *px = address(x), *pw = address(w), *pg = address(g), *pdw = dw.data_ptr(), *pdx = want ? dx.data_ptr() : nullptr, *pws = ws.data_ptr();
-    bool weights = true;  // (which of the two a status is of)
     int status;
     if constexpr (DENSE) {
         const phx_qdense_desc c = *d->den();
         status = unlocked([&] {
-            const int s = L.phx_qdense_bwd_weights(&c, st, px, pg, pdw, pws, weights_bytes);
-            if (s != PHX_OK || !pdx) return s;
-            weights = false;
-            return L.phx_qdense_bwd_data(&c, st, pg, pw, pdx, pws, data_bytes);
+            return pdx ? L.phx_qdense_bwd(&c, st, px, pw, pg, pdw, pdx, pws, std::max(weights_bytes, data_bytes))
+                       : L.phx_qdense_bwd_weights(&c, st, px, pg, pdw, pws, weights_bytes);
         });
-        if (!ok(status, weights ? "phx_qdense_bwd_weights" : "phx_qdense_bwd_data")) return nullptr;
+        if (!ok(status, pdx ? "phx_qdense_bwd" : "phx_qdense_bwd_weights")) return nullptr;
     } else {
         const phx_qconv_desc c = *d->conv();
+        bool weights = true;  // (which of the two a status is of)
         status = unlocked([&] {
             const int s = L.phx_qconv2d_bwd_weights(&c, st, px, pg, pdw, pws, weights_bytes);
             if (s != PHX_OK || !pdx) return s;
