@@ -42,8 +42,24 @@ struct RegArgs {
 struct RegNormArgs : RegArgs {
     NormArgs norm;
 };
-template <bool NORM>
-using RegArgsOf = std::conditional_t<NORM, RegNormArgs, RegArgs>;
+// The phases of a strided input gradient in one launch: the results whose row is oh and whose column ow modulo the stride, a unit-
+// stride correlation of the gradient with the filter's taps that reach them.  Each phase has tiles of its own and writes its
+// results where they belong; one that no tap reaches writes zeros (and the addend).
+constexpr int REG_PHASES_MAX = 4;
+struct RegPhase {
+    int first;              // its first tile
+    int Kh, kw, dh, pt, pl; // filter rows; taps of a row (at most the kernel's, those behind them are zero); as in RegArgs
+    int Hout, Wout;         // its results
+    int oh, ow;             // ... and where they lie
+    int flat, rpr, tpi, items, zitems;
+    int image;              // its packed filters, 16-byte vectors behind the first one's
+};
+struct RegPhaseArgs : RegArgs {
+    RegPhase phase[REG_PHASES_MAX];
+    int phases, step_h, step_w;  // and the strides; Hout, Wout: the whole result
+};
+template <bool NORM, bool PHASE = false>
+using RegArgsOf = std::conditional_t<PHASE, RegPhaseArgs, std::conditional_t<NORM, RegNormArgs, RegArgs>>;
 
 // Pixels that a pair reads under a filter row, as a power of two.  (Memory bounds a CU: its L1 hands out some 30 bytes a clock
 // of these loads.  Runs of four pixels with 16-byte loads measured the same rate per pixel, 0.84 against 0.76 us for the 3x3
@@ -100,10 +116,17 @@ __device__ __forceinline__ RegWords<W> reg_shift(const RegWords<W>& a, int n) {
     return r;
 }
 
-// KW taps a filter row, dilation D and stride S along the row; CL: channels-last tensors
-template <int KW, int D, int S, bool CL, bool NORM>
-__global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const RegArgsOf<NORM> P) {
-    static_assert(!(CL && NORM), "channels-last passes take no norm");
+// KW taps a filter row, dilation D and stride S along the row; CL: channels-last tensors; PHASE: see RegPhase
+template <int KW, int D, int S, bool CL, bool NORM, bool PHASE = false>
+__global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const RegArgsOf<NORM, PHASE> P0) {
+    static_assert(!(CL && NORM) && !(PHASE && NORM), "channels-last passes and input gradients take no norm");
+    [[maybe_unused]] RegArgs one;  // (PHASE: this tile's phase as a correlation of its own)
+    [[maybe_unused]] RegPhase phase;
+    const auto& P = [&]() -> const auto& {
+        if constexpr (PHASE) return one;
+        else return P0;
+    }();
+    if constexpr (PHASE) one = P0;
     constexpr int PX = REG_PX, SPAN = reg_span(KW, D, S);
     constexpr int W = CL ? 4 : SPAN / 2;                  // words of a load
     constexpr int NL = CL ? (KW - 1) * D + (PX - 1) * S + 1 : 8;     // loads of a component's part of an item
@@ -120,14 +143,30 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
     const int rest = wg / P.co_tiles;
     const int groups = (P.tiles + subs - 1) / subs;
     const int z = rest / groups;
-    const int tile = (rest - z * groups) * subs + (wave >> P.kslog);
+    int tile = (rest - z * groups) * subs + (wave >> P.kslog);
     const bool live = tile < P.tiles;
+    if constexpr (PHASE) {
+        int which = 0;
+#pragma unroll
+        for (int i = 1; i < REG_PHASES_MAX; ++i)
+            if (live && i < P0.phases && tile >= P0.phase[i].first) which = i;
+        phase = P0.phase[which];
+        tile -= phase.first;
+        one.Kh = phase.Kh; one.dh = phase.dh; one.pt = phase.pt; one.pl = phase.pl;
+        one.Hout = phase.Hout; one.Wout = phase.Wout;
+        one.flat = phase.flat; one.rpr = phase.rpr; one.tpi = phase.tpi; one.items = phase.items; one.zitems = phase.zitems;
+        one.wpk += phase.image;
+    }
     const int img = live ? tile / P.tpi : 0;
     const int first_pair = (tile - img * P.tpi) * REG_TM;
     const int pair = first_pair + r;
 
     // the pair's pixels: (ho[e], wo[e]), q0 the first one's place in the plane
-    const int HWin = P.Hin * P.Win, HWout = P.Hout * P.Wout;
+    const int HWin = P.Hin * P.Win, HWout = P0.Hout * P0.Wout;  // (PHASE: of the whole result)
+    auto pixel = [&](int h, int w) __attribute__((always_inline)) {  // a result's place in its plane
+        if constexpr (PHASE) return (h * P0.step_h + phase.oh) * P0.Wout + w * P0.step_w + phase.ow;
+        else return h * P0.Wout + w;
+    };
     int ho[PX], wo[PX];
     bool ok[PX];
     const int per_row = P.flat ? P.Wout : P.rpr * PX;  // pixels of a row as the pairs count them
@@ -147,7 +186,7 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
 #pragma unroll
         for (int kw = 0; kw < KW; ++kw) {
             const int iw = wo[e] * S - P.pl + kw * D;
-            if (ok[e] && iw >= 0 && iw < P.Win) cols[e] |= 1u << kw;
+            if (ok[e] && iw >= 0 && iw < P.Win && (!PHASE || kw < phase.kw)) cols[e] |= 1u << kw;
         }
     }
 
@@ -325,7 +364,7 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
 #pragma unroll
             for (int e = 0; e < PX; ++e) {
                 if (!ok[e]) continue;
-                const long at = q * P.out_cs + ((long)img * HWout + q0 + e) * P.Cout + co;
+                const long at = q * P.out_cs + ((long)img * HWout + (PHASE ? pixel(ho[e], wo[e]) : q0 + e)) * P.Cout + co;
                 _Float16 h[NI];
 #pragma unroll
                 for (int i = 0; i < NI; ++i) {
@@ -373,7 +412,7 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
             };
             const int r0 = first_pair + 4 * kg + i0;  // the first of NI pairs
             // (rows of an odd number of pixels end in half a pair, unless the pairs go through the plane)
-            const bool whole = P.flat || P.Wout % PX == 0;  // (uniform)
+            const bool whole = !PHASE && (P.flat || P.Wout % PX == 0);  // (uniform)
             if (whole && PX * (r0 + NI) <= HWout) {
                 const long at = plane + PX * r0;
                 if (P.partial) {
@@ -409,11 +448,11 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
                 for (int i = 0; i < PX * NI; ++i)
                     if (PX * r0 + i < HWout) store(PX * r0 + i, v[i]);
             } else {
-                int row = r0 / P.rpr, col = PX * (r0 - row * P.rpr);
+                int row = PX * r0 / per_row, col = PX * r0 - row * per_row;
 #pragma unroll
                 for (int i = 0; i < PX * NI; ++i) {
-                    if (row < P.Hout && col < P.Wout) store(row * P.Wout + col, v[i]);
-                    if (++col == PX * P.rpr) { col = 0; ++row; }
+                    if (row < P.Hout && col < P.Wout) store(pixel(row, col), v[i]);
+                    if (++col == per_row) { col = 0; ++row; }
                 }
             }
         }
@@ -468,7 +507,7 @@ __device__ __forceinline__ void pack_filters_reg_body(const PackArgs& P, long fi
         const int want = chunk * REG_CK + (lane >> 4) * 8, base = min(want, P.red - 8);
         if (MAP == MAP_DGRAD) {
             kh = P.khm - kh * P.khs;
-            kw = P.kwm - kw * P.kws;
+            kw = P.kwm - kw * P.kws;  // (negative: a tap that the phase does not have)
         }
         const float sgn = (MAP == MAP_DGRAD && c > 0) ? -1.f : 1.f;
         const long at = c * P.wcs + kh * P.skh + kw * P.skw;
@@ -477,7 +516,7 @@ __device__ __forceinline__ void pack_filters_reg_body(const PackArgs& P, long fi
         for (int i = 0; i < 8; ++i) {
             const int red = base + i;
             float v = 0.f;
-            if (row < P.rows && red >= want) v = sgn * (float)w[at + (MAP == MAP_DGRAD ? red * P.so + row * P.si : row * P.so + red * P.si)];
+            if (row < P.rows && red >= want && kw >= 0) v = sgn * (float)w[at + (MAP == MAP_DGRAD ? red * P.so + row * P.si : row * P.so + red * P.si)];
             vec[i] = (_Float16)v;
         }
         outv[idx] = vec;

@@ -78,7 +78,9 @@ int launch_pack_filters_pwx(int map, int WCO, int nsteps, const PackArgs& a, hip
 // fp16 convolutions of few output tiles, operands straight in registers (phx_kernels_reg16.h); cl = channels-last tensors;
 // norm.gamma null: none; waves of a workgroup
 struct RegArgs;
+struct RegPhaseArgs;
 int launch_reg_f16(int kw, int dw, int sw, bool cl, const RegArgs& a, const NormArgs& norm, int waves, int blocks, hipStream_t st);  // < 0: no such instance
+int launch_reg_phases(int kw, bool cl, const RegPhaseArgs& a, int waves, int blocks, hipStream_t st);  // kw: 1 to 3 taps a filter row at most
 bool reg_row_shape(int kw, int dw, int sw);  // whether there are instances for filter rows of this shape
 int launch_pack_filters_reg(int map, const PackArgs& a, int blocks, hipStream_t st);
 

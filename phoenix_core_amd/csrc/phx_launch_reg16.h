@@ -6,9 +6,9 @@
 
 namespace phx {
 
-template <int KW, int D, int S, bool CL, bool NORM>
-static int launch_reg_one(const RegArgsOf<NORM>& a, int waves, int blocks, hipStream_t st) {
-    constexpr auto kernel = qconv_reg_f16_kernel<KW, D, S, CL, NORM>;
+template <int KW, int D, int S, bool CL, bool NORM, bool PHASE = false>
+static int launch_reg_one(const RegArgsOf<NORM, PHASE>& a, int waves, int blocks, hipStream_t st) {
+    constexpr auto kernel = qconv_reg_f16_kernel<KW, D, S, CL, NORM, PHASE>;
     if (!BigLds<kernel>::registered || waves > reg_waves(KW)) return -1;  // dynamic LDS opt-in at set-up, see BigLds
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * waves), a.kslog ? waves * REG_WAVE_LDS : 0, st, a);
     return 0;

@@ -47,6 +47,60 @@ def _close(got, want, sums, terms, roundings=1):
     assert not bad.any(), (int(bad.sum()), float(np.abs(got - want).max()))
 
 
+# n, ci, co, h, w, kh, kw, stride, dilation, padding: input gradients by phases
+STRIDED = [
+    (2, 17, 40, 9, 8, 3, 3, 2, 1, "SAME"),           # 2 and 1 taps; planes of the phases as wide as the gradient's
+    (1, 33, 9, 11, 13, 3, 3, 2, 1, "SAME"),          # ... and one narrower; nine reduced channels
+    (3, 16, 64, 7, 6, 1, 1, 2, 1, "SAME"),           # phases that no tap reaches
+    (2, 20, 33, 10, 12, 5, 5, 2, 1, "SAME"),         # 3 and 2 taps
+    (1, 24, 32, 12, 12, 3, 3, 2, 2, "SAME"),         # dilated by the stride: one phase has all taps
+    (1, 16, 32, 13, 10, 2, 3, (3, 1), (2, 1), (1, 0, 2, 1)),
+    (2, 16, 24, 8, 9, 4, 2, (1, 2), 1, (3, 1, 0, 2)),
+    (1, 40, 16, 6, 17, 3, 4, (1, 4), 1, "VALID"),    # columns that no window covers
+    (1, 18, 72, 16, 15, 6, 6, 2, 1, (2, 2, 2, 3)),
+]
+
+
+@pytest.mark.parametrize("layout", ["NCHW", "NHWC"])
+@pytest.mark.parametrize("split", ["1,0,1", "1,2,1", "1,3,1", "1,1,2", "1,3,3"])
+@pytest.mark.parametrize("case", STRIDED, ids=lambda c: "n%d_%d-%d_%dx%d_%dx%d_s%s_d%s_%s" % c)
+def test_strided_input_gradients(case, split, layout, tune_env):
+    n, ci, co, h, w, kh, kw, stride, dilation, padding = case
+    r = np.random.default_rng(ci * h + w)
+    g = oracle.make_geom(n, ci, co, h, w, kh, kw, stride, dilation, padding)
+    x = r.standard_normal((4 * n, ci, h, w)).astype(np.float16)
+    wt = (r.standard_normal((4, co, ci, kh, kw)) * (4 * co * kh * kw) ** -0.5).astype(np.float16)
+    gr = r.standard_normal((4 * n, co, g.ho, g.wo)).astype(np.float16)
+    _, want = oracle.conv2d_bwd(g, x.astype(np.float64), wt.astype(np.float64), gr.astype(np.float64), "hamilton")
+    _, sums = oracle.conv2d_bwd(g, x.astype(np.float64), np.stack([np.abs(wt.astype(np.float64)).sum(0)] + [0 * wt[0].astype(np.float64)] * 3),
+                                np.tile(np.abs(gr.astype(np.float64)).reshape((4, n) + gr.shape[1:]).sum(0), (4, 1, 1, 1)), "hamilton")
+    last = (lambda t: t.permute(0, 2, 3, 1).contiguous()) if layout == "NHWC" else (lambda t: t)
+    back = (lambda t: t.permute(0, 3, 1, 2)) if layout == "NHWC" else (lambda t: t)
+    gd, wd = last(torch.from_numpy(gr)).cuda(), torch.from_numpy(wt).cuda()
+    shape = tuple(last(torch.from_numpy(x)).shape)
+    desc = ops.Conv2DDescriptor(shape, wd.shape, stride, dilation, padding, dtype=torch.float16, context=phx.Context(POLICIES["f16"]), data_format=layout)
+    tune_env(PHX_TUNE_REG=split)
+    dx = ops.conv2d_bwd_data(wd, gd, desc)
+    assert "phases_qconv_dgrad" in capi.last_kernel_name() and "mfmareg" in capi.last_kernel_name(), capi.last_kernel_name()
+    _close(back(dx).cpu().numpy(), want, np.abs(sums), 4 * co * kh * kw)
+    packed = ops.conv2d_pack_filters(wd, desc)
+    assert torch.equal(ops.conv2d_bwd_data(torch.zeros_like(wd), gd, desc, packed=packed), dx)
+    addend = torch.from_numpy(x).cuda()
+    assert torch.equal(ops.conv2d_bwd_data(wd, gd, desc, addend=last(addend)), dx + last(addend))
+
+
+def test_strided_input_gradients_keep_what_is_not_finite_in_its_windows(tune_env):
+    """A filter value that is not finite meets no gradient of a phase without its tap."""
+    tune_env(PHX_TUNE_REG="1,1,1")
+    wt, gr = torch.ones(4, 32, 16, 3, 3, device="cuda").half(), torch.ones(8, 32, 5, 5, device="cuda").half()
+    wt[0, 3, 2, 1, 1] = float("inf")  # (reaches rows and columns of one parity)
+    desc = ops.Conv2DDescriptor((8, 16, 10, 10), wt.shape, 2, 1, (1, 1, 1, 1), dtype=torch.float16, context=phx.Context(POLICIES["f16"]))
+    dx = ops.conv2d_bwd_data(wt, gr, desc)
+    assert "mfmareg" in capi.last_kernel_name()
+    bad = ~torch.isfinite(dx)
+    assert bool(bad[:, 2, 0::2, 0::2].all()) and int(bad.sum()) == 8 * 25
+
+
 @pytest.mark.parametrize("layout", ["NCHW", "NHWC"])
 @pytest.mark.parametrize("split", ["1,0,1", "1,1,1", "1,2,1", "1,3,1", "1,2,2", "1,3,3"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "n%d_%d-%d_%dx%d_%dx%d_s%s_d%s_%s" % c)
