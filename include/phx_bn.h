@@ -6,7 +6,8 @@
  * components stacked on the batch axis, src/backend/tensor.hpp:489-581); every channel is normalised
  * over rows x H x W, i.e. the four components of a quaternion channel share one mean and variance,
  * exactly what torch.nn.BatchNorm2d computes on such a tensor.  HBM-bound: two reads and one write of
- * the activations forward, four reads and one write backward, spread over many workgroups per channel
+ * the activations forward, four reads and one write backward (large tensors, whose workgroups keep what they have
+ * summed: one and one, two and one), spread over many workgroups per channel
  * (a library kernel with one workgroup per channel leaves a 16-channel layer on 16 of 256 CUs).
  *
  * Same conventions as phx_qconv.h: device pointers, work enqueued on the given stream, non-zero

@@ -7,6 +7,7 @@
 
 #include "../../include/phx_bn.h"
 #include "phx_device.h"
+#include "phx_launch.h"
 
 namespace phx {
 
@@ -30,6 +31,9 @@ struct BnArgs {
     int nchunk;             // 16-byte chunks per (row, channel) plane, the last one possibly partial
     float eps, momentum;
     int relu;
+    int total, per_split;   // bn_held_kernel: chunks of a channel and those of a split,
+    int rows_step, chunks_step;  // a workgroup's threads' chunks as rows and what is left,
+    int waits;              // how often a workgroup looks for its channel's other partial sums
 };
 
 template <typename TS>
@@ -88,6 +92,7 @@ __device__ __forceinline__ void store_chunk(TS* p, int n, const float (&v)[Vec<T
 }
 
 // Sum of two values over the workgroup (256 threads), result in every thread.
+template <int T = 256>
 __device__ __forceinline__ void wg_sum2(float& a, float& b, float (*red)[2]) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -100,6 +105,8 @@ __device__ __forceinline__ void wg_sum2(float& a, float& b, float (*red)[2]) {
     __syncthreads();
     a = red[0][0] + red[1][0] + red[2][0] + red[3][0];
     b = red[0][1] + red[1][1] + red[2][1] + red[3][1];
+#pragma unroll
+    for (int w = 4; w < T / 64; ++w) { a += red[w][0]; b += red[w][1]; }
 }
 
 // The channel's totals from its S partial pairs (fixed order inside the reduction tree).
@@ -248,6 +255,215 @@ __global__ void __launch_bounds__(256) bn_apply_kernel(const BnArgs P) {
     }
 }
 
+// ---- both passes in one: a workgroup holds its part of a channel in registers ----
+// The two kernels above read x (and dy) twice, with the whole tensor between the two reads: 2.0 GB for the two 128-channel norms
+// of a bottleneck block at 128 images of 28x28 where 1.3 are needed.  Here a workgroup keeps the chunks that it has summed (and
+// the forward pass's residual, requested with them), publishes its two sums, waits for those of its channel's other
+// workgroups, which are its neighbours in the launch, and applies the result to what it holds.  206 MB of a forward pass take
+// 44 us (4.7 TB/s, a copy's 5.05), backward 309 MB 72 us; what is missing is the wait, a store and a load behind the tensor's own
+// traffic, which the other workgroups of the CU fill in part.  (Neighbouring channels on one XCD: 49 and 102 us; the residual
+// of the backward pass requested three chunks ahead: 139 us for 128.)
+//
+// A pair of sums is one 64-bit word, written and read by relaxed atomics of the device's scope, and differs from BN_NONE, which
+// a launch in front sets the words to: nothing else passes between workgroups, so no cache is written back or dropped.
+// No workgroup depends on another's progress: one that has looked P.waits times (some milliseconds) without seeing all words
+// forms them itself from memory, in the order of their owners.  What is written is therefore never what is read (one_pass).
+constexpr unsigned long long BN_NONE = ~0ull;
+constexpr int BN_HELD_ONE = 16, BN_HELD_TWO = 8;  // chunks a thread holds of a single tensor, of each of two
+
+__global__ void __launch_bounds__(256) bn_none_kernel(unsigned long long* words, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) words[i] = BN_NONE;
+}
+
+template <typename TS>
+__device__ __forceinline__ void unpack_chunk(const u32x4 raw, float (&v)[Vec<TS>::N]) {
+    if constexpr (sizeof(TS) == 2) {
+        const f16x8 h = __builtin_bit_cast(f16x8, raw);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = (float)h[i];
+    } else {
+        const f32x4 f = __builtin_bit_cast(f32x4, raw);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = f[i];
+    }
+}
+template <typename TS>
+__device__ __forceinline__ u32x4 pack_chunk(const float (&v)[Vec<TS>::N]) {
+    if constexpr (sizeof(TS) == 2) {
+        f16x8 h;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) h[i] = (_Float16)v[i];
+        return __builtin_bit_cast(u32x4, h);
+    } else {
+        f32x4 f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f[i] = v[i];
+        return __builtin_bit_cast(u32x4, f);
+    }
+}
+template <typename TS>
+__device__ __forceinline__ u32x4 load_raw(const TS* p) { return load16_a2(reinterpret_cast<const _Float16*>(p)); }
+template <typename TS>
+__device__ __forceinline__ void store_raw(TS* p, u32x4 raw) {
+    *reinterpret_cast<__attribute__((address_space(1))) u32x4_a2*>((__attribute__((address_space(1))) _Float16*)p) = raw;
+}
+
+// A thread's walk over the chunks first, first + T, ... of channel c: the element offset of each, and how many of its
+// elements belong to the chunk before (a plane's last chunk ends where the plane ends; hw >= a chunk here).
+struct ChunkWalk {
+    int row, chunk;
+    __device__ __forceinline__ ChunkWalk(const BnArgs& P, int first) : row(first / P.nchunk), chunk(first - row * P.nchunk) {}
+    template <int V>
+    __device__ __forceinline__ unsigned int offset(const BnArgs& P, int c, int& seen) const {
+        seen = max(chunk * V + V - P.hw, 0);
+        return ((unsigned int)row * P.C + c) * (unsigned int)P.hw + (unsigned int)(chunk * V - seen);
+    }
+    __device__ __forceinline__ void next(const BnArgs& P) {
+        chunk += P.chunks_step;
+        row += P.rows_step;
+        if (chunk >= P.nchunk) { chunk -= P.nchunk; ++row; }
+    }
+};
+
+template <typename TS, int MODE, bool RES, int HELD, int T>
+__global__ void __launch_bounds__(T, 4) bn_held_kernel(const BnArgs P) {
+    constexpr int V = Vec<TS>::N;
+    __shared__ float red[T / 64][2];
+    const int tid = threadIdx.x;
+    const int c = blockIdx.x / P.S, s = blockIdx.x - c * P.S;
+    const TS* x = static_cast<const TS*>(P.x);
+    const TS* dy = static_cast<const TS*>(P.dy);
+    const TS* res = static_cast<const TS*>(P.res);
+    const float g = P.gamma[c], be = P.beta[c];
+    float mean = 0.f, invstd = 0.f;
+    if constexpr (MODE == 1) { mean = P.save_mean[c]; invstd = P.save_invstd[c]; }
+    const float shift = MODE == 0 ? (float)x[(long)c * P.hw] : 0.f;
+
+    u32x4 hx[HELD], hd[HELD];  // hd: dy, then the gradient behind the ReLU (MODE 1); the residual (forward pass)
+    // One chunk's part of the sums.  MODE 1 leaves the gradient behind the ReLU in `d`.
+    const auto add = [&](u32x4 xc, u32x4& d, unsigned int off, int seen, float& a0, float& a1) {
+        float xv[V], dv[V], rv[V];
+        unpack_chunk<TS>(xc, xv);
+        if constexpr (MODE == 1) unpack_chunk<TS>(d, dv);
+        if constexpr (MODE == 1 && RES) unpack_chunk<TS>(load_raw(res + off), rv);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            if constexpr (MODE == 0) {
+                const float e = i < seen ? 0.f : xv[i] - shift;
+                a0 += e;
+                a1 += e * e;
+            } else {
+                const float xh = (xv[i] - mean) * invstd;
+                dv[i] = (P.relu && g * xh + be + (RES ? rv[i] : 0.f) <= 0.f) ? 0.f : dv[i];
+                const float e = i < seen ? 0.f : dv[i];
+                a0 += e;
+                a1 += e * xh;
+            }
+        }
+        if constexpr (MODE == 1) d = pack_chunk<TS>(dv);  // (values of the tensor's type: exact)
+    };
+
+    const int mine = min(P.per_split, P.total - s * P.per_split);  // chunks of this workgroup
+    const ChunkWalk start(P, s * P.per_split + tid);
+    ChunkWalk walk = start;
+    int seen;
+#pragma unroll
+    for (int k = 0; k < HELD; ++k, walk.next(P)) {
+        if (k * T + tid < mine) {
+            const unsigned int off = walk.offset<V>(P, c, seen);
+            hx[k] = load_raw(x + off);
+            if constexpr (MODE == 1) hd[k] = load_raw(dy + off);
+            else if constexpr (RES) hd[k] = load_raw(res + off);
+        }
+    }
+    float a0 = 0.f, a1 = 0.f;
+    walk = start;
+    asm volatile("" : "+v"(walk.row), "+v"(walk.chunk));
+#pragma unroll
+    for (int k = 0; k < HELD; ++k, walk.next(P)) {
+        if (k * T + tid < mine) {
+            const unsigned int off = walk.offset<V>(P, c, seen);
+            add(hx[k], hd[k], off, seen, a0, a1);
+            if (MODE == 1 && RES && P.dres) store_raw(static_cast<TS*>(P.dres) + off, hd[k]);
+        }
+    }
+    // the channel's totals
+    const auto word = [](float a, float b) {
+        const unsigned long long w = (unsigned long long)__float_as_uint(b) << 32 | __float_as_uint(a);
+        return w == BN_NONE ? 0x7fc000007fc00000ull : w;  // (a NaN for a NaN)
+    };
+    unsigned long long* words = reinterpret_cast<unsigned long long*>(P.partial) + (long)c * P.S;
+    wg_sum2<T>(a0, a1, red);
+    if (tid == 0) __hip_atomic_store(words + s, word(a0, a1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long w = tid < P.S ? BN_NONE : 0;
+    for (int i = 0; i < P.waits && w == BN_NONE; ++i) {
+        w = __hip_atomic_load(words + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (w == BN_NONE) __builtin_amdgcn_s_sleep(10);
+    }
+    if (__syncthreads_or(w == BN_NONE)) {
+        for (int t = 0; t < P.S; ++t) {
+            const int count = min(P.per_split, P.total - t * P.per_split);
+            ChunkWalk again(P, t * P.per_split + tid);
+            a0 = a1 = 0.f;
+            for (int i = tid; i < count; i += T, again.next(P)) {
+                const unsigned int off = again.offset<V>(P, c, seen);
+                u32x4 d{};
+                if constexpr (MODE == 1) d = load_raw(dy + off);
+                add(load_raw(x + off), d, off, seen, a0, a1);
+            }
+            wg_sum2<T>(a0, a1, red);
+            if (tid == t) w = word(a0, a1);
+        }
+    }
+    float t0 = __uint_as_float((unsigned int)w), t1 = __uint_as_float((unsigned int)(w >> 32));  // (zeros past the splits)
+    wg_sum2<T>(t0, t1, red);
+
+    // (what the sums formed of the held values -- conversions, offsets -- is formed again: kept, it would take more registers than they do)
+    walk = start;
+    asm volatile("" : "+v"(walk.row), "+v"(walk.chunk));
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) {
+        asm volatile("" : "+v"(hx[k]));
+        if constexpr (MODE == 1 || RES) asm volatile("" : "+v"(hd[k]));
+    }
+    const float m = (float)P.rows * (float)P.hw;
+    const float k0 = t0 / m, k1 = t1 / m;
+    if constexpr (MODE == 0) {
+        mean = shift + k0;
+        const float var = fmaxf(k1 - k0 * k0, 0.f);
+        invstd = 1.f / sqrtf(var + P.eps);
+        if (s == 0 && tid == 0) {
+            P.save_mean[c] = mean;
+            P.save_invstd[c] = invstd;
+            if (P.run_mean) P.run_mean[c] = (1.f - P.momentum) * P.run_mean[c] + P.momentum * mean;
+            if (P.run_var) P.run_var[c] = (1.f - P.momentum) * P.run_var[c] + P.momentum * var * (m > 1.f ? m / (m - 1.f) : 1.f);
+        }
+    } else if (s == 0 && tid == 0) {
+        P.dbeta[c] = t0;
+        P.dgamma[c] = t1;
+    }
+    const float scale = g * invstd;
+#pragma unroll
+    for (int k = 0; k < HELD; ++k, walk.next(P)) {
+        if (k * T + tid < mine) {
+            float xv[V], dv[V], ov[V];
+            unpack_chunk<TS>(hx[k], xv);
+            if constexpr (MODE == 1 || RES) unpack_chunk<TS>(hd[k], dv);
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                if constexpr (MODE == 0) {
+                    const float y = scale * (xv[i] - mean) + be + (RES ? dv[i] : 0.f);
+                    ov[i] = (P.relu && y < 0.f) ? 0.f : y;
+                } else {
+                    ov[i] = scale * (dv[i] - k0 - (xv[i] - mean) * invstd * k1);
+                }
+            }
+            store_raw(static_cast<TS*>(P.out) + walk.offset<V>(P, c, seen), pack_chunk<TS>(ov));
+        }
+    }
+}
+
 // Evaluation: y = gamma / sqrt(running_var + eps) * (x - running_mean) + beta (+ residual, ReLU), one pass.
 //
 // Bound by HBM at the large layers and by its launch at the deep ones (a 512-channel 7x7 layer of 8 images is 1.6 MB).
@@ -364,8 +580,81 @@ static int plan(const phx_bn_desc* d, BnArgs& a) {
     return PHX_OK;
 }
 
+// The plan of bn_held_kernel: its workgroup's threads, or 0 for sizes it does not take or where it is not the faster one.
+// A thread holds 16 chunks, of one tensor or eight each of two (64 of 128 registers; half as many in twice the workgroups took
+// 1.3 times as long).  Measured, us, two launches / one pass, forward, forward with residual, backward, backward with residual:
+//   fp16 [512, 128, 28, 28] 55/44 74/69 87/72 147/128     fp16 [512, 64, 28, 28] 30/23 37/35 46/36 60/50
+//   fp16 [256, 512, 7, 7]   16/14 21/18 27/19  35/25      fp32 [512, 128, 28, 28] 115/94 155/136 209/138 289/232
+//   fp16 [64, 64, 28, 28]    9/11 10/11 10/10  12/12      fp32 [64, 64, 28, 28] 11/11 11/11 12/11 17/16
+// * The backward pass gains from 8 MB on; the forward pass, whose second reading of x the 256 MB cache serves in part, from
+//   32 MB, or 16 MB where a channel's workgroups are few ([128, 256, 14, 14], 12.8 MB in fp16 and 26 in fp32: 12/12, 14/14 and
+//   16/14, 21/18).
+// * A channel of many workgroups waits longer: from 50 on they have 512 threads (fp32 [256, 64, 56, 56], backward, 98 of 256
+//   threads or 49 of 512: 157 or 137 us, two launches 209) and beyond 64 of those the two launches are as fast ([256, 16, 112, 112]
+//   in fp16 83/90), as they are for a forward pass with a residual of more than 40 that the cache holds ([256, 64, 56, 56] in
+//   fp16 68/70; 567/454 at 695 MB).
+static int plan_held(BnArgs& a, int dtype, bool backward, bool residual) {
+    const int pinned = tuning_bn_held();
+    if (pinned == 0) return 0;
+    const int V = dtype == PHX_F16 ? Vec<_Float16>::N : Vec<float>::N;
+    const long elements = (long)a.rows * a.C * a.hw, bytes = elements * (dtype == PHX_F16 ? 2 : 4), total = (long)a.rows * a.nchunk;
+    if (a.hw < V || elements >= 1L << 31) return 0;  // (offsets are 32-bit)
+    const int chunks = !backward && !residual ? BN_HELD_ONE : BN_HELD_TWO;
+    int threads = 256;
+    if ((total + 256 * chunks - 1) / (256 * chunks) > (!backward && residual ? 40 : 50)) {
+        if (!backward && residual && bytes < 160000000 && pinned < 0) return 0;
+        threads = 512;
+    }
+    const long held = (long)threads * chunks;
+    // (no fewer workgroups than the GPU holds at once, as long as each has a chunk a thread)
+    long S = std::max((total + held - 1) / held, std::min((1024L + a.C - 1) / a.C, (total + threads - 1) / threads));
+    const long per = std::min(held, ((total + S - 1) / S + 63) / 64 * 64);
+    S = (total + per - 1) / per;
+    if (S > 64) return 0;
+    if (pinned < 0 && bytes < (backward ? 8000000 : S <= 8 ? 16000000 : 32000000)) return 0;
+    a.S = (int)S;
+    a.total = (int)total;
+    a.per_split = (int)per;
+    a.rows_step = threads / a.nchunk;
+    a.chunks_step = threads % a.nchunk;
+    a.waits = tuning_bn_waits();
+    return threads;
+}
+
+static bool apart(const void* out, const void* in, size_t bytes) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+    return !out || !in || o + bytes <= i || i + bytes <= o;
+}
+
+template <typename TS, int T>
+static void launch_held(const BnArgs& a, bool backward, hipStream_t st) {
+    const int words = a.C * a.S;
+    hipLaunchKernelGGL(bn_none_kernel, dim3((words + 255) / 256), dim3(256), 0, st, reinterpret_cast<unsigned long long*>(a.partial), words);
+    const dim3 grid(words);
+    if (!backward && !a.res) hipLaunchKernelGGL((bn_held_kernel<TS, 0, false, BN_HELD_ONE, T>), grid, dim3(T), 0, st, a);
+    else if (!backward) hipLaunchKernelGGL((bn_held_kernel<TS, 0, true, BN_HELD_TWO, T>), grid, dim3(T), 0, st, a);
+    else if (!a.res) hipLaunchKernelGGL((bn_held_kernel<TS, 1, false, BN_HELD_TWO, T>), grid, dim3(T), 0, st, a);
+    else hipLaunchKernelGGL((bn_held_kernel<TS, 1, true, BN_HELD_TWO, T>), grid, dim3(T), 0, st, a);
+}
+
+// One pass where its plan takes the call, the workspace holds its words and nothing that it writes is read.
 template <typename TS>
-static void launch_all(const BnArgs& a, bool backward, hipStream_t st) {
+static bool one_pass(BnArgs a, bool backward, size_t workspace_bytes, hipStream_t st) {
+    const int threads = plan_held(a, sizeof(TS) == 2 ? PHX_F16 : PHX_F32, backward, a.res != nullptr);
+    if (!threads || (size_t)a.C * a.S * 8 > workspace_bytes || reinterpret_cast<uintptr_t>(a.partial) % 8) return false;
+    const size_t bytes = sizeof(TS) * (size_t)a.rows * a.C * a.hw;
+    for (const void* w : {static_cast<const void*>(a.out), static_cast<const void*>(a.dres)})
+        for (const void* r : {a.x, a.dy, a.res})
+            if (!apart(w, r, bytes)) return false;
+    if (!apart(a.out, a.dres, bytes)) return false;
+    if (threads == 256) launch_held<TS, 256>(a, backward, st);
+    else launch_held<TS, 512>(a, backward, st);
+    return true;
+}
+
+template <typename TS>
+static void launch_all(const BnArgs& a, bool backward, size_t workspace_bytes, hipStream_t st) {
+    if (one_pass<TS>(a, backward, workspace_bytes, st)) return;
     const dim3 grid(a.C, a.S);
     if (!backward) {
         hipLaunchKernelGGL((bn_sums_kernel<TS, 0>), grid, dim3(256), 0, st, a);
@@ -385,7 +674,12 @@ extern "C" {
 size_t phx_bn_workspace_bytes(const phx_bn_desc* desc) {
     BnArgs a{};
     if (plan(desc, a) != PHX_OK) return 0;
-    return ((size_t)a.C * a.S * 2 * sizeof(float) + 255) / 256 * 256;
+    int splits = a.S;
+    for (int pass = 0; pass < 4 && desc->rows > 0 && desc->hw > 0; ++pass) {
+        BnArgs held = a;
+        if (plan_held(held, desc->dtype, pass & 1, pass & 2)) splits = std::max(splits, held.S);
+    }
+    return ((size_t)a.C * splits * 2 * sizeof(float) + 255) / 256 * 256;
 }
 
 int phx_bn_fwd_train(const phx_bn_desc* desc, phx_stream_t stream, const void* x, const void* residual_or_null,
@@ -400,8 +694,8 @@ int phx_bn_fwd_train(const phx_bn_desc* desc, phx_stream_t stream, const void* x
     a.x = x; a.res = residual_or_null; a.out = y; a.gamma = gamma; a.beta = beta; a.partial = static_cast<float*>(workspace);
     a.save_mean = save_mean; a.save_invstd = save_invstd; a.run_mean = running_mean_or_null; a.run_var = running_var_or_null;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (desc->dtype == PHX_F16) launch_all<_Float16>(a, false, st);
-    else launch_all<float>(a, false, st);
+    if (desc->dtype == PHX_F16) launch_all<_Float16>(a, false, workspace_bytes, st);
+    else launch_all<float>(a, false, workspace_bytes, st);
     if (hipGetLastError() != hipSuccess) return PHX_ERR_RUNTIME;
     return PHX_OK;
 }
@@ -436,8 +730,8 @@ int phx_bn_bwd(const phx_bn_desc* desc, phx_stream_t stream, const void* x, cons
     a.save_mean = const_cast<float*>(save_mean); a.save_invstd = const_cast<float*>(save_invstd);
     a.dgamma = dgamma; a.dbeta = dbeta;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (desc->dtype == PHX_F16) launch_all<_Float16>(a, true, st);
-    else launch_all<float>(a, true, st);
+    if (desc->dtype == PHX_F16) launch_all<_Float16>(a, true, workspace_bytes, st);
+    else launch_all<float>(a, true, workspace_bytes, st);
     if (hipGetLastError() != hipSuccess) return PHX_ERR_RUNTIME;
     return PHX_OK;
 }

@@ -25,6 +25,8 @@ inline unsigned int grid_rows(int groups) { return groups > 1 ? (unsigned int)gr
 
 bool tuning_noearly();  // PHX_TUNE_NOEARLY, read once with the other planner overrides
 bool tuning_thin_notile();  // PHX_TUNE_THIN_NOTILE
+int tuning_bn_held();       // PHX_TUNE_BN_HELD
+int tuning_bn_waits();      // PHX_TUNE_BN_WAITS
 
 // which instantiation of the forward / input-gradient kernel to run
 struct FwdVariant {
