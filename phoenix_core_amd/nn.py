@@ -200,16 +200,18 @@ class QConv2d(nn.Module):
         for ent in self._packed.values():
             ent[0] = None
 
-    def _descriptors(self, x):
+    def _descriptors(self, x, backward=True):
+        """(forward, backward) for tensors like x; the second is made when it is first asked for (in evaluation it never is)."""
         key = (tuple(x.shape), x.dtype)
-        if key not in self._descs:
+        pair = self._descs.get(key)
+        if pair is None or (backward and pair[1] is None):
             common = dict(stride=self.stride, dilation=self.dilation, padding=self.padding, dtype=x.dtype,
                           context=self.context, real_valued_input=self.real_input, groups=self.groups,
                           data_format=self.data_format)
-            fwd = ops.Conv2DDescriptor(x.shape, self.weight.shape, use_bias=self.bias is not None, **common)
-            bwd = ops.Conv2DDescriptor(x.shape, self.weight.shape, require_input_grad=self.input_requires_grad, **common)
-            self._descs[key] = (fwd, bwd)
-        return self._descs[key]
+            fwd = pair[0] if pair else ops.Conv2DDescriptor(x.shape, self.weight.shape, use_bias=self.bias is not None, **common)
+            bwd = ops.Conv2DDescriptor(x.shape, self.weight.shape, require_input_grad=self.input_requires_grad, **common) if backward else None
+            pair = self._descs[key] = (fwd, bwd)
+        return pair
 
     def forward(self, x, passthrough=False):
         """passthrough: returns (y, x') with x' an alias of x for the OTHER consumers of x (the identity branch of a
@@ -373,7 +375,7 @@ def _conv_norm(conv, norm, x, residual=None):
         own = (np.get("weight"), np.get("bias"), buffers.get("running_mean"), buffers.get("running_var"))
         if type(w) is nn.Parameter and norm._eval_on_kernel(x, None, own, w.shape[1]):
             device, dtype = x.device, x.dtype
-            fwd, _ = conv._descriptors(x)
+            fwd, _ = conv._descriptors(x, backward=False)
             shape = fwd.output_shape
             n4, c, h, wd = shape
             # (what the operators ask of these tensors, and what the pass behind a convolution that does not normalise what it
