@@ -52,3 +52,20 @@ def test_one_pass_under_capture_and_on_nonfinite_values():
     y = run()[0]
     bad = [c for c in range(24) if not torch.isfinite(y[:, c]).all() or bool((y[:, c] == 0).all())]
     assert bad == [5, 7]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(64, 33, 9, 5), (37, 6, 31, 17), (700, 2, 21, 20)], ids=lambda s: "x".join(map(str, s)))
+def test_results_do_not_depend_on_who_forms_the_sums(shape, dtype, tune_env):
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, dy, res = (torch.randn(shape, generator=gen, device="cuda").to(dtype) for _ in range(3))
+    gamma, beta = torch.rand(shape[1], device="cuda") + 0.5, torch.randn(shape[1], device="cuda")
+    results = []
+    for waits in ("4096", "0"):
+        tune_env(PHX_TUNE_BN_HELD="1", PHX_TUNE_BN_WAITS=waits)
+        for r in (None, res):
+            run = [torch.zeros(shape[1], device="cuda") for _ in range(2)]
+            y, mean, invstd = ops.batch_norm_fwd(x, gamma, beta, *run, 1e-5, 0.1, True, r)
+            results += [y, mean, invstd, *run, *(t for t in ops.batch_norm_bwd(x, dy, gamma, beta, mean, invstd, 1e-5, True, r) if t is not None)]
+    half = len(results) // 2
+    assert all(torch.equal(a, b) for a, b in zip(results[:half], results[half:]))
