@@ -9,8 +9,8 @@
 // the operators' definition and reports their errors, runs instead.
 //
 // What is kept between calls: per descriptor (in its own dictionary) its shapes and workspace sizes, checked against the
-// descriptor's fields each time; per device and stream one scratch buffer that only grows.  All under the interpreter's lock,
-// which is released around the library's calls.
+// descriptor's fields each time; per device and stream one scratch buffer that only grows (captured calls: see scratch).  All
+// under the interpreter's lock, which is released around the library's calls.
 #include <torch/csrc/python_headers.h>
 
 #include <ATen/core/Tensor.h>
@@ -19,7 +19,7 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
-#include <c10/hip/HIPGraphsC10Utils.h>
+#include <c10/hip/HIPException.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/DynamicTypes.h>
@@ -108,14 +108,41 @@ size_t bytes_of(const at::Tensor* t) { return t ? (size_t)t->numel() : 0; }
 struct PairHash {
     size_t operator()(const std::pair<int, uintptr_t>& k) const { return k.second * 31 + (size_t)k.first; }
 };
-std::unordered_map<std::pair<int, uintptr_t>, at::Tensor, PairHash>& buffers() {
-    static auto* b = new std::unordered_map<std::pair<int, uintptr_t>, at::Tensor, PairHash>;  // (tensors outlive the runtime's own shutdown)
+struct Buffer {
+    at::Tensor memory;
+    bool reserved = false;  // asked for in front of a capture (ops.reserve_workspace)
+};
+std::unordered_map<std::pair<int, uintptr_t>, Buffer, PairHash>& buffers() {
+    static auto* b = new std::unordered_map<std::pair<int, uintptr_t>, Buffer, PairHash>;  // (tensors outlive the runtime's own shutdown)
     return *b;
 }
-at::Tensor scratch(c10::Device device, uintptr_t stream, size_t bytes) {
-    at::Tensor& b = buffers()[{device.index(), stream}];
-    if (!b.defined() || (size_t)b.numel() < bytes) b = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, c10::TensorOptions().dtype(c10::kByte).device(device));
-    return b;
+bool holds(const Buffer& b, size_t bytes) { return b.memory.defined() && (size_t)b.memory.numel() >= bytes; }
+bool captured(uintptr_t stream) {
+    if (!stream) return false;  // (the default stream cannot be)
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    C10_HIP_CHECK(hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &status));
+    return status != hipStreamCaptureStatusNone;
+}
+// A graph replays with the addresses that it was captured with, on any stream and whatever eager calls do meanwhile.  A captured
+// call therefore gets memory of its own, from the allocator, which under capture takes it from the graph's pool and gives it to
+// later calls of the same capture and stream only.  Nothing of a graph's pool is kept here, and no graph is left with a buffer of
+// this table that grows away.  One that was reserved for a capture serves that capture, and is never given back.
+at::Tensor scratch(c10::Device device, uintptr_t stream, size_t bytes, bool reserve = false) {
+    Buffer& b = buffers()[{device.index(), stream}];
+    const bool capture = captured(stream);
+    if (holds(b, bytes) && (!capture || b.reserved)) {
+        b.reserved |= reserve;
+        return b.memory;
+    }
+    at::Tensor memory = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, c10::TensorOptions().dtype(c10::kByte).device(device));
+    if (capture) return memory;
+    if (b.reserved) {
+        static auto* kept = new std::vector<at::Tensor>;
+        kept->push_back(b.memory);
+    }
+    b.memory = memory;
+    b.reserved |= reserve;
+    return memory;
 }
 uintptr_t current_stream(c10::Device device) { return reinterpret_cast<uintptr_t>(c10::hip::getCurrentHIPStream(device.index()).stream()); }
 
@@ -579,7 +606,7 @@ PyObject* conv_norm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
             PyErr_Clear();
             return plain_no();
         }
-        if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return plain_no();
+        if (captured(current_stream(device))) return plain_no();
     }
     if (!packed_image(d, packed, true, image)) return plain_no();
     PyObject* own_o[4] = {member(norm, N._parameters, N.weight), member(norm, N._parameters, N.bias), member(norm, N._buffers, N.running_mean), member(norm, N._buffers, N.running_var)};
@@ -606,15 +633,17 @@ PyObject* conv_norm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// workspace(device index, stream handle, bytes) -> the stream's scratch buffer, grown to at least that
+// workspace(device index, stream handle, bytes, whether for a capture to come) -> the stream's scratch buffer, grown to at least
+// that; memory of the capture's own under one (see scratch)
 PyObject* workspace(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    PHX_ARGS(3)
+    PHX_ARGS(4)
     const long device = PyLong_AsLong(a[0]);
     const uintptr_t stream = (uintptr_t)PyLong_AsUnsignedLongLong(a[1]);
     const size_t bytes = (size_t)PyLong_AsUnsignedLongLong(a[2]);
+    const int reserve = PyObject_IsTrue(a[3]);
     if (PyErr_Occurred()) return nullptr;
-    return THPVariable_Wrap(scratch(c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)device), stream, bytes));
+    return THPVariable_Wrap(scratch(c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)device), stream, bytes, reserve == 1));
     END_HANDLE_TH_ERRORS
 }
 
@@ -626,7 +655,7 @@ PyObject* workspace_holds(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const size_t bytes = (size_t)PyLong_AsUnsignedLongLong(a[2]);
     if (PyErr_Occurred()) return nullptr;
     const auto it = buffers().find({(int)device, stream});
-    return PyBool_FromLong(it != buffers().end() && (size_t)it->second.numel() >= bytes);
+    return PyBool_FromLong(it != buffers().end() && holds(it->second, bytes));
 }
 
 // bind(addresses of the C ABI by name, capi's namespace, capi.check, torch.nn.Parameter, forward_ad's namespace)

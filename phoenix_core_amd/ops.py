@@ -277,11 +277,12 @@ def _ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
-def _scratch(device, nbytes, stream=None):
+def _scratch(device, nbytes, stream=None, reserve=False):
     """Grow-only scratch buffer per device and stream, shared by the operations enqueued there (the reference's
     Device keeps one workspace for all its operations, src/backend/device.hpp:75-84, and serializes them with a
-    mutex; here the stream's own order serializes them, and calls on different streams get different buffers)."""
-    return _host.workspace(_index(device), current_stream_handle(device) if stream is None else stream, nbytes)
+    mutex; here the stream's own order serializes them, and calls on different streams get different buffers).
+    A captured call gets memory of its own, from the graph's pool."""
+    return _host.workspace(_index(device), current_stream_handle(device) if stream is None else stream, nbytes, reserve)
 
 
 def _index(device):
@@ -294,10 +295,11 @@ def workspace_holds(device, stream, nbytes):
 
 
 def reserve_workspace(nbytes, device=None):
-    """Grows the scratch buffer of the current stream to at least nbytes ahead of time -- in front of a stream
-    capture, inside which the buffer must not be reallocated."""
+    """Grows the scratch buffer of the current stream to at least nbytes ahead of time, for a capture of the stream to come:
+    captured calls that need no more then use this buffer, which stays where it is for good.  (torch.cuda.graph needs
+    no such call: what it captures takes its scratch memory from the graph's pool.)"""
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
-    return _scratch(device, int(nbytes))
+    return _scratch(device, int(nbytes), reserve=True)
 
 
 def _stream(device, stream=None):
