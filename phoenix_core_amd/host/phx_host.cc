@@ -20,6 +20,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPException.h>
+#include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/DynamicTypes.h>
@@ -134,7 +135,12 @@ at::Tensor scratch(c10::Device device, uintptr_t stream, size_t bytes, bool rese
         b.reserved |= reserve;
         return b.memory;
     }
-    at::Tensor memory = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, c10::TensorOptions().dtype(c10::kByte).device(device));
+    at::Tensor memory;
+    {
+        // (of the stream that works in it: given back, it is that stream's again, behind what is enqueued there)
+        const c10::hip::HIPStreamGuard guard(c10::hip::getStreamFromExternal(reinterpret_cast<hipStream_t>(stream), device.index()));
+        memory = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, c10::TensorOptions().dtype(c10::kByte).device(device));
+    }
     if (capture) return memory;
     if (b.reserved) {
         static auto* kept = new std::vector<at::Tensor>;

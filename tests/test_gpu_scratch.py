@@ -93,3 +93,22 @@ def test_a_reserved_buffer_serves_captures_and_stays():
     graph.replay()
     torch.cuda.synchronize()
     assert all(torch.equal(a, e) for a, e in zip(out, want)) and all(bool((t == 77).all()) for t in others)
+
+
+@pytest.mark.parametrize("stream", ["default", "own"])
+def test_memory_is_of_the_stream_that_works_in_it(stream):
+    """... also where a call names a stream that is not the current one (ops.conv2d_bwd_weights): a buffer that grows away is given
+    back to the stream whose kernels may still write it."""
+    conv, x = _layer(64, 14)
+    desc = ops.Conv2DDescriptor(x.shape, conv.weight.shape, padding="SAME", dtype=torch.float16)
+    grad = torch.randn(desc.output_shape, device="cuda").half()
+    want = ops.conv2d_bwd_weights(x.detach(), grad, desc)
+    handle = torch.cuda.Stream().cuda_stream if stream == "own" else 0
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got = ops.conv2d_bwd_weights(x.detach(), grad, desc, stream=handle)
+        places = [ops._scratch(x.device, n, handle).data_ptr() for n in (desc.workspace_bytes(capi.PHX_PASS_BWD_WEIGHTS), 48 << 20)]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    of = lambda place: [s["stream"] for s in torch.cuda.memory_snapshot() if s["address"] <= place < s["address"] + s["total_size"]]
+    assert of(places[1]) == [handle] and (stream == "default" or of(places[0]) == [handle])
