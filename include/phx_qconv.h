@@ -255,7 +255,8 @@ int phx_qdense_bwd_data(const phx_qdense_desc* desc, phx_stream_t stream, const 
                         void* dx, void* workspace, size_t workspace_bytes);
 int phx_qdense_bwd_weights(const phx_qdense_desc* desc, phx_stream_t stream, const void* x, const void* grad,
                            void* dw, void* workspace, size_t workspace_bytes);
-/* phx_qdense_bwd_weights and phx_qdense_bwd_data behind each other, with a workspace for either; small problems in one launch. */
+/* phx_qdense_bwd_weights and phx_qdense_bwd_data behind each other, with a workspace for either; small problems in one launch, where
+ * neither result lies on an operand or on the other. */
 int phx_qdense_bwd(const phx_qdense_desc* desc, phx_stream_t stream, const void* x, const void* w, const void* grad,
                    void* dw, void* dx, void* workspace, size_t workspace_bytes);
 

@@ -621,11 +621,6 @@ static int plan_held(BnArgs& a, int dtype, bool backward, bool residual) {
     return threads;
 }
 
-static bool apart(const void* out, const void* in, size_t bytes) {
-    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
-    return !out || !in || o + bytes <= i || i + bytes <= o;
-}
-
 template <typename TS, int T>
 static void launch_held(const BnArgs& a, bool backward, hipStream_t st) {
     const int words = a.C * a.S;
@@ -645,8 +640,8 @@ static bool one_pass(BnArgs a, bool backward, size_t workspace_bytes, hipStream_
     const size_t bytes = sizeof(TS) * (size_t)a.rows * a.C * a.hw;
     for (const void* w : {static_cast<const void*>(a.out), static_cast<const void*>(a.dres)})
         for (const void* r : {a.x, a.dy, a.res})
-            if (!apart(w, r, bytes)) return false;
-    if (!apart(a.out, a.dres, bytes)) return false;
+            if (!apart(w, bytes, r, bytes)) return false;
+    if (!apart(a.out, bytes, a.dres, bytes)) return false;
     if (threads == 256) launch_held<TS, 256>(a, backward, st);
     else launch_held<TS, 512>(a, backward, st);
     return true;

@@ -23,6 +23,12 @@ struct BigLds {
 // grid rows of a launch that runs every group of a grouped convolution (one row otherwise)
 inline unsigned int grid_rows(int groups) { return groups > 1 ? (unsigned int)groups : 1u; }
 
+// whether two buffers (null: none) share no byte
+inline bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return !a || !b || p + a_bytes <= q || q + b_bytes <= p;
+}
+
 bool tuning_noearly();  // PHX_TUNE_NOEARLY, read once with the other planner overrides
 bool tuning_thin_notile();  // PHX_TUNE_THIN_NOTILE
 int tuning_bn_held();       // PHX_TUNE_BN_HELD

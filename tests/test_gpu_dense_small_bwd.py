@@ -42,6 +42,37 @@ def test_both_gradients_in_one_launch(n, ci, co, layout, dtype):
         assert (np.abs(got - want) <= terms * 2.0 ** -24 * sums + once * np.abs(want) * 1.01 + 1e-7).all()
 
 
+@pytest.mark.parametrize("place", ["x", "half of x", "w", "dw"])
+def test_results_on_operands_are_those_of_the_two_passes(place):
+    """What the two passes behind each other allow stays allowed, and is not run at once."""
+    n, c = 24, 40
+    size = 4 * n * c
+    desc = ops.DenseDescriptor((4 * n, c), (4, c, c), dtype=torch.float32, context=phx.Context({}))
+    L, stream = capi.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    results = []
+    for both in (False, True):
+        gen = torch.Generator(device="cuda").manual_seed(3)
+        memory = torch.randn(5 * size + 8 * c * c, generator=gen, device="cuda")
+        at = lambda element: memory.data_ptr() + 4 * element
+        x, g, w, dx, dw = at(0), at(2 * size), at(4 * size), at(4 * size + 4 * c * c), at(5 * size + 4 * c * c)
+        if place == "x":
+            dx = x
+        elif place == "half of x":
+            x, dx, g = at(0), at(size // 2), at(size + size // 2)  # (dx: the second half of x and what lies between the two)
+        elif place == "w":
+            dw = w
+        else:
+            dx = dw  # (the input gradient is left, and behind it what the filter gradient is longer by)
+        if both:
+            assert L.phx_qdense_bwd(ctypes.byref(desc.c), stream, x, w, g, dw, dx, None, 0) == capi.PHX_OK
+            assert "dgrad_wgrad" not in capi.last_kernel_name()
+        else:
+            assert L.phx_qdense_bwd_weights(ctypes.byref(desc.c), stream, x, g, dw, None, 0) == capi.PHX_OK
+            assert L.phx_qdense_bwd_data(ctypes.byref(desc.c), stream, g, w, dx, None, 0) == capi.PHX_OK
+        results.append(memory)
+    assert torch.equal(*results)
+
+
 def test_refusals_are_those_of_the_two_passes():
     desc = ops.DenseDescriptor((8, 4), (4, 4, 4), dtype=torch.float32, context=phx.Context({}))
     x = torch.zeros(8, 4, device="cuda")
