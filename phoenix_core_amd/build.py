@@ -36,6 +36,18 @@ def _host_command():
             "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
 
+def _build_host(verbose):
+    """None, or why there is no host path: torch's headers or a host compiler may be missing where the library is built alone."""
+    try:
+        cmd = _host_command()
+        if verbose:
+            print("+", " ".join(cmd), flush=True)
+        proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    except (ImportError, AttributeError, OSError) as e:
+        return "%s: %s" % (type(e).__name__, e)
+    return "%s failed on %s:\n%s" % (cmd[0], HOST_SOURCE, proc.stdout) if proc.returncode != 0 else None
+
+
 def sources():
     return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
 
@@ -49,7 +61,8 @@ def _compile_one(job):
 
 
 def build(verbose=True, extra_flags=()):
-    """Compile every csrc/*.hip to an object (in parallel) and link libphx_qconv.so."""
+    """Compile every csrc/*.hip to an object (in parallel) and link libphx_qconv.so; beside it the operators' host path, whose failure
+    is raised behind the library's link."""
     from concurrent.futures import ThreadPoolExecutor
     os.makedirs(LIB_DIR, exist_ok=True)
     objdir = os.path.join(HERE, "build")
@@ -58,15 +71,9 @@ def build(verbose=True, extra_flags=()):
     jobs = [(src, os.path.join(objdir, os.path.basename(src)[:-4] + ".o"), flags) for src in sources()]
     if verbose:
         print("+ %s %s -c {%s}" % (HIPCC, " ".join(flags), ", ".join(os.path.basename(j[0]) for j in jobs)), flush=True)
-    host = _host_command()
-    if verbose:
-        print("+", " ".join(host), flush=True)
-    with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as pool:
-        host_result = pool.submit(subprocess.run, host, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    with ThreadPoolExecutor(max_workers=min(8, len(jobs) + 1)) as pool:
+        host = pool.submit(_build_host, verbose)
         results = list(pool.map(_compile_one, jobs))
-    host_done = host_result.result()
-    if host_done.returncode != 0:
-        raise RuntimeError("%s failed on %s:\n%s" % (host[0], HOST_SOURCE, host_done.stdout))
     for src, rc, out in results:
         if verbose and out.strip():
             print(out, flush=True)
@@ -78,6 +85,8 @@ def build(verbose=True, extra_flags=()):
     proc = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError("link failed:\n" + proc.stdout)
+    if host.result():
+        raise RuntimeError("%s is built, the Python operators' host path is not: %s" % (LIB_PATH, host.result()))
     return LIB_PATH
 
 
