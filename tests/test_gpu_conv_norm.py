@@ -23,7 +23,8 @@ CASES = [
     (2, 40, 72, 13, 9, 3, 1, FACTORIZED, {}, "lanes"),
     (64, 64, 64, 16, 16, 3, 1, FACTORIZED, {}, "lanes"),
     (16, 72, 130, 16, 14, 3, 2, MIXED, {}, "ldsc"),
-    (1, 256, 64, 7, 7, 3, 1, FACTORIZED, {}, "kslices"),          # partial tensors, normalised by their sum
+    (1, 256, 64, 7, 7, 3, 1, FACTORIZED, {"staged": True}, "kslices"),  # partial tensors, normalised by their sum
+    (1, 256, 64, 7, 7, 3, 1, FACTORIZED, {}, "mfmareg"),          # ... and on registers
     (2, 32, 48, 14, 14, 1, 2, FACTORIZED, {}, "sub_"),
     (2, 3, 16, 33, 35, 7, 2, FACTORIZED, {"real": True}, ""),
     (2, 24, 40, 11, 9, 3, 1, FACTORIZED, {"f32": True}, ""),      # a pass behind the convolution
@@ -44,8 +45,9 @@ def _gap(y, conv, own, res):
 
 @pytest.mark.parametrize("residual,relu", [(False, False), (False, True), (True, True)])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "%dx%d-%d_%dx%d_k%ds%d_%s" % (c[:7] + (c[9] or "-".join(c[8]),)))
-def test_normalised_on_the_way_out(case, residual, relu):
+def test_normalised_on_the_way_out(case, residual, relu, tune_env):
     n, ci, co, h, w, k, stride, env, opt, path = case
+    tune_env(PHX_TUNE_REG="0" if opt.get("staged") else None)
     dtype = torch.float32 if opt.get("f32") else torch.float16
     groups, real = opt.get("groups", 1), opt.get("real", False)
     g = torch.Generator(device="cuda").manual_seed(5)
@@ -73,8 +75,9 @@ def test_normalised_on_the_way_out(case, residual, relu):
 @pytest.mark.parametrize("case", CASES + [(64, 64, 128, 14, 14, 1, 1, FACTORIZED, {"bias": True}, "mfmapw"),
                                           (5, 128, 96, 7, 9, 1, 1, FACTORIZED, {}, ""), (32, 16, 64, 28, 28, 1, 1, FACTORIZED, {}, "mfmapw")],
                          ids=lambda c: "%dx%d-%d_%dx%d_k%ds%d_%s" % (c[:7] + (c[9] or "-".join(c[8]),)))
-def test_the_bits_of_the_two_operators(case, residual, relu):
+def test_the_bits_of_the_two_operators(case, residual, relu, tune_env):
     n, ci, co, h, w, k, stride, env, opt, path = case
+    tune_env(PHX_TUNE_REG="0" if opt.get("staged") else None)
     dtype = torch.float32 if opt.get("f32") else torch.float16
     groups, real = opt.get("groups", 1), opt.get("real", False)
     g = torch.Generator(device="cuda").manual_seed(6)

@@ -21,11 +21,13 @@ def Ctx(mode, policy):
     return phx.Context(env)
 
 
-# (the second shape is a small batch on a deep layer: forward and input gradient run in reduction slices, partial
-# tensors in the workspace and the pass that adds them inside the graph)
+# (the second shape is a small batch on a deep layer: on the staged kernels forward and input gradient run in reduction slices,
+# partial tensors in the workspace and the pass that adds them inside the graph; by the rule fp16 goes to the kernel on registers)
+@pytest.mark.parametrize("kernel", ["rule", "staged"])
 @pytest.mark.parametrize("shape", [(4, 32, 64, 14), (1, 256, 128, 7)], ids=lambda s: "n%d_%dto%d_%dx%d" % (s + s[-1:]))
 @pytest.mark.parametrize("dtype,policy", [(torch.float16, "full16"), (torch.float32, "fp32")], ids=["f16", "f32"])
-def test_captured_conv_replays_match_eager(dtype, policy, shape):
+def test_captured_conv_replays_match_eager(dtype, policy, shape, kernel, tune_env):
+    tune_env(PHX_TUNE_REG="0" if kernel == "staged" else None)
     capi.init()
     torch.manual_seed(11)
     n, ci, co, h = shape
@@ -39,7 +41,10 @@ def test_captured_conv_replays_match_eager(dtype, policy, shape):
         ops.reserve_workspace(max(desc.workspace_bytes(p) for p in range(3)))
         # eager reference and warm-up on the capture stream (fills the plan cache, sizes the scratch buffer)
         y0 = phx.conv2d_fwd(x, w, None, desc)
-        assert ("_kslices" in capi.last_kernel_name()) == (n == 1)
+        name = capi.last_kernel_name()
+        if "mfmareg" not in name:
+            assert ("_kslices" in name) == (n == 1), name
+        assert ("mfmareg" in name) == (kernel == "rule" and dtype == torch.float16), name
         dw0, dx0 = phx.conv2d_bwd(x, w, g, desc)
     side.synchronize()
     graph = torch.cuda.CUDAGraph()
