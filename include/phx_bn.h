@@ -34,6 +34,10 @@ typedef struct phx_bn_desc {
 
 size_t phx_bn_workspace_bytes(const phx_bn_desc* desc);
 
+/* The kernels of the calling thread's last batch-norm call ("" if none): bn_fwd_f16_res_held256_s49 is a forward pass with a
+ * residual in one pass, 49 workgroups of 256 threads a channel; ..._two_s16 two launches; bn_eval_f32 an evaluation pass. */
+const char* phx_bn_last_kernel_name(void);
+
 /* y = gamma * (x - mean) / sqrt(var + eps) + beta (+ residual) with the batch statistics of x, then the
  * optional ReLU; save_mean and save_invstd ([C] each) receive the statistics for the backward pass;
  * running_mean / running_var ([C]) are updated when non-null.  The residual (same shape as x, e.g. the

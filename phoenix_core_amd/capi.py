@@ -37,7 +37,7 @@ EXPORTS = (
 
 
 # every symbol include/phx_bn.h declares (batch normalisation for the ResNet harness)
-EXPORTS_BN = ("phx_bn_workspace_bytes", "phx_bn_fwd_train", "phx_bn_fwd_eval", "phx_bn_bwd")
+EXPORTS_BN = ("phx_bn_workspace_bytes", "phx_bn_fwd_train", "phx_bn_fwd_eval", "phx_bn_bwd", "phx_bn_last_kernel_name")
 
 
 # every symbol include/phx_pool.h declares (max pooling for the same harness)
@@ -108,6 +108,7 @@ def lib():
         L.phx_qdense_bwd.argtypes = [dd, vp, vp, vp, vp, vp, vp, vp, sz]
         bd = ctypes.POINTER(BnDesc)
         L.phx_bn_workspace_bytes.restype = sz
+        L.phx_bn_last_kernel_name.restype = ctypes.c_char_p
         L.phx_bn_workspace_bytes.argtypes = [bd]
         L.phx_bn_fwd_train.argtypes = [bd, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz]
         L.phx_bn_fwd_eval.argtypes = [bd, vp, vp, vp, vp, vp, vp, vp, vp]
@@ -136,6 +137,10 @@ def status_string(status):
 
 def last_kernel_name():
     return lib().phx_last_kernel_name().decode()
+
+
+def bn_last_kernel_name():
+    return lib().phx_bn_last_kernel_name().decode()
 
 
 def check(status, what):

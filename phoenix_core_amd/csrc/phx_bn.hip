@@ -632,6 +632,14 @@ static void launch_held(const BnArgs& a, bool backward, hipStream_t st) {
     else hipLaunchKernelGGL((bn_held_kernel<TS, 1, true, BN_HELD_TWO, T>), grid, dim3(T), 0, st, a);
 }
 
+// What the calling thread's last call ran (phx_bn_last_kernel_name puts it into words)
+struct BnRan {
+    const char* pass = "";
+    bool half, residual;
+    int threads, splits;  // of one pass; threads 0: two launches
+};
+static thread_local BnRan g_bn_ran;
+
 // One pass where its plan takes the call, the workspace holds its words and nothing that it writes is read.
 template <typename TS>
 static bool one_pass(BnArgs a, bool backward, size_t workspace_bytes, hipStream_t st) {
@@ -644,11 +652,14 @@ static bool one_pass(BnArgs a, bool backward, size_t workspace_bytes, hipStream_
     if (!apart(a.out, bytes, a.dres, bytes)) return false;
     if (threads == 256) launch_held<TS, 256>(a, backward, st);
     else launch_held<TS, 512>(a, backward, st);
+    g_bn_ran.threads = threads;
+    g_bn_ran.splits = a.S;
     return true;
 }
 
 template <typename TS>
 static void launch_all(const BnArgs& a, bool backward, size_t workspace_bytes, hipStream_t st) {
+    g_bn_ran = {backward ? "bwd" : "fwd", sizeof(TS) == 2, a.res != nullptr, 0, a.S};
     if (one_pass<TS>(a, backward, workspace_bytes, st)) return;
     const dim3 grid(a.C, a.S);
     if (!backward) {
@@ -665,6 +676,16 @@ static void launch_all(const BnArgs& a, bool backward, size_t workspace_bytes, h
 using namespace phx;
 
 extern "C" {
+
+const char* phx_bn_last_kernel_name(void) {
+    static thread_local char name[64];
+    const BnRan& r = g_bn_ran;
+    if (!*r.pass) return "";
+    const int n = snprintf(name, sizeof(name), "bn_%s_%s%s", r.pass, r.half ? "f16" : "f32", r.residual ? "_res" : "");
+    if (r.threads) snprintf(name + n, sizeof(name) - n, "_held%d_s%d", r.threads, r.splits);
+    else if (r.splits) snprintf(name + n, sizeof(name) - n, "_two_s%d", r.splits);
+    return name;
+}
 
 size_t phx_bn_workspace_bytes(const phx_bn_desc* desc) {
     BnArgs a{};
@@ -704,6 +725,7 @@ int phx_bn_fwd_eval(const phx_bn_desc* desc, phx_stream_t stream, const void* x,
     BnEvalArgs a{x, residual_or_null, y, gamma, beta, running_mean, running_var, (long)desc->rows * desc->c * desc->hw,
                  desc->c, desc->hw, desc->eps, desc->relu};
     hipStream_t st = static_cast<hipStream_t>(stream);
+    g_bn_ran = {"eval", desc->dtype == PHX_F16, residual_or_null != nullptr, 0, 0};
     if (desc->dtype == PHX_F16) launch_eval<_Float16>(a, st);
     else launch_eval<float>(a, st);
     if (hipGetLastError() != hipSuccess) return PHX_ERR_RUNTIME;

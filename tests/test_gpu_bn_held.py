@@ -1,17 +1,32 @@
 """The one-pass batch-norm kernels, whose workgroups hold their part of a channel in registers and wait for their neighbours'
 sums, at the edges of their plan: planes of one 16-byte chunk and of one element more, a partial last chunk in every plane, one
 workgroup a channel, as many as ask for 512 threads, and more than 64 of those, which stay on two launches.  Against fp64 with
-test_gpu_bn's tolerances; with no wait allowed every workgroup forms the channel's sums itself, and the results are the same."""
+test_gpu_bn's tolerances; with no wait allowed every workgroup forms the channel's sums itself, and the results are the same.
+What ran is read from the kernels' names."""
+import ctypes
+
 import pytest
 import torch
 
 import test_gpu_bn
-from phoenix_core_amd import ops
+from phoenix_core_amd import capi, ops
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(8, 16, 14, 14), (12, 5, 7, 7), (64, 33, 9, 5), (2, 3, 2, 4), (5, 1100, 3, 3), (65, 2, 4, 8), (37, 6, 31, 17), (1, 1, 64, 96), (257, 1, 40, 41),
-          (700, 2, 21, 20), (330, 1, 56, 57), (40, 512, 7, 7)]
+# threads of a workgroup, 0: two launches; (fp32, fp16), where they differ by the pass (forward, with a residual, backward)
+SHAPES = {(8, 16, 14, 14): (256, 256), (12, 5, 7, 7): (256, 256), (64, 33, 9, 5): (256, 256), (2, 3, 2, 4): (256, 256), (5, 1100, 3, 3): (256, 256),
+          (65, 2, 4, 8): (256, 256), (37, 6, 31, 17): (256, 256), (1, 1, 64, 96): (256, 256), (257, 1, 40, 41): (0, 0), (700, 2, 21, 20): (0, 0),
+          (40, 512, 7, 7): (256, 256), (131, 17, 57, 55): ((256, 512, 512), 256)}
+MANY = {(293, 17, 57, 55): (512, (256, 512, 512))}  # (61 and 60 workgroups a channel)
+
+
+def _ran(shape, dtype, passes):
+    """The start of the names of these passes of a shape."""
+    threads = {**SHAPES, **MANY}[shape][dtype == torch.float16]
+    threads = threads if isinstance(threads, tuple) else (threads,) * 3
+    names = {"fwd": ("bn_fwd_%s", threads[0]), "fwd_res": ("bn_fwd_%s_res", threads[1]), "bwd": ("bn_bwd_%s", threads[2]), "bwd_res": ("bn_bwd_%s_res", threads[2])}
+    of = lambda name, t: (name + ("_held%d_s" % t if t else "_two_s")) % ("f16" if dtype == torch.float16 else "f32")
+    return [of(*names[p]) for p in passes]
 
 
 @pytest.fixture(params=["4096", "0"], ids=["waits", "alone"])
@@ -19,11 +34,76 @@ def held(request, tune_env):
     tune_env(PHX_TUNE_BN_HELD="1", PHX_TUNE_BN_WAITS=request.param)
 
 
+@pytest.fixture
+def names(monkeypatch):
+    """What the operators' batch-norm calls ran, in their order."""
+    seen = []
+
+    def watched(op):
+        def call(*args):
+            result = op(*args)
+            seen.append(capi.bn_last_kernel_name())
+            return result
+        return call
+
+    for op in ("batch_norm_fwd", "batch_norm_bwd"):
+        monkeypatch.setattr(ops, op, watched(getattr(ops, op)))
+    return seen
+
+
+def _are(names, expected):
+    assert len(names) == len(expected) and all(n.startswith(e) for n, e in zip(names, expected)), (names, expected)
+
+
 @pytest.mark.parametrize("relu,residual", [(False, False), (True, False), (True, True)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
-def test_one_pass_matches_torch(held, shape, dtype, relu, residual):
+def test_one_pass_matches_torch(held, names, shape, dtype, relu, residual):
     test_gpu_bn.test_batch_norm_matches_torch(shape, dtype, relu, residual)
+    _are(names, _ran(shape, dtype, ("fwd_res", "bwd_res") if residual else ("fwd", "bwd")))
+
+
+@pytest.mark.parametrize("shape,dtype,residual", [(s, d, r) for s in MANY for d, r in ((torch.float32, False), (torch.float16, True))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_many_workgroups_a_channel_match_torch(shape, dtype, residual, names, tune_env):
+    tune_env(PHX_TUNE_BN_HELD="1")
+    test_gpu_bn.test_batch_norm_matches_torch(shape, dtype, True, residual)
+    _are(names, _ran(shape, dtype, ("fwd_res", "bwd_res") if residual else ("fwd", "bwd")))
+
+
+def test_calls_that_stay_on_two_launches():
+    """By the rule's sizes, a workspace that does not hold the words, one that is not aligned for them, and results on operands."""
+    rows, c, hw = 8, 64, 112 * 112
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x, dy = (torch.randn(rows, c, 112, 112, generator=gen, device="cuda").half() for _ in range(2))
+    gamma, beta = torch.rand(c, device="cuda") + 0.5, torch.randn(c, device="cuda")
+    mean, invstd, dgamma, dbeta = (torch.empty(c, device="cuda") for _ in range(4))
+    desc = capi.BnDesc(capi.PHX_F16, rows, c, hw, 1e-5, 0.1, 1)
+    L, stream, at = capi.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), lambda t: t.data_ptr()
+    size = L.phx_bn_workspace_bytes(ctypes.byref(desc))
+    memory = torch.empty(size + 256, dtype=torch.uint8, device="cuda")
+
+    def bwd(dx, offset=0, nbytes=size):
+        x0 = x.clone()
+        out = x0 if dx == "x" else dy.clone() if dx == "dy" else torch.empty_like(x)
+        grad = out if dx == "dy" else dy
+        assert L.phx_bn_bwd(ctypes.byref(desc), stream, at(x0), None, at(grad), at(gamma), at(beta), at(mean), at(invstd), at(out), None, at(dgamma),
+                            at(dbeta), at(memory) + offset, nbytes) == capi.PHX_OK
+        return capi.bn_last_kernel_name(), [out, dgamma.clone(), dbeta.clone()]
+
+    y = torch.empty_like(x)
+    fwd = lambda out: L.phx_bn_fwd_train(ctypes.byref(desc), stream, at(out), None, at(gamma), at(beta), at(y), at(mean), at(invstd), None, None, at(memory), size)
+    assert fwd(x) == capi.PHX_OK and capi.bn_last_kernel_name().startswith("bn_fwd_f16_two_s")  # (12.8 MB)
+    name, want = bwd("own")
+    assert name == "bn_bwd_f16_held256_s16"
+    words = 8 * c * 16  # (two launches ask for half of that)
+    assert bwd("own", nbytes=words)[0] == name
+    for args in (dict(dx="x"), dict(dx="dy"), dict(dx="own", offset=4), dict(dx="own", nbytes=words - 8)):
+        name, got = bwd(**args)
+        assert name == "bn_bwd_f16_two_s8", (args, name)
+        # (fp32 sums of 100352 terms in another order, then one rounding to fp16)
+        for a, e in zip(got, want):
+            assert float((a.double() - e.double()).norm() / e.double().norm()) < 1e-3
 
 
 def test_one_pass_under_capture_and_on_nonfinite_values():
@@ -43,6 +123,7 @@ def test_one_pass_under_capture_and_on_nonfinite_values():
     for seed in range(3):
         x.copy_(torch.randn(shape, generator=torch.Generator().manual_seed(seed)).half())
         eager = run()
+        assert capi.bn_last_kernel_name().startswith("bn_fwd_f16_held256_s")
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
@@ -55,8 +136,8 @@ def test_one_pass_under_capture_and_on_nonfinite_values():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
-@pytest.mark.parametrize("shape", [(64, 33, 9, 5), (37, 6, 31, 17), (700, 2, 21, 20)], ids=lambda s: "x".join(map(str, s)))
-def test_results_do_not_depend_on_who_forms_the_sums(shape, dtype, tune_env):
+@pytest.mark.parametrize("shape", [(64, 33, 9, 5), (37, 6, 31, 17), (131, 17, 57, 55)], ids=lambda s: "x".join(map(str, s)))
+def test_results_do_not_depend_on_who_forms_the_sums(shape, dtype, names, tune_env):
     gen = torch.Generator(device="cuda").manual_seed(5)
     x, dy, res = (torch.randn(shape, generator=gen, device="cuda").to(dtype) for _ in range(3))
     gamma, beta = torch.rand(shape[1], device="cuda") + 0.5, torch.randn(shape[1], device="cuda")
@@ -67,5 +148,6 @@ def test_results_do_not_depend_on_who_forms_the_sums(shape, dtype, tune_env):
             run = [torch.zeros(shape[1], device="cuda") for _ in range(2)]
             y, mean, invstd = ops.batch_norm_fwd(x, gamma, beta, *run, 1e-5, 0.1, True, r)
             results += [y, mean, invstd, *run, *(t for t in ops.batch_norm_bwd(x, dy, gamma, beta, mean, invstd, 1e-5, True, r) if t is not None)]
+    _are(names, _ran(shape, dtype, ("fwd", "bwd", "fwd_res", "bwd_res") * 2))
     half = len(results) // 2
     assert all(torch.equal(a, b) for a, b in zip(results[:half], results[half:]))
