@@ -337,10 +337,10 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
         }
     }
 
-    // The waves of a tile add their sums.  Wave `rank` finishes the components q with q % min(KS, 4) == rank % 4 and, of more than
-    // four waves, the rows i0 .. i0 + 4 / (KS / 4) - 1 of them.
+    // The waves of a tile add their sums.  Wave `rank` finishes the components q with q % min(KS, 4) == rank % 4 and, of eight
+    // waves, the rows i0 and i0 + 1 of them.
     const int qmask = min(KS, 4) - 1;
-    const int i0 = KS > 4 ? (rank >> 2) * (16 >> P.kslog) : 0;
+    const int i0 = reg_waves(KW) > 4 && KS > 4 ? (rank >> 2) * 2 : 0;
     const float* sums = red + (wave - rank) * (REG_SUMS * 64) + lane;
     if (KS > 1) {
         float* mine = red + wave * (REG_SUMS * 64) + lane;
@@ -479,12 +479,10 @@ __global__ void __launch_bounds__(64 * reg_waves(KW)) qconv_reg_f16_kernel(const
                 for (int i = 0; i < 4; ++i) v[PX * i + e] = acc[q][e][i];
             finish(std::integral_constant<int, 4>{}, q, v);
         }
-    } else if (KS <= 4) {
+    } else if (reg_waves(KW) <= 4 || KS <= 4) {
         finish_sums(std::integral_constant<int, 4>{});
-    } else if (KS == 8) {
+    } else if constexpr (reg_waves(KW) > 4) {
         finish_sums(std::integral_constant<int, 2>{});
-    } else {
-        finish_sums(std::integral_constant<int, 1>{});
     }
 }
 
