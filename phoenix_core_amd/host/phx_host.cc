@@ -5,7 +5,7 @@
 // evaluation ResNet's 53 convolutions 15.5 each and 7.5.
 //
 // Every function answers NotImplemented for a call that is not a plain one -- tensors of another type, shape, device or order
-// than the descriptor's, subclasses and wrapped tensors, function and dispatch modes -- and the Python code behind it, which is
+// than the descriptor's, subclasses (of tensors and of descriptors) and wrapped tensors, function and dispatch modes -- and the Python code behind it, which is
 // the operators' definition and reports their errors, runs instead.
 //
 // What is kept between calls: per descriptor (in its own dictionary) its shapes and workspace sizes, checked against the
@@ -51,6 +51,8 @@ struct Library {
 PyObject* g_check = nullptr;       // capi.check(status, name): raises
 PyObject* g_capi_dict = nullptr;   // capi's namespace: tuning_generation
 PyObject* g_parameter = nullptr;   // torch.nn.Parameter
+PyObject* g_conv_type = nullptr;   // ops.Conv2DDescriptor
+PyObject* g_dense_type = nullptr;  // ops.DenseDescriptor
 PyObject* g_forward_ad = nullptr;  // torch.autograd.forward_ad's namespace: _current_level
 
 struct Names {
@@ -153,9 +155,10 @@ at::Tensor scratch(c10::Device device, uintptr_t stream, size_t bytes, bool rese
 uintptr_t current_stream(c10::Device device) { return reinterpret_cast<uintptr_t>(c10::hip::getCurrentHIPStream(device.index()).stream()); }
 
 // ---- what is kept of a descriptor ----
+enum { FIELD_C, FIELD_INPUT, FIELD_FILTER, FIELD_OUTPUT, FIELD_DTYPE, FIELD_USE_BIAS, FIELD_BIAS_SHAPE, FIELD_REAL, DESC_FIELDS };
 struct Desc {
     PyObject_HEAD
-    PyObject *c, *input_shape, *filter_shape, *output_shape, *dtype, *use_bias;  // the fields it was made from (owned)
+    PyObject* fields[DESC_FIELDS];  // what it was made from (owned; null: not there)
     const void* abi;      // the ctypes structure's memory
     bool dense, bias, real;
     c10::ScalarType type;
@@ -171,7 +174,7 @@ struct Desc {
 };
 void desc_dealloc(PyObject* self) {
     Desc* d = reinterpret_cast<Desc*>(self);
-    Py_XDECREF(d->c); Py_XDECREF(d->input_shape); Py_XDECREF(d->filter_shape); Py_XDECREF(d->output_shape); Py_XDECREF(d->dtype); Py_XDECREF(d->use_bias);
+    for (PyObject* f : d->fields) Py_XDECREF(f);
     d->in.~vector(); d->filter.~vector(); d->out.~vector(); d->bias_shape.~vector();
     Py_TYPE(self)->tp_free(self);
 }
@@ -194,26 +197,25 @@ long tuning_generation() {
 }
 
 // The kept part of a descriptor of the quaternion algebra, made (again) where there is none or a field is another object now;
-// nullptr: a descriptor of another kind.
+// nullptr: a descriptor of another kind or type.
 Desc* desc_of(PyObject* o, bool dense) {
+    if (reinterpret_cast<PyObject*>(Py_TYPE(o)) != (dense ? g_dense_type : g_conv_type)) return nullptr;
     PyObject** dictptr = _PyObject_GetDictPtr(o);
     if (!dictptr || !*dictptr) return nullptr;
     PyObject* dict = *dictptr;
-    PyObject* fields[6] = {PyDict_GetItem(dict, N.c),            PyDict_GetItem(dict, N.input_shape), PyDict_GetItem(dict, N.filter_shape),
-                           PyDict_GetItem(dict, N.output_shape), PyDict_GetItem(dict, N.dtype),       PyDict_GetItem(dict, N.use_bias)};
+    PyObject* fields[DESC_FIELDS] = {PyDict_GetItem(dict, N.c),     PyDict_GetItem(dict, N.input_shape), PyDict_GetItem(dict, N.filter_shape), PyDict_GetItem(dict, N.output_shape),
+                                     PyDict_GetItem(dict, N.dtype), PyDict_GetItem(dict, N.use_bias),    PyDict_GetItem(dict, N.bias_shape),   PyDict_GetItem(dict, N.real_valued_input)};
     PyObject* held = PyDict_GetItem(dict, N._host);
     if (held && Py_TYPE(held) == &DescType) {
         Desc* d = reinterpret_cast<Desc*>(held);
-        if (d->dense == dense && d->c == fields[0] && d->input_shape == fields[1] && d->filter_shape == fields[2] && d->output_shape == fields[3] &&
-            d->dtype == fields[4] && d->use_bias == fields[5])
-            return d;
+        if (d->dense == dense && std::memcmp(d->fields, fields, sizeof(fields)) == 0) return d;
     }
     PyObject* algebra = PyDict_GetItem(dict, N.algebra);
-    for (PyObject* f : fields)
-        if (!f) return nullptr;
-    if (!algebra || !PyLong_Check(algebra) || PyLong_AsLong(algebra) != 2 /* ops.QUATERNION */ || !THPDtype_Check(fields[4])) return nullptr;
+    for (int i = 0; i <= FIELD_USE_BIAS; ++i)
+        if (!fields[i]) return nullptr;
+    if (!algebra || !PyLong_Check(algebra) || PyLong_AsLong(algebra) != 2 /* ops.QUATERNION */ || !THPDtype_Check(fields[FIELD_DTYPE])) return nullptr;
     Py_buffer view;
-    if (PyObject_GetBuffer(fields[0], &view, PyBUF_SIMPLE) != 0) { PyErr_Clear(); return nullptr; }
+    if (PyObject_GetBuffer(fields[FIELD_C], &view, PyBUF_SIMPLE) != 0) { PyErr_Clear(); return nullptr; }
     const void* abi = view.buf;
     const bool size_ok = (size_t)view.len == (dense ? sizeof(phx_qdense_desc) : sizeof(phx_qconv_desc));
     PyBuffer_Release(&view);  // (the structure owns its memory as long as it lives, and this holds it)
@@ -221,18 +223,15 @@ Desc* desc_of(PyObject* o, bool dense) {
     Desc* d = reinterpret_cast<Desc*>(DescType.tp_alloc(&DescType, 0));
     if (!d) { PyErr_Clear(); return nullptr; }
     new (&d->in) std::vector<int64_t>; new (&d->filter) std::vector<int64_t>; new (&d->out) std::vector<int64_t>; new (&d->bias_shape) std::vector<int64_t>;
-    PyObject** own[6] = {&d->c, &d->input_shape, &d->filter_shape, &d->output_shape, &d->dtype, &d->use_bias};
-    for (int i = 0; i < 6; ++i) { Py_INCREF(fields[i]); *own[i] = fields[i]; }
+    for (int i = 0; i < DESC_FIELDS; ++i) { Py_XINCREF(fields[i]); d->fields[i] = fields[i]; }
     d->abi = abi;
     d->dense = dense;
-    d->bias = PyObject_IsTrue(fields[5]) == 1;
-    PyObject* real = PyDict_GetItem(dict, N.real_valued_input);
-    d->real = real && PyObject_IsTrue(real) == 1;
-    d->type = reinterpret_cast<THPDtype*>(fields[4])->scalar_type;
+    d->bias = PyObject_IsTrue(fields[FIELD_USE_BIAS]) == 1;
+    d->real = fields[FIELD_REAL] && PyObject_IsTrue(fields[FIELD_REAL]) == 1;
+    d->type = reinterpret_cast<THPDtype*>(fields[FIELD_DTYPE])->scalar_type;
     d->generation = -1;
-    const bool good = to_sizes(fields[1], d->in) && to_sizes(fields[2], d->filter) && to_sizes(fields[3], d->out) &&
-                      (!d->bias || to_sizes(PyDict_GetItem(dict, N.bias_shape), d->bias_shape)) &&
-                      PyDict_SetItem(dict, N._host, reinterpret_cast<PyObject*>(d)) == 0;
+    const bool good = to_sizes(fields[FIELD_INPUT], d->in) && to_sizes(fields[FIELD_FILTER], d->filter) && to_sizes(fields[FIELD_OUTPUT], d->out) &&
+                      (!d->bias || to_sizes(fields[FIELD_BIAS_SHAPE], d->bias_shape)) && PyDict_SetItem(dict, N._host, reinterpret_cast<PyObject*>(d)) == 0;
     Py_DECREF(d);  // (the dictionary holds it)
     if (!good) { PyErr_Clear(); return nullptr; }
     return d;
@@ -664,9 +663,9 @@ PyObject* workspace_holds(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     return PyBool_FromLong(it != buffers().end() && holds(it->second, bytes));
 }
 
-// bind(addresses of the C ABI by name, capi's namespace, capi.check, torch.nn.Parameter, forward_ad's namespace)
+// bind(addresses of the C ABI by name, capi's namespace, capi.check, torch.nn.Parameter, forward_ad's namespace, the descriptors' types)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
-    PHX_ARGS(5)
+    PHX_ARGS(7)
 #define PHX_FIELD(f)                                                                                         \
     {                                                                                                        \
         PyObject* p = PyDict_GetItemString(a[0], #f);                                                        \
@@ -676,8 +675,8 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
     PHX_HOST_FUNCTIONS(PHX_FIELD)
 #undef PHX_FIELD
-    PyObject** kept[4] = {&g_capi_dict, &g_check, &g_parameter, &g_forward_ad};
-    for (int i = 0; i < 4; ++i) { Py_INCREF(a[1 + i]); Py_XDECREF(*kept[i]); *kept[i] = a[1 + i]; }
+    PyObject** kept[6] = {&g_capi_dict, &g_check, &g_parameter, &g_forward_ad, &g_conv_type, &g_dense_type};
+    for (int i = 0; i < 6; ++i) { Py_INCREF(a[1 + i]); Py_XDECREF(*kept[i]); *kept[i] = a[1 + i]; }
     Py_RETURN_NONE;
 }
 

@@ -34,7 +34,7 @@ class _Unloaded:
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_phx_host", loader))
         loader.exec_module(module)
         addresses = {f: ctypes.cast(getattr(lib, f), ctypes.c_void_p).value for f in capi.EXPORTS + capi.EXPORTS_BN}
-        module.bind(addresses, vars(capi), capi.check, torch.nn.Parameter, vars(torch.autograd.forward_ad))
+        module.bind(addresses, vars(capi), capi.check, torch.nn.Parameter, vars(torch.autograd.forward_ad), Conv2DDescriptor, DenseDescriptor)
         _host = module
         return getattr(module, name)
 

@@ -123,6 +123,40 @@ def test_what_is_kept_follows_the_descriptor(tune_env, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("field,value,error", [("bias_shape", (4, 9), ValueError), ("real_valued_input", True, RuntimeError), ("use_bias", False, None),
+                                               ("filter_shape", (4, 10, 12, 3, 2), ValueError), ("output_shape", (8, 10, 9, 6), None)])
+def test_every_field_of_a_descriptor_is_read_again(field, value, error):
+    """A field that is set after the first call is the next one's, as the definitions read it."""
+    x, w, b, g, desc, back, rnd = _case()
+    y = phx.conv2d_fwd(x, w, b, desc)
+    setattr(desc, field, value)
+    if error:
+        with pytest.raises(error):
+            phx.conv2d_fwd(x, w, b, desc)
+    else:
+        try:
+            assert phx.conv2d_fwd(x, w, b, desc).shape == desc.output_shape
+        except (ValueError, capi.PhxError):  # (the structure asks for a bias that the call leaves out)
+            assert field == "use_bias"
+    assert torch.equal(phx.conv2d_fwd(x, w, b, _case()[4]), y)
+
+
+@pytest.mark.gpu
+def test_descriptors_of_another_type_reach_the_definitions():
+    """What a subclass changes of a descriptor is heard."""
+    asked = []
+
+    class Roomy(ops.Conv2DDescriptor):
+        def workspace_bytes(self, which):
+            asked.append(which)
+            return super().workspace_bytes(which) + 512
+
+    x, w, b, g, desc, back, rnd = _case()
+    roomy = Roomy(x.shape, w.shape, padding="SAME", use_bias=True, dtype=torch.float16, context=phx.Context({}))
+    assert torch.equal(phx.conv2d_fwd(x, w, b, roomy), phx.conv2d_fwd(x, w, b, desc)) and asked == [capi.PHX_PASS_FWD]
+
+
+@pytest.mark.gpu
 def test_modes_and_wrapped_tensors_reach_the_definitions(monkeypatch):
     x, w, b, g, desc, back, rnd = _case()
 
