@@ -1,8 +1,7 @@
 // The host path of the operators on torch tensors: what ops.py and nn.py do per call -- checks of the tensors against a
 // descriptor, the result's allocation, the stream's scratch buffer, the call of the C ABI -- without the interpreter's share of it.
-// Layers of a few microseconds are bound by that: a forward call with a packed filter took 9.2 us of the host and takes 5.9, of
-// which the library and its launch are 4.2; both gradients of a convolution 21.4 and 14.1, a Dense step 22.2 and 13.2, the
-// evaluation ResNet's 53 convolutions 15.5 each and 7.5.
+// Layers of a few microseconds are bound by that: of the host's time a forward call with a packed filter took 9.1 us and takes 5.2,
+// both gradients of a convolution 22.1 and 14.6, a Dense step 22.1 and 10.4, a convolution with its norm in evaluation 13.3 and 6.2.
 //
 // Every function answers NotImplemented for a call that is not a plain one -- tensors of another type, shape, device or order
 // than the descriptor's, subclasses (of tensors and of descriptors) and wrapped tensors, function and dispatch modes -- and the Python code behind it, which is
