@@ -113,6 +113,7 @@ struct PairHash {
 struct Buffer {
     at::Tensor memory;
     bool reserved = false;  // asked for in front of a capture (ops.reserve_workspace)
+    bool in_graph = false;  // ... and met by one
 };
 std::unordered_map<std::pair<int, uintptr_t>, Buffer, PairHash>& buffers() {
     static auto* b = new std::unordered_map<std::pair<int, uintptr_t>, Buffer, PairHash>;  // (tensors outlive the runtime's own shutdown)
@@ -128,12 +129,13 @@ bool captured(uintptr_t stream) {
 // A graph replays with the addresses that it was captured with, on any stream and whatever eager calls do meanwhile.  A captured
 // call therefore gets memory of its own, from the allocator, which under capture takes it from the graph's pool and gives it to
 // later calls of the same capture and stream only.  Nothing of a graph's pool is kept here, and no graph is left with a buffer of
-// this table that grows away.  One that was reserved for a capture serves that capture, and is never given back.
+// this table that grows away.  One that was reserved for a capture serves that capture, and is never given back then.
 at::Tensor scratch(c10::Device device, uintptr_t stream, size_t bytes, bool reserve = false) {
     Buffer& b = buffers()[{device.index(), stream}];
     const bool capture = captured(stream);
     if (holds(b, bytes) && (!capture || b.reserved)) {
         b.reserved |= reserve;
+        b.in_graph |= capture;
         return b.memory;
     }
     at::Tensor memory;
@@ -143,9 +145,10 @@ at::Tensor scratch(c10::Device device, uintptr_t stream, size_t bytes, bool rese
         memory = at::empty({(int64_t)std::max<size_t>(bytes, 1)}, c10::TensorOptions().dtype(c10::kByte).device(device));
     }
     if (capture) return memory;
-    if (b.reserved) {
+    if (b.in_graph) {
         static auto* kept = new std::vector<at::Tensor>;
         kept->push_back(b.memory);
+        b.in_graph = false;
     }
     b.memory = memory;
     b.reserved |= reserve;

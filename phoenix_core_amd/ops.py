@@ -296,7 +296,7 @@ def workspace_holds(device, stream, nbytes):
 
 def reserve_workspace(nbytes, device=None):
     """Grows the scratch buffer of the current stream to at least nbytes ahead of time, for a capture of the stream to come:
-    captured calls that need no more then use this buffer, which stays where it is for good.  (torch.cuda.graph needs
+    captured calls that need no more then use this buffer, which from then on stays where it is.  (torch.cuda.graph needs
     no such call: what it captures takes its scratch memory from the graph's pool.)"""
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     return _scratch(device, int(nbytes), reserve=True)

@@ -93,6 +93,10 @@ def test_a_reserved_buffer_serves_captures_and_stays():
     graph.replay()
     torch.cuda.synchronize()
     assert all(torch.equal(a, e) for a, e in zip(out, want)) and all(bool((t == 77).all()) for t in others)
+    before = torch.cuda.memory_allocated()
+    with torch.cuda.stream(stream):
+        ops.reserve_workspace(1 << 25)
+    assert torch.cuda.memory_allocated() == before + (1 << 24)  # (one that no capture has met is given back)
 
 
 @pytest.mark.parametrize("stream", ["default", "own"])
