@@ -151,3 +151,21 @@ def test_results_do_not_depend_on_who_forms_the_sums(shape, dtype, names, tune_e
     _are(names, _ran(shape, dtype, ("fwd", "bwd", "fwd_res", "bwd_res") * 2))
     half = len(results) // 2
     assert all(torch.equal(a, b) for a, b in zip(results[:half], results[half:]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_statistics_are_rounded_at_their_end(dtype):
+    """Over 256 channels' root mean square: 1/deviation carries its own last roundings (the variance's, the root's, the quotient's: 0.3
+    of 2^-23 each, the variance's halved) and next to nothing of the 401408 additions in front, the mean its last one at most.
+    A thread's elements one behind the other and the channel's words added in fp32 gave two and three times as much."""
+    errors = torch.zeros(2, dtype=torch.float64, device="cuda")
+    for seed in range(4):
+        x = (torch.randn(128, 64, 56, 56, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda") * 1.5 + 0.3).to(dtype)
+        run = [torch.zeros(64, device="cuda"), torch.ones(64, device="cuda")]
+        _, mean, invstd = ops.batch_norm_fwd(x, torch.ones(64, device="cuda"), torch.zeros(64, device="cuda"), *run, 1e-5, 0.1, False, None)
+        assert "_held" in capi.bn_last_kernel_name()
+        exact = x.double()
+        m, i = exact.mean((0, 2, 3)), (exact.var((0, 2, 3), unbiased=False) + 1e-5).rsqrt()
+        errors += torch.stack([((mean.double() - m) * i).square().mean(), (invstd.double() / i - 1).square().mean()])
+    errors = (errors / 4).sqrt()
+    assert float(errors[0]) < 2.0 ** -25 and float(errors[1]) < 2.0 ** -24, errors.tolist()
